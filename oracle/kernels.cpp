@@ -133,6 +133,32 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
       }
       continue;
     }
+    if (nm == "bc_open_xy") {
+      // the merged halo launch of a domain with an open side: per field the
+      // periodic passes, then the open ones (timestep.js haloFill)
+      const uint32_t* dm = w + A[4];
+      const uint32_t nx = dm[0], ny = dm[1], nz = dm[2];
+      const uint32_t* P = w + A[4 + 9];
+      for (uint32_t q = 0; q < P[0] && q < 8; ++q) {
+        auto pass = [&](const char* kn, uint32_t other, const uint32_t* stag) {
+          uint32_t X[64] = {0};
+          X[0] = 4; X[1] = other + 7; X[2] = nz + 1;
+          X[4] = A[4]; X[5] = A[5 + q]; X[34] = A[34];
+          if (stag) X[6] = (uint32_t)(stag - w);
+          K<T> k1{w, v, X};
+          call(find_kernel(kn), k1);
+        };
+        // (the passes' stagger argument: the field's own word, set for each)
+        if (!P[1]) pass("bc_periodic_x", ny, nullptr);
+        if (!P[2]) pass("bc_periodic_y", nx, nullptr);
+        uint32_t* flag = w + A[4 + 9] + 3 + q;
+        const uint32_t on = *flag;
+        if (P[1]) { *flag = on == 1u; pass("bc_open_x", ny, flag); }
+        if (P[2]) { *flag = on == 2u; pass("bc_open_y", nx, flag); }
+        *flag = on;
+      }
+      continue;
+    }
     if (nm == "ac_column") {
       // the dispatches one acoustic substep launch stands for: on the stage's
       // first substep acoustic_prepare and acoustic_begin, then acoustic_fpk,

@@ -45,6 +45,63 @@ __global__ __launch_bounds__(256) void k_bc_periodic_xy(uint32_t* M, KArg a) {
   }
 }
 
+// Halos of up to 8 fields on a domain with an open side, in one launch.
+// Replaces, per field, bc_periodic_x or bc_open_x and bc_periodic_y or
+// bc_open_y in haloFill's order (timestep.js haloFill: the periodic passes,
+// then the open ones).  Each pass copies whole lines of the other direction,
+// halo included, so a halo cell ends as the value at (sx(i), sy(j)): on a
+// periodic axis the image modulo n; on an open one the nearest cell of
+// [0, last], last = n - 1 (n for a field on that axis' faces), for the three
+// cells past either end, and the cell itself beyond them (bc_open_x.wgsl:111-131
+// fills three).  No source is itself filled, so every cell can be written at
+// once.  The fill moves a few percent of the field and is bound by the launch:
+// 120 x 120 x 40 with 7 species has 188 of these passes per step at 3.0-3.4 us
+// each; one launch for the 4 fields of a substep takes about what one pass did.
+// Grid as k_bc_periodic_xy.  p[1..8] fields, p[9] -> count, open x, open y and
+// per field 1 (on x faces), 2 (on y faces) or 0.
+__global__ __launch_bounds__(256) void k_bc_open_xy(uint32_t* M, KArg a) {
+  TE_TID3
+  const Dims g = dims(a.q[0], 0);
+  const int k = gy;
+  if (k > g.nz) return;
+  const int rowCells = 7 * g.sJ;
+  int i, j;
+  if (gx < rowCells) {
+    const int r = gx / g.sJ;           // 0..6 -> j = -3..-1, ny..ny+3
+    i = gx - r * g.sJ - 3;
+    j = r < 3 ? r - 3 : g.ny + (r - 3);
+  } else {
+    const int t = gx - rowCells;       // ny rows x 7 halo columns, row by row
+    j = t / 7;
+    const int cidx = t - j * 7;
+    if (j >= g.ny) return;
+    i = cidx < 3 ? cidx - 3 : g.nx + (cidx - 3);
+  }
+  const uint32_t* P = a.q[9];
+  const int n = ldi(P, 0);
+  const bool openx = ldi(P, 1) != 0, openy = ldi(P, 2) != 0;
+  auto source = [](int q, int cells, bool open, int last) {
+    if (!open) return ((q % cells) + cells) % cells;
+    return q < 0 ? 0 : (q > last && q <= last + 3 ? last : q);
+  };
+  const int64_t dst = g.idx(i, j, k);
+  float v[8];
+  bool fill[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    fill[q] = false;
+    if (q < n) {
+      const int on = ldi(P, 3 + q);
+      const int64_t src = g.idx(source(i, g.nx, openx, g.nx - 1 + (on == 1)), source(j, g.ny, openy, g.ny - 1 + (on == 2)), k);
+      fill[q] = src != dst;
+      if (fill[q]) v[q] = fq(a.q[1 + q])[src];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (fill[q]) fq(a.q[1 + q])[dst] = v[q];
+}
+
 // rk_update of a scalar (stagger 1) then its halo fill (rk_update.wgsl:111-132,
 // timestep.js:1593 haloFill); arguments as rk_update's.
 __global__ __launch_bounds__(256) void k_rk_update_xy(uint32_t* M, KArg a) {

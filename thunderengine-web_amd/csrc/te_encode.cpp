@@ -117,9 +117,9 @@ class Encoder {
   }
   Bytes acoustic;  // current stage's acoustic parameter bytes
 
-  // Periodic halo fills queue here when both directions are periodic and
-  // fusion is on; they are written by one bc_periodic_xy launch (up to 8
-  // fields) just before the next op that is not a halo fill.
+  // Halo fills queue here when fusion is on; they are written by one
+  // bc_periodic_xy launch (bc_open_xy where a side is open; up to 8 fields)
+  // just before the next op that is not a halo fill.
   bool mergeHalo = false;
   // fuse = 1 on a periodic domain (nx, ny >= 4): the halo fill after a
   // scalar's RK update, TKE's advance and the stage's pressure is written by
@@ -177,14 +177,21 @@ class Encoder {
       const int n = (int)std::min<size_t>(8, q.size() - s);
       Op o;
       std::memset(&o, 0, sizeof(o));
-      o.kid = kernel_id("bc_periodic_xy");
+      const char* kn = openX || openY ? "bc_open_xy" : "bc_periodic_xy";
+      o.kid = kernel_id(kn);
       o.A[0] = (uint32_t)(7 * (cfg.nx + 7) + 7 * cfg.ny); o.A[1] = (uint32_t)(cfg.nz + 1); o.A[2] = 1;
       o.A[4 + 0] = (uint32_t)dimsOff;
       o.A[4 + 30] = (uint32_t)hmOff;
       for (int q2 = 0; q2 < n; ++q2) o.A[4 + 1 + q2] = (uint32_t)off(q[s + q2]);
-      o.A[4 + 9] = (uint32_t)bytes(I1(n));
+      Bytes b = I1(n);
+      if (openX || openY) {  // the open sides, and per field 1 = on x faces, 2 = on y faces
+        b.push_back(openX ? 1u : 0u);
+        b.push_back(openY ? 1u : 0u);
+        for (int q2 = 0; q2 < 8; ++q2) b.push_back(q2 >= n ? 0u : isU(q[s + q2]) ? 1u : isV(q[s + q2]) ? 2u : 0u);
+      }
+      o.A[4 + 9] = (uint32_t)bytes(b);
       E.ops.push_back(o);
-      E.names.push_back("bc_periodic_xy");
+      E.names.push_back(kn);
     }
   }
 
@@ -279,8 +286,8 @@ void Encoder::setup() {
   rayleigh = cfg.rayleigh != 0;
   openX = cfg.open_x != 0; openY = cfg.open_y != 0;
   periodicX = !openX; periodicY = !openY;
-  mergeHalo = cfg.fuse != 0 && periodicX && periodicY;
-  foldHalo = mergeHalo && cfg.fuse == 1 && cfg.nx >= 4 && cfg.ny >= 4;
+  mergeHalo = cfg.fuse != 0;
+  foldHalo = periodicX && periodicY && cfg.fuse == 1 && cfg.nx >= 4 && cfg.ny >= 4;
   wenoS = cfg.weno_scalars != 0;
   wenoM = cfg.weno_momentum != 0;
   explicitZ = cfg.explicit_vdiff != 0;
