@@ -271,6 +271,63 @@ __global__ __launch_bounds__(256) void k_ac_pp_accumulate(uint32_t* M, KArg a) {
 
 namespace te {
 
+// One acoustic substep's accumulation of u and v over the whole grid
+// (acoustic_accumulate's rru, rrv) and the halo fill of u and v, by workgroups of their own in the same
+// launch: none of it waits for the column sweep, whose workgroups leave the
+// memory idle while they pass it on.  A wave takes AC_UV_UNITS (row, 64
+// columns) pairs, all loads before the first store (4: 2, 8 and 16 were slower
+// from 160 x 160 x 40 on, by up to 3, 1 and 7% of a step); the pairs are
+// numbered level by level within a row j, so that an XCD takes the rows its
+// column workgroups read.  u at (nx, j) and v at (i, ny) of interior rows /
+// columns belong to the column workgroups, which read them.
+TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t wg, int wave, int lane) {
+  const uint32_t n = a.n[2], q8 = n >> 3, r8 = n & 7u, xcd = wg & 7u;  // a.n[2]: workgroups of this kind
+  const uint32_t l = xcd * q8 + min(xcd, r8) + (wg >> 3);
+  const int nc = (g.sJ + 63) / 64, nl = g.nz + 1, units = g.sK * nl * nc;
+  auto F = [&](int q) { return FieldB(reinterpret_cast<float*>(M) + a.p[q]); };
+  const FieldB u = F(2), v = F(3), rru = F(13), rrv = F(14);
+  const bool first = ldi(a.q[33], 0) != 0;
+  const float tavg = ldf(a.q[17], 0), tv = tavg > 0.0f ? tavg : 1.0f;
+  const uint32_t sjb = 4u * (uint32_t)g.sJ, skb = sjb * (uint32_t)g.sK;
+  const int u0 = (int)(l * AC_WAVES + (uint32_t)wave) * AC_UV_UNITS;
+  uint32_t h[AC_UV_UNITS];
+  int todo[AC_UV_UNITS];  // 1 rru, 2 rrv, 4 u and v from their image
+  float uo[AC_UV_UNITS], vo[AC_UV_UNITS], ru[AC_UV_UNITS], rv[AC_UV_UNITS], us[AC_UV_UNITS], vs[AC_UV_UNITS];
+#pragma unroll
+  for (int d = 0; d < AC_UV_UNITS; ++d) {
+    const int id = u0 + d;
+    todo[d] = 0;
+    if (id >= units) continue;
+    const int row = id / nc, c = id - row * nc, jr = row / nl, k = row - jr * nl;
+    const int i = c * 64 + lane - 3, j = jr - 3;
+    if (i > g.nx + 3) continue;
+    const bool hx = i < 0 || i >= g.nx, hy = j < 0 || j >= g.ny;
+    const uint32_t lv = skb * (uint32_t)k;
+    h[d] = lv + 4u * (uint32_t)(i + 3) + sjb * (uint32_t)jr;
+    todo[d] = (!hy && i == g.nx ? 0 : 1) | (!hx && j == g.ny ? 0 : 2) | (hx || hy ? 4 : 0);
+    uo[d] = u(h[d]);
+    vo[d] = v(h[d]);
+    ru[d] = rv[d] = 0.0f;
+    if (!first) {
+      ru[d] = rru(h[d]);
+      rv[d] = rrv(h[d]);
+    }
+    if (todo[d] & 4) {
+      const int si = i < 0 ? i + g.nx : i >= g.nx ? i - g.nx : i, sj = j < 0 ? j + g.ny : j >= g.ny ? j - g.ny : j;
+      const uint32_t src = lv + 4u * (uint32_t)(si + 3) + sjb * (uint32_t)(sj + 3);
+      us[d] = u(src);
+      vs[d] = v(src);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < AC_UV_UNITS; ++d) {
+    if (todo[d] & 1) rru.put(h[d], (ru[d] + uo[d]) * tv);
+    if (todo[d] & 2) rrv.put(h[d], (rv[d] + vo[d]) * tv);
+    if ((todo[d] & 5) == 5) u.put(h[d], us[d]);
+    if ((todo[d] & 6) == 6) v.put(h[d], vs[d]);
+  }
+}
+
 // One acoustic substep after acoustic_uv, on a periodic domain, in one launch:
 // acoustic_fpk, acoustic_w_solve, acoustic_pp and acoustic_accumulate, then
 // the periodic halo fill of ppd, u, v and w, and on the stage's last substep
@@ -289,18 +346,39 @@ namespace te {
 // levels' coefficients in registers.  Values of the sweep are the reference's
 // sequential Thomas recurrence, level by level.
 //
+// The nz levels are dealt nz / AC_WAVES or one more to each wave, so only the
+// last of a wave's L rows is conditional; lanes past nx follow column nx - 1
+// and store nothing.  The elimination forms a row's coefficients while the
+// pivot before it is inverted, and takes the division only where a wave meets a
+// pivot outside the refined reciprocal's range (one uniform branch per row).
+//
 // Halo cells (every halo cell of ppd, u, v, w is the image of interior cell
 // (i mod nx, j mod ny), as the halo fill leaves it), each updated by the
-// workgroup of its interior cell, at each level by the wave that owns the
-// level, after that wave's own stores:
+// workgroup of its interior cell, at each level by the wave that owns it:
 //  * w and ppd: rrw accumulates the image's old w (the accumulate runs
 //    before the fill), then the new values are copied in.
 //  * u and v: rru, rrv accumulate the value there (acoustic_uv's at i = nx or
 //    j = ny, else the old image), then the image is copied in.  u at
 //    (nx, j) and v at (i, ny) are updated by the workgroup of column nx-1 /
-//    row ny-1, the only one that reads them (acoustic_fpk), after its reads.
-// The row's own images (hx = i) go column by column, lane = column; the
-// x-images and corners through a short per-workgroup list.
+//    row ny-1, the only one that reads them (acoustic_fpk), after its reads;
+//    all the others, with the accumulation at interior points, by
+//    ac_accumulate_uv's workgroups.
+// Only the new w, ppd and pp3d wait for the sweep.  The rest (`early`) is done
+// where the wave would wait for the sweep: before the elimination in the upper
+// waves, before the back substitution in the lower ones.  What follows the
+// sweep then holds stores only.  (gfx950 retires a wave's loads and stores in
+// order, so a load behind stores waits for their acknowledgement: 2-4 k cycles
+// with the grid's traffic, and every turn from stores to loads costs that.)
+// What bounds it: below about 256 workgroups the chain of one workgroup's
+// phases, above them the memory (212 MB of fields at 192 x 192 x 80).  Clock
+// stamps of the form before (a branch around each reciprocal, loads and stores
+// in turn after the sweep, halos last): 300 cycles to eliminate a row and 150 to
+// substitute it back, 45 k cycles in a row without y images and 60 k in one
+// with them at 64 x 64 x 40, 125 k and 180 k at 192 x 192 x 80; now 120 and 60
+// per row, 26 k and 32 k, 105 k and 145 k.  us per launch, before and now:
+// 64 x 64 x 40 24.3 and 15.0, 192 x 192 x 80 69 and 51, 256 x 256 x 120 203 and
+// 164 (1 level of loads in flight for 9 to 12 levels per wave: 2 spill, and a
+// reload behind stores waits for them, 58 us at 192 x 192 x 80).
 // p: 0 dims, 1 acoustic, 2 u, 3 v, 4 w, 5 piadv, 6 ppten, 7 ppterm, 8 thv,
 //    9 wten, 10 pp3d, 11 ppd, 12 ppx, 13 rru, 14 rrv, 15 rrw, 16 -> save ppx,
 //    17 -> tavg, 18 rr0, 19 rf0, 20 mh, 21 mf, 22 c1, 23 c2, 30 metric,
@@ -308,52 +386,63 @@ namespace te {
 //    too (with ppd's, group 4 below); the fields the replaced dispatches
 //    write as scratch (for expansions of this launch into them): 24 qk,
 //    25 pk1, 26 pk2, 27 mm, 28 fpk, 29 cA, 31 cB, and 32 rho0.
-// Grid: 64 x AC_WAVES threads per workgroup, ceil(nx / 64) x ny workgroups.
-// Needs nx, ny >= 4 and 4 <= nz <= AC_WAVES * LMAX.
+// Grid: 64 x AC_WAVES threads per workgroup, ceil(nx / 64) * ny workgroups of
+// columns (padded to a multiple of 8), then a.n[2] of ac_accumulate_uv.
+// Needs nx, ny >= 4, 4 <= nz <= AC_WAVES * 16, and fields below 2^32 bytes
+// (word offsets into M are 32 bits and a program's fields share that range).
 #define AC_HALO_CELLS 40  // per workgroup: at most 7 x-images, 1 (nx, j) cell, 14 corners
-template <int LMAX>
+template <int L>
 __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
-  constexpr int KMAX = AC_WAVES * 16 + 1;
+  // Few levels per wave: the later phases' operands are kept or loaded ahead
+  // of the sweep (registers to spare); many: the w rows wait in LDS and the
+  // loads come in chunks, so that three workgroups stay resident per CU.
+  constexpr bool AHEAD = L <= 6;
+  constexpr int CH = AHEAD ? L : L >= 9 && L <= 12 ? 1 : 2;  // levels of loads in flight, pointwise part
   __shared__ float xa[AC_WAVES][3][64];  // pk1+qk, pk2-qk, pp3d+fpk at each wave's last level
   __shared__ float xb[2][64];            // elimination carry between waves
-  __shared__ float xw[AC_WAVES][64];     // new w at each wave's first level
-  __shared__ float lv[6][KMAX];          // acoustic_prepare's per-level factors: tem, r1, r2, tem1, c1, c2
+  __shared__ float xw[64];               // new w at the first level of the wave above
+  __shared__ int fwd_done, back_next;    // the sweep's hand-offs between waves
   __shared__ int hcnt;
-  __shared__ int fwd_done, back_next;  // the sweep's hand-offs between waves
   __shared__ short hcell[AC_HALO_CELLS][3];
-  // dynamic: per level and lane mm (then cA, then the new w) and the w
-  // row's right-hand side part (then cB): 2 * nz * 64 floats
+  // acoustic_prepare's per-level factors tem, r1, r2, tem1, c1, c2: scalar
+  // loads where a wave has few levels, else a table
+  __shared__ float lv[AHEAD ? 1 : 6][AHEAD ? 1 : AC_WAVES * 16 + 1];
+  // dynamic (L > 6): per level and lane mm and the w row's right-hand side
+  // part, then the elimination coefficients
   float* me0 = te_lds;
-  const Blk blk = te_block(a);
   const int lane = (int)threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);  // one wave per threadIdx.y
   const Dims g = dims(a.q[0], 0);
+  const uint32_t solvers = (a.lg[9] + 7u) & ~7u;  // workgroups of columns, padded to the XCDs
+  if (blockIdx.x >= solvers) {
+    ac_accumulate_uv(M, a, g, blockIdx.x - solvers, wave, lane);
+    return;
+  }
+  if (blockIdx.x >= a.lg[9]) return;
+  const Blk blk = te_block(a);
   const int i = blk.x * 64 + lane, j = blk.y, nx = g.nx, ny = g.ny, nz = g.nz;
   float* me1 = te_lds + nz * 64;
-  const bool active = i < nx && j < ny;
-  const int Lw = (nz + AC_WAVES - 1) / AC_WAVES, k0 = wave * Lw, k1 = min(nz, k0 + Lw), Lq = max(0, k1 - k0);
-  const bool top = k1 == nz && Lq > 0;
+  const bool active = i < nx;
+  const int ic = min(i, nx - 1);
+  const int base = nz / AC_WAVES, rem = nz % AC_WAVES;
+  const int Lq = base + (wave < rem ? 1 : 0), k0 = wave * base + min(wave, rem);
+  const bool full = Lq == L;  // else Lq == L - 1
+  const bool top = Lq > 0 && k0 + Lq == nz;
   const Acoustic ac = acoustic(a.q[1], 0);
-  // fields as 32-bit word offsets into M (fewer scalar registers than pointers)
-  auto F = [&](int q) { return reinterpret_cast<float*>(M) + a.p[q]; };
+  auto F = [&](int q) { return FieldB(reinterpret_cast<float*>(M) + a.p[q]); };
+  auto prof = [&](int q, int k) { return (reinterpret_cast<const float*>(M) + a.p[q])[k]; };
   const bool saveX = ldi(a.q[16], 0) != 0, first = ldi(a.q[33], 0) != 0;
   const bool imgP = a.p[34] != 0 && ldi(a.q[34], 0) != 0;
   const float tavg = ldf(a.q[17], 0);
   if (threadIdx.x == 0 && threadIdx.y == 0) {
-    hcnt = 0;
     fwd_done = 0;
     back_next = AC_WAVES - 1;
+    hcnt = 0;
   }
-  // Halo cells this workgroup updates, (hx, hy, groups):
-  // group 1 = u, rru; 2 = v, rrv; 4 = w, rrw, ppd.  A halo cell's groups are
-  // handled by the workgroup of its image (i mod nx, j mod ny), except u at
-  // (nx, j) and v at (i, ny): acoustic_fpk of column nx-1 / row ny-1 reads
-  // them, so that column's / row's workgroup updates them after its reads.
-  // The images of the workgroup's own row (hx = i: hy = j -+ ny, and v at
-  // (i, ny) for row ny-1) are handled column by column (row_images); the list
-  // holds the x-images, the corners and u at (nx, j).
+  // Halo cells of the x-images and corners of this workgroup's columns,
+  // (hx, hy, 4), and (nx, j, 1): what `early` does with them
   const int ys[2] = {j >= ny - 3 ? j - ny : j, j <= 3 ? j + ny : j};
-  if (active && wave == 0) {
+  if (active && wave == 0) {  // (one wave: its LDS operations keep their order)
     const int xs[2] = {i >= nx - 3 ? i - nx : i, i <= 3 ? i + nx : i};
     const int nxi = (i >= nx - 3) + (i <= 3), nyi = (j >= ny - 3) + (j <= 3);
     const int n = nxi * (1 + nyi) + (i == nx - 1);
@@ -364,205 +453,250 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
         ++q;
       };
       for (int by = 0; by < 3; ++by)
-        for (int bx = 1; bx < 3; ++bx) {
-          const int hx = xs[bx - 1], hy = by == 0 ? j : ys[by - 1];
+        for (int bx = 0; bx < 2; ++bx) {
+          const int hx = xs[bx], hy = by == 0 ? j : ys[by - 1];
           if (hx == i || (by > 0 && hy == j)) continue;
-          put(hx, hy, 7 & ~(hx == nx && hy == j ? 1 : 0));
+          put(hx, hy, 4);
         }
       if (i == nx - 1) put(nx, j, 1);
     }
   }
-
-  {
-    const float *rr0 = F(18), *rf0 = F(19), *mh = F(20), *mf = F(21), *c1 = F(22), *c2 = F(23);
+  auto prep = [&](int k, float f[6]) {
+    const int kp = min(k + 1, nz);
+    const float tem = (ac.dts * g.rdz) * prof(20, k), rr0k = prof(18, k);
+    f[0] = tem;
+    f[1] = (tem * rr0k) * prof(19, k);
+    f[2] = (tem * rr0k) * prof(19, kp);
+    f[3] = ((ac.dts * g.rdz) * CP) * prof(21, k);
+    f[4] = prof(22, k);
+    f[5] = prof(23, k);
+  };
+  if constexpr (!AHEAD) {
     for (int k = (int)(threadIdx.y * 64 + threadIdx.x); k <= nz; k += 64 * AC_WAVES) {
-      if (k < nz) {
-        const float tem = (ac.dts * g.rdz) * mh[k];
-        lv[0][k] = tem;
-        lv[1][k] = (tem * rr0[k]) * rf0[k];
-        lv[2][k] = (tem * rr0[k]) * rf0[k + 1];
-      }
-      lv[3][k] = ((ac.dts * g.rdz) * CP) * mf[k];
-      lv[4][k] = c1[k];
-      lv[5][k] = c2[k];
+      float f[6];
+      prep(k, f);
+      for (int q = 0; q < 6; ++q) lv[q][k] = f[q];
     }
   }
   __syncthreads();
-  const int64_t sj = g.sJ, sk = g.sk();
+  const FieldB u = F(2), v = F(3), w = F(4), piadv = F(5), ppten = F(6), ppterm = F(7), thv = F(8), wten = F(9),
+               pp3d = F(10), ppd = F(11), ppx = F(12), rru = F(13), rrv = F(14), rrw = F(15);
+  // byte offset of this lane's column at level k (the same in every field)
+  const uint32_t sjb = 4u * (uint32_t)g.sJ, skb = sjb * (uint32_t)g.sK;
+  const uint32_t o00 = 4u * (uint32_t)(ic + 3) + sjb * (uint32_t)(j + 3);
+  auto at = [&](int k) { return o00 + skb * (uint32_t)k; };
   const float asq = ac.alph * ac.alph;
   const float temx = (ac.dts * 0.5f) * g.rdx, temy = (ac.dts * 0.5f) * g.rdy;
   const bool vec_v = nx > 3 && i < (nx / 4) * 4;
-  auto acc = [&](float base, float x) { return tavg > 0.0f ? (base + x) * tavg : base + x; };
-  auto accw = [&](float base, float x) { return tavg > 0.0f ? fma_(x, ac.alph, base) * tavg : base + x; };
-  // Halo cells, each wave at its own levels (and level nz for the top wave)
-  // once its stores above are done.  u, v (groups 1, 2): rru, rrv accumulate
-  // the value there (acoustic_uv's at i = nx or j = ny, else the old image),
-  // then the image is copied in; the interior values are acoustic_uv's, and
-  // the wave's own acoustic_fpk reads of u at i = nx and v at j = ny came
-  // first.  w, ppd (group 4): rrw accumulates the old w there, then the new w
-  // and ppd of the interior cell are copied in; the interior cell is in this
-  // workgroup's row at the same level, written by this wave.  pp3d (with
-  // group 4 when imgP) likewise: no thread of the launch reads its halo.
-  // halo(): the cells of the list, 2 (cell, level) items per lane per round
-  // with their loads before their stores.
-  // The row's own images, lane = column, 2 levels of loads before their
-  // stores: r = 0, 1 the images at hy = j -+ ny (v excluded at hy = ny: row
-  // ny-1's workgroup handles v there), r = 2 v at (i, ny) for row ny-1.
-  auto row_images = [&](auto G) {
-    constexpr int groups = decltype(G)::value;
-    if (!active) return;
-    float *u = F(2), *v = F(3), *w = F(4), *pp3d = F(10), *ppd = F(11), *rru = F(13), *rrv = F(14), *rrw = F(15);
-    const int nl = Lq + (top ? 1 : 0);
-    for (int r = 0; r < 3; ++r) {
-      int hy, m;
-      if (r < 2) {
-        hy = ys[r];
-        if (hy == j || (r == 1 && ys[0] == ys[1])) continue;
-        m = 7 & ~(hy == ny ? 2 : 0);
-      } else {
-        if (j != ny - 1) continue;
-        hy = ny;
-        m = 2;
-      }
-      m &= groups;
-      if (m == 0) continue;
-      const int sy = hy < 0 ? hy + ny : (hy >= ny ? hy - ny : hy);
-      for (int t0 = 0; t0 < nl; t0 += 2) {
-        float x[2][11];
-#pragma unroll
-        for (int d = 0; d < 2; ++d)
-          if (t0 + d < nl) {
-            const int t = t0 + d, k = t < Lq ? k0 + t : nz;
-            const int64_t ch = g.idx(i, hy, k), cs = g.idx(i, sy, k);
-            if (m & 1) { x[d][0] = u[ch]; x[d][1] = u[cs]; x[d][2] = rru[ch]; }
-            if (m & 2) { x[d][3] = v[ch]; x[d][4] = v[cs]; x[d][5] = rrv[ch]; }
-            if (m & 4) {
-              x[d][6] = w[ch]; x[d][7] = rrw[ch]; x[d][8] = w[cs]; x[d][9] = ppd[cs];
-              if (imgP) x[d][10] = pp3d[cs];
-            }
-          }
-#pragma unroll
-        for (int d = 0; d < 2; ++d)
-          if (t0 + d < nl) {
-            const int t = t0 + d, k = t < Lq ? k0 + t : nz;
-            const int64_t ch = g.idx(i, hy, k);
-            if (m & 1) {
-              rru[ch] = acc(first ? 0.0f : x[d][2], x[d][0]);
-              u[ch] = x[d][1];
-            }
-            if (m & 2) {
-              rrv[ch] = acc(first ? 0.0f : x[d][5], x[d][3]);
-              v[ch] = x[d][4];
-            }
-            if (m & 4) {
-              rrw[ch] = accw(first ? x[d][6] * ac.beta : x[d][7], x[d][6]);
-              w[ch] = x[d][8];
-              ppd[ch] = x[d][9];
-              if (imgP) pp3d[ch] = x[d][10];
-            }
-          }
-      }
-    }
-  };
-  auto halo = [&](auto G) {
-    constexpr int groups = decltype(G)::value;
-    float *u = F(2), *v = F(3), *w = F(4), *pp3d = F(10), *ppd = F(11), *rru = F(13), *rrv = F(14), *rrw = F(15);
-    const int nc = hcnt, nl = Lq + (top ? 1 : 0), items = nc * nl;
-    constexpr int B = 2;
-    for (int it0 = lane; it0 < items; it0 += B * 64) {
-      float x[B][11];
-      int64_t hc[B];
-      int mask[B];
-#pragma unroll
-      for (int d = 0; d < B; ++d) {
-        const int it = it0 + d * 64;
-        mask[d] = 0;
-        if (it < items) {
-          const int kk = it / nc, q = it - kk * nc, k = kk < Lq ? k0 + kk : nz;
-          const int hx = hcell[q][0], hy = hcell[q][1];
-          const int sx = hx < 0 ? hx + nx : (hx >= nx ? hx - nx : hx), sy = hy < 0 ? hy + ny : (hy >= ny ? hy - ny : hy);
-          const int64_t ch = g.idx(hx, hy, k), cs = g.idx(sx, sy, k);
-          hc[d] = ch;
-          mask[d] = hcell[q][2] & groups;
-          if (mask[d] & 1) { x[d][0] = u[ch]; x[d][1] = u[cs]; x[d][2] = rru[ch]; }
-          if (mask[d] & 2) { x[d][3] = v[ch]; x[d][4] = v[cs]; x[d][5] = rrv[ch]; }
-          if (mask[d] & 4) {
-            x[d][6] = w[ch]; x[d][7] = rrw[ch]; x[d][8] = w[cs]; x[d][9] = ppd[cs];
-            if (imgP) x[d][10] = pp3d[cs];
-          }
-        }
-      }
-#pragma unroll
-      for (int d = 0; d < B; ++d) {
-        const int64_t ch = hc[d];
-        if (mask[d] & 1) {
-          rru[ch] = acc(first ? 0.0f : x[d][2], x[d][0]);
-          u[ch] = x[d][1];
-        }
-        if (mask[d] & 2) {
-          rrv[ch] = acc(first ? 0.0f : x[d][5], x[d][3]);
-          v[ch] = x[d][4];
-        }
-        if (mask[d] & 4) {
-          rrw[ch] = accw(first ? x[d][6] * ac.beta : x[d][7], x[d][6]);
-          w[ch] = x[d][8];
-          ppd[ch] = x[d][9];
-          if (imgP) pp3d[ch] = x[d][10];
-        }
-      }
-    }
-  };
-  float PQ[LMAX], P2Q[LMAX], PF[LMAX];
+  // the accumulation, scaled on the last substep; before it the factors are 1
+  // (exact in both operations)
+  const float tv = tavg > 0.0f ? tavg : 1.0f, al = tavg > 0.0f ? ac.alph : 1.0f;
+  auto acc = [&](float b, float x) { return (b + x) * tv; };
+  auto accw = [&](float b, float x) { return fma_(x, al, b) * tv; };
+#define ROW(t) ((t) < L - 1 || full)
+  float PQ[L], P2Q[L], PF[L], ME[L], EE[L];
   // ---- pointwise: acoustic_prepare's terms, acoustic_fpk, the w row's
-  // right-hand side (levels -1 and nz, read at the column's ends and not
-  // used, lie in the field slot or the memory's front guard)
-  if (active) {
-    const float *u = F(2), *v = F(3), *w = F(4), *piadv = F(5), *ppten = F(6), *ppterm = F(7), *thv = F(8),
-                *wten = F(9), *pp3d = F(10), *hm = F(30);
-    const float uh = hm_uh(hm, g, i), vh = hm_vh(hm, g, j);
-    float pp_prev = pp3d[g.idx(i, j, min(k0, nz) - 1)];
+  // right-hand side.  Row L - 1 of a wave with L - 1 levels is formed from
+  // the level above (or level nz) and not used.
+  float PP[L];  // pp3d before the substep
+  {
+    const float* hm = reinterpret_cast<const float*>(M) + a.p[30];
+    const float uh = hm_uh(hm, g, ic), vh = hm_vh(hm, g, j);
+    const uint32_t om = at(max(k0 - 1, 0));  // level -1 is not used
+    float pam = piadv(om), thm0 = thv(om), ppm = pp3d(om);
 #pragma unroll
-    for (int t = 0; t < LMAX; ++t) {
-      if (t < Lq) {
-        const int k = k0 + t;
-        const int64_t c = g.idx(i, j, k);
-        const float uc = u[c], up = u[c + 1], vc = v[c], vp = v[c + sj], wk = w[c], wk1 = w[c + sk];
-        const float pa0 = piadv[c], paxm = piadv[c - 1], paxp = piadv[c + 1], paym = piadv[c - sj],
-                    payp = piadv[c + sj], pzp0 = piadv[c + sk], pzm0 = piadv[c - sk];
-        const float ppt = ppterm[c], ppn = ppten[c], pp = pp3d[c], th = thv[c], thm0 = thv[c - sk], wt = wten[c];
-        const bool bot = k == 0, ktop = k == nz - 1;
-        const float pzp = ktop ? 0.0f : pzp0, pzm = bot ? 0.0f : pzm0, thm = bot ? th : thm0;
-        const float tem = lv[0][k], r1 = lv[1][k], r2 = lv[2][k], tem1 = lv[3][k];
-        const float c1a = lv[4][k], c2a = lv[5][k], c1b = lv[4][k + 1], c2b = lv[5][k + 1];
-        const float qk = tem * ppt;
-        const float p2 = ktop ? 0.0f : (vec_v ? fma_(-c2b, pzp, (1.0f - c1b) * pa0) : fma_(1.0f - c1b, pa0, -(c2b * pzp)));
-        const float p1 = bot ? 0.0f : (vec_v ? fma_(c2a - 1.0f, pa0, c1a * pzm) : fma_(c1a, pzm, (c2a - 1.0f) * pa0));
-        const float pk2 = ktop ? 0.0f : r2 * p2;
-        const float pk1 = bot ? 0.0f : r1 * p1;
-        const float mm = tem1 * fma_(c2a, th, c1a * thm);
-        float div = fma_((up - uc) * g.rdx, uh, ((vp - vc) * g.rdy) * vh);
-        if (ab(div) < ac.smeps) div = 0.0f;
-        const float Au = fma_(uc, pa0 - paxm, up * (paxp - pa0));
-        const float Av = fma_(vc, pa0 - paym, vp * (payp - pa0));
-        const float advPi = fma_((-Au) * temx, uh, -((Av * temy) * vh));
-        const float fpk = fma_(ac.beta, fma_(wk, pk1 + qk, wk1 * (pk2 - qk)),
-                               fma_(ac.dts, fma_(-ppt, div, ppn), advPi));
-        PQ[t] = pk1 + qk;
-        P2Q[t] = pk2 - qk;
-        PF[t] = pp + fpk;
-        me0[k * 64 + lane] = mm;
-        me1[k * 64 + lane] = bot ? 0.0f : wk + fma_(ac.dts, wt, ac.beta * ((-mm) * (pp - pp_prev)));
-        pp_prev = pp;
+    for (int t0 = 0; t0 < L; t0 += CH) {
+      float U[CH], UP[CH], V[CH], VP[CH], W[CH + 1], PA[CH + 1], XM[CH], XP[CH], YM[CH], YP[CH], PT[CH], PN[CH], TH[CH],
+          WT[CH];
+#pragma unroll
+      for (int d = 0; d < CH; ++d)
+        if (t0 + d < L) {
+          const uint32_t o = at(min(k0 + t0 + d, nz));
+          U[d] = u(o); UP[d] = u(o + 4u); V[d] = v(o); VP[d] = v(o + sjb);
+          W[d] = w(o); PA[d] = piadv(o);
+          XM[d] = piadv(o - 4u); XP[d] = piadv(o + 4u); YM[d] = piadv(o - sjb); YP[d] = piadv(o + sjb);
+          PT[d] = ppterm(o); PN[d] = ppten(o); PP[t0 + d] = pp3d(o); TH[d] = thv(o); WT[d] = wten(o);
+        }
+      {
+        const int n = t0 + CH < L ? CH : L - t0;  // rows of this chunk; the level above its last
+        const uint32_t o = at(min(k0 + t0 + n, nz));
+        W[n] = w(o);
+        PA[n] = piadv(o);
+      }
+#pragma unroll
+      for (int d = 0; d < CH; ++d)
+        if (t0 + d < L) {
+          const int t = t0 + d, k = min(k0 + t, nz), kp = min(k + 1, nz);
+          const float pa0 = PA[d];
+          const bool bot = k == 0, ktop = k == nz - 1;
+          const float pzp = ktop ? 0.0f : PA[d + 1], pzm = bot ? 0.0f : pam, thm = bot ? TH[d] : thm0;
+          float f[6];
+          if constexpr (AHEAD) {
+            prep(k, f);
+          } else {
+            for (int q = 0; q < 6; ++q) f[q] = lv[q][k];
+          }
+          const float tem = f[0], r1 = f[1], r2 = f[2], tem1 = f[3], c1a = f[4], c2a = f[5];
+          const float c1b = AHEAD ? prof(22, kp) : lv[AHEAD ? 0 : 4][AHEAD ? 0 : kp], c2b = AHEAD ? prof(23, kp) : lv[AHEAD ? 0 : 5][AHEAD ? 0 : kp];
+          const float qk = tem * PT[d];
+          const float p2 = ktop ? 0.0f : (vec_v ? fma_(-c2b, pzp, (1.0f - c1b) * pa0) : fma_(1.0f - c1b, pa0, -(c2b * pzp)));
+          const float p1 = bot ? 0.0f : (vec_v ? fma_(c2a - 1.0f, pa0, c1a * pzm) : fma_(c1a, pzm, (c2a - 1.0f) * pa0));
+          const float pk2 = ktop ? 0.0f : r2 * p2;
+          const float pk1 = bot ? 0.0f : r1 * p1;
+          const float mm = tem1 * fma_(c2a, TH[d], c1a * thm);
+          float div = fma_((UP[d] - U[d]) * g.rdx, uh, ((VP[d] - V[d]) * g.rdy) * vh);
+          if (ab(div) < ac.smeps) div = 0.0f;
+          const float Au = fma_(U[d], pa0 - XM[d], UP[d] * (XP[d] - pa0));
+          const float Av = fma_(V[d], pa0 - YM[d], VP[d] * (YP[d] - pa0));
+          const float advPi = fma_((-Au) * temx, uh, -((Av * temy) * vh));
+          const float fpk = fma_(ac.beta, fma_(W[d], pk1 + qk, W[d + 1] * (pk2 - qk)),
+                                 fma_(ac.dts, fma_(-PT[d], div, PN[d]), advPi));
+          PQ[t] = pk1 + qk;
+          P2Q[t] = pk2 - qk;
+          PF[t] = PP[t] + fpk;
+          ME[t] = mm;
+          EE[t] = bot ? 0.0f : W[d] + fma_(ac.dts, WT[d], ac.beta * ((-mm) * (PP[t] - ppm)));
+          te_pin(PQ[t]); te_pin(P2Q[t]); te_pin(PF[t]); te_pin(ME[t]); te_pin(EE[t]);
+          if constexpr (!AHEAD)
+            if (ROW(t)) {
+              me0[k * 64 + lane] = ME[t];
+              me1[k * 64 + lane] = EE[t];
+            }
+          ppm = PP[t];
+          pam = pa0;
+          thm0 = TH[d];
+        }
+    }
+    if (Lq > 0) {
+      xa[wave][0][lane] = full ? PQ[L - 1] : PQ[L > 1 ? L - 2 : 0];
+      xa[wave][1][lane] = full ? P2Q[L - 1] : P2Q[L > 1 ? L - 2 : 0];
+      xa[wave][2][lane] = full ? PF[L - 1] : PF[L > 1 ? L - 2 : 0];
+    }
+  }
+  float RW[L], ppdz = 0.0f, ppz = 0.0f;  // rrw before the substep; ppd, pp3d of level nz
+  // What does not wait for the sweep (see above).  Level nz goes with the top
+  // wave: w stays 0 there (acoustic_w_solve clears it), ppd is not updated.
+  auto early = [&]() {
+    const int nl = Lq + (top ? 1 : 0);
+    if (top) {
+      const uint32_t o = at(nz);
+      const float rw = first ? w(o) * ac.beta : rrw(o);
+      ppdz = ppd(o);
+      ppz = pp3d(o);
+      if (active) {
+        rrw.put(o, accw(rw, 0.0f));
+        w.put(o, 0.0f);
       }
     }
-#pragma unroll
-    for (int t = 0; t < LMAX; ++t)
-      if (t == Lq - 1) {
-        xa[wave][0][lane] = PQ[t];
-        xa[wave][1][lane] = P2Q[t];
-        xa[wave][2][lane] = PF[t];
+    // a halo cell's rrw accumulates the old w there; u at (nx, j) and v at
+    // (i, ny) are accumulated, then replaced by their images
+    struct Item {
+      uint32_t h;
+      int m;
+      float x, y, z;
+    };
+    // the x-images, the corners and (nx, j): the list, a (cell, level) pair per
+    // lane, the first 64 pairs loaded before the first store
+    const int nc = hcnt, items = nc * nl;
+    auto item = [&](int it) {
+      Item c = {0u, 0, 0.0f, 0.0f, 0.0f};
+      if (it < items) {
+        const int kk = it / nc, q = it - kk * nc, hx = hcell[q][0], hy = hcell[q][1];
+        const uint32_t l0 = skb * (uint32_t)(k0 + kk) + 12u + sjb * 3u;
+        c.m = hcell[q][2];
+        c.h = l0 + 4u * (uint32_t)hx + sjb * (uint32_t)hy;
+        if (c.m == 4) {
+          c.x = w(c.h);
+          c.y = first ? c.x * ac.beta : rrw(c.h);
+        } else {
+          c.x = u(c.h);
+          c.y = first ? 0.0f : rru(c.h);
+          c.z = u(l0 + sjb * (uint32_t)j);  // u at (0, j)
+        }
       }
-  }
+      return c;
+    };
+    auto store = [&](const Item& c) {
+      if (c.m == 4) {
+        rrw.put(c.h, accw(c.y, c.x));
+      } else if (c.m != 0) {
+        rru.put(c.h, acc(c.y, c.x));
+        u.put(c.h, c.z);
+      }
+    };
+    const Item ia = item(lane);
+    // the row's own images, lane = column: rows t0 .. t0 + CI - 1 of the wave
+    // (and level nz as row Lq), loads without a branch between them
+    constexpr int CI = AHEAD ? L : 5;
+    auto batch = [&](int t0, auto&& f) {
+#pragma unroll
+      for (int d = 0; d < CI; ++d)
+        if (t0 + d < L && ROW(t0 + d)) f(d, at(k0 + t0 + d));
+    };
+#pragma unroll 1
+    for (int r = 0; r < 2; ++r) {
+      const int hy = ys[r];
+      if (hy == j) continue;
+      const uint32_t off = sjb * (uint32_t)(hy - j);
+#pragma unroll
+      for (int t0 = 0; t0 < L; t0 += CI) {
+        float x[CI], y[CI], xz = 0.0f, yz = 0.0f;
+        const bool z = top && t0 + CI >= L;
+        batch(t0, [&](int d, uint32_t o) { x[d] = w(o + off); });
+        if (z) xz = w(at(nz) + off);
+        if (first) {
+          batch(t0, [&](int d, uint32_t) { y[d] = x[d] * ac.beta; });
+          yz = xz * ac.beta;
+        } else {
+          batch(t0, [&](int d, uint32_t o) { y[d] = rrw(o + off); });
+          if (z) yz = rrw(at(nz) + off);
+        }
+        if (active) {
+          batch(t0, [&](int d, uint32_t o) { rrw.put(o + off, accw(y[d], x[d])); });
+          if (z) rrw.put(at(nz) + off, accw(yz, xz));
+        }
+      }
+    }
+    store(ia);
+#pragma unroll 1
+    for (int it = lane + 64; it < items; it += 64) store(item(it));
+    if (j == ny - 1) {  // v at (i, ny)
+      const uint32_t src = sjb * (uint32_t)(-j);
+#pragma unroll
+      for (int t0 = 0; t0 < L; t0 += CI) {
+        float x[CI], y[CI], s[CI], xz = 0.0f, yz = 0.0f, sz = 0.0f;
+        const bool z = top && t0 + CI >= L;
+        batch(t0, [&](int d, uint32_t o) { x[d] = v(o + sjb); s[d] = v(o + src); y[d] = 0.0f; });
+        if (!first) batch(t0, [&](int d, uint32_t o) { y[d] = rrv(o + sjb); });
+        if (z) {
+          const uint32_t o = at(nz);
+          xz = v(o + sjb);
+          sz = v(o + src);
+          yz = first ? 0.0f : rrv(o + sjb);
+        }
+        if (active) {
+          batch(t0, [&](int d, uint32_t o) {
+            rrv.put(o + sjb, acc(y[d], x[d]));
+            v.put(o + sjb, s[d]);
+          });
+          if (z) {
+            rrv.put(at(nz) + sjb, acc(yz, xz));
+            v.put(at(nz) + sjb, sz);
+          }
+        }
+      }
+    }
+  };
+  const FieldB rw0 = first ? w : rrw;  // acoustic_begin's rrw is w * beta
+  const float bf = first ? ac.beta : 1.0f;
+  auto load_rrw = [&]() {
+#pragma unroll
+    for (int t = 0; t < L; ++t) {
+      RW[t] = 0.0f;
+      if (ROW(t)) RW[t] = rw0(at(k0 + t));
+    }
+  };
+  const bool upper = wave >= AC_WAVES / 2;
   // The sweep passes from wave to wave through LDS counters instead of
   // workgroup barriers, so a wave's share of the serial recurrence overlaps
   // the loads of the waves above it (forward) and the stores of the waves
@@ -571,150 +705,161 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   // elimination) and for back_next == w (set by wave w+1 after its back
   // substitution; the top wave is the last of the forward chain), so each
   // wait ends once the waves below / above it have run.  The waits are
-  // bounded (2^22 polls) all the same.
+  // bounded (2^22 polls) all the same.  What is handed over lies in LDS, whose
+  // operations a wave issues and the LDS executes in order: the flag needs the
+  // LDS counter only, not a release of the wave's global loads and stores
+  // (192 x 192 x 80: the top wave waited 43 k cycles there for rrw).
   auto wait_for = [&](int* flag, int want) {
     for (int s = 0; s < (1 << 22); ++s) {
-      const int v = __builtin_amdgcn_readfirstlane(
-          __hip_atomic_load(flag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
-      if (v == want) break;
+      const int f = __builtin_amdgcn_readfirstlane(
+          __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+      if (f == want) break;
       __builtin_amdgcn_s_sleep(1);
     }
+    asm volatile("" ::: "memory");
   };
-  auto pass = [&](int* flag, int v) { __hip_atomic_store(flag, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP); };
-  // ---- forward elimination, wave after wave (cA over mm, cB over the
-  // right-hand side part; the top row leaves w at nz-1 there).  Rows k = 1
-  // and k = nz-1 are the reference's special cases, taken by selects.  Lanes
-  // past nx compute on unset values and touch no global memory here.
-  // The rows' operands from LDS into registers before the wait (the
-  // recurrence then waits on nothing but itself).
-  float ME[LMAX], EE[LMAX];
+  auto pass = [&](int* flag, int f) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __hip_atomic_store(flag, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  // ---- forward elimination, wave after wave: (mm, right-hand side) of a row
+  // become its elimination coefficients (the top row's leave w at nz-1).
+  // Row k = 1 has no row below it (row 1 of wave 0, or row 0 of wave 1 when
+  // waves hold one level); level 0 is no row.
+  float CA[L], CB[L];
+  struct Row {
+    float aa, cc, bb, dd;
+  };
+  // row t from PQ, P2Q and PF of its own level and of the one below
+  auto row = [&](int t, float pq_m, float p2q_m, float ppf_m) {
+    const float m = AHEAD ? ME[t] : me0[(k0 + t) * 64 + lane], e = AHEAD ? EE[t] : me1[(k0 + t) * 64 + lane];
+    Row r = {(-asq) * (m * pq_m), (-asq) * ((-m) * P2Q[t]), fma_(-asq, m * ((-PQ[t]) + p2q_m), 1.0f),
+             fma_(ac.alph, (-m) * (PF[t] - ppf_m), e)};
+    te_pin(r.aa); te_pin(r.cc); te_pin(r.bb); te_pin(r.dd);
+    return r;
+  };
+  // AHEAD: every row but the first (which waits for the wave below's last
+  // level) before the wait; else row t + 1 between row t's pivot and the test
+  // that waits for its reciprocal
+  Row R[AHEAD ? L : 2];
+  if constexpr (AHEAD) {
 #pragma unroll
-  for (int t = 0; t < LMAX; ++t)
-    if (t < Lq) {
-      ME[t] = me0[(k0 + t) * 64 + lane];
-      EE[t] = me1[(k0 + t) * 64 + lane];
-    }
+    for (int t = 1; t < L; ++t) R[t] = row(t, PQ[t - 1], P2Q[t - 1], PF[t - 1]);
+  }
+  if (upper && Lq > 0) early();
   wait_for(&fwd_done, wave);
-  {
-    if (Lq > 0) {
-      float pa = 0.0f, pb = 0.0f, pq_m = 0.0f, p2q_m = 0.0f, ppf_m = 0.0f;
-      if (wave > 0) {
-        pa = xb[0][lane];
-        pb = xb[1][lane];
-        pq_m = xa[wave - 1][0][lane];
-        p2q_m = xa[wave - 1][1][lane];
-        ppf_m = xa[wave - 1][2][lane];
-      }
-#pragma unroll
-      for (int t = 0; t < LMAX; ++t) {
-        const int k = k0 + t;
-        if (t < Lq) {
-          if (k >= 1) {
-            const float m = ME[t], e = EE[t];
-            const float aa = (-asq) * (m * pq_m);
-            const float cc = (-asq) * ((-m) * P2Q[t]);
-            const float bb = fma_(-asq, m * ((-PQ[t]) + p2q_m), 1.0f);
-            const float dd = fma_(ac.alph, (-m) * (PF[t] - ppf_m), e);
-            const bool first_row = k == 1;
-            const float r = recip(first_row ? bb : fma_(aa, pa, bb));
-            pa = (-cc) * r;
-            pb = (first_row ? dd : fma_(-aa, pb, dd)) * r;
-            ME[t] = pa;  // not read for the top row (w there is pb)
-            EE[t] = pb;
-          }
-          pq_m = PQ[t];
-          p2q_m = P2Q[t];
-          ppf_m = PF[t];
-        }
-      }
-      xb[0][lane] = pa;
-      xb[1][lane] = pb;
+  if (Lq > 0) {
+    float pa = 0.0f, pb = 0.0f;
+    if (wave > 0) {
+      pa = xb[0][lane];
+      pb = xb[1][lane];
+      R[0] = row(0, xa[wave - 1][0][lane], xa[wave - 1][1][lane], xa[wave - 1][2][lane]);
     }
-    pass(&fwd_done, wave + 1);
+#pragma unroll
+    for (int t = 0; t < L; ++t) {
+      const bool first_row = t == (L > 1 ? 1 : 0) && k0 + t == 1;
+      const Row& r = R[AHEAD ? t : t % 2];
+      if (t == 0 ? (wave > 0 && ROW(0)) : ROW(t)) {
+        const float x = first_row ? r.bb : fma_(r.aa, pa, r.bb);
+        float y = recip_refined(x);
+        if constexpr (!AHEAD)
+          if (t + 1 < L) R[(t + 1) % 2] = row(t + 1, PQ[t], P2Q[t], PF[t]);
+        if (__builtin_expect(__any(recip_far(x) > kRecipRange), 0)) y = recip(x);
+        pb = (first_row ? r.dd : fma_(-r.aa, pb, r.dd)) * y;
+        pa = (-r.cc) * y;
+        if constexpr (AHEAD) {
+          CA[t] = pa;  // not read for the top row (w there is pb)
+          CB[t] = pb;
+        } else {
+          me0[(k0 + t) * 64 + lane] = pa;
+          me1[(k0 + t) * 64 + lane] = pb;
+        }
+      } else if constexpr (!AHEAD) {
+        if (t + 1 < L) R[(t + 1) % 2] = row(t + 1, PQ[t], P2Q[t], PF[t]);
+      }
+    }
+    xb[0][lane] = pa;
+    xb[1][lane] = pb;
   }
-  // ---- back substitution, wave after wave downwards (new w over cA); the
-  // elimination coefficients of the wave's levels stayed in registers (ME, EE)
+  pass(&fwd_done, wave + 1);
+  if (!upper && Lq > 0) early();
+  if (Lq > 0) load_rrw();
+  // ---- back substitution, wave after wave downwards: CA becomes the new w
   wait_for(&back_next, wave);
-  {
-    if (Lq > 0) {
-      float wn = top ? 0.0f : xw[wave + 1][lane];
+  float wnext = 0.0f;
+  if (Lq > 0) {
+    if (!top) wnext = xw[lane];
+    float wn = wnext;
 #pragma unroll
-      for (int t = LMAX - 1; t >= 0; --t) {
-        const int k = k0 + t;
-        if (t < Lq) {
-          wn = k == nz - 1 ? EE[t] : (k >= 1 ? fma_(ME[t], wn, EE[t]) : 0.0f);
-          me0[k * 64 + lane] = wn;
-        }
+    for (int t = L - 1; t >= 0; --t)
+      if (ROW(t)) {
+        const float ca = AHEAD ? CA[t] : me0[(k0 + t) * 64 + lane], cb = AHEAD ? CB[t] : me1[(k0 + t) * 64 + lane];
+        wn = t >= L - 2 && k0 + t == nz - 1 ? cb : fma_(ca, wn, cb);
+        if (t == 0 && wave == 0) wn = 0.0f;  // level 0
+        CA[t] = wn;
+        // (the coefficients of a few rows in registers at a time)
+        if constexpr (!AHEAD)
+          if (t % 4 == 0) __builtin_amdgcn_sched_barrier(0);
       }
-      xw[wave][lane] = wn;
-    }
-    pass(&back_next, wave - 1);
+    xw[lane] = wn;
   }
-  // ---- acoustic_pp, the rru / rrv / rrw accumulation (acoustic_begin's
-  // values first on the stage's first substep), new w; the loads of 4 levels
-  // before their stores
-  if (active && Lq > 0) {
-    float *u = F(2), *v = F(3), *w = F(4), *pp3d = F(10), *ppd = F(11), *ppx = F(12), *rru = F(13), *rrv = F(14),
-          *rrw = F(15);
-    const float wnext = top ? 0.0f : xw[wave + 1][lane];
+  pass(&back_next, wave - 1);
+  // ---- acoustic_pp, the rrw accumulation, new w; CB keeps ppd, PF pp3d
 #pragma unroll
-    for (int t0 = 0; t0 < LMAX; t0 += 4) {
-      float RU[4], RV[4], RW[4], UU[4], VV[4], PV[4];
-#pragma unroll
-      for (int d = 0; d < 4; ++d)
-        if (t0 + d < Lq) {
-          const int64_t c = g.idx(i, j, k0 + t0 + d);
-          PV[d] = pp3d[c];
-          UU[d] = u[c];
-          VV[d] = v[c];
-          RU[d] = first ? 0.0f : rru[c];
-          RV[d] = first ? 0.0f : rrv[c];
-          RW[d] = first ? w[c] * ac.beta : rrw[c];
-        }
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const int t = t0 + d;
-        if (t < Lq) {
-          const int k = k0 + t;
-          const int64_t c = g.idx(i, j, k);
-          const float w0 = me0[k * 64 + lane];
-          const float w1 = t + 1 < Lq ? me0[(k + 1) * 64 + lane] : wnext;
-          float p = fma_(ac.alph, fma_(w0, PQ[t], w1 * P2Q[t]), PF[t]);
-          if (ab(p) < ac.smeps) p = 0.0f;
-          pp3d[c] = p;
-          const float dum1 = ac.kdiv * (p - PV[d]);
-          ppd[c] = p + dum1;
-          if (saveX) ppx[c] = dum1;
-          w[c] = w0;
-          rru[c] = acc(RU[d], UU[d]);
-          rrv[c] = acc(RV[d], VV[d]);
-          rrw[c] = accw(RW[d], w0);
-        }
+  for (int t = 0; t < L; ++t)
+    if (ROW(t)) {
+      const uint32_t o = at(k0 + t);
+      const float w0 = CA[t];
+      const float w1 = t == L - 1 || (t == L - 2 && !full) ? wnext : CA[t + 1 < L ? t + 1 : t];
+      float p = fma_(ac.alph, fma_(w0, PQ[t], w1 * P2Q[t]), PF[t]);
+      if (ab(p) < ac.smeps) p = 0.0f;
+      const float dum1 = ac.kdiv * (p - PP[t]);
+      PF[t] = p;
+      CB[t] = p + dum1;
+      if (active) {
+        pp3d.put(o, p);
+        ppd.put(o, CB[t]);
+        if (saveX) ppx.put(o, dum1);
+        w.put(o, w0);
+        rrw.put(o, accw(RW[t] * bf, w0));
       }
     }
-    if (top) {  // level nz: w stays 0 (acoustic_w_solve clears it); ppd there is not updated
-      const int64_t c = g.idx(i, j, nz);
-      const float uo = u[c], vo = v[c], ru = first ? 0.0f : rru[c], rv = first ? 0.0f : rrv[c];
-      const float rw = first ? w[c] * ac.beta : rrw[c];
-      w[c] = 0.0f;
-      rru[c] = acc(ru, uo);
-      rrv[c] = acc(rv, vo);
-      rrw[c] = accw(rw, 0.0f);
+  // ---- the halo cells' w, ppd and pp3d, lane = column: images of the row in
+  // y (dy rows away), of the column in x (dx columns), and both
+  const bool lo = i >= nx - 3, hi = i <= 3;
+#pragma unroll 1
+  for (int q = 1; q < 9; ++q) {
+    const int xi = q % 3, yi = q / 3;
+    const int dy = yi == 0 ? 0 : yi == 1 ? (j >= ny - 3 ? -ny : 0) : (j <= 3 ? ny : 0);
+    if (yi > 0 && dy == 0) continue;
+    const int dx = xi == 0 ? 0 : xi == 1 ? (lo ? -nx : hi ? nx : 0) : (lo && hi ? nx : 0);
+    if (!active || (xi > 0 && dx == 0)) continue;
+    const uint32_t h0 = at(k0) + (uint32_t)(4 * dx) + sjb * (uint32_t)dy;
+#pragma unroll
+    for (int t = 0; t < L; ++t)
+      if (ROW(t)) {
+        const uint32_t h = h0 + skb * (uint32_t)t;
+        w.put(h, CA[t]);
+        ppd.put(h, CB[t]);
+        if (imgP) pp3d.put(h, PF[t]);
+      }
+    if (top) {
+      const uint32_t h = h0 + skb * (uint32_t)Lq;
+      w.put(h, 0.0f);
+      ppd.put(h, ppdz);
+      if (imgP) pp3d.put(h, ppz);
     }
   }
-  // ---- halo cells of the wave's levels, after its own stores above
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  row_images(std::integral_constant<int, 7>());
-  halo(std::integral_constant<int, 7>());
+#undef ROW
 }
 // instantiations by levels per wave: the runtime picks the one with
 // ceil(nz / AC_WAVES) levels (k_ac_column: 16)
-__global__ __launch_bounds__(64 * AC_WAVES) void k_ac_column(uint32_t* M, KArg a) { ac_column<16>(M, a); }
-#define AC_INST(L) \
-  __global__ __launch_bounds__(64 * AC_WAVES) void k_ac_column##L(uint32_t* M, KArg a) { ac_column<L>(M, a); }
-AC_INST(1) AC_INST(2) AC_INST(3) AC_INST(4) AC_INST(5) AC_INST(6) AC_INST(7) AC_INST(8) AC_INST(9) AC_INST(10)
-AC_INST(11) AC_INST(12) AC_INST(13) AC_INST(14) AC_INST(15)
+#define AC_INST(L, name, waves) \
+  __global__ __launch_bounds__(64 * AC_WAVES) __attribute__((amdgpu_waves_per_eu(waves))) void name(uint32_t* M, KArg a) { ac_column<L>(M, a); }
+AC_INST(1, k_ac_column1, 4) AC_INST(2, k_ac_column2, 4) AC_INST(3, k_ac_column3, 4) AC_INST(4, k_ac_column4, 4)
+AC_INST(5, k_ac_column5, 4) AC_INST(6, k_ac_column6, 4) AC_INST(7, k_ac_column7, 6) AC_INST(8, k_ac_column8, 6)
+AC_INST(9, k_ac_column9, 6) AC_INST(10, k_ac_column10, 6) AC_INST(11, k_ac_column11, 6) AC_INST(12, k_ac_column12, 6)
+AC_INST(13, k_ac_column13, 4) AC_INST(14, k_ac_column14, 4) AC_INST(15, k_ac_column15, 4) AC_INST(16, k_ac_column, 4)
 #undef AC_INST
 
 const void* ac_column_kernel(int levels_per_wave) {

@@ -306,6 +306,17 @@ TE_DEV float fast_pow(float x, float p) {
   return f32_clear(exp((double)p * log((double)x)), f, 0x1p-32) ? f : rr_pow(x, p);
 }
 
+// recip without its range test, for recurrences that must not branch: the
+// same value where the bits of |x| lie within [2^-64, 2^64], that is where
+// recip_far(x) <= kRecipRange (zero and smaller x wrap around, infinities and
+// NaN lie above); a caller that meets another x takes recip.
+TE_DEV float recip_refined(float x) {
+  const float y = __builtin_amdgcn_rcpf(x);
+  return fma_(fma_(-x, y, 1.0f), y, y);
+}
+TE_DEV uint32_t recip_far(float x) { return (__float_as_uint(x) & 0x7fffffffu) - 0x1f800000u; }
+constexpr uint32_t kRecipRange = 0x5f800000u - 0x1f800000u;
+
 // 1 / x rounded to nearest even, for the tridiagonal recurrences' pivots:
 // the hardware reciprocal estimate (within 1 ulp) refined by one
 // Newton-Raphson step with an FMA residual (Markstein's reciprocal
@@ -317,8 +328,7 @@ TE_DEV float fast_pow(float x, float p) {
 TE_DEV float recip(float x) {
   const float a = __builtin_fabsf(x);
   if (!(a >= 0x1p-64f && a <= 0x1p64f)) return 1.0f / x;
-  const float y = __builtin_amdgcn_rcpf(x);
-  return fma_(fma_(-x, y, 1.0f), y, y);
+  return recip_refined(x);
 }
 
 // global thread ids of a 3-D launch

@@ -18,6 +18,7 @@ struct Op {
   int32_t kid;
   uint32_t A[64];
   int32_t nz = 0;  // levels of the op's grid (set before the first launch)
+  int32_t sJ = 0, sK = 0;  // its row and plane strides (set with nz)
   bool flat = false;  // launched flat over its words (set with nz)
   bool plane = false;  // launched over its (i, j) plane's points (set with nz)
   // launch shape chosen by te_autotune (generic 3-D kernels only)

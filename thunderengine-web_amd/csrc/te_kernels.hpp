@@ -32,6 +32,8 @@
 // Fused launches of 64 x AC_WAVES threads per workgroup (one acoustic
 // substep per launch, k_fused.hip).
 #define AC_WAVES 8
+// (row, 64 columns) pairs per wave of ac_column's accumulation of u and v
+#define AC_UV_UNITS 4
 #define TE_WIDE_LIST(X) X(ac_column)
 
 namespace te {

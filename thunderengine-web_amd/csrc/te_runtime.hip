@@ -134,13 +134,19 @@ static hipError_t launch(te_ctx* c, const Op& op) {
     const dim3 g((a.n[0] + 63) / 64, a.n[1], 1);
     if (!launch_shape(a, b, g)) return hipErrorInvalidConfiguration;
     const void* fn = ac_column_kernel((int)lw);
-    const size_t dyn = (size_t)2 * nz * 64 * sizeof(float);  // per level and lane: mm / cA / w and cB
+    // beyond 6 levels per wave the w rows wait in LDS: 2 floats per level and lane
+    const size_t dyn = lw > 6 ? (size_t)2 * nz * 64 * sizeof(float) : 0;
     if (dyn > 65536) {
       const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn);
       if (e != hipSuccess) return e;
     }
+    // then the workgroups that accumulate u and v (ac_accumulate_uv)
+    const uint64_t units = (uint64_t)op.sK * (nz + 1) * ((op.sJ + 63) / 64), per = AC_WAVES * AC_UV_UNITS;
+    const uint64_t uv = (units + per - 1) / per, all = (((uint64_t)a.lg[9] + 7) & ~7ull) + uv;
+    if (units >= (1ull << 31) || all >= (1ull << 31)) return hipErrorInvalidConfiguration;
+    a.n[2] = (uint32_t)uv;
     void* args[] = {(void*)&c->dM, (void*)&a};
-    return hipLaunchKernel(fn, g, b, args, dyn, c->stream);
+    return hipLaunchKernel(fn, dim3((uint32_t)all, 1, 1), b, args, dyn, c->stream);
   }
   if (a.n[2] == 1 && op.nz >= 4 && wave_sweep(op.kid)) {
     // 64 columns of a row per workgroup, AC_WAVES waves over the levels
@@ -404,6 +410,8 @@ static int grow_guards(te_ctx* c) {
     if (nz < 1 || sJ < 1 || sK < 1 || nz > 100000 || sJ > 100000 || sK > 100000)
       return fail(c, TE_ERR_ARG, std::string("op ") + te::kernel_name(op.kid) + ": invalid grid parameters");
     op.nz = nz;
+    op.sJ = sJ;
+    op.sK = sK;
     if (fl != flatOps.end()) {
       const bool wholeGrid = op.A[0] == (uint32_t)sJ && op.A[1] == (uint32_t)sK && op.A[2] == (uint32_t)(nz + 1);
       const bool words1d = std::strcmp(kn, "copy_fields") == 0 && op.A[1] == 1 && op.A[2] == 1;
@@ -419,6 +427,8 @@ static int grow_guards(te_ctx* c) {
     // the wave sweeps address a column within a level by a 32-bit byte offset
     if (te::wave_sweep(op.kid) && (uint64_t)sJ * sK >= (1ull << 30))
       return fail(c, TE_ERR_UNSUPPORTED, std::string(te::kernel_name(op.kid)) + ": a level spans 2^32 bytes or more");
+    if (std::strcmp(kn, "ac_column") == 0 && (uint64_t)sJ * sK * (uint64_t)(nz + 2) >= (1ull << 30))
+      return fail(c, TE_ERR_UNSUPPORTED, "ac_column: a field spans 2^32 bytes or more");
     need = std::max<uint64_t>(need, (uint64_t)sJ * sK * (uint64_t)(nz + 3));
     if (std::strcmp(kn, "adv_fused") == 0) {
       int32_t stag = 0, kind = 0;
