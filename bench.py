@@ -132,6 +132,14 @@ def alg_bytes_per_launch(run, names, A, op):
         io = [(1 + q, False, True) for q in range(3)] + [(4 + q, True, False) for q in range(3)]
     elif name == "adv_fused":
         io = adv_fused_io(run, A, op)
+    elif name == "adv_pdef":
+        io = ([(i, True, False) for i in (2, 4, 6, 7, 9, 13, 14, 15, 16, 30, 46)] +
+              [(i, False, True) for i in (11, 22, 23, 24, 43, 44, 45)])
+    elif name == "pdef_update":
+        flags = _flag(run, A, op, 17)
+        io = [(i, True, False) for i in (9, 10, 11, 16)]  # fluxes and operands of corrected cells only: not counted
+        io += ([(18, True, False)] if flags & 1 else [])
+        io += [(20, True, False), (21, False, True)] if flags & 2 else [(16, True, True)]
     elif name == "massflux_div":
         io = [(1, True, False), (2, True, False), (3, True, False), (6, False, True), (7, False, True),
               (8, False, True), (10, False, True)]

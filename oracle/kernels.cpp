@@ -83,6 +83,30 @@ static void fill_periodic(uint32_t* w, T* v, const uint32_t* A, uint32_t f) {
   call(find_kernel("bc_periodic_y"), ky);
 }
 
+// haloFill of a cell-centred field on a domain with open sides (flags ox, oy;
+// word `tmp` of memory carries the open passes' stagger argument, 0, and is
+// put back): the periodic passes, then the open ones.
+template <class T>
+static void fill_halo(uint32_t* w, T* v, const uint32_t* A, uint32_t f, bool ox, bool oy, uint32_t tmp) {
+  const uint32_t* dm = w + A[4];
+  const uint32_t nx = dm[0], ny = dm[1], nz = dm[2];
+  auto pass = [&](const char* kn, uint32_t other, bool open) {
+    uint32_t X[64] = {0};
+    X[0] = 4; X[1] = other + 7; X[2] = nz + 1;
+    X[4] = A[4]; X[5] = f; X[34] = A[34];
+    if (open) X[6] = tmp;
+    K<T> k1{w, v, X};
+    call(find_kernel(kn), k1);
+  };
+  if (!ox) pass("bc_periodic_x", ny, false);
+  if (!oy) pass("bc_periodic_y", nx, false);
+  const uint32_t keep = w[tmp];
+  w[tmp] = 0;
+  if (ox) pass("bc_open_x", ny, true);
+  if (oy) pass("bc_open_y", nx, true);
+  w[tmp] = keep;
+}
+
 template <class T>
 static int run_program(uint32_t* w, T* v, const char* const* names, const uint32_t* args, int nops, int first,
                        int last, char* err, int errlen) {
@@ -231,7 +255,35 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
       call(e1, k1); call(e2, k2);
       continue;
     }
-    if (nm == "adv_fused") {
+    if (nm == "pdef_update") {
+      // pdef_apply, then the SGS add (flag 1), rk_update and halo fill (flag 2)
+      auto P = [&](int q) { return A[4 + q]; };
+      auto run1 = [&](const char* kn, std::array<uint32_t, 3> g3, std::vector<std::pair<int, uint32_t>> ps) {
+        uint32_t X[64] = {0};
+        X[0] = g3[0]; X[1] = g3[1]; X[2] = g3[2];
+        X[4] = A[4]; X[34] = A[34];
+        for (auto& pr : ps) X[4 + pr.first] = pr.second;
+        K<T> k1{w, v, X};
+        call(find_kernel(kn), k1);
+      };
+      const uint32_t* dm = w + A[4];
+      const std::array<uint32_t, 3> full = {dm[0], dm[1], dm[2]}, whole = {dm[0] + 7, dm[1] + 7, dm[2] + 1};
+      std::vector<std::pair<int, uint32_t>> ps;
+      for (int q = 1; q <= 16; ++q) ps.push_back({q, P(q)});
+      run1("pdef_apply", full, ps);
+      const uint32_t flags = w[P(17)];
+      if (flags & 1u) run1("turb_add_tendency", whole, {{1, P(18)}, {2, P(16)}, {3, P(19)}});
+      if (flags & 2u) {
+        const uint32_t one = w[P(17)];
+        w[P(17)] = 1u;  // rk_update's stagger: a cell-centred field
+        run1("rk_update", full, {{1, P(17)}, {2, P(20)}, {3, P(16)}, {4, P(21)}, {5, P(14)}});
+        w[P(17)] = one;
+        fill_halo(w, v, A, P(21), w[P(15)] != 0u, w[P(15) + 1] != 0u, P(17));
+      }
+      continue;
+    }
+    if (nm == "adv_fused" || nm == "adv_pdef") {
+      const bool pd = nm == "adv_pdef";  // no chain; the three pdef_dum and two halo fills after the assembly
       // the three flux dispatches it stands for, then adv_assemble
       const uint32_t* dm = w + A[4];
       const uint32_t nx = dm[0], ny = dm[1], nz = dm[2];
@@ -270,7 +322,7 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
         K<T> k1{w, v, X};
         call(e1, k1);
       }
-      if (w[A[4 + 32]] & 16u) {  // turb_zero of the accumulating sink
+      if (!pd && (w[A[4 + 32]] & 16u)) {  // turb_zero of the accumulating sink
         uint32_t Z[64] = {0};
         Z[0] = nx + 7; Z[1] = ny + 7; Z[2] = nz + 1;
         Z[4] = A[4]; Z[5] = A[4 + 11]; Z[34] = A[34];
@@ -285,7 +337,7 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
       K<T> ka{w, v, Y};
       call(ea, ka);
       // the scalar follow-ups chained into the launch, as their own dispatches
-      const uint32_t chain = w[A[4 + 32]], TEND = A[4 + 11];
+      const uint32_t chain = pd ? 0u : w[A[4 + 32]], TEND = A[4 + 11];
       auto run1 = [&](const char* kn, const uint32_t* g3, std::vector<std::pair<int, uint32_t>> ps) {
         uint32_t X[64] = {0};
         X[0] = g3[0]; X[1] = g3[1]; X[2] = g3[2];
@@ -297,6 +349,17 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
         call(e1, k1);
       };
       const uint32_t full[3] = {nx, ny, nz}, whole[3] = {nx + 7, ny + 7, nz + 1}, asz[3] = {A[0], A[1], A[2]};
+      if (pd) {
+        const uint32_t F[3] = {FX, FY, FZ}, R[3] = {RU, RV, RW}, keep = w[ST];
+        for (uint32_t d = 0; d < 3; ++d) {
+          w[ST] = d;  // the direction argument
+          run1("pdef_dum", full, {{1, ST}, {2, S}, {3, A[4 + 46]}, {4, F[d]}, {5, R[d]}, {6, A[4 + 7]}, {7, A[4 + 9]},
+                                  {8, A[4 + 41]}, {9, A[4 + 17]}, {10, A[4 + 43 + d]}});
+        }
+        w[ST] = keep;
+        for (int d = 0; d < 2; ++d)
+          fill_halo(w, v, A, A[4 + 43 + d], w[A[4 + 17]] != 0u, w[A[4 + 17] + 1] != 0u, ST);
+      }
       if (chain & 1) run1("apply_thterm", full, {{1, A[4 + 33]}, {2, A[4 + 34]}, {3, TEND}});
       if (chain & 2) run1("turb_add_tendency", whole, {{1, A[4 + 35]}, {2, TEND}, {3, A[4 + 36]}});
       if (chain & 4) run1("turb_add_tendency", whole, {{1, A[4 + 37]}, {2, TEND}, {3, A[4 + 38]}});

@@ -280,7 +280,8 @@ __global__ __launch_bounds__(256) void k_pdef_dum(uint32_t* M, KArg a) {
 }
 // pdef_dum, then the halo fill of its output on a periodic domain (nx, ny >=
 // 4; timestep.js:1593 haloFill): each cell writes its periodic images.
-// Arguments as pdef_dum's.
+// Arguments as pdef_dum's.  The encoder emits k_adv_pdef instead; programs
+// recorded with this launch still replay.
 __global__ __launch_bounds__(256) void k_pdef_dum_xy(uint32_t* M, KArg a) {
   TE_TID3
   const Dims g = dims(a.q[0], 0);
@@ -311,19 +312,15 @@ TE_DEV float pdef_mass(float dm2, float dm1, float d0, float dp1, float dp2, boo
   return mass;
 }
 
-// pdef_apply.wgsl:207-282
-__global__ __launch_bounds__(256) void k_pdef_apply(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx, j = gy, k = gz;
-  if (i >= g.nx || j >= g.ny || k >= g.nz) return;
+// pdef_apply.wgsl:207-282: the corrected tendency of cell (i, j, k)
+TE_DEV float pdef_apply_at(uint32_t* M, const KArg& a, const Dims& g, int i, int j, int k) {
   const float *s = fq(a.q[1]), *s0 = fq(a.q[2]), *fx = fq(a.q[3]), *fy = fq(a.q[4]), *fz = fq(a.q[5]),
               *rru = fq(a.q[6]), *rrv = fq(a.q[7]), *rrw = fq(a.q[8]), *dx = fq(a.q[9]),
               *dy = fq(a.q[10]), *dz = fq(a.q[11]), *rho0 = fq(a.q[12]), *mh = fq(a.q[13]),
               *hm = fq(a.q[30]);
   float dt = ldf(a.q[14], 0);
   int openx = ldi(a.q[15], 0), openy = ldi(a.q[15], 1);
-  float* tend = fq(a.q[16]);
+  const float* tend = fq(a.q[16]);
   const int64_t sj = g.sJ, sk = g.sk(), c = g.idx(i, j, k);
   float rdt = 1.0f / dt;
   float base = rho0[k] * s0[c];
@@ -363,7 +360,50 @@ __global__ __launch_bounds__(256) void k_pdef_apply(uint32_t* M, KArg a) {
       delta = delta + (advNew - advOld);
     }
   }
-  tend[c] = t0 + delta / rho0[k];
+  return t0 + delta / rho0[k];
+}
+__global__ __launch_bounds__(256) void k_pdef_apply(uint32_t* M, KArg a) {
+  TE_TID3
+  const Dims g = dims(a.q[0], 0);
+  if (gx >= g.nx || gy >= g.ny || gz >= g.nz) return;
+  fq(a.q[16])[g.idx(gx, gy, gz)] = pdef_apply_at(M, a, g, gx, gy, gz);
+}
+
+// pdef_apply, the SGS tendency's add, rk_update and the halo fill of the
+// scalar in one launch: everything after the three dum fields is pointwise.
+// Arguments as pdef_apply's, with 17 -> flags (1 add, 2 rk_update and halo
+// fill; without 2 the tendency is stored), 18 the added tendency, 19 -> scale,
+// 20 phi_a, 21 phi (may be the advected field: it is read at the own cell
+// only), 15 -> open x, open y.
+// With k_adv_pdef this replaces the 9 launches of a scalar's last stage (10
+// with an SGS add, two more with an open side): three fluxes, the assembly,
+// three pdef_dum, pdef_apply, add, update, halo fills.  Those were bound by
+// their launches on small grids (3.2-4.5 us each at 64 x 64 x 40) and by their
+// passes over memory on large ones (10-18 us each at 192 x 192 x 80).  A step of
+// 64 x 64 x 40 with two such scalars went from 508 to 479 us, one of
+// 192 x 192 x 80 with TKE from 2980 to 2860.
+__global__ __launch_bounds__(256) void k_pdef_update(uint32_t* M, KArg a) {
+  TE_TID3
+  const Dims g = dims(a.q[0], 0);
+  const int i = gx, j = gy, k = gz;
+  if (i >= g.nx || j >= g.ny || k >= g.nz) return;
+  const int64_t c = g.idx(i, j, k), sk = g.sk();
+  const int flags = ldi(a.q[17], 0);
+  float* phi = fq(a.q[21]);
+  const bool top = (flags & 2) && k == g.nz - 1;
+  const float add = (flags & 1) ? fq(a.q[18])[c] : 0.0f, phi_a = (flags & 2) ? fq(a.q[20])[c] : 0.0f;
+  const float ptop = top ? phi[c + sk] : 0.0f;
+  float v = pdef_apply_at(M, a, g, i, j, k);
+  if (flags & 1) v = fma_(ldf(a.q[19], 0), add, v);
+  if (flags & 2) {
+    const bool openx = ldi(a.q[15], 0) != 0, openy = ldi(a.q[15], 1) != 0;
+    const float nv = fma_(ldf(a.q[14], 0), v, phi_a);
+    phi[c] = nv;
+    halo_from(g, openx, openy, phi, i, j, c, nv);
+    if (top) halo_from(g, openx, openy, phi, i, j, c + sk, ptop);
+  } else {
+    fq(a.q[16])[c] = v;
+  }
 }
 
 }  // namespace te

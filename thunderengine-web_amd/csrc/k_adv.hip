@@ -544,7 +544,9 @@ struct FusedFlux {
   }
 };
 
-template <int KIND, int STC>
+// PD: the fluxes of a positive-definite scalar (stagger 1) with its three
+// partial updates (pdef_dum.wgsl:177-231, see k_adv_pdef).
+template <int KIND, int STC, bool PD = false>
 __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
   // launched as 64 x Y x Z blocks (Y * Z <= 4; runtime launch(), te_autotune):
   // a wave is one row of cells, so j and k are wave-uniform and branches on
@@ -569,7 +571,7 @@ __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
   const FacePre pyl = F.template pre<1>(k, cy), pyh = F.template pre<1>(k, cy + sj);
   const FacePre pzl = F.template pre<2>(zlo, cz), pzh = F.template pre<2>(zlo + 1, cz + sk);
   const AsmPre P = asm_pre<STC>(a, g, c);
-  const int chain = ldi(a.q[32], 0), acc = ldi(a.q[12], 0);
+  const int chain = PD ? 0 : ldi(a.q[32], 0), acc = PD ? 0 : ldi(a.q[12], 0);
   float* tend = fq(a.q[11]);
   const float t_old = (chain & 16) == 0 && acc != 0 ? tend[c] : 0.0f;
   const float d3 = (chain & 1) ? fq(a.q[33])[c] : 0.0f, th3 = (chain & 1) ? fq(a.q[34])[c] : 0.0f;
@@ -581,6 +583,34 @@ __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
   const float fxl = F.template eval<0>(pxl, xlo, j, k), fxh = F.template eval<0>(pxh, xlo + 1, j, k);
   const float fyl = F.template eval<1>(pyl, i, ylo, k), fyh = F.template eval<1>(pyh, i, ylo + 1, k);
   const float fzl = F.template eval<2>(pzl, i, j, zlo), fzh = F.template eval<2>(pzh, i, j, zlo + 1);
+  if (PD) {
+    // each cell stores its low faces, the last ones their high face too
+    float *fx = fq(a.q[22]), *fy = fq(a.q[23]), *fz = fq(a.q[24]);
+    fx[c] = fxl;
+    fy[c] = fyl;
+    fz[c] = fzl;
+    if (i == g.nx - 1) fx[c + 1] = fxh;
+    if (j == g.ny - 1) fy[c + sj] = fyh;
+    if (k == g.nz - 1) fz[c + sk] = fzh;
+    const float* hm = fq(a.q[30]);
+    const bool openx = ldi(a.q[17], 0) != 0, openy = ldi(a.q[17], 1) != 0;
+    const float dt = ldf(a.q[41], 0), base = fq(a.q[7])[k] * fq(a.q[46])[c];
+    auto dum = [&](bool inflow, float lo, float hi, float rlo, float rhi, float rd, float m) {
+      const float adv = ((-(hi - lo)) * rd) * m, sdiv = ((P.s * (rhi - rlo)) * rd) * m;
+      return inflow ? base : fma_(dt, adv + sdiv, base);
+    };
+    const bool inx = openx && ((i == 0 && pxl.a >= 0.0f) || (i == g.nx - 1 && pxh.a <= 0.0f));
+    const bool iny = openy && ((j == 0 && pyl.a >= 0.0f) || (j == g.ny - 1 && pyh.a <= 0.0f));
+    const float dx = dum(inx, fxl, fxh, pxl.a, pxh.a, g.rdx, hm_uh(hm, g, i));
+    const float dy = dum(iny, fyl, fyh, pyl.a, pyh.a, g.rdy, hm_vh(hm, g, j));
+    const float dz = dum(false, fzl, fzh, pzl.a, pzh.a, g.rdz, fq(a.q[9])[k]);
+    float *ox = fq(a.q[43]), *oy = fq(a.q[44]);
+    ox[c] = dx;
+    oy[c] = dy;
+    fq(a.q[45])[c] = dz;
+    halo_from(g, openx, openy, ox, i, j, c, dx);
+    halo_from(g, openx, openy, oy, i, j, c, dy);
+  }
   // p[32] -> chain flags: the pointwise dispatches around a field's assembly
   // in the reference, applied to the tendency in registers:
   // 16 turb_zero of the accumulating sink before it (tend = 0 + t),
@@ -639,6 +669,24 @@ const void* adv_fused_kernel(int kind, int stag) {
   if (kind == 2 && stag == 4) return (const void*)&k_adv_fused_v<2, 4>;
   if (kind == 3 && stag == 4) return (const void*)&k_adv_fused_v<3, 4>;
   return nullptr;
+}
+
+// A positive-definite scalar's fluxes, adv_assemble and its three pdef_dum
+// dispatches with the halo fill of the first two: a cell that has its six
+// faces in registers forms its three partial updates from them.  k_pdef_update
+// reads the result.  Parameters as adv_fused's (no chain), with 22-24 the
+// fluxes (written: a corrected cell reads its old ones), 41 -> dt, 43-45 the
+// partial updates, 46 the start-of-step field, 17 -> open x, open y.
+template <int KIND>
+__global__ __launch_bounds__(256) void k_adv_pdef_v(uint32_t* M, KArg a) {
+  adv_fused_body<KIND, 1, true>(M, a);
+}
+const void* adv_pdef_kernel(int kind) {
+  return kind == 0 ? (const void*)&k_adv_pdef_v<0> : kind == 1 ? (const void*)&k_adv_pdef_v<1> : nullptr;
+}
+__global__ __launch_bounds__(256) void k_adv_pdef(uint32_t* M, KArg a) {
+  if (ldi(a.q[3], 0) == 0) adv_fused_body<0, 1, true>(M, a);
+  else adv_fused_body<1, 1, true>(M, a);
 }
 
 // The three flux dispatches of one advected field and adv_assemble in one

@@ -98,6 +98,38 @@ TE_DEV void update_with_images(const Dims& g, float* f, int i, int j, int k, int
     if (hi) f[c + sk + o] = fhi;
   });
 }
+// The halo cells of a level that a haloFill of a cell-centred field gives the
+// value v of interior cell (i, j) (index c), written by that cell (nx, ny >= 4).
+// A periodic axis copies from the image modulo n, an open one from the nearest
+// cell for the three cells past either end (bc_open_x.wgsl:111-131).  The
+// fourth column or row past the open east or north end is filled by no pass
+// along its own axis, but the passes along the other axis copy it too, from
+// the words as they are.  No thread of the launch may read the field's halo.
+TE_DEV void halo_from(const Dims& g, bool openx, bool openy, float* f, int i, int j, int64_t c, float v) {
+  const int nX = openx ? (i == 0 || i == g.nx - 1 ? 4 : 1) : 1 + (i >= g.nx - 3) + (i <= 3);
+  const int nY = openy ? (j == 0 || j == g.ny - 1 ? 4 : 1) : 1 + (j >= g.ny - 3) + (j <= 3);
+  if (nX == 1 && nY == 1) return;
+  const int64_t sj = g.sJ;
+  auto ox = [&](int a) -> int64_t {
+    if (openx) return i == 0 ? -a : a;
+    return a == 0 ? 0 : (a == 1 && i >= g.nx - 3 ? -g.nx : g.nx);
+  };
+  auto oy = [&](int b) -> int64_t {
+    if (openy) return (j == 0 ? -b : b) * sj;
+    return b == 0 ? 0 : (b == 1 && j >= g.ny - 3 ? -g.ny : g.ny) * sj;
+  };
+  for (int b = 0; b < nY; ++b)
+    for (int a = 0; a < nX; ++a)
+      if (a != 0 || b != 0) f[c + ox(a) + oy(b)] = v;
+  if (openx && i == g.nx - 1 && nY > 1) {
+    const float e = f[c + 4];
+    for (int b = 1; b < nY; ++b) f[c + 4 + oy(b)] = e;
+  }
+  if (openy && j == g.ny - 1 && nX > 1) {
+    const float e = f[c + 4 * sj];
+    for (int a = 1; a < nX; ++a) f[c + 4 * sj + ox(a)] = e;
+  }
+}
 // GridDims bytes: nx ny nz strideJ strideK 1/dx 1/dy 1/dz (timestep.js:88-90).
 TE_DEV Dims dims(const uint32_t* M, uint32_t o) {
   Dims g;

@@ -263,6 +263,9 @@ class Encoder {
   void afterAssemble(int nrk, const std::string& s, int stagger, const std::string& into, bool accumulate,
                      const std::string& target, const std::array<int, 3>& asmSize, const Bytes& dttmp,
                      const Bytes& open);
+  void advectPdef(int nrk, const std::string& target, const Bytes& dttmp, const Bytes& open);
+  void sgsAndUpdate(int nrk, int stagger, const std::string& target, const std::array<int, 3>& asmSize,
+                    const Bytes& dttmp);
   void stages();
   void end();
 };
@@ -542,6 +545,10 @@ void Encoder::advect(int nrk, const std::string& s, int stagger, const std::stri
   const std::string target = state.empty() ? s : state;
   const std::array<int, 3> asmSize{nx + (stagger == 2 ? 1 : 0), ny + (stagger == 3 ? 1 : 0), nz};
   const bool pdefAfter = !accumulate && stagger == 1 && moist && nrk == 2 && target != scalars[0];
+  if (pdefAfter && cfg.fuse == 1) {
+    advectPdef(nrk, target, dttmp, open);
+    return;
+  }
   const bool wenoUVm = (stagger == 2 || stagger == 3) && wenoM && nrk == 2;
   if (cfg.fuse != 0 && !pdefAfter && !wenoUVm) {
     // fluxes + assembly in one launch (pdef needs the fluxes in memory; the
@@ -642,6 +649,39 @@ void Encoder::advect(int nrk, const std::string& s, int stagger, const std::stri
   afterAssemble(nrk, s, stagger, into, accumulate, target, asmSize, dttmp, open);
 }
 
+// The last stage of a positive-definite scalar, fuse = 1: k_adv_pdef, then
+// k_pdef_update with the SGS add, the RK update and the halo fill unless
+// something else adds to the tendency in between (advect's rule for a chain).
+void Encoder::advectPdef(int nrk, const std::string& target, const Bytes& dttmp, const Bytes& open) {
+  const std::array<int, 3> full{cfg.nx, cfg.ny, cfg.nz};
+  const bool weno = wenoS;
+  const bool moistSgs = tke, chained = (!moistSgs || cacheMT) && !(hasMicro && usePT);
+  std::vector<Bind> bs = {bb(1, I1(1)), fb(2, target), bb(3, I1(weno ? 1 : 0)), fb(4, "rrw"),
+                          bb(5, F1(weno ? wenoEps(target) : 0.0f)), fb(6, "divx"), rb(7, "rho0"), rb(8, "rf0"),
+                          rb(9, "mh"), rb(10, "mf"), fb(11, "tend"), bb(12, I1(0)), fb(13, "rru"), fb(14, "rrv"),
+                          rb(15, "c1"), rb(16, "c2"), bb(17, open), rb(18, "rr0"), fb(19, "tend"),
+                          bb(20, I1(weno ? 1 : 0)), bb(21, I1(weno && target != "qv" ? 1 : 0)), fb(22, "fx"),
+                          fb(23, "fy"), fb(24, "fz"), bb(27, F1(0.0f)), bb(41, dttmp), fb(43, "pk1"), fb(44, "pk2"),
+                          fb(45, "fpk"), fb(46, target + "_a")};
+  op("adv_pdef", full, {});
+  for (const Bind& bd : bs) E.ops.back().A[4 + bd.idx] = (uint32_t)bd.off;
+  const bool add = chained && moistSgs;
+  bs = {fb(1, target), fb(2, target + "_a"), fb(3, "fx"), fb(4, "fy"), fb(5, "fz"), fb(6, "rru"), fb(7, "rrv"),
+        fb(8, "rrw"), fb(9, "pk1"), fb(10, "pk2"), fb(11, "fpk"), rb(12, "rho0"), rb(13, "mh"), bb(14, dttmp),
+        bb(15, open), fb(16, "tend"), bb(17, I1((add ? 1 : 0) | (chained ? 2 : 0)))};
+  if (add) {
+    bs.push_back(fb(18, "qturb_" + target));
+    bs.push_back(bb(19, F1(1.0f)));
+  }
+  if (chained) {
+    bs.push_back(fb(20, target + "_a"));
+    bs.push_back(fb(21, target));
+  }
+  op("pdef_update", full, {});
+  for (const Bind& bd : bs) E.ops.back().A[4 + bd.idx] = (uint32_t)bd.off;
+  if (!chained) sgsAndUpdate(nrk, 1, target, full, dttmp);
+}
+
 void Encoder::advectFluxes(int nrk, const std::string& s, int stagger, const std::string& target) {
   const int nx = cfg.nx, ny = cfg.ny, nz = cfg.nz;
   const std::array<int, 3> fullU{nx + 1, ny, nz}, fullV{nx, ny + 1, nz}, fullW{nx, ny, nz + 1};
@@ -709,25 +749,30 @@ void Encoder::moistureTurbulence(int nrk, const std::string& target) {
 void Encoder::afterAssemble(int nrk, const std::string& s, int stagger, const std::string& into, bool accumulate,
                             const std::string& target, const std::array<int, 3>& asmSize, const Bytes& dttmp,
                             const Bytes& open) {
-  const int nx = cfg.nx, ny = cfg.ny, nz = cfg.nz;
-  const std::array<int, 3> full{nx, ny, nz}, whole{nx + 7, ny + 7, nz + 1}, stag{nx + 1, ny + 1, nz}, cols{nx, ny, 1};
   if (accumulate) return;
   if (stagger == 1 && moist && nrk == 2 && target != scalars[0]) {
     const std::string s0 = target + "_a";
     const char* names[3][3] = {{"fx", "rru", "pk1"}, {"fy", "rrv", "pk2"}, {"fz", "rrw", "fpk"}};
     for (int dd = 0; dd < 3; ++dd)
-      op(foldHalo && dd < 2 ? "pdef_dum_xy" : "pdef_dum", asmSize,
+      op("pdef_dum", asmSize,
          {bb(1, I1(dd)), fb(2, s), fb(3, s0), fb(4, names[dd][0]), fb(5, names[dd][1]), rb(6, "rho0"), rb(7, "mh"),
           bb(8, dttmp), bb(9, open), fb(10, names[dd][2])});
-    if (!foldHalo) {
-      haloFill("pk1");
-      haloFill("pk2");
-    }
+    haloFill("pk1");
+    haloFill("pk2");
     op("pdef_apply", asmSize,
        {fb(1, s), fb(2, s0), fb(3, "fx"), fb(4, "fy"), fb(5, "fz"), fb(6, "rru"), fb(7, "rrv"), fb(8, "rrw"),
         fb(9, "pk1"), fb(10, "pk2"), fb(11, "fpk"), rb(12, "rho0"), rb(13, "mh"), bb(14, dttmp), bb(15, open),
         fb(16, "tend")});
   }
+  sgsAndUpdate(nrk, stagger, target, asmSize, dttmp);
+}
+
+// The SGS and microphysics adds of a scalar's tendency, its RK update and the
+// halo fill.
+void Encoder::sgsAndUpdate(int nrk, int stagger, const std::string& target, const std::array<int, 3>& asmSize,
+                           const Bytes& dttmp) {
+  const int nx = cfg.nx, ny = cfg.ny, nz = cfg.nz;
+  const std::array<int, 3> full{nx, ny, nz}, whole{nx + 7, ny + 7, nz + 1};
   if (moist && target == scalars[0]) op("apply_thterm", full, {fb(1, "div3d"), fb(2, "thterm"), fb(3, "tend")});
   if ((tke || rayleigh) && target == scalars[0])
     op("turb_add_tendency", whole, {fb(1, "thten_t"), fb(2, "tend"), bb(3, F1(1.0f))});

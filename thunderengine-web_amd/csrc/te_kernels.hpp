@@ -27,7 +27,7 @@
 #define TE_FUSED_LIST(X) X(bc_periodic_xy) X(zero_fields) X(copy_fields) X(ac_pp_accumulate) \
   X(adv_fused) X(add_fields) X(tendency_reset_add) X(acoustic_w_solve_lds) X(turb_scalar_vert_implicit_lds) X(turb_u_tendency_lds) \
   X(turb_v_tendency_lds) X(turb_w_tendency_lds) X(tke_transport_lds) X(rk_update_xy) X(tke_advance_xy) \
-  X(pdef_dum_xy) X(ppx_finish_xy) X(turb_km_kh_xy) X(massflux_div) X(bc_open_xy)
+  X(pdef_dum_xy) X(ppx_finish_xy) X(turb_km_kh_xy) X(massflux_div) X(bc_open_xy) X(adv_pdef) X(pdef_update)
 
 // Fused launches of 64 x AC_WAVES threads per workgroup (one acoustic
 // substep per launch, k_fused.hip).
@@ -51,6 +51,7 @@ const void* svi_waves_kernel(int levels_per_wave);
 // adv_fused specialised on (flux kind, stagger) (k_adv.hip); null for the
 // pairs only the run-time dispatch of k_adv_fused serves
 const void* adv_fused_kernel(int kind, int stag);
+const void* adv_pdef_kernel(int kind);
 // turb_u_tendency_lds (dir 0) / turb_v_tendency_lds (dir 1) in the same form
 const void* uv_waves_kernel(int dir, int levels_per_wave);
 // turb_w_tendency_lds (which 0) / tke_transport_lds (which 1): levels 1 .. nz-1

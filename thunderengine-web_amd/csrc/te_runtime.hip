@@ -109,6 +109,11 @@ static bool wave_sweep(int kid) {
     if (kid == id) return true;
   return false;
 }
+// Launched as 64 x Y x Z blocks, a wave per row of cells (adv_fused_body).
+static bool row_waves(int kid) {
+  static const int kAdvFused = kernel_id("adv_fused"), kAdvPdef = kernel_id("adv_pdef");
+  return kid == kAdvFused || kid == kAdvPdef;
+}
 static uint32_t column_lanes() {
   static uint32_t lanes = [] {
     const char* e = std::getenv("TE_COLUMN_LANES");
@@ -123,8 +128,8 @@ static hipError_t launch(te_ctx* c, const Op& op) {
   for (int q = 0; q < 48; ++q) a.q[q] = c->dM + a.p[q];
   if (a.n[0] == 0 || a.n[1] == 0 || a.n[2] == 0) return hipSuccess;
   dim3 b = block_for(a.n);
-  static const int kAdvFused = kernel_id("adv_fused"), kTkeEpst = kernel_id("tke_epst");
-  if (op.kid == kAdvFused) b = dim3(64, 4, 1);  // one row of cells per wave (k_adv_fused)
+  static const int kTkeEpst = kernel_id("tke_epst");
+  if (row_waves(op.kid)) b = dim3(64, 4, 1);  // one row of cells per wave (k_adv_fused)
   if (op.kid == kTkeEpst) a.n[2] = (a.n[2] + 1) / 2;  // two levels per thread (k_tke_epst)
   static const int kAcColumn = kernel_id("ac_column");
   if (op.kid == kAcColumn) {  // 64 columns of a row per workgroup, AC_WAVES waves over the levels
@@ -304,6 +309,12 @@ static int validate_ops(te_ctx* c) {
           return fail(c, TE_ERR_ARG, "copy_fields op " + std::to_string(i) + " leaves the memory");
     for (int q = 0; q < 48; ++q)
       if (op.A[4 + q] >= c->words) return fail(c, TE_ERR_ARG, "op " + std::to_string(i) + " (" + nm + ") parameter offset outside memory");
+    if (std::strcmp(nm, "adv_pdef") == 0) {  // likewise its tendency, fluxes and partial updates
+      for (int w : {11, 22, 23, 24, 43, 44, 45})
+        for (int r : {2, 4, 13, 14})
+          if (op.A[4 + w] == op.A[4 + r])
+            return fail(c, TE_ERR_ARG, "adv_pdef op " + std::to_string(i) + " writes a field its stencil reads");
+    }
     if (std::strcmp(nm, "adv_fused") == 0) {
       // the fields a fused advection writes (tendency, chained update) must
       // not be ones its workgroups read at neighbouring points
@@ -361,7 +372,7 @@ static int ctx_alloc(te_ctx* c, uint64_t words) {
 // kernels that map threads themselves (columns, fused advection, copies)
 static const std::set<std::string>& own_mapping() {
   static const std::set<std::string> s = {
-      "acoustic_w_solve", "acoustic_w_solve_lds", "adv_fused", "_copy", "copy_fields", "turb_sfcstress",
+      "acoustic_w_solve", "acoustic_w_solve_lds", "adv_fused", "adv_pdef", "_copy", "copy_fields", "turb_sfcstress",
       "turb_u_tendency", "turb_u_tendency_lds", "turb_v_tendency", "turb_v_tendency_lds", "turb_w_tendency",
       "turb_w_tendency_lds", "turb_scalar_vert_implicit", "turb_scalar_vert_implicit_lds", "tke_transport",
       "tke_transport_lds", "ac_column"};
@@ -435,6 +446,11 @@ static int grow_guards(te_ctx* c) {
       TE_HIP(hipMemcpy(&stag, c->dM + op.A[4 + 1], 4, hipMemcpyDeviceToHost), "read stagger");
       TE_HIP(hipMemcpy(&kind, c->dM + op.A[4 + 3], 4, hipMemcpyDeviceToHost), "read flux kind");
       op.fn = te::adv_fused_kernel(kind, stag);
+    }
+    if (std::strcmp(kn, "adv_pdef") == 0) {
+      int32_t kind = 0;
+      TE_HIP(hipMemcpy(&kind, c->dM + op.A[4 + 3], 4, hipMemcpyDeviceToHost), "read flux kind");
+      op.fn = te::adv_pdef_kernel(kind);
     }
     if (std::strcmp(te::kernel_name(op.kid), "turb_sfcstress") == 0) {
       int32_t mode = 0;
@@ -639,12 +655,11 @@ int te_autotune(te_ctx* c, int32_t reps, int32_t force) {
   // dispatches on the generic 3-D path: not the column sweeps, the fused
   // advection or the flat copies, which fix their own thread mapping
   // (adv_fused too, among the shapes that keep one row of cells per wave)
-  static const int kAdvFused = te::kernel_id("adv_fused");
   std::vector<char> eligible(n, 0), planeOk(n, 0);
   for (int i = 0; i < n; ++i) {
     const te::Op& op = c->ops[i];
     const char* kn = te::kernel_name(op.kid);
-    if (op.flat || (own_mapping().count(kn) && op.kid != kAdvFused) ||
+    if (op.flat || (own_mapping().count(kn) && !te::row_waves(op.kid)) ||
         (op.A[2] == 1 && te::is_column_kernel(op.kid)))
       continue;
     if (op.A[0] == 0 || op.A[1] == 0 || op.A[2] == 0) continue;
@@ -666,10 +681,10 @@ int te_autotune(te_ctx* c, int32_t reps, int32_t force) {
     const te::Op& op = c->ops[i];
     if (sh.plane) {
       const uint64_t pts = (uint64_t)op.A[0] * op.A[1];
-      return op.kid != kAdvFused && planeOk[i] != 0 && grid_ok((pts + 255) / 256, op.A[2], 1);
+      return !te::row_waves(op.kid) && planeOk[i] != 0 && grid_ok((pts + 255) / 256, op.A[2], 1);
     }
     if (!grid_ok((op.A[0] + sh.x - 1) / sh.x, (op.A[1] + sh.y - 1) / sh.y, (op.A[2] + sh.z - 1) / sh.z)) return false;
-    if (op.kid == kAdvFused) return sh.x == 64 && sh.y * sh.z <= 4;
+    if (te::row_waves(op.kid)) return sh.x == 64 && sh.y * sh.z <= 4;
     return sh.x <= std::max<uint32_t>(64, p2(op.A[0])) && sh.y <= p2(op.A[1]) && sh.z <= p2(op.A[2]);
   };
   const std::vector<te::Op> base = c->ops;  // shapes as the context had them
