@@ -115,19 +115,24 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
     std::string nm(names[o]);
     {
       // the library's pointwise updates with the halo fill of their output
-      // folded in: the update, then bc_periodic_x and bc_periodic_y of the
+      // folded in: the update, then haloFill (bc_periodic_x, bc_periodic_y, or
+      // the open passes of the sides that parameter `open` names) of the
       // field it writes (parameter slot of that field)
-      struct Folded { const char* name; int out[4]; int n; };
-      static const Folded kFolded[] = {{"rk_update_xy", {4}, 1},    {"tke_advance_xy", {4}, 1},
-                                       {"pdef_dum_xy", {10}, 1},    {"ppx_finish_xy", {2}, 1},
-                                       {"turb_km_kh_xy", {4, 5, 6, 7}, 4}};
+      struct Folded { const char* name; int out[4]; int n, open; };
+      static const Folded kFolded[] = {{"rk_update_xy", {4}, 1, 6},    {"tke_advance_xy", {4}, 1, 5},
+                                       {"pdef_dum_xy", {10}, 1, 0},    {"ppx_finish_xy", {2}, 1, 3},
+                                       {"turb_km_kh_xy", {4, 5, 6, 7}, 4, 0}};
       const Folded* fo = nullptr;
       for (const auto& f : kFolded)
         if (nm == f.name) fo = &f;
       if (fo) {
         K<T> k1{w, v, A};
         call(find_kernel(nm.substr(0, nm.size() - 3)), k1);
-        for (int q = 0; q < fo->n; ++q) fill_periodic(w, v, A, A[4 + fo->out[q]]);
+        const uint32_t so = fo->open ? A[4 + fo->open] : 0;  // -> open x, open y; 0: none bound
+        for (int q = 0; q < fo->n; ++q) {
+          if (so == 0) fill_periodic(w, v, A, A[4 + fo->out[q]]);
+          else fill_halo(w, v, A, A[4 + fo->out[q]], w[so] != 0u, w[so + 1] != 0u, so + 1);
+        }
         continue;
       }
     }
@@ -364,7 +369,7 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
       if (chain & 2) run1("turb_add_tendency", whole, {{1, A[4 + 35]}, {2, TEND}, {3, A[4 + 36]}});
       if (chain & 4) run1("turb_add_tendency", whole, {{1, A[4 + 37]}, {2, TEND}, {3, A[4 + 38]}});
       if (chain & 8) run1("rk_update", asz, {{1, A[4 + 1]}, {2, A[4 + 39]}, {3, TEND}, {4, A[4 + 40]}, {5, A[4 + 41]}});
-      if (chain & 32) fill_periodic(w, v, A, A[4 + 40]);  // the updated field's halo fill, folded in
+      if (chain & 32) fill_halo(w, v, A, A[4 + 40], w[A[4 + 17]] != 0u, w[A[4 + 17] + 1] != 0u, A[4 + 17]);  // the updated field's halo fill, folded in
       if (chain & 64) {  // buoyancy_apply on the assembled tendency of w
         const uint32_t bg[3] = {nx, ny, std::max<uint32_t>(nz - 1, 1)};
         run1("buoyancy_apply", bg, {{1, A[4 + 42]}, {2, A[4 + 15]}, {3, A[4 + 16]}, {4, TEND}});

@@ -287,7 +287,7 @@ __global__ __launch_bounds__(256) void k_pdef_dum_xy(uint32_t* M, KArg a) {
   const Dims g = dims(a.q[0], 0);
   const int i = gx, j = gy, k = gz;
   if (i >= g.nx || j >= g.ny || k >= g.nz) return;
-  update_with_images(g, fq(a.q[10]), i, j, k, 0, g.nz, [&](int64_t c) { return pdef_dum_at(M, a, g, i, j, k, c); });
+  update_with_halo(g, {false, false}, fq(a.q[10]), i, j, k, 0, [&](int64_t c) { return pdef_dum_at(M, a, g, i, j, k, c); });
 }
 
 struct PdefCell { bool neg; float f1, f2, foo3; };
@@ -381,29 +381,27 @@ __global__ __launch_bounds__(256) void k_pdef_apply(uint32_t* M, KArg a) {
 // their launches on small grids (3.2-4.5 us each at 64 x 64 x 40) and by their
 // passes over memory on large ones (10-18 us each at 192 x 192 x 80).  A step of
 // 64 x 64 x 40 with two such scalars went from 508 to 479 us, one of
-// 192 x 192 x 80 with TKE from 2980 to 2860.
+// 192 x 192 x 80 with TKE from 3277 to 3145.
+template <bool OPEN>
+TE_DEV void pdef_update_at(uint32_t* M, const KArg& a, const Dims& g, Sides open, int i, int j, int k) {
+  const int64_t c = g.idx(i, j, k);
+  const int flags = ldi(a.q[17], 0);
+  float* phi = fq(a.q[21]);
+  HaloCell h{};
+  if (flags & 2) h = halo_cell<OPEN>(g, open, phi, i, j, k, 0, c);
+  const float add = (flags & 1) ? fq(a.q[18])[c] : 0.0f, phi_a = (flags & 2) ? fq(a.q[20])[c] : 0.0f;
+  float v = pdef_apply_at(M, a, g, i, j, k);
+  if (flags & 1) v = fma_(ldf(a.q[19], 0), add, v);
+  if (flags & 2) halo_put<OPEN>(g, open, phi, i, j, c, fma_(ldf(a.q[14], 0), v, phi_a), h);
+  else fq(a.q[16])[c] = v;
+}
 __global__ __launch_bounds__(256) void k_pdef_update(uint32_t* M, KArg a) {
   TE_TID3
   const Dims g = dims(a.q[0], 0);
-  const int i = gx, j = gy, k = gz;
-  if (i >= g.nx || j >= g.ny || k >= g.nz) return;
-  const int64_t c = g.idx(i, j, k), sk = g.sk();
-  const int flags = ldi(a.q[17], 0);
-  float* phi = fq(a.q[21]);
-  const bool top = (flags & 2) && k == g.nz - 1;
-  const float add = (flags & 1) ? fq(a.q[18])[c] : 0.0f, phi_a = (flags & 2) ? fq(a.q[20])[c] : 0.0f;
-  const float ptop = top ? phi[c + sk] : 0.0f;
-  float v = pdef_apply_at(M, a, g, i, j, k);
-  if (flags & 1) v = fma_(ldf(a.q[19], 0), add, v);
-  if (flags & 2) {
-    const bool openx = ldi(a.q[15], 0) != 0, openy = ldi(a.q[15], 1) != 0;
-    const float nv = fma_(ldf(a.q[14], 0), v, phi_a);
-    phi[c] = nv;
-    halo_from(g, openx, openy, phi, i, j, c, nv);
-    if (top) halo_from(g, openx, openy, phi, i, j, c + sk, ptop);
-  } else {
-    fq(a.q[16])[c] = v;
-  }
+  if (gx >= g.nx || gy >= g.ny || gz >= g.nz) return;
+  const Sides open = open_sides(a, 15);
+  if (open.x || open.y) pdef_update_at<true>(M, a, g, open, gx, gy, gz);
+  else pdef_update_at<false>(M, a, g, open, gx, gy, gz);
 }
 
 }  // namespace te

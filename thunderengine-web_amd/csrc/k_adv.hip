@@ -546,7 +546,8 @@ struct FusedFlux {
 
 // PD: the fluxes of a positive-definite scalar (stagger 1) with its three
 // partial updates (pdef_dum.wgsl:177-231, see k_adv_pdef).
-template <int KIND, int STC, bool PD = false>
+// OPEN: the launch's halo fill may meet an open side.
+template <int KIND, int STC, bool OPEN, bool PD = false>
 __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
   // launched as 64 x Y x Z blocks (Y * Z <= 4; runtime launch(), te_autotune):
   // a wave is one row of cells, so j and k are wave-uniform and branches on
@@ -577,6 +578,14 @@ __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
   const float d3 = (chain & 1) ? fq(a.q[33])[c] : 0.0f, th3 = (chain & 1) ? fq(a.q[34])[c] : 0.0f;
   const float add1 = (chain & 2) ? fq(a.q[35])[c] : 0.0f, add2 = (chain & 4) ? fq(a.q[37])[c] : 0.0f;
   const float phi_a = (chain & 8) ? fq(a.q[39])[c] : 0.0f;
+  const Sides open = open_sides(a, 17);
+  HaloCell hc{};
+  if ((chain & 40) == 40) hc = halo_cell<OPEN>(g, open, fq(a.q[40]), i, j, k, 0, c);
+  HaloOwn hx{}, hy{};
+  if (PD) {
+    hx = halo_own<OPEN>(g, open, fq(a.q[43]), i, j, c);
+    hy = halo_own<OPEN>(g, open, fq(a.q[44]), i, j, c);
+  }
   const bool buoy = (chain & 64) && k >= 1 && k <= g.nz - 1;
   const float bm = buoy ? fq(a.q[42])[c - sk] : 0.0f, b0 = buoy ? fq(a.q[42])[c] : 0.0f;
   const float bc1 = buoy ? fq(a.q[15])[k] : 0.0f, bc2 = buoy ? fq(a.q[16])[k] : 0.0f;
@@ -593,14 +602,13 @@ __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
     if (j == g.ny - 1) fy[c + sj] = fyh;
     if (k == g.nz - 1) fz[c + sk] = fzh;
     const float* hm = fq(a.q[30]);
-    const bool openx = ldi(a.q[17], 0) != 0, openy = ldi(a.q[17], 1) != 0;
     const float dt = ldf(a.q[41], 0), base = fq(a.q[7])[k] * fq(a.q[46])[c];
     auto dum = [&](bool inflow, float lo, float hi, float rlo, float rhi, float rd, float m) {
       const float adv = ((-(hi - lo)) * rd) * m, sdiv = ((P.s * (rhi - rlo)) * rd) * m;
       return inflow ? base : fma_(dt, adv + sdiv, base);
     };
-    const bool inx = openx && ((i == 0 && pxl.a >= 0.0f) || (i == g.nx - 1 && pxh.a <= 0.0f));
-    const bool iny = openy && ((j == 0 && pyl.a >= 0.0f) || (j == g.ny - 1 && pyh.a <= 0.0f));
+    const bool inx = open.x && ((i == 0 && pxl.a >= 0.0f) || (i == g.nx - 1 && pxh.a <= 0.0f));
+    const bool iny = open.y && ((j == 0 && pyl.a >= 0.0f) || (j == g.ny - 1 && pyh.a <= 0.0f));
     const float dx = dum(inx, fxl, fxh, pxl.a, pxh.a, g.rdx, hm_uh(hm, g, i));
     const float dy = dum(iny, fyl, fyh, pyl.a, pyh.a, g.rdy, hm_vh(hm, g, j));
     const float dz = dum(false, fzl, fzh, pzl.a, pzh.a, g.rdz, fq(a.q[9])[k]);
@@ -608,8 +616,8 @@ __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
     ox[c] = dx;
     oy[c] = dy;
     fq(a.q[45])[c] = dz;
-    halo_from(g, openx, openy, ox, i, j, c, dx);
-    halo_from(g, openx, openy, oy, i, j, c, dy);
+    halo_from<OPEN>(g, open, ox, i, j, c, dx, hx);
+    halo_from<OPEN>(g, open, oy, i, j, c, dy, hy);
   }
   // p[32] -> chain flags: the pointwise dispatches around a field's assembly
   // in the reference, applied to the tendency in registers:
@@ -618,9 +626,9 @@ __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
   // 2 / 4 turb_add_tendency (tend = fma(scale, src, tend); p35/p36, p37/p38),
   // 8 rk_update (phi = fma(dttmp, tend, phi_a); p39 phi_a, p40 phi, p41 dttmp;
   // phi must not be the advected field, which other workgroups still read),
-  // 32 with 8 on a periodic domain (nx, ny >= 4, cell-centred field): the
-  // halo fill of phi after it, each cell's periodic images written by the
-  // cell, level nz's by the cell below it (no thread of the launch reads phi),
+  // 32 with 8 (nx, ny >= 4, cell-centred field): the halo fill of phi after
+  // it, the halo cells a cell is the source of written by the cell, level nz's
+  // by the cell below it (no thread of the launch reads phi),
   // 64 buoyancy_apply after the assembly of w (tend = tend + fma(c1[k],
   // buoy[k-1], c2[k] * buoy[k]) at levels 1 .. nz-1; p42 buoy, p15 c1, p16 c2).
   // With an update in the chain the tendency itself is not stored.
@@ -640,15 +648,8 @@ __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
         if (chain & 8) {
           float* phi = fq(a.q[40]);
           const float nv = fma_(ldf(a.q[41], 0), v, phi_a);
-          phi[c] = nv;
-          if (chain & 32) {
-            const bool top = k == g.nz - 1;
-            const float ptop = top ? phi[c + sk] : 0.0f;
-            periodic_images(g, i, j, [&](int64_t o) {
-              phi[c + o] = nv;
-              if (top) phi[c + sk + o] = ptop;
-            });
-          }
+          if (chain & 32) halo_put<OPEN>(g, open, phi, i, j, c, nv, hc);
+          else phi[c] = nv;
         } else {
           tend[c] = v;
         }
@@ -657,17 +658,18 @@ __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
 
 // One kernel per specialised body (adv_fused_kernel), so that each carries
 // only its own registers; k_adv_fused selects the body at run time.
-template <int KIND, int STC>
+template <int KIND, int STC, bool OPEN>
 __global__ __launch_bounds__(256) void k_adv_fused_v(uint32_t* M, KArg a) {
-  adv_fused_body<KIND, STC>(M, a);
+  adv_fused_body<KIND, STC, OPEN>(M, a);
 }
-const void* adv_fused_kernel(int kind, int stag) {
-  if (kind == 0 && stag == 1) return (const void*)&k_adv_fused_v<0, 1>;
-  if (kind == 1 && stag == 1) return (const void*)&k_adv_fused_v<1, 1>;
-  if (kind == 2 && stag == 2) return (const void*)&k_adv_fused_v<2, 2>;
-  if (kind == 2 && stag == 3) return (const void*)&k_adv_fused_v<2, 3>;
-  if (kind == 2 && stag == 4) return (const void*)&k_adv_fused_v<2, 4>;
-  if (kind == 3 && stag == 4) return (const void*)&k_adv_fused_v<3, 4>;
+const void* adv_fused_kernel(int kind, int stag, bool open) {
+  if (kind == 0 && stag == 1) return open ? (const void*)&k_adv_fused_v<0, 1, true> : (const void*)&k_adv_fused_v<0, 1, false>;
+  if (kind == 1 && stag == 1) return open ? (const void*)&k_adv_fused_v<1, 1, true> : (const void*)&k_adv_fused_v<1, 1, false>;
+  if (open) return nullptr;
+  if (kind == 2 && stag == 2) return (const void*)&k_adv_fused_v<2, 2, false>;
+  if (kind == 2 && stag == 3) return (const void*)&k_adv_fused_v<2, 3, false>;
+  if (kind == 2 && stag == 4) return (const void*)&k_adv_fused_v<2, 4, false>;
+  if (kind == 3 && stag == 4) return (const void*)&k_adv_fused_v<3, 4, false>;
   return nullptr;
 }
 
@@ -677,33 +679,28 @@ const void* adv_fused_kernel(int kind, int stag) {
 // reads the result.  Parameters as adv_fused's (no chain), with 22-24 the
 // fluxes (written: a corrected cell reads its old ones), 41 -> dt, 43-45 the
 // partial updates, 46 the start-of-step field, 17 -> open x, open y.
-template <int KIND>
+template <int KIND, bool OPEN>
 __global__ __launch_bounds__(256) void k_adv_pdef_v(uint32_t* M, KArg a) {
-  adv_fused_body<KIND, 1, true>(M, a);
+  adv_fused_body<KIND, 1, OPEN, true>(M, a);
 }
-const void* adv_pdef_kernel(int kind) {
-  return kind == 0 ? (const void*)&k_adv_pdef_v<0> : kind == 1 ? (const void*)&k_adv_pdef_v<1> : nullptr;
+const void* adv_pdef_kernel(int kind, bool open) {
+  if (kind == 0) return open ? (const void*)&k_adv_pdef_v<0, true> : (const void*)&k_adv_pdef_v<0, false>;
+  if (kind == 1) return open ? (const void*)&k_adv_pdef_v<1, true> : (const void*)&k_adv_pdef_v<1, false>;
+  return nullptr;
 }
 __global__ __launch_bounds__(256) void k_adv_pdef(uint32_t* M, KArg a) {
-  if (ldi(a.q[3], 0) == 0) adv_fused_body<0, 1, true>(M, a);
-  else adv_fused_body<1, 1, true>(M, a);
+  if (ldi(a.q[3], 0) == 0) adv_fused_body<0, 1, true, true>(M, a);
+  else adv_fused_body<1, 1, true, true>(M, a);
 }
 
 // The three flux dispatches of one advected field and adv_assemble in one
 // launch (see above); the flux kind selects one specialised body.
 __global__ __launch_bounds__(256) void k_adv_fused(uint32_t* M, KArg a) {
-  const int kind = ldi(a.q[3], 0), stag = ldi(a.q[1], 0);
-  // the (kind, stagger) pairs the encoder emits get bodies specialised on both
-  if (kind == 0 && stag == 1) adv_fused_body<0, 1>(M, a);
-  else if (kind == 1 && stag == 1) adv_fused_body<1, 1>(M, a);
-  else if (kind == 2 && stag == 2) adv_fused_body<2, 2>(M, a);
-  else if (kind == 2 && stag == 3) adv_fused_body<2, 3>(M, a);
-  else if (kind == 2 && stag == 4) adv_fused_body<2, 4>(M, a);
-  else if (kind == 3 && stag == 4) adv_fused_body<3, 4>(M, a);
-  else if (kind == 0) adv_fused_body<0, 0>(M, a);
-  else if (kind == 1) adv_fused_body<1, 0>(M, a);
-  else if (kind == 2) adv_fused_body<2, 0>(M, a);
-  else adv_fused_body<3, 0>(M, a);
+  const int kind = ldi(a.q[3], 0);
+  if (kind == 0) adv_fused_body<0, 0, true>(M, a);
+  else if (kind == 1) adv_fused_body<1, 0, true>(M, a);
+  else if (kind == 2) adv_fused_body<2, 0, true>(M, a);
+  else adv_fused_body<3, 0, true>(M, a);
 }
 
 }  // namespace te

@@ -365,7 +365,7 @@ __global__ __launch_bounds__(256) void k_ppx_finish_xy(uint32_t* M, KArg a) {
   if (gx >= g.nx || gy >= g.ny || gz >= g.nz) return;
   const float* pp = fq(a.q[1]);
   float* ppx = fq(a.q[2]);
-  update_with_images(g, ppx, gx, gy, gz, 0, g.nz, [&](int64_t c) { return pp[c] + ppx[c]; });
+  update_with_halo(g, open_sides(a, 3), ppx, gx, gy, gz, 0, [&](int64_t c) { return pp[c] + ppx[c]; });
 }
 
 // diabatic_unapply.wgsl:111-140

@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256) void k_bc_open_xy(uint32_t* M, KArg a) {
 }
 
 // rk_update of a scalar (stagger 1) then its halo fill (rk_update.wgsl:111-132,
-// timestep.js:1593 haloFill); arguments as rk_update's.
+// timestep.js:1593 haloFill); arguments as rk_update's, 6 -> open x, open y.
 __global__ __launch_bounds__(256) void k_rk_update_xy(uint32_t* M, KArg a) {
   TE_TID3
   const Dims g = dims(a.q[0], 0);
@@ -111,12 +111,12 @@ __global__ __launch_bounds__(256) void k_rk_update_xy(uint32_t* M, KArg a) {
   if (i >= g.nx || j >= g.ny || k >= g.nz) return;
   const float *phiA = fq(a.q[2]), *tend = fq(a.q[3]);
   const float dttmp = ldf(a.q[5], 0);
-  update_with_images(g, fq(a.q[4]), i, j, k, 0, g.nz, [&](int64_t c) { return fma_(dttmp, tend[c], phiA[c]); });
+  update_with_halo(g, open_sides(a, 6), fq(a.q[4]), i, j, k, 0, [&](int64_t c) { return fma_(dttmp, tend[c], phiA[c]); });
 }
 
 // tke_advance (levels 1 .. nz-1) then the halo fill of tke
 // (tke_advance.wgsl:111-129, timestep.js:1593 haloFill); arguments as
-// tke_advance's.
+// tke_advance's, 5 -> open x, open y.
 __global__ __launch_bounds__(256) void k_tke_advance_xy(uint32_t* M, KArg a) {
   TE_TID3
   const Dims g = dims(a.q[0], 0);
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) void k_tke_advance_xy(uint32_t* M, KArg a) {
   if (i >= g.nx || j >= g.ny || k > g.nz - 1) return;
   const float *tkea = fq(a.q[1]), *tketen = fq(a.q[2]);
   const float dttmp = ldf(a.q[3], 0);
-  update_with_images(g, fq(a.q[4]), i, j, k, 1, g.nz, [&](int64_t c) {
+  update_with_halo(g, open_sides(a, 5), fq(a.q[4]), i, j, k, 1, [&](int64_t c) {
     const float v = fma_(dttmp, tketen[c], tkea[c]);
     return (v < 1e-10f) ? 0.0f : v;
   });

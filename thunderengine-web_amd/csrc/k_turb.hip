@@ -301,13 +301,11 @@ __device__ __forceinline__ void turb_km_kh_body(uint32_t* M, const KArg& a) {
       ev[q] = e != 0 ? F[q][c + e] : 0.0f;
       ev2[q] = e2 != 0 ? F[q][c + e2] : 0.0f;
     }
-    periodic_images(g, i, j, [&](int64_t o) {
-      for (int q = 0; q < 4; ++q) {
-        F[q][c + o] = v[q];
-        if (e != 0) F[q][c + e + o] = ev[q];
-        if (e2 != 0) F[q][c + e2 + o] = ev2[q];
-      }
-    });
+    for (int q = 0; q < 4; ++q) {
+      halo_from<false>(g, {false, false}, F[q], i, j, c, v[q], {});
+      if (e != 0) halo_from<false>(g, {false, false}, F[q], i, j, c + e, ev[q], {});
+      if (e2 != 0) halo_from<false>(g, {false, false}, F[q], i, j, c + e2, ev2[q], {});
+    }
   }
 }
 __global__ __launch_bounds__(256) void k_turb_km_kh(uint32_t* M, KArg a) { turb_km_kh_body<false>(M, a); }

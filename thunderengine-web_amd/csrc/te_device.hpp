@@ -62,72 +62,129 @@ struct Dims {
   TE_DEV int64_t sk() const { return (int64_t)sJ * sK; }
   TE_DEV int64_t idx(int i, int j, int k) const { return (int64_t)(i + 3) + (int64_t)sJ * ((j + 3) + (int64_t)sK * k); }
 };
-// The periodic halo cells whose image is interior cell (i, j) of a level:
-// hx in {i, i - nx (i >= nx - 3), i + nx (i <= 3)}, hy likewise with ny, all
-// pairs but (i, j) itself -- the cells bc_periodic_x then bc_periodic_y
-// (bc_periodic_x.wgsl:111-133, bc_periodic_y.wgsl:111-133) copy from it,
-// for nx, ny >= 4.  put(o) gets each one's word offset from (i, j).
-template <class F>
-TE_DEV void periodic_images(const Dims& g, int i, int j, F&& put) {
-  int64_t dx[3] = {0, 0, 0}, dy[3] = {0, 0, 0};
-  int nxo = 1, nyo = 1;
-  if (i >= g.nx - 3) dx[nxo++] = -g.nx;
-  if (i <= 3) dx[nxo++] = g.nx;
-  if (j >= g.ny - 3) dy[nyo++] = -(int64_t)g.ny * g.sJ;
-  if (j <= 3) dy[nyo++] = (int64_t)g.ny * g.sJ;
-  for (int b = 0; b < nyo; ++b)
-    for (int a = 0; a < nxo; ++a)
-      if (a != 0 || b != 0) put(dx[a] + dy[b]);
-}
-// A pointwise update of levels [k0, k1) of a cell-centred field on a
-// periodic domain (nx, ny >= 4) followed by the field's halo fill
-// (bc_periodic_x, bc_periodic_y): each cell writes its new value and its
-// periodic images, the cells next to levels 0 and nz also the images of
-// those levels (copied as they are: the update does not write them, and no
-// thread of the launch reads the field's halo).
-template <class F>
-TE_DEV void update_with_images(const Dims& g, float* f, int i, int j, int k, int k0, int k1, F value) {
-  const int64_t c = g.idx(i, j, k), sk = g.sk();
-  const bool lo = k == k0 && k0 == 1, hi = k == k1 - 1 && k1 == g.nz;
-  const float flo = lo ? f[c - sk] : 0.0f, fhi = hi ? f[c + sk] : 0.0f;
-  const float v = value(c);
-  f[c] = v;
-  periodic_images(g, i, j, [&](int64_t o) {
-    f[c + o] = v;
-    if (lo) f[c - sk + o] = flo;
-    if (hi) f[c + sk + o] = fhi;
-  });
+// The open sides of a launch that fills halos: parameter q -> open x, open y;
+// none where the parameter is not bound.
+struct Sides { bool x, y; };
+TE_DEV Sides open_sides(const KArg& a, int q) {
+  if (a.p[q] == 0) return {false, false};
+  return {ldi(a.q[q], 0) != 0, ldi(a.q[q], 1) != 0};
 }
 // The halo cells of a level that a haloFill of a cell-centred field gives the
-// value v of interior cell (i, j) (index c), written by that cell (nx, ny >= 4).
-// A periodic axis copies from the image modulo n, an open one from the nearest
-// cell for the three cells past either end (bc_open_x.wgsl:111-131).  The
-// fourth column or row past the open east or north end is filled by no pass
-// along its own axis, but the passes along the other axis copy it too, from
-// the words as they are.  No thread of the launch may read the field's halo.
-TE_DEV void halo_from(const Dims& g, bool openx, bool openy, float* f, int i, int j, int64_t c, float v) {
-  const int nX = openx ? (i == 0 || i == g.nx - 1 ? 4 : 1) : 1 + (i >= g.nx - 3) + (i <= 3);
-  const int nY = openy ? (j == 0 || j == g.ny - 1 ? 4 : 1) : 1 + (j >= g.ny - 3) + (j <= 3);
-  if (nX == 1 && nY == 1) return;
-  const int64_t sj = g.sJ;
-  auto ox = [&](int a) -> int64_t {
-    if (openx) return i == 0 ? -a : a;
-    return a == 0 ? 0 : (a == 1 && i >= g.nx - 3 ? -g.nx : g.nx);
-  };
-  auto oy = [&](int b) -> int64_t {
-    if (openy) return (j == 0 ? -b : b) * sj;
-    return b == 0 ? 0 : (b == 1 && j >= g.ny - 3 ? -g.ny : g.ny) * sj;
-  };
-  for (int b = 0; b < nY; ++b)
-    for (int a = 0; a < nX; ++a)
-      if (a != 0 || b != 0) f[c + ox(a) + oy(b)] = v;
-  if (openx && i == g.nx - 1 && nY > 1) {
-    const float e = f[c + 4];
-    for (int b = 1; b < nY; ++b) f[c + 4 + oy(b)] = e;
+// value of interior cell (i, j), written by that cell (nx, ny >= 4): a periodic
+// axis copies from the image modulo n, an open one from the nearest cell for
+// the three cells past either end (bc_open_x.wgsl:111-131).  The fourth column
+// or row past an open east or north end is filled by no pass along its own
+// axis, but the passes along the other axis copy it too, from the words as
+// they are: HaloOwn holds those words next to cell (i, j), loaded ahead of the
+// launch's stores (a load behind a store waits for it).  OPEN false: no side is
+// open; the two forms are compiled apart, as the open one in a periodic run's
+// launches cost them up to 20% (RK update at 192 x 192 x 80: 14.2, not 11.9 us).
+TE_DEV bool halo_source(Sides open, const Dims& g, int i, int j) {
+  const bool x = open.x ? i == 0 || i == g.nx - 1 : i <= 3 || i >= g.nx - 3;
+  const bool y = open.y ? j == 0 || j == g.ny - 1 : j <= 3 || j >= g.ny - 3;
+  return x || y;
+}
+struct HaloOwn { float x, y; };
+template <bool OPEN>
+TE_DEV HaloOwn halo_own(const Dims& g, Sides open, const float* f, int i, int j, int64_t c) {
+  HaloOwn o{0.0f, 0.0f};
+  if (OPEN) {
+    if (open.x && i == g.nx - 1 && halo_source({true, open.y}, g, 1, j)) o.x = f[c + 4];
+    if (open.y && j == g.ny - 1 && halo_source({open.x, true}, g, i, 1)) o.y = f[c + 4 * (int64_t)g.sJ];
   }
-  if (openy && j == g.ny - 1 && nX > 1) {
-    const float e = f[c + 4 * sj];
-    for (int a = 1; a < nX; ++a) f[c + 4 * sj + ox(a)] = e;
+  return o;
+}
+// Writes the halo cells of a level whose source is interior cell (i, j) (index
+// c, value v).  No thread of the launch may read the halo.  Straight-line
+// predicated stores: counted loops over the copies cost the corner waves, which
+// the launch waits for, 5 us at 120 x 120 x 40.
+template <bool OPEN>
+TE_DEV void halo_from(const Dims& g, Sides open, float* f, int i, int j, int64_t c, float v, HaloOwn own) {
+  const int64_t sj = g.sJ, wx = g.nx, wy = (int64_t)g.ny * sj;
+  const bool xlo = i <= 3, xhi = i >= g.nx - 3, ylo = j <= 3, yhi = j >= g.ny - 3;
+  float* p = f + c;
+  if (!OPEN) {
+    if (!(xlo || xhi || ylo || yhi)) return;
+    auto row = [&](float* r) {
+      if (xlo) r[wx] = v;
+      if (xhi) r[-wx] = v;
+    };
+    row(p);
+    if (ylo) {
+      p[wy] = v;
+      row(p + wy);
+    }
+    if (yhi) {
+      p[-wy] = v;
+      row(p - wy);
+    }
+    return;
+  }
+  if (!halo_source(open, g, i, j)) return;
+  const bool xe = i == 0 || i == g.nx - 1, ye = j == 0 || j == g.ny - 1;
+  const int64_t dx = i == 0 ? -1 : 1, dy = j == 0 ? -sj : sj;
+  auto copies = [&](float* r, float x) {  // the copies along x of the word at r
+    if (open.x) {
+      if (xe) {
+        r[dx] = x;
+        r[2 * dx] = x;
+        r[3 * dx] = x;
+      }
+    } else {
+      if (xlo) r[wx] = x;
+      if (xhi) r[-wx] = x;
+    }
+  };
+  auto row = [&](float* r) {
+    r[0] = v;
+    copies(r, v);
+    if (open.x && i == g.nx - 1) r[4] = own.x;
+  };
+  copies(p, v);
+  if (open.y) {
+    if (ye) {
+      row(p + dy);
+      row(p + 2 * dy);
+      row(p + 3 * dy);
+      if (j == g.ny - 1) copies(p + 4 * sj, own.y);
+    }
+  } else {
+    if (ylo) row(p + wy);
+    if (yhi) row(p - wy);
+  }
+}
+// A field's update at cell (i, j, k) with its halo fill: the cell's new value
+// and the halo cells it is the source of; the cells next to levels 0 (k0 = 1)
+// and nz also those of these levels, whose words the update leaves.  halo_cell
+// loads, halo_put stores.
+struct HaloCell { HaloOwn c, lo, hi; float flo, fhi; bool l, h; };
+template <bool OPEN>
+TE_DEV HaloCell halo_cell(const Dims& g, Sides open, const float* f, int i, int j, int k, int k0, int64_t c) {
+  HaloCell p{{0, 0}, {0, 0}, {0, 0}, 0.0f, 0.0f, k == k0 && k0 == 1, k == g.nz - 1};
+  const int64_t sk = g.sk();
+  p.c = halo_own<OPEN>(g, open, f, i, j, c);
+  if (p.l) { p.flo = f[c - sk]; p.lo = halo_own<OPEN>(g, open, f, i, j, c - sk); }
+  if (p.h) { p.fhi = f[c + sk]; p.hi = halo_own<OPEN>(g, open, f, i, j, c + sk); }
+  return p;
+}
+template <bool OPEN>
+TE_DEV void halo_put(const Dims& g, Sides open, float* f, int i, int j, int64_t c, float v, const HaloCell& p) {
+  f[c] = v;
+  halo_from<OPEN>(g, open, f, i, j, c, v, p.c);
+  if (p.l) halo_from<OPEN>(g, open, f, i, j, c - g.sk(), p.flo, p.lo);
+  if (p.h) halo_from<OPEN>(g, open, f, i, j, c + g.sk(), p.fhi, p.hi);
+}
+// A pointwise update of levels k0 .. nz-1 (k0 = 0 or 1) of a cell-centred field
+// followed by the field's halo fill.
+template <class F>
+TE_DEV void update_with_halo(const Dims& g, Sides open, float* f, int i, int j, int k, int k0, F value) {
+  const int64_t c = g.idx(i, j, k);
+  if (open.x || open.y) {
+    const HaloCell p = halo_cell<true>(g, open, f, i, j, k, k0, c);
+    halo_put<true>(g, open, f, i, j, c, value(c), p);
+  } else {
+    const HaloCell p = halo_cell<false>(g, open, f, i, j, k, k0, c);
+    halo_put<false>(g, open, f, i, j, c, value(c), p);
   }
 }
 // GridDims bytes: nx ny nz strideJ strideK 1/dx 1/dy 1/dz (timestep.js:88-90).

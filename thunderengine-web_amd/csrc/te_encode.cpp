@@ -121,10 +121,12 @@ class Encoder {
   // bc_periodic_xy launch (bc_open_xy where a side is open; up to 8 fields)
   // just before the next op that is not a halo fill.
   bool mergeHalo = false;
-  // fuse = 1 on a periodic domain (nx, ny >= 4): the halo fill after a
-  // scalar's RK update, TKE's advance and the stage's pressure is written by
-  // the launch that produces the field (each cell writes its periodic images)
-  // instead of by a bc_periodic_xy launch
+  // fuse = 1 (nx, ny >= 4): the halo fill after a scalar's RK update, TKE's
+  // advance, ppx and (periodic domains) the eddy coefficients and the stage's
+  // pressure is written by the launch that produces the field, each cell the
+  // halo cells it is the source of, instead of by a bc_periodic_xy or
+  // bc_open_xy launch.  At 120 x 120 x 40 open with 7 species 25 launches of
+  // 3.1-4.4 us fewer per step, the others 0.8-1.4 us longer: 1922 -> 1846 us.
   bool foldHalo = false;
   std::vector<std::string> pendingHalo, pendingZero;
   // turb_zero runs queue likewise (fusion on): one zero_fields launch per 8.
@@ -237,6 +239,10 @@ class Encoder {
   Bind rb(int i, const std::string& n) const { return {i, region(n)}; }
   Bind bb(int i, const Bytes& w) { return {i, bytes(w)}; }
 
+  // the open sides of the *_xy launch just emitted (its parameter q), if any
+  void foldSides(int q) {
+    if (foldHalo && (openX || openY)) E.ops.back().A[4 + q] = (uint32_t)bytes(I2(openX ? 1 : 0, openY ? 1 : 0));
+  }
   std::string species(const std::string& n, const std::string& suf) const {
     return std::find(scalars.begin(), scalars.end(), n) != scalars.end() ? n + suf : "qzero";
   }
@@ -290,7 +296,7 @@ void Encoder::setup() {
   openX = cfg.open_x != 0; openY = cfg.open_y != 0;
   periodicX = !openX; periodicY = !openY;
   mergeHalo = cfg.fuse != 0;
-  foldHalo = periodicX && periodicY && cfg.fuse == 1 && cfg.nx >= 4 && cfg.ny >= 4;
+  foldHalo = cfg.fuse == 1 && cfg.nx >= 4 && cfg.ny >= 4;
   wenoS = cfg.weno_scalars != 0;
   wenoM = cfg.weno_momentum != 0;
   explicitZ = cfg.explicit_vdiff != 0;
@@ -472,10 +478,12 @@ void Encoder::turbulence() {
     for (const Bind& bd : bs) o.A[4 + bd.idx] = (uint32_t)bd.off;
     E.ops.back() = o;
   }
-  op(foldHalo ? "turb_km_kh_xy" : "turb_km_kh", full,
+  // (open sides: four fields' copies in one launch are slower than their own)
+  const bool foldK = foldHalo && !openX && !openY;
+  op(foldK ? "turb_km_kh_xy" : "turb_km_kh", full,
      {fb(1, "tke_a"), fb(2, "nm"), rb(3, "mf"), fb(4, "kmh"), fb(5, "kmv"), fb(6, "khh"), fb(7, "khv"), fb(8, "lenscl"),
       fb(9, "dissten"), bb(10, F1(1.0f)), bb(11, F1(0.0f)), bb(12, F1(1.0f))});
-  if (!foldHalo)
+  if (!foldK)
     for (const char* n : {"kmh", "kmv", "khh", "khv"}) haloFill(n);
   if (diss) {
     const char* ks[] = {"qv", "qc", "qr", "qi", "qs", "qg"};
@@ -633,6 +641,7 @@ void Encoder::advect(int nrk, const std::string& s, int stagger, const std::stri
       if (!update)
         op(foldHalo ? "rk_update_xy" : "rk_update", asmSize,
            {bb(1, I1(stagger)), fb(2, target + "_a"), fb(3, "tend"), fb(4, target), bb(5, dttmp)});
+      if (!update) foldSides(6);
       if (!foldHalo) haloFill(target);
       return;
     }
@@ -787,7 +796,8 @@ void Encoder::sgsAndUpdate(int nrk, int stagger, const std::string& target, cons
   const bool fold = foldHalo && stagger == 1;
   op(fold ? "rk_update_xy" : "rk_update", asmSize,
      {bb(1, I1(stagger)), fb(2, target + "_a"), fb(3, "tend"), fb(4, target), bb(5, dttmp)});
-  if (!fold) haloFill(target);
+  if (fold) foldSides(6);
+  else haloFill(target);
 }
 
 void Encoder::stages() {
@@ -843,6 +853,7 @@ void Encoder::stages() {
         advect(nrk, "tke", 4, "tketen_s", true, "");
         op(foldHalo ? "tke_advance_xy" : "tke_advance", full,
            {fb(1, "tke_a"), fb(2, "tketen_s"), bb(3, dttmp), fb(4, "tke")});
+        foldSides(5);
       } else {
         op("turb_zero", whole, {fb(1, "tketen_s")});
         advect(nrk, "tke", 4, "tketen_s", true, "");
@@ -983,6 +994,7 @@ void Encoder::end() {
        {bb(1, F1(dtf)), fb(2, "pp3d"), fb(3, "th"), fb(4, "qv"), fb(5, "qc"), fb(6, "qpten"), fb(7, "qtten"),
         fb(8, "qvten"), fb(9, "qcten")});
   op(foldHalo ? "ppx_finish_xy" : "ppx_finish", full, {fb(1, "pp3d"), fb(2, "ppx")});
+  foldSides(3);
   if (!foldHalo) haloFill("ppx");
   flushAdd();
   flushHalo();

@@ -50,8 +50,8 @@ const void* ac_column_kernel(int levels_per_wave);
 const void* svi_waves_kernel(int levels_per_wave);
 // adv_fused specialised on (flux kind, stagger) (k_adv.hip); null for the
 // pairs only the run-time dispatch of k_adv_fused serves
-const void* adv_fused_kernel(int kind, int stag);
-const void* adv_pdef_kernel(int kind);
+const void* adv_fused_kernel(int kind, int stag, bool open);
+const void* adv_pdef_kernel(int kind, bool open);
 // turb_u_tendency_lds (dir 0) / turb_v_tendency_lds (dir 1) in the same form
 const void* uv_waves_kernel(int dir, int levels_per_wave);
 // turb_w_tendency_lds (which 0) / tke_transport_lds (which 1): levels 1 .. nz-1

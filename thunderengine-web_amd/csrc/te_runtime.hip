@@ -441,16 +441,15 @@ static int grow_guards(te_ctx* c) {
     if (std::strcmp(kn, "ac_column") == 0 && (uint64_t)sJ * sK * (uint64_t)(nz + 2) >= (1ull << 30))
       return fail(c, TE_ERR_UNSUPPORTED, "ac_column: a field spans 2^32 bytes or more");
     need = std::max<uint64_t>(need, (uint64_t)sJ * sK * (uint64_t)(nz + 3));
-    if (std::strcmp(kn, "adv_fused") == 0) {
-      int32_t stag = 0, kind = 0;
+    if (te::row_waves(op.kid)) {  // the body for its flux kind, stagger and halo fill
+      const bool pdef = std::strcmp(kn, "adv_pdef") == 0;
+      int32_t stag = 0, kind = 0, chain = 0, open[2] = {0, 0};
       TE_HIP(hipMemcpy(&stag, c->dM + op.A[4 + 1], 4, hipMemcpyDeviceToHost), "read stagger");
       TE_HIP(hipMemcpy(&kind, c->dM + op.A[4 + 3], 4, hipMemcpyDeviceToHost), "read flux kind");
-      op.fn = te::adv_fused_kernel(kind, stag);
-    }
-    if (std::strcmp(kn, "adv_pdef") == 0) {
-      int32_t kind = 0;
-      TE_HIP(hipMemcpy(&kind, c->dM + op.A[4 + 3], 4, hipMemcpyDeviceToHost), "read flux kind");
-      op.fn = te::adv_pdef_kernel(kind);
+      TE_HIP(hipMemcpy(&chain, c->dM + op.A[4 + 32], 4, hipMemcpyDeviceToHost), "read chain flags");
+      if (op.A[4 + 17] != 0) TE_HIP(hipMemcpy(open, c->dM + op.A[4 + 17], 8, hipMemcpyDeviceToHost), "read open sides");
+      const bool side = open[0] != 0 || open[1] != 0;
+      op.fn = pdef ? te::adv_pdef_kernel(kind, side) : te::adv_fused_kernel(kind, stag, side && (chain & 32) != 0);
     }
     if (std::strcmp(te::kernel_name(op.kid), "turb_sfcstress") == 0) {
       int32_t mode = 0;
