@@ -132,6 +132,8 @@ def alg_bytes_per_launch(run, names, A, op):
         io = [(1 + q, False, True) for q in range(3)] + [(4 + q, True, False) for q in range(3)]
     elif name == "adv_fused":
         io = adv_fused_io(run, A, op)
+    elif name == "mean_massflux":
+        io = ([(i, True, False) for i in (1, 2, 3, 13)] + [(i, False, True) for i in (6, 7, 8, 10, 11, 14)])
     elif name == "adv_pdef":
         io = ([(i, True, False) for i in (2, 4, 6, 7, 9, 13, 14, 15, 16, 30, 46)] +
               [(i, False, True) for i in (11, 22, 23, 24, 43, 44, 45)])

@@ -188,7 +188,49 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
       }
       continue;
     }
+    if (nm == "mean_massflux") {
+      // divergence3d (if bound), velocity_to_massflux, div_massflux and
+      // build_sadv, on the mean velocities copied into rru, rrv, rrw
+      auto P = [&](int q) { return A[4 + q]; };
+      auto run1 = [&](const char* kn, std::array<uint32_t, 3> g3, std::vector<std::pair<int, uint32_t>> ps) {
+        uint32_t X[64] = {0};
+        X[0] = g3[0]; X[1] = g3[1]; X[2] = g3[2];
+        X[4] = A[4]; X[34] = A[34];
+        for (auto& pr : ps) X[4 + pr.first] = pr.second;
+        K<T> k1{w, v, X};
+        call(find_kernel(kn), k1);
+      };
+      const uint32_t* dm = w + A[4];
+      const std::array<uint32_t, 3> full = {dm[0], dm[1], dm[2]}, whole = {dm[0] + 7, dm[1] + 7, dm[2] + 1};
+      const uint64_t n = (uint64_t)whole[0] * whole[1] * whole[2];
+      for (int q = 0; q < 3; ++q)
+        for (uint64_t c = 0; c < n; ++c) v[P(6 + q) + c] = v[P(1 + q) + c];
+      if (P(11) != 0) run1("divergence3d", full, {{1, P(6)}, {2, P(7)}, {3, P(8)}, {4, P(9)}, {5, P(11)}});
+      run1("velocity_to_massflux", whole, {{1, P(4)}, {2, P(5)}, {3, P(6)}, {4, P(7)}, {5, P(8)}});
+      run1("div_massflux", whole, {{1, P(6)}, {2, P(7)}, {3, P(8)}, {4, P(9)}, {5, P(10)}});
+      run1("build_sadv", whole, {{1, P(12)}, {2, P(13)}, {3, P(14)}});
+      continue;
+    }
+    // an accumulation whose result goes to other fields (slots `out`, if
+    // bound): run in place, copied there, and rru, rrv, rrw (slots `in`) put back
+    struct Redirect {
+      T* v; const uint32_t* A; int in, out; uint64_t n; std::vector<T> keep;
+      Redirect(T* v_, const uint32_t* A_, int in_, int out_, uint64_t n_) : v(v_), A(A_), in(in_), out(out_), n(n_) {
+        if (A[4 + out] == 0) return;
+        for (int q = 0; q < 3; ++q) keep.insert(keep.end(), v + A[4 + in + q], v + A[4 + in + q] + n);
+      }
+      ~Redirect() {
+        if (keep.empty()) return;
+        for (int q = 0; q < 3; ++q)
+          for (uint64_t c = 0; c < n; ++c) {
+            v[A[4 + out + q] + c] = v[A[4 + in + q] + c];
+            v[A[4 + in + q] + c] = keep[(uint64_t)q * n + c];
+          }
+      }
+    };
+    auto fieldWords = [&] { const uint32_t* dm = w + A[4]; return (uint64_t)(dm[0] + 7) * (dm[1] + 7) * (dm[2] + 1); };
     if (nm == "ac_column") {
+      const Redirect redirect(v, A, 13, 35, fieldWords());
       // the dispatches one acoustic substep launch stands for: on the stage's
       // first substep acoustic_prepare and acoustic_begin, then acoustic_fpk,
       // acoustic_w_solve, acoustic_pp, acoustic_accumulate and the periodic
@@ -244,6 +286,7 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
     }
     if (nm == "ac_pp_accumulate") {
       // acoustic_pp then acoustic_accumulate, the dispatches it stands for
+      const Redirect redirect(v, A, 13, 17, fieldWords());
       const uint32_t* dm = w + A[4];
       const uint32_t nx = dm[0], ny = dm[1], nz = dm[2];
       uint32_t X[64] = {0}, Y[64] = {0};

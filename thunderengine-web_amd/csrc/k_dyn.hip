@@ -189,6 +189,43 @@ __global__ __launch_bounds__(256) void k_massflux_div(uint32_t* M, KArg a) {
   if (div) fq(a.q[10])[c] = d;
 }
 
+// After the stage's substeps: divergence3d of the mean velocities,
+// velocity_to_massflux, div_massflux of the fluxes and build_sadv
+// (timestep.js:2056-2075) in one launch.  The mean velocities are read from
+// fields of their own (the last substep writes them there), so that no thread
+// of the launch reads what another one writes.  10 words per cell instead of
+// 16, one launch instead of four: 17.3 us became 6 at 64 x 64 x 40, 42 became
+// 30 at 192 x 192 x 80.
+// p: 1-3 mean u, v, w, 4 rho0, 5 rf0, 6-8 rru, rrv, rrw, 9 mh, 10 divx,
+// 11 div3d (if bound), 12 th0, 13 th, 14 sadv, 30 metric.  Grid: whole.
+__global__ __launch_bounds__(256) void k_mean_massflux(uint32_t* M, KArg a) {
+  TE_TID3
+  const Dims g = dims(a.q[0], 0);
+  const int i = gx - 3, j = gy - 3, k = gz;
+  if (i > g.nx + 3 || j > g.ny + 3 || k > g.nz) return;
+  const float *u = fq(a.q[1]), *v = fq(a.q[2]), *w = fq(a.q[3]), *rho0 = fq(a.q[4]), *rf0 = fq(a.q[5]),
+              *mh = fq(a.q[9]), *hm = fq(a.q[30]);
+  const int64_t sj = g.sJ, sk = g.sk(), c = g.idx(i, j, k);
+  const bool below = k < g.nz, div = i <= g.nx + 2 && j <= g.ny + 2 && below;
+  const bool inner = a.p[11] != 0 && below && i >= 0 && i < g.nx && j >= 0 && j < g.ny;
+  const float uc = u[c], vc = v[c], wc = w[c], th = below ? fq(a.q[13])[c] : 0.0f;
+  const float up = div ? u[c + 1] : 0.0f, vp = div ? v[c + sj] : 0.0f, wp = div ? w[c + sk] : 0.0f;
+  const float r = below ? rho0[k] : 1.0f, t0 = below ? fq(a.q[12])[k] - 3e+02f : 0.0f;
+  auto fw = [&](int kk, float x) { return (kk == 0 || kk == g.nz) ? 0.0f : x * rf0[kk]; };
+  const float mu = uc * r, mv = vc * r, mw = fw(k, wc), mwp = div ? fw(k + 1, wp) : 0.0f;
+  const float uh = div ? hm_uh(hm, g, i) : 0.0f, vh = div ? hm_vh(hm, g, j) : 0.0f, mhk = div ? mh[k] : 0.0f;
+  auto divergence = [&](float u0, float u1, float v0, float v1, float w0, float w1) {
+    return fma_((w1 - w0) * g.rdz, mhk, fma_((u1 - u0) * g.rdx, uh, ((v1 - v0) * g.rdy) * vh));
+  };
+  const float dx = divergence(mu, up * r, mv, vp * r, mw, mwp), d3 = divergence(uc, up, vc, vp, wc, wp);
+  fq(a.q[6])[c] = below ? mu : uc;  // level nz keeps the mean velocity
+  fq(a.q[7])[c] = below ? mv : vc;
+  fq(a.q[8])[c] = mw;
+  if (div) fq(a.q[10])[c] = dx;
+  if (inner) fq(a.q[11])[c] = (ab(d3) < 1e-30f) ? 0.0f : d3;
+  if (below) fq(a.q[14])[c] = t0 + th;
+}
+
 // velocity_to_massflux.wgsl:111-134
 __global__ __launch_bounds__(256) void k_velocity_to_massflux(uint32_t* M, KArg a) {
   {

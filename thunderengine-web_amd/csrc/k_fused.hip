@@ -232,7 +232,8 @@ __global__ __launch_bounds__(256) void k_copy_fields(uint32_t* M, KArg a) {
 // acoustic_accumulate (acoustic_accumulate.wgsl:129-158) at every point of
 // the whole grid.  Neither reads what the other writes, so one pass does
 // both.  p: 0 dims, 1 acoustic, 2 w, 3 pk1, 4 pk2, 5 qk, 6 fpk, 7 pp3d, 8 ppd,
-// 9 ppx, 10 -> saveX, 11 u, 12 v, 13 rru, 14 rrv, 15 rrw, 16 -> tavg.
+// 9 ppx, 10 -> saveX, 11 u, 12 v, 13 rru, 14 rrv, 15 rrw, 16 -> tavg, 17-19
+// (if bound) the fields the accumulated rru, rrv, rrw go to instead.
 __global__ __launch_bounds__(256) void k_ac_pp_accumulate(uint32_t* M, KArg a) {
   TE_TID3
   Dims g = dims(a.q[0], 0);
@@ -254,16 +255,18 @@ __global__ __launch_bounds__(256) void k_ac_pp_accumulate(uint32_t* M, KArg a) {
     if (ldi(a.q[10], 0) != 0) ppx[c] = dum1;
   }
   const float *u = fq(a.q[11]), *v = fq(a.q[12]);
-  float *rru = fq(a.q[13]), *rrv = fq(a.q[14]), *rrw = fq(a.q[15]);
+  const float *rru = fq(a.q[13]), *rrv = fq(a.q[14]), *rrw = fq(a.q[15]);
+  auto out = [&](int q, int in) { return fq(a.p[q] != 0 ? a.q[q] : a.q[in]); };
+  float *ru = out(17, 13), *rv = out(18, 14), *rw = out(19, 15);
   const float tavg = ldf(a.q[16], 0);
   if (tavg > 0.0f) {
-    rru[c] = (rru[c] + u[c]) * tavg;
-    rrv[c] = (rrv[c] + v[c]) * tavg;
-    rrw[c] = fma_(wc, ac.alph, rrw[c]) * tavg;
+    ru[c] = (rru[c] + u[c]) * tavg;
+    rv[c] = (rrv[c] + v[c]) * tavg;
+    rw[c] = fma_(wc, ac.alph, rrw[c]) * tavg;
   } else {
-    rru[c] = rru[c] + u[c];
-    rrv[c] = rrv[c] + v[c];
-    rrw[c] = rrw[c] + wc;
+    ru[c] = rru[c] + u[c];
+    rv[c] = rrv[c] + v[c];
+    rw[c] = rrw[c] + wc;
   }
 }
 
@@ -286,6 +289,7 @@ TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t
   const int nc = (g.sJ + 63) / 64, nl = g.nz + 1, units = g.sK * nl * nc;
   auto F = [&](int q) { return FieldB(reinterpret_cast<float*>(M) + a.p[q]); };
   const FieldB u = F(2), v = F(3), rru = F(13), rrv = F(14);
+  const FieldB rruO = a.p[35] != 0 ? F(35) : rru, rrvO = a.p[36] != 0 ? F(36) : rrv;
   const bool first = ldi(a.q[33], 0) != 0;
   const float tavg = ldf(a.q[17], 0), tv = tavg > 0.0f ? tavg : 1.0f;
   const uint32_t sjb = 4u * (uint32_t)g.sJ, skb = sjb * (uint32_t)g.sK;
@@ -321,8 +325,8 @@ TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t
   }
 #pragma unroll
   for (int d = 0; d < AC_UV_UNITS; ++d) {
-    if (todo[d] & 1) rru.put(h[d], (ru[d] + uo[d]) * tv);
-    if (todo[d] & 2) rrv.put(h[d], (rv[d] + vo[d]) * tv);
+    if (todo[d] & 1) rruO.put(h[d], (ru[d] + uo[d]) * tv);
+    if (todo[d] & 2) rrvO.put(h[d], (rv[d] + vo[d]) * tv);
     if ((todo[d] & 5) == 5) u.put(h[d], us[d]);
     if ((todo[d] & 6) == 6) v.put(h[d], vs[d]);
   }
@@ -385,7 +389,8 @@ TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t
 //    33 -> first substep of the stage, 34 -> (if bound) fill pp3d's halo
 //    too (with ppd's, group 4 below); the fields the replaced dispatches
 //    write as scratch (for expansions of this launch into them): 24 qk,
-//    25 pk1, 26 pk2, 27 mm, 28 fpk, 29 cA, 31 cB, and 32 rho0.
+//    25 pk1, 26 pk2, 27 mm, 28 fpk, 29 cA, 31 cB, and 32 rho0; 35-37 (if
+//    bound) the fields the accumulated rru, rrv, rrw go to instead, every word.
 // Grid: 64 x AC_WAVES threads per workgroup, ceil(nx / 64) * ny workgroups of
 // columns (padded to a multiple of 8), then a.n[2] of ac_accumulate_uv.
 // Needs nx, ny >= 4, 4 <= nz <= AC_WAVES * 16, and fields below 2^32 bytes
@@ -481,6 +486,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   __syncthreads();
   const FieldB u = F(2), v = F(3), w = F(4), piadv = F(5), ppten = F(6), ppterm = F(7), thv = F(8), wten = F(9),
                pp3d = F(10), ppd = F(11), ppx = F(12), rru = F(13), rrv = F(14), rrw = F(15);
+  const FieldB rruO = a.p[35] != 0 ? F(35) : rru, rrvO = a.p[36] != 0 ? F(36) : rrv, rrwO = a.p[37] != 0 ? F(37) : rrw;
   // byte offset of this lane's column at level k (the same in every field)
   const uint32_t sjb = 4u * (uint32_t)g.sJ, skb = sjb * (uint32_t)g.sK;
   const uint32_t o00 = 4u * (uint32_t)(ic + 3) + sjb * (uint32_t)(j + 3);
@@ -584,7 +590,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
       ppdz = ppd(o);
       ppz = pp3d(o);
       if (active) {
-        rrw.put(o, accw(rw, 0.0f));
+        rrwO.put(o, accw(rw, 0.0f));
         w.put(o, 0.0f);
       }
     }
@@ -618,9 +624,9 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
     };
     auto store = [&](const Item& c) {
       if (c.m == 4) {
-        rrw.put(c.h, accw(c.y, c.x));
+        rrwO.put(c.h, accw(c.y, c.x));
       } else if (c.m != 0) {
-        rru.put(c.h, acc(c.y, c.x));
+        rruO.put(c.h, acc(c.y, c.x));
         u.put(c.h, c.z);
       }
     };
@@ -652,8 +658,8 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
           if (z) yz = rrw(at(nz) + off);
         }
         if (active) {
-          batch(t0, [&](int d, uint32_t o) { rrw.put(o + off, accw(y[d], x[d])); });
-          if (z) rrw.put(at(nz) + off, accw(yz, xz));
+          batch(t0, [&](int d, uint32_t o) { rrwO.put(o + off, accw(y[d], x[d])); });
+          if (z) rrwO.put(at(nz) + off, accw(yz, xz));
         }
       }
     }
@@ -676,11 +682,11 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
         }
         if (active) {
           batch(t0, [&](int d, uint32_t o) {
-            rrv.put(o + sjb, acc(y[d], x[d]));
+            rrvO.put(o + sjb, acc(y[d], x[d]));
             v.put(o + sjb, s[d]);
           });
           if (z) {
-            rrv.put(at(nz) + sjb, acc(yz, xz));
+            rrvO.put(at(nz) + sjb, acc(yz, xz));
             v.put(at(nz) + sjb, sz);
           }
         }
@@ -821,7 +827,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
         ppd.put(o, CB[t]);
         if (saveX) ppx.put(o, dum1);
         w.put(o, w0);
-        rrw.put(o, accw(RW[t] * bf, w0));
+        rrwO.put(o, accw(RW[t] * bf, w0));
       }
     }
   // ---- the halo cells' w, ppd and pp3d, lane = column: images of the row in

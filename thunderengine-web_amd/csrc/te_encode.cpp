@@ -880,6 +880,12 @@ void Encoder::stages() {
       op("acoustic_begin", whole, {fb(2, "w"), fb(3, "rru"), fb(4, "rrv"), fb(5, "rrw")}, true);
     }
     const int nloop = sch.count[nrk];
+    // the last substep's mean velocities go to dead flux fields, which
+    // mean_massflux reads
+    auto meanOut = [&](int q) {
+      const char* out[] = {"fx", "fy", "fz"};
+      for (int d = 0; d < 3; ++d) E.ops.back().A[4 + q + d] = (uint32_t)off(out[d]);
+    };
     for (int n = 0; n < nloop; ++n) {
       if (openX || openY)
         op("openbc_uv_tendency", {std::max(nx, ny), nz, 1},
@@ -898,6 +904,7 @@ void Encoder::stages() {
             fb(27, "mm"), fb(28, "fpk"), fb(29, "cA"), fb(31, "cB"), rb(32, "rho0"), bb(33, I1(n == 0 ? 1 : 0)),
             bb(34, I1(foldHalo && n == nloop - 1 ? 1 : 0))},
            true);
+        if (n == nloop - 1) meanOut(35);
         continue;
       }
       if (cfg.fuse != 0) {  // pp + accumulate in one pass; accumulate reads no ppd, so ppd's
@@ -916,6 +923,7 @@ void Encoder::stages() {
             fb(9, "ppx"), bb(10, I1(nrk == 2 ? 1 : 0)), fb(11, "u"), fb(12, "v"), fb(13, "rru"), fb(14, "rrv"),
             fb(15, "rrw"), bb(16, F1(tavg))},
            true);
+        if (cfg.fuse == 1 && n == nloop - 1) meanOut(17);
         for (const char* h : {"ppd", "u", "v", "w"}) haloFill(h);
         continue;
       }
@@ -944,12 +952,19 @@ void Encoder::stages() {
       op("radbc_ew", {ny, 1, 1}, {fb(1, "u_a"), fb(2, "u"), bb(3, dttmp), rb(4, "radbcw"), rb(5, "radbce")});
     if (openY)
       op("radbc_ns", {nx, 1, 1}, {fb(1, "v_a"), fb(2, "v"), bb(3, dttmp), rb(4, "radbcs"), rb(5, "radbcn")});
-    if (moist) op("divergence3d", full, {fb(1, "rru"), fb(2, "rrv"), fb(3, "rrw"), rb(4, "mh"), fb(5, "div3d")});
-    op("velocity_to_massflux", whole, {rb(1, "rho0"), rb(2, "rf0"), fb(3, "rru"), fb(4, "rrv"), fb(5, "rrw")});
-    computeDiv();
+    if (cfg.fuse == 1) {
+      op("mean_massflux", whole,
+         {fb(1, "fx"), fb(2, "fy"), fb(3, "fz"), rb(4, "rho0"), rb(5, "rf0"), fb(6, "rru"), fb(7, "rrv"), fb(8, "rrw"),
+          rb(9, "mh"), fb(10, "divx"), rb(12, "th0"), fb(13, scalars[0]), fb(14, "sadv")});
+      if (moist) E.ops.back().A[4 + 11] = (uint32_t)off("div3d");
+    } else {
+      if (moist) op("divergence3d", full, {fb(1, "rru"), fb(2, "rrv"), fb(3, "rrw"), rb(4, "mh"), fb(5, "div3d")});
+      op("velocity_to_massflux", whole, {rb(1, "rho0"), rb(2, "rf0"), fb(3, "rru"), fb(4, "rrv"), fb(5, "rrw")});
+      computeDiv();
+    }
     for (size_t q = 0; q < scalars.size(); ++q) {
       if (q == 0) {
-        op("build_sadv", whole, {rb(1, "th0"), fb(2, scalars[0]), fb(3, "sadv")});
+        if (cfg.fuse != 1) op("build_sadv", whole, {rb(1, "th0"), fb(2, scalars[0]), fb(3, "sadv")});
         advect(nrk, "sadv", 1, "tend", false, scalars[0]);
       } else {
         advect(nrk, scalars[q], 1, "tend", false, "");
