@@ -339,6 +339,12 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
       const uint32_t S = A[4 + 2], RU = A[4 + 13], RV = A[4 + 14], RW = A[4 + 4], C1 = A[4 + 15], C2 = A[4 + 16];
       const uint32_t ST = A[4 + 1], WE = A[4 + 5], PD = A[4 + 20], PW = A[4 + 21];
       const uint32_t FX = A[4 + 22], FY = A[4 + 23], FZ = A[4 + 24];
+      // the launch keeps its fluxes in registers: the fields it names for them
+      // are put back
+      const uint64_t fluxWords = (uint64_t)(nx + 7) * (ny + 7) * (nz + 1);
+      std::vector<T> flux[3];
+      if (!pd)
+        for (int q = 0; q < 3; ++q) flux[q].assign(v + A[4 + 22 + q], v + A[4 + 22 + q] + fluxWords);
       struct Slot { const char* k; uint32_t g[3]; std::vector<std::pair<int, uint32_t>> p; };
       std::vector<Slot> fl;
       if (kind == 0) {
@@ -384,6 +390,8 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
       const KernelEntry* ea = find_kernel("adv_assemble");
       K<T> ka{w, v, Y};
       call(ea, ka);
+      if (!pd)
+        for (int q = 0; q < 3; ++q) std::copy(flux[q].begin(), flux[q].end(), v + A[4 + 22 + q]);
       // the scalar follow-ups chained into the launch, as their own dispatches
       const uint32_t chain = pd ? 0u : w[A[4 + 32]], TEND = A[4 + 11];
       auto run1 = [&](const char* kn, const uint32_t* g3, std::vector<std::pair<int, uint32_t>> ps) {

@@ -548,11 +548,10 @@ struct FusedFlux {
 // partial updates (pdef_dum.wgsl:177-231, see k_adv_pdef).
 // OPEN: the launch's halo fill may meet an open side.
 template <int KIND, int STC, bool OPEN, bool PD = false>
-__device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
+__device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a, const Blk b_) {
   // launched as 64 x Y x Z blocks (Y * Z <= 4; runtime launch(), te_autotune):
   // a wave is one row of cells, so j and k are wave-uniform and branches on
   // them are scalar
-  const Blk b_ = te_block(a);
   const int i = b_.x * 64 + (int)threadIdx.x,
             j = b_.y * TE_BY + (int)__builtin_amdgcn_readfirstlane(threadIdx.y),
             k = b_.z * TE_BZ + (int)__builtin_amdgcn_readfirstlane(threadIdx.z);
@@ -660,7 +659,7 @@ __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a) {
 // only its own registers; k_adv_fused selects the body at run time.
 template <int KIND, int STC, bool OPEN>
 __global__ __launch_bounds__(256) void k_adv_fused_v(uint32_t* M, KArg a) {
-  adv_fused_body<KIND, STC, OPEN>(M, a);
+  adv_fused_body<KIND, STC, OPEN>(M, a, te_block(a));
 }
 const void* adv_fused_kernel(int kind, int stag, bool open) {
   if (kind == 0 && stag == 1) return open ? (const void*)&k_adv_fused_v<0, 1, true> : (const void*)&k_adv_fused_v<0, 1, false>;
@@ -681,7 +680,7 @@ const void* adv_fused_kernel(int kind, int stag, bool open) {
 // partial updates, 46 the start-of-step field, 17 -> open x, open y.
 template <int KIND, bool OPEN>
 __global__ __launch_bounds__(256) void k_adv_pdef_v(uint32_t* M, KArg a) {
-  adv_fused_body<KIND, 1, OPEN, true>(M, a);
+  adv_fused_body<KIND, 1, OPEN, true>(M, a, te_block(a));
 }
 const void* adv_pdef_kernel(int kind, bool open) {
   if (kind == 0) return open ? (const void*)&k_adv_pdef_v<0, true> : (const void*)&k_adv_pdef_v<0, false>;
@@ -689,18 +688,65 @@ const void* adv_pdef_kernel(int kind, bool open) {
   return nullptr;
 }
 __global__ __launch_bounds__(256) void k_adv_pdef(uint32_t* M, KArg a) {
-  if (ldi(a.q[3], 0) == 0) adv_fused_body<0, 1, true, true>(M, a);
-  else adv_fused_body<1, 1, true, true>(M, a);
+  if (ldi(a.q[3], 0) == 0) adv_fused_body<0, 1, true, true>(M, a, te_block(a));
+  else adv_fused_body<1, 1, true, true>(M, a, te_block(a));
 }
 
 // The three flux dispatches of one advected field and adv_assemble in one
 // launch (see above); the flux kind selects one specialised body.
 __global__ __launch_bounds__(256) void k_adv_fused(uint32_t* M, KArg a) {
   const int kind = ldi(a.q[3], 0);
-  if (kind == 0) adv_fused_body<0, 0, true>(M, a);
-  else if (kind == 1) adv_fused_body<1, 0, true>(M, a);
-  else if (kind == 2) adv_fused_body<2, 0, true>(M, a);
-  else adv_fused_body<3, 0, true>(M, a);
+  if (kind == 0) adv_fused_body<0, 0, true>(M, a, te_block(a));
+  else if (kind == 1) adv_fused_body<1, 0, true>(M, a, te_block(a));
+  else if (kind == 2) adv_fused_body<2, 0, true>(M, a, te_block(a));
+  else adv_fused_body<3, 0, true>(M, a, te_block(a));
+}
+
+// Independent advections (adv_fused, adv_pdef) in one launch.  A stage's u, v,
+// w and TKE, and its scalars, read common fields and write their own: one
+// launch fills the chip once instead of draining it between them, and the
+// tiles of one place share an L2 (te_batch_part).
+// MASK: the bodies (adv_body) the launch may meet; body 0 or 8 is served by
+// 1 or 9, which take open sides too.  Blocks of 64 x 4 x 1.
+template <uint32_t MASK>
+__global__ __launch_bounds__(256) void k_adv_batch(uint32_t* M, KBatch) {
+  const BatchPart p = te_batch_part();
+  if (!p.in) return;
+  const Blk b = te_block_at(p.a, p.w);
+  auto is = [&](int v, int alt = -1) {
+    return (MASK >> v & 1u) != 0 && (p.body == v || (alt >= 0 && !(MASK >> alt & 1u) && p.body == alt));
+  };
+  if (is(0)) adv_fused_body<0, 1, false>(M, p.a, b);
+  if (is(1, 0)) adv_fused_body<0, 1, true>(M, p.a, b);
+  if (is(2)) adv_fused_body<1, 1, false>(M, p.a, b);
+  if (is(3)) adv_fused_body<1, 1, true>(M, p.a, b);
+  if (is(4)) adv_fused_body<2, 2, false>(M, p.a, b);
+  if (is(5)) adv_fused_body<2, 3, false>(M, p.a, b);
+  if (is(6)) adv_fused_body<2, 4, false>(M, p.a, b);
+  if (is(7)) adv_fused_body<3, 4, false>(M, p.a, b);
+  if (is(8)) adv_fused_body<0, 1, false, true>(M, p.a, b);
+  if (is(9)) adv_fused_body<0, 1, true, true>(M, p.a, b);
+  if (is(10)) adv_fused_body<1, 1, false, true>(M, p.a, b);
+  if (is(11)) adv_fused_body<1, 1, true, true>(M, p.a, b);
+}
+int adv_body(bool pdef, int kind, int stag, bool open) {
+  if (pdef) return kind == 0 || kind == 1 ? 8 + 2 * kind + open : -1;
+  if (stag == 1 && (kind == 0 || kind == 1)) return 2 * kind + open;
+  if (open) return -1;
+  if (kind == 2 && stag >= 2 && stag <= 4) return 2 + stag;
+  return kind == 3 && stag == 4 ? 7 : -1;
+}
+const void* adv_batch_kernel(uint32_t bodies) {
+  // momentum; with TKE; scalars; the last stage's theta and first moisture
+  // scalar (WENO, 5th order), each for periodic and open domains
+#define SET(m, with) {m, with, (const void*)&k_adv_batch<m>}
+  static const struct { uint32_t mask, serves; const void* fn; } sets[] = {
+      SET(0x70u, 0x70u), SET(0xf0u, 0xf0u), SET(0x01u, 0x01u), SET(0x02u, 0x03u),
+      SET(0x404u, 0x404u), SET(0x808u, 0x808u), SET(0x101u, 0x101u), SET(0x202u, 0x202u)};
+#undef SET
+  for (const auto& s : sets)
+    if ((bodies & ~s.serves) == 0) return s.fn;
+  return nullptr;
 }
 
 }  // namespace te

@@ -512,7 +512,7 @@ __global__ __launch_bounds__(256) void k_stability_max(uint32_t* M, KArg a) {
   }
   __syncthreads();
   int gx, gy, gz;
-  te_tid3(a, gx, gy, gz);
+  te_tid3(a, te_block(a), gx, gy, gz);
   const Dims g = dims(a.q[0], 0);
   float c2 = 0.0f, m = 0.0f;
   if (gx < (int)a.n[0] && gy < (int)a.n[1] && gz < (int)a.n[2] && gx < g.nx && gy < g.ny && gz < g.nz) {

@@ -104,14 +104,21 @@ __global__ __launch_bounds__(256) void k_bc_open_xy(uint32_t* M, KArg a) {
 
 // rk_update of a scalar (stagger 1) then its halo fill (rk_update.wgsl:111-132,
 // timestep.js:1593 haloFill); arguments as rk_update's, 6 -> open x, open y.
-__global__ __launch_bounds__(256) void k_rk_update_xy(uint32_t* M, KArg a) {
-  TE_TID3
+TE_DEV void rk_update_xy_body(uint32_t* M, const KArg& a, const Blk blk) {
+  int gx, gy, gz;
+  te_tid3(a, blk, gx, gy, gz);
   const Dims g = dims(a.q[0], 0);
   const int i = gx, j = gy, k = gz;
   if (i >= g.nx || j >= g.ny || k >= g.nz) return;
   const float *phiA = fq(a.q[2]), *tend = fq(a.q[3]);
   const float dttmp = ldf(a.q[5], 0);
   update_with_halo(g, open_sides(a, 6), fq(a.q[4]), i, j, k, 0, [&](int64_t c) { return fma_(dttmp, tend[c], phiA[c]); });
+}
+__global__ __launch_bounds__(256) void k_rk_update_xy(uint32_t* M, KArg a) { rk_update_xy_body(M, a, te_block(a)); }
+// the scalars of a stage in one launch
+__global__ __launch_bounds__(256) void k_rk_update_xy_batch(uint32_t* M, KBatch) {
+  const BatchPart p = te_batch_part();
+  if (p.in) rk_update_xy_body(M, p.a, te_block_at(p.a, p.w));
 }
 
 // tke_advance (levels 1 .. nz-1) then the halo fill of tke

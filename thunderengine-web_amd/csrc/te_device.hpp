@@ -455,20 +455,49 @@ struct Blk {
 TE_DEV uint32_t te_div(uint32_t l, uint32_t mlo, uint32_t mhi) {
   return (uint32_t)((((uint64_t)mhi << 32 | mlo) * (uint64_t)l) >> 40);
 }
-__device__ __forceinline__ Blk te_block(const KArg& a) {
+// the workgroup numbered w of a's grid (te_block: this launch's own)
+__device__ __forceinline__ Blk te_block_at(const KArg& a, uint32_t w) {
   const uint32_t nbx = a.lg[3], nby = a.lg[4];
 #if TE_XCD_REMAP
   const uint32_t n = a.lg[9];
-  const uint32_t w = blockIdx.x + nbx * (blockIdx.y + nby * blockIdx.z);
   const uint32_t q = n >> 3, r = n & 7u, x = w & 7u;
   const uint32_t l = x * q + (x < r ? x : r) + (w >> 3);
   const uint32_t yz = te_div(l, a.lg[5], a.lg[6]), z = te_div(yz, a.lg[7], a.lg[8]);
   return Blk{(int)(l - yz * nbx), (int)(yz - z * nby), (int)z};
 #else
-  (void)nbx;
-  (void)nby;
-  return Blk{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z};
+  return Blk{(int)(w % nbx), (int)(w / nbx % nby), (int)(w / nbx / nby)};
 #endif
+}
+__device__ __forceinline__ Blk te_block(const KArg& a) {
+  return te_block_at(a, blockIdx.x + a.lg[3] * (blockIdx.y + a.lg[4] * blockIdx.z));
+}
+// Launches of independent dispatches side by side (the runtime's batches): the
+// arguments of each lie in the kernel's argument segment (a by-value array
+// argument indexed by a variable would be copied to scratch memory; it is read
+// in place here).  Workgroup b runs on XCD b % 8; each XCD takes its share of
+// the dispatches one after the other, start[i] .. start[i+1] of its workgroups
+// for dispatch i.  (Tile by tile in turn instead, for the fields they share:
+// their stencils' levels then exceed an L2, u, v, w and TKE at 192 x 192 x 80
+// 143 us instead of 118 in four launches.)
+#define TE_BATCH 6
+struct KBatch {
+  KArg a[TE_BATCH];
+  uint32_t start[TE_BATCH + 1], body[TE_BATCH];
+};
+struct BatchPart {
+  const KArg& a;
+  int body;
+  uint32_t w;
+  bool in;
+};
+TE_DEV BatchPart te_batch_part() {
+  const KBatch& B = *(const KBatch*)((const char*)__builtin_amdgcn_kernarg_segment_ptr() + 8);
+  const uint32_t s = blockIdx.x >> 3;
+  uint32_t i = 0;
+#pragma unroll
+  for (int q = 1; q < TE_BATCH; ++q) i += s >= B.start[q];
+  const uint32_t w = (s - B.start[i]) * 8u + (blockIdx.x & 7u);
+  return {B.a[i], (int)B.body[i], w, w < B.a[i].lg[9]};
 }
 // block dims as the runtime launched them (kernel arguments, not the
 // dispatch packet)
@@ -535,8 +564,7 @@ TE_DEV void st4(uint32_t* p, uint32_t w, int width, const F4& r) {
 // not a multiple of 64: whole-field rows of nx+7, staggered rows of nx+1)
 // number the (i, j) plane's points consecutively, 256 per workgroup, with
 // the level on the grid's y axis, so no wave idles at a row's end.
-TE_DEV void te_tid3(const KArg& a, int& gx, int& gy, int& gz) {
-  const Blk b = te_block(a);
+TE_DEV void te_tid3(const KArg& a, const Blk b, int& gx, int& gy, int& gz) {
   if (a.lg[11] != 0) {
     const uint32_t t = (uint32_t)b.x * 256u + threadIdx.x;
     const uint32_t row = te_div(t, a.lg[12], a.lg[13]);
@@ -551,7 +579,7 @@ TE_DEV void te_tid3(const KArg& a, int& gx, int& gy, int& gz) {
 }
 #define TE_TID3                                                          \
   int gx, gy, gz;                                                        \
-  te_tid3(a, gx, gy, gz);                                                \
+  te_tid3(a, te_block(a), gx, gy, gz);                                   \
   if (gx >= (int)a.n[0] || gy >= (int)a.n[1] || gz >= (int)a.n[2]) return;
 
 }  // namespace te

@@ -610,7 +610,7 @@ void Encoder::advect(int nrk, const std::string& s, int stagger, const std::stri
       bs.push_back(fb(35, "tketen"));
       bs.push_back(bb(36, F1(1.0f)));
     } else if (chained) {
-      if (moistSgs) moistureTurbulence(nrk, target);
+      if (moistSgs && cfg.fuse != 1) moistureTurbulence(nrk, target);  // (fuse = 1: before all scalars, stages)
       int flags = 0;
       if (moist && target == scalars[0]) {
         flags |= 1;
@@ -635,13 +635,16 @@ void Encoder::advect(int nrk, const std::string& s, int stagger, const std::stri
     } else {
       bs.push_back(bb(32, I1(0)));
     }
+    if (into == "fx" || into == "fy" || into == "fz")  // (the flux fields are scratch of an expansion only)
+      for (Bind& bd : bs)
+        if (bd.idx >= 22 && bd.idx <= 24) bd.off = off(bd.idx == 22 ? "pk1" : bd.idx == 23 ? "pk2" : "fpk");
     op("adv_fused", asmSize, {});
     for (const Bind& bd : bs) E.ops.back().A[4 + bd.idx] = (uint32_t)bd.off;
     if (chained) {
+      if (!update && cfg.fuse == 1) return;  // rk_update_xy after all scalars' advection (stages)
       if (!update)
         op(foldHalo ? "rk_update_xy" : "rk_update", asmSize,
            {bb(1, I1(stagger)), fb(2, target + "_a"), fb(3, "tend"), fb(4, target), bb(5, dttmp)});
-      if (!update) foldSides(6);
       if (!foldHalo) haloFill(target);
       return;
     }
@@ -962,14 +965,28 @@ void Encoder::stages() {
       op("velocity_to_massflux", whole, {rb(1, "rho0"), rb(2, "rf0"), fb(3, "rru"), fb(4, "rrv"), fb(5, "rrw")});
       computeDiv();
     }
+    // fuse = 1, unless moisture SGS or microphysics tendencies add to `tend`
+    // scalar by scalar: each scalar's tendency in a (dead) field of its own, so
+    // that the advections are independent and their RK updates follow together
+    // (the runtime launches each group at once)
+    static const char* const own[] = {"cA", "cB", "qk", "mm", "pk1", "pk2", "fpk", "fx", "fy", "fz"};
+    const bool chains = cfg.fuse == 1 && moist && (!tke || cacheMT) && !(hasMicro && usePT), grouped = chains && nrk < 2;
+    if (chains && tke)
+      for (size_t q = 1; q < scalars.size(); ++q) moistureTurbulence(nrk, scalars[q]);
     for (size_t q = 0; q < scalars.size(); ++q) {
       if (q == 0) {
         if (cfg.fuse != 1) op("build_sadv", whole, {rb(1, "th0"), fb(2, scalars[0]), fb(3, "sadv")});
         advect(nrk, "sadv", 1, "tend", false, scalars[0]);
       } else {
-        advect(nrk, scalars[q], 1, "tend", false, "");
+        advect(nrk, scalars[q], 1, grouped ? own[q - 1] : "tend", false, "");
       }
     }
+    if (grouped)
+      for (size_t q = 1; q < scalars.size(); ++q) {
+        op("rk_update_xy", full,
+           {bb(1, I1(1)), fb(2, scalars[q] + "_a"), fb(3, own[q - 1]), fb(4, scalars[q]), bb(5, dttmp)});
+        foldSides(6);
+      }
     if (nrk == 2) {
       if (moist && usePT)
         op("diabatic_unapply", full,

@@ -27,6 +27,10 @@ struct Op {
   // the kernel launched in place of the op's table entry: a body specialised
   // on parameters the op fixes (set with nz; null: the table's kernel)
   const void* fn = nullptr;
+  // adv_fused, adv_pdef: the chain flags and specialised body (-1: none)
+  int32_t chain = 0, body = -1;
+  // ops, from this one on, that one launch runs side by side (set with nz)
+  int32_t batch = 1;
 };
 
 int kernel_id(const char* name);

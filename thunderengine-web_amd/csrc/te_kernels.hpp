@@ -52,6 +52,11 @@ const void* svi_waves_kernel(int levels_per_wave);
 // pairs only the run-time dispatch of k_adv_fused serves
 const void* adv_fused_kernel(int kind, int stag, bool open);
 const void* adv_pdef_kernel(int kind, bool open);
+// the specialised body of an adv_fused (pdef: adv_pdef) dispatch, -1 if none,
+// and the kernel that runs a set of them (bit n: body n) side by side, or null
+int adv_body(bool pdef, int kind, int stag, bool open);
+const void* adv_batch_kernel(uint32_t bodies);
+__global__ __launch_bounds__(256) void k_rk_update_xy_batch(uint32_t* M, KBatch);
 // turb_u_tendency_lds (dir 0) / turb_v_tendency_lds (dir 1) in the same form
 const void* uv_waves_kernel(int dir, int levels_per_wave);
 // turb_w_tendency_lds (which 0) / tke_transport_lds (which 1): levels 1 .. nz-1

@@ -123,10 +123,25 @@ static uint32_t column_lanes() {
   return lanes;
 }
 
-static hipError_t launch(te_ctx* c, const Op& op) {
-  KArg a = karg_of(op);
+// A dispatch's kernel, arguments, grid, block and dynamic LDS bytes.
+struct Shape {
+  const void* fn = nullptr;
+  KArg a;
+  dim3 g, b;
+  size_t lds = 0;
+};
+static hipError_t shape_of(te_ctx* c, const Op& op, Shape& s) {
+  KArg& a = s.a;
+  a = karg_of(op);
   for (int q = 0; q < 48; ++q) a.q[q] = c->dM + a.p[q];
   if (a.n[0] == 0 || a.n[1] == 0 || a.n[2] == 0) return hipSuccess;
+  auto done = [&](const void* fn, const dim3& g, const dim3& b, size_t lds) {
+    s.fn = fn;
+    s.g = g;
+    s.b = b;
+    s.lds = lds;
+    return hipSuccess;
+  };
   dim3 b = block_for(a.n);
   static const int kTkeEpst = kernel_id("tke_epst");
   if (row_waves(op.kid)) b = dim3(64, 4, 1);  // one row of cells per wave (k_adv_fused)
@@ -150,8 +165,7 @@ static hipError_t launch(te_ctx* c, const Op& op) {
     const uint64_t uv = (units + per - 1) / per, all = (((uint64_t)a.lg[9] + 7) & ~7ull) + uv;
     if (units >= (1ull << 31) || all >= (1ull << 31)) return hipErrorInvalidConfiguration;
     a.n[2] = (uint32_t)uv;
-    void* args[] = {(void*)&c->dM, (void*)&a};
-    return hipLaunchKernel(fn, dim3((uint32_t)all, 1, 1), b, args, dyn, c->stream);
+    return done(fn, dim3((uint32_t)all, 1, 1), b, dyn);
   }
   if (a.n[2] == 1 && op.nz >= 4 && wave_sweep(op.kid)) {
     // 64 columns of a row per workgroup, AC_WAVES waves over the levels
@@ -167,11 +181,10 @@ static hipError_t launch(te_ctx* c, const Op& op) {
     const uint64_t nb = ((uint64_t)a.n[0] * a.n[1] + 63) / 64;
     const dim3 g = nb <= 65535 ? dim3((uint32_t)nb, 1, 1) : dim3(4096, (uint32_t)((nb + 4095) / 4096), 1);
     if (!launch_shape(a, b, g)) return hipErrorInvalidConfiguration;
-    void* args[] = {(void*)&c->dM, (void*)&a};
     const void* fn = op.kid == kSviLds ? svi_waves_kernel((int)lw)
                      : !face       ? uv_waves_kernel(op.kid == kULds ? 0 : 1, (int)lw)
                                    : face_waves_kernel(op.kid == kWLds ? 0 : 1, (int)lw);
-    return hipLaunchKernel(fn, g, b, args, 0, c->stream);
+    return done(fn, g, b, 0);
   }
   size_t lds = 0;
   if (op.flat) {  // runs of 4 words per thread over the op's n0*n1*n2 words (te_flat)
@@ -180,8 +193,7 @@ static hipError_t launch(te_ctx* c, const Op& op) {
     const dim3 g((uint32_t)((runs + 255) / 256), 1, 1);
     if (!launch_shape(a, b, g)) return hipErrorInvalidConfiguration;
     a.lg[10] = 1;
-    void* args[] = {(void*)&c->dM, (void*)&a};
-    return hipLaunchKernel(kKernels[op.kid].fn, g, b, args, 0, c->stream);
+    return done(kKernels[op.kid].fn, g, b, 0);
   }
   if (a.n[2] == 1 && is_column_kernel(op.kid)) {
     b = dim3(column_lanes(), 1, 1);
@@ -197,13 +209,108 @@ static hipError_t launch(te_ctx* c, const Op& op) {
     a.lg[11] = 1;
     a.lg[12] = (uint32_t)m;
     a.lg[13] = (uint32_t)(m >> 32);
-    void* args[] = {(void*)&c->dM, (void*)&a};
-    return hipLaunchKernel(kKernels[op.kid].fn, g, b, args, 0, c->stream);
+    return done(kKernels[op.kid].fn, g, b, 0);
   }
   dim3 g((a.n[0] + b.x - 1) / b.x, (a.n[1] + b.y - 1) / b.y, (a.n[2] + b.z - 1) / b.z);
   if (!launch_shape(a, b, g)) return hipErrorInvalidConfiguration;  // beyond te_block()'s exact range
-  void* args[] = {(void*)&c->dM, (void*)&a};
-  return hipLaunchKernel(op.fn ? op.fn : kKernels[op.kid].fn, g, b, args, lds, c->stream);
+  return done(op.fn ? op.fn : kKernels[op.kid].fn, g, b, lds);
+}
+static hipError_t launch(te_ctx* c, const Op& op) {
+  Shape s;
+  const hipError_t e = shape_of(c, op, s);
+  if (e != hipSuccess || !s.fn) return e;
+  void* args[] = {(void*)&c->dM, (void*)&s.a};
+  return hipLaunchKernel(s.fn, s.g, s.b, args, s.lds, c->stream);
+}
+
+// ---- batches: consecutive dispatches none of which reads or writes what
+// another one writes, run side by side by one launch (KBatch).  The fields of
+// a dispatch, by parameter:
+static void op_fields(const Op& op, std::vector<uint32_t>& reads, std::vector<uint32_t>& writes) {
+  static const int kAdvFused = kernel_id("adv_fused"), kAdvPdef = kernel_id("adv_pdef");
+  auto add = [&](std::vector<uint32_t>& to, std::initializer_list<int> ps) {
+    for (int q : ps) to.push_back(op.A[4 + q]);
+  };
+  if (op.kid == kAdvFused) {
+    add(reads, {2, 4, 6, 13, 14});
+    if (op.chain & 1) add(reads, {33, 34});
+    if (op.chain & 2) add(reads, {35});
+    if (op.chain & 4) add(reads, {37});
+    if (op.chain & 8) add(reads, {39});
+    if (op.chain & 64) add(reads, {42});
+    if (op.chain & 8) add(writes, {40});
+    else add(writes, {11});
+  } else if (op.kid == kAdvPdef) {
+    add(reads, {2, 4, 6, 13, 14, 46});
+    add(writes, {11, 22, 23, 24, 43, 44, 45});
+  } else {  // rk_update_xy
+    add(reads, {2, 3});
+    add(writes, {4});
+  }
+}
+static const void* batch_kernel(const Op* ops, int n) {
+  static const int kRk = kernel_id("rk_update_xy");
+  if (n < 2 || n > TE_BATCH) return nullptr;
+  uint32_t bodies = 0;
+  for (int i = 0; i < n; ++i) {
+    if (ops[i].kid == kRk && ops[0].kid == kRk) {
+      // one block shape for all
+      if (ops[i].tuned || std::memcmp(ops[i].A, ops[0].A, 12) != 0 || ops[i].plane != ops[0].plane) return nullptr;
+    } else {
+      if (!row_waves(ops[i].kid) || ops[i].body < 0 || ops[0].kid == kRk) return nullptr;
+      bodies |= 1u << ops[i].body;
+    }
+  }
+  const uint64_t words = (uint64_t)ops[0].sJ * ops[0].sK * (ops[0].nz + 1);
+  auto meets = [&](const std::vector<uint32_t>& v, uint32_t f) {
+    for (uint32_t x : v)
+      if ((x > f ? x - f : f - x) < words) return true;
+    return false;
+  };
+  std::vector<uint32_t> r, w;
+  for (int i = 0; i < n; ++i) {
+    if (ops[i].A[4] != ops[0].A[4]) return nullptr;  // one grid
+    std::vector<uint32_t> ri, wi;
+    op_fields(ops[i], ri, wi);
+    for (uint32_t f : wi)
+      if (meets(r, f) || meets(w, f)) return nullptr;
+    for (uint32_t f : ri)
+      if (meets(w, f)) return nullptr;
+    r.insert(r.end(), ri.begin(), ri.end());
+    w.insert(w.end(), wi.begin(), wi.end());
+  }
+  return ops[0].kid == kRk ? (const void*)&k_rk_update_xy_batch : adv_batch_kernel(bodies);
+}
+static hipError_t launch_batch(te_ctx* c, const Op* ops, int n) {
+  const void* fn = batch_kernel(ops, n);
+  bool fits = fn != nullptr;
+  KBatch B;
+  std::memset(&B, 0, sizeof(B));
+  uint64_t per = 0;  // workgroups per XCD
+  dim3 b;
+  for (int i = 0; i < n && fits; ++i) {
+    Op op = ops[i];
+    op.tuned = false;
+    Shape s;
+    const hipError_t e = shape_of(c, op, s);
+    if (e != hipSuccess) return e;
+    fits = s.fn != nullptr;
+    B.a[i] = s.a;
+    B.body[i] = (uint32_t)std::max(op.body, 0);
+    b = s.b;
+    B.start[i] = (uint32_t)per;
+    per += (s.a.lg[9] + 7) / 8;
+  }
+  for (int i = n; i <= TE_BATCH; ++i) B.start[i] = (uint32_t)per;
+  if (!fits || per * 8 >= (1ull << 31)) {  // one by one
+    for (int i = 0; i < n; ++i) {
+      const hipError_t e = launch(c, ops[i]);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+  void* args[] = {(void*)&c->dM, (void*)&B};
+  return hipLaunchKernel(fn, dim3((uint32_t)per * 8, 1, 1), b, args, 0, c->stream);
 }
 
 // region_hash (replay.js:408-418): per-lane sums of a 32-bit mix, reduced
@@ -382,6 +489,7 @@ static const std::set<std::string>& own_mapping() {
 static int grow_guards(te_ctx* c) {
   if (c->guard_ok) return TE_OK;
   uint64_t need = 0;
+  std::map<uint32_t, int32_t> words;                 // parameter words already read
   std::map<uint32_t, std::array<uint32_t, 5>> seen;  // grid parameter blocks already read
   // pointwise ops that may run flat (te_flat): kernel -> the parameters it
   // accesses in 16-byte runs (fields; profiles are read per level)
@@ -444,12 +552,26 @@ static int grow_guards(te_ctx* c) {
     if (te::row_waves(op.kid)) {  // the body for its flux kind, stagger and halo fill
       const bool pdef = std::strcmp(kn, "adv_pdef") == 0;
       int32_t stag = 0, kind = 0, chain = 0, open[2] = {0, 0};
-      TE_HIP(hipMemcpy(&stag, c->dM + op.A[4 + 1], 4, hipMemcpyDeviceToHost), "read stagger");
-      TE_HIP(hipMemcpy(&kind, c->dM + op.A[4 + 3], 4, hipMemcpyDeviceToHost), "read flux kind");
-      TE_HIP(hipMemcpy(&chain, c->dM + op.A[4 + 32], 4, hipMemcpyDeviceToHost), "read chain flags");
-      if (op.A[4 + 17] != 0) TE_HIP(hipMemcpy(open, c->dM + op.A[4 + 17], 8, hipMemcpyDeviceToHost), "read open sides");
+      auto read = [&](uint32_t at, int32_t* to, const char* what) -> int {  // each word once (they are shared)
+        const auto known = words.find(at);
+        if (known != words.end()) {
+          *to = known->second;
+          return TE_OK;
+        }
+        TE_HIP(hipMemcpy(to, c->dM + at, 4, hipMemcpyDeviceToHost), what);
+        words[at] = *to;
+        return TE_OK;
+      };
+      int rc = read(op.A[4 + 1], &stag, "read stagger");
+      if (rc == TE_OK) rc = read(op.A[4 + 3], &kind, "read flux kind");
+      if (rc == TE_OK) rc = read(op.A[4 + 32], &chain, "read chain flags");
+      for (int q = 0; q < 2 && rc == TE_OK && op.A[4 + 17] != 0; ++q) rc = read(op.A[4 + 17] + q, &open[q], "read open sides");
+      if (rc != TE_OK) return rc;
       const bool side = open[0] != 0 || open[1] != 0;
-      op.fn = pdef ? te::adv_pdef_kernel(kind, side) : te::adv_fused_kernel(kind, stag, side && (chain & 32) != 0);
+      const bool openBody = side && (pdef || (chain & 32) != 0);
+      op.fn = pdef ? te::adv_pdef_kernel(kind, side) : te::adv_fused_kernel(kind, stag, openBody);
+      op.chain = pdef ? 0 : chain;
+      op.body = te::adv_body(pdef, kind, stag, openBody);
     }
     if (std::strcmp(te::kernel_name(op.kid), "turb_sfcstress") == 0) {
       int32_t mode = 0;
@@ -463,6 +585,13 @@ static int grow_guards(te_ctx* c) {
     int rc = alloc_memory(c, std::max(want, c->words), need);
     if (rc != TE_OK) return rc;
   }
+  // batches: as many of the following dispatches as can join
+  for (size_t i = 0; i < c->ops.size(); i += c->ops[i].batch) {
+    int n = 1;
+    while (i + n < c->ops.size() && te::batch_kernel(&c->ops[i], n + 1)) ++n;
+    c->ops[i].batch = n;
+    for (int q = 1; q < n; ++q) c->ops[i + q].batch = 1;
+  }
   c->guard_ok = true;
   return TE_OK;
 }
@@ -470,9 +599,12 @@ static int grow_guards(te_ctx* c) {
 int te::ensure_guard(te_ctx* c) { return grow_guards(c); }
 
 static int run_ops(te_ctx* c, int first, int last) {
-  for (int i = first; i <= last; ++i) {
-    hipError_t e = te::launch(c, c->ops[i]);
+  for (int i = first; i <= last;) {
+    const int n = c->ops[i].batch;
+    const bool together = n > 1 && i + n - 1 <= last;
+    hipError_t e = together ? te::launch_batch(c, &c->ops[i], n) : te::launch(c, c->ops[i]);
     if (e != hipSuccess) return hip_fail(c, e, (std::string("launch ") + te::kernel_name(c->ops[i].kid)).c_str());
+    i += together ? n : 1;
   }
   return TE_OK;
 }
