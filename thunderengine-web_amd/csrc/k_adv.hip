@@ -712,7 +712,7 @@ template <uint32_t MASK>
 __global__ __launch_bounds__(256) void k_adv_batch(uint32_t* M, KBatch) {
   const BatchPart p = te_batch_part();
   if (!p.in) return;
-  const Blk b = te_block_at(p.a, p.w);
+  const Blk b = p.blk();
   auto is = [&](int v, int alt = -1) {
     return (MASK >> v & 1u) != 0 && (p.body == v || (alt >= 0 && !(MASK >> alt & 1u) && p.body == alt));
   };

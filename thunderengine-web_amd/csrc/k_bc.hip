@@ -2,6 +2,7 @@
 // radiative speeds and normal-velocity tendencies, turbulence edge copies.
 #include "te_device.hpp"
 #include "te_kernels.hpp"
+#include "pointwise.hpp"
 
 namespace te {
 
@@ -92,23 +93,7 @@ __device__ void radbc(uint32_t* M, const KArg& a, int t) {
 __global__ __launch_bounds__(256) void k_radbc_ew(uint32_t* M, KArg a) { TE_TID3 radbc<0>(M, a, gx); }
 __global__ __launch_bounds__(256) void k_radbc_ns(uint32_t* M, KArg a) { TE_TID3 radbc<1>(M, a, gx); }
 
-// turb_openbc_flux.wgsl:111-140
-__global__ __launch_bounds__(256) void k_turb_openbc_flux(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  const int n = gx, k = gy;
-  if (k > g.nz) return;
-  float *fx = fq(a.q[1]), *fy = fq(a.q[2]);
-  int openx = ldi(a.q[3], 0), openy = ldi(a.q[3], 1);
-  if (openx != 0 && n <= g.ny) {
-    fx[g.idx(0, n, k)] = fx[g.idx(1, n, k)];
-    fx[g.idx(g.nx, n, k)] = fx[g.idx(g.nx - 1, n, k)];
-  }
-  if (openy != 0 && n <= g.nx) {
-    fy[g.idx(n, 0, k)] = fy[g.idx(n, 1, k)];
-    fy[g.idx(n, g.ny, k)] = fy[g.idx(n, g.ny - 1, k)];
-  }
-}
+__global__ __launch_bounds__(256) void k_turb_openbc_flux(uint32_t* M, KArg a) { turb_openbc_flux_body(M, a, te_block(a)); }
 
 // turb_openbc_stress_x.wgsl:111-137 / turb_openbc_stress_y.wgsl
 template <int DIR>
@@ -130,7 +115,7 @@ __global__ __launch_bounds__(256) void k_turb_openbc_stress_y(uint32_t* M, KArg 
 
 // copy_words (replay.js:403-406): end-of-step state swap copies.
 __global__ __launch_bounds__(256) void k__copy(uint32_t* M, KArg a) {
-  if (te_flat(a, [&](uint32_t w, int width) { st4(a.q[1], w, width, ld4(a.q[0], w, width)); })) return;
+  if (te_flat(a, te_block(a), [&](uint32_t w, int width) { st4(a.q[1], w, width, ld4(a.q[0], w, width)); })) return;
   const uint32_t q = (uint32_t)(te_block(a).x * TE_BX) + threadIdx.x;
   if (q >= a.n[0]) return;
   a.q[1][q] = a.q[0][q];

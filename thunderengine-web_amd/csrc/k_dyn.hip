@@ -4,126 +4,23 @@
 // launch it by name; the thread mapping follows the reference dispatch grid.
 #include "te_device.hpp"
 #include "te_kernels.hpp"
+#include "pointwise.hpp"
 
 namespace te {
 
-// update_diagnostics_moist.wgsl:128-184
-__global__ __launch_bounds__(256) void k_update_diagnostics_moist(uint32_t* M, KArg a) {
-  {
-    const Dims g = dims(a.q[0], 0);
-    if (te_flat_levels(a, (uint32_t)(g.sJ * g.sK), [&](uint32_t w, int width, int k) {
-          if (k >= g.nz) return;
-          const float reps = RV / RD, repsm1 = reps - 1.0f;
-          const float t0 = fq(a.q[3])[k], p0 = fq(a.q[4])[k], qv0k = fq(a.q[5])[k], qc0k = fq(a.q[6])[k],
-                      qi0k = fq(a.q[7])[k], rt0 = fq(a.q[8])[k];
-          const F4 thP = ld4(a.q[1], w, width), ppP = ld4(a.q[2], w, width), qv = ld4(a.q[9], w, width),
-                   qc = ld4(a.q[10], w, width), qr = ld4(a.q[11], w, width), qi = ld4(a.q[12], w, width),
-                   qs = ld4(a.q[13], w, width), qg = ld4(a.q[14], w, width);
-          F4 thv, ppterm, piadv, thterm, buoy;
-          for (int e = 0; e < width; ++e) {
-            const float qvv = mx(qv.v[e], 0.0f);
-            const float liq = qc.v[e] + qr.v[e];
-            const float ice = (qi.v[e] + qs.v[e]) + qg.v[e];
-            const float qli = mx(0.0f, liq + ice);
-            const float cpli = fma_(CPL, mx(0.0f, liq), CPI * mx(0.0f, ice));
-            const float th = t0 + thP.v[e];
-            const float pi = p0 + ppP.v[e];
-            const float cpm = fma_(CPV, qvv, CP) + cpli;
-            const float cvm = 1.0f / (fma_(CVV, qvv, CV) + cpli);
-            thv.v[e] = (th * fma_(reps, qvv, 1.0f)) / ((1.0f + qvv) + qli);
-            piadv.v[e] = pi;
-            ppterm.v[e] = ((pi * ROVCP) * cpm) * cvm;
-            thterm.v[e] = (th * fma_(-ROVCP, cpm, fma_(RV, qvv, RD))) * cvm;
-            buoy.v[e] = GRAV * (fma_(thP.v[e], rt0, repsm1 * (qvv - qv0k)) - ((qli - qc0k) - qi0k));
-          }
-          st4(a.q[15], w, width, thv);
-          st4(a.q[16], w, width, ppterm);
-          st4(a.q[17], w, width, piadv);
-          st4(a.q[18], w, width, thterm);
-          st4(a.q[19], w, width, buoy);
-        }))
-      return;
-  }
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx - 3, j = gy - 3, k = gz;
-  if (i > g.nx + 3 || j > g.ny + 3 || k >= g.nz) return;
-  const float *thP = fq(a.q[1]), *ppP = fq(a.q[2]), *th0 = fq(a.q[3]), *pi0 = fq(a.q[4]),
-              *qv0 = fq(a.q[5]), *qc0 = fq(a.q[6]), *qi0 = fq(a.q[7]), *rth0 = fq(a.q[8]),
-              *qv = fq(a.q[9]), *qc = fq(a.q[10]), *qr = fq(a.q[11]), *qi = fq(a.q[12]),
-              *qs = fq(a.q[13]), *qg = fq(a.q[14]);
-  float *thv = fq(a.q[15]), *ppterm = fq(a.q[16]), *piadv = fq(a.q[17]), *thterm = fq(a.q[18]),
-        *buoy = fq(a.q[19]);
-  int64_t c = g.idx(i, j, k);
-  const float reps = RV / RD, repsm1 = reps - 1.0f;
-  float qvv = mx(qv[c], 0.0f);
-  float liq = qc[c] + qr[c];
-  float ice = (qi[c] + qs[c]) + qg[c];
-  float qli = mx(0.0f, liq + ice);
-  float cpli = fma_(CPL, mx(0.0f, liq), CPI * mx(0.0f, ice));
-  float th = th0[k] + thP[c];
-  float pi = pi0[k] + ppP[c];
-  float cpm = fma_(CPV, qvv, CP) + cpli;
-  float cvm = 1.0f / (fma_(CVV, qvv, CV) + cpli);
-  thv[c] = (th * fma_(reps, qvv, 1.0f)) / ((1.0f + qvv) + qli);
-  piadv[c] = pi;
-  ppterm[c] = ((pi * ROVCP) * cpm) * cvm;
-  thterm[c] = (th * fma_(-ROVCP, cpm, fma_(RV, qvv, RD))) * cvm;
-  buoy[c] = GRAV * (fma_(thP[c], rth0[k], repsm1 * (qvv - qv0[k])) - ((qli - qc0[k]) - qi0[k]));
-}
+__global__ __launch_bounds__(256) void k_update_diagnostics_moist(uint32_t* M, KArg a) { update_diagnostics_moist_body(M, a, te_block(a)); }
 
-// update_diagnostics.wgsl:114-144 (dry)
-__global__ __launch_bounds__(256) void k_update_diagnostics(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx - 3, j = gy - 3, k = gz;
-  if (i > g.nx + 3 || j > g.ny + 3 || k >= g.nz) return;
-  const float *thP = fq(a.q[1]), *ppP = fq(a.q[2]), *th0 = fq(a.q[3]), *pi0 = fq(a.q[4]),
-              *rth0 = fq(a.q[8]);
-  float *thv = fq(a.q[5]), *ppterm = fq(a.q[6]), *piadv = fq(a.q[7]), *buoy = fq(a.q[9]);
-  const float rddcv = RD / (CP - RD);
-  int64_t c = g.idx(i, j, k);
-  float pi = pi0[k] + ppP[c];
-  thv[c] = th0[k] + thP[c];
-  piadv[c] = pi;
-  ppterm[c] = pi * rddcv;
-  buoy[c] = (GRAV * thP[c]) * rth0[k];
-}
+__global__ __launch_bounds__(256) void k_update_diagnostics(uint32_t* M, KArg a) { update_diagnostics_body(M, a, te_block(a)); }
 
-// stage_tendency_reset.wgsl:110-129
-__global__ __launch_bounds__(256) void k_stage_tendency_reset(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx - 3, j = gy - 3, k = gz;
-  if (i > g.nx + 3 || j > g.ny + 3 || k > g.nz) return;
-  int64_t c = g.idx(i, j, k);
-  fq(a.q[1])[c] = 0.0f;
-  fq(a.q[2])[c] = 0.0f;
-  fq(a.q[3])[c] = 0.0f;
-}
+__global__ __launch_bounds__(256) void k_stage_tendency_reset(uint32_t* M, KArg a) { stage_tendency_reset_body(M, a, te_block(a)); }
 
-// stage_state_reset.wgsl:110-138
-__global__ __launch_bounds__(256) void k_stage_state_reset(uint32_t* M, KArg a) {
-  if (te_flat(a, [&](uint32_t w, int width) {
-        const int src[5] = {1, 2, 3, 4, 10};
-        for (int q = 0; q < 5; ++q) st4(a.q[5 + q], w, width, ld4(a.q[src[q]], w, width));
-      }))
-    return;
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx - 3, j = gy - 3, k = gz;
-  if (i > g.nx + 3 || j > g.ny + 3 || k > g.nz) return;
-  int64_t c = g.idx(i, j, k);
-  // u <- u_a, v <- v_a, w <- w_a, pp3d <- ppi, ppd <- ppx
-  const int src[5] = {1, 2, 3, 4, 10};
-  for (int q = 0; q < 5; ++q) fq(a.q[5 + q])[c] = fq(a.q[src[q]])[c];
-}
+__global__ __launch_bounds__(256) void k_stage_state_reset(uint32_t* M, KArg a) { stage_state_reset_body(M, a, te_block(a)); }
 
 // massflux_from_state.wgsl:111-137
 __global__ __launch_bounds__(256) void k_massflux_from_state(uint32_t* M, KArg a) {
   {
     const Dims g = dims(a.q[0], 0);
-    if (te_flat_levels(a, (uint32_t)(g.sJ * g.sK), [&](uint32_t w, int width, int k) {
+    if (te_flat_levels(a, te_block(a), (uint32_t)(g.sJ * g.sK), [&](uint32_t w, int width, int k) {
           if (k < g.nz) {
             const float r = fq(a.q[4])[k];
             F4 u = ld4(a.q[1], w, width), v = ld4(a.q[2], w, width);
@@ -156,38 +53,7 @@ __global__ __launch_bounds__(256) void k_massflux_from_state(uint32_t* M, KArg a
   rrw[c] = (k == 0 || k == g.nz) ? 0.0f : rf0[k] * w[c];
 }
 
-// massflux_from_state then div_massflux (div_massflux.wgsl:125-147) in one
-// launch: each cell stores its mass fluxes and forms the divergence from its
-// own and its i+1, j+1, k+1 neighbours' fluxes, each the product
-// massflux_from_state stores there (so the same bits), instead of reading them
-// back.  p: 1-8 as massflux_from_state's, 9 mh, 10 divx.  Grid: whole.
-__global__ __launch_bounds__(256) void k_massflux_div(uint32_t* M, KArg a) {
-  TE_TID3
-  const Dims g = dims(a.q[0], 0);
-  const int i = gx - 3, j = gy - 3, k = gz;
-  if (i > g.nx + 3 || j > g.ny + 3 || k > g.nz) return;
-  const float *u = fq(a.q[1]), *v = fq(a.q[2]), *w = fq(a.q[3]), *rho0 = fq(a.q[4]), *rf0 = fq(a.q[5]),
-              *mh = fq(a.q[9]), *hm = fq(a.q[30]);
-  const int64_t sj = g.sJ, sk = g.sk(), c = g.idx(i, j, k);
-  auto fw = [&](int kk, int64_t cc) { return (kk == 0 || kk == g.nz) ? 0.0f : rf0[kk] * w[cc]; };
-  const bool div = i <= g.nx + 2 && j <= g.ny + 2 && k < g.nz;
-  const float r = k < g.nz ? rho0[k] : 0.0f;
-  const float uc = k < g.nz ? u[c] : 0.0f, vc = k < g.nz ? v[c] : 0.0f;
-  const float up = div ? u[c + 1] : 0.0f, vp = div ? v[c + sj] : 0.0f;
-  const float mw = fw(k, c), mwp = div ? fw(k + 1, c + sk) : 0.0f;
-  const float mu = r * uc, mv = r * vc;
-  // the divergence formed before the first store (its profile and metric
-  // loads go out with the others)
-  const float d = div ? fma_((mwp - mw) * g.rdz, mh[k],
-                             fma_((r * up - mu) * g.rdx, hm_uh(hm, g, i), ((r * vp - mv) * g.rdy) * hm_vh(hm, g, j)))
-                      : 0.0f;
-  if (k < g.nz) {
-    fq(a.q[6])[c] = mu;
-    fq(a.q[7])[c] = mv;
-  }
-  fq(a.q[8])[c] = mw;
-  if (div) fq(a.q[10])[c] = d;
-}
+__global__ __launch_bounds__(256) void k_massflux_div(uint32_t* M, KArg a) { massflux_div_body(M, a, te_block(a)); }
 
 // After the stage's substeps: divergence3d of the mean velocities,
 // velocity_to_massflux, div_massflux of the fluxes and build_sadv
@@ -230,7 +96,7 @@ __global__ __launch_bounds__(256) void k_mean_massflux(uint32_t* M, KArg a) {
 __global__ __launch_bounds__(256) void k_velocity_to_massflux(uint32_t* M, KArg a) {
   {
     const Dims g = dims(a.q[0], 0);
-    if (te_flat_levels(a, (uint32_t)(g.sJ * g.sK), [&](uint32_t w, int width, int k) {
+    if (te_flat_levels(a, te_block(a), (uint32_t)(g.sJ * g.sK), [&](uint32_t w, int width, int k) {
           if (k < g.nz) {
             const float r = fq(a.q[1])[k];
             F4 u = ld4(a.q[3], w, width), v = ld4(a.q[4], w, width);
@@ -318,27 +184,7 @@ __global__ __launch_bounds__(256) void k_rk_update(uint32_t* M, KArg a) {
   phi[c] = fma_(dttmp, tend[c], phiA[c]);
 }
 
-// build_sadv.wgsl:111-127
-__global__ __launch_bounds__(256) void k_build_sadv(uint32_t* M, KArg a) {
-  {
-    const Dims g = dims(a.q[0], 0);
-    if (te_flat_levels(a, (uint32_t)(g.sJ * g.sK), [&](uint32_t w, int width, int k) {
-          if (k >= g.nz) return;
-          const float t0 = fq(a.q[1])[k] - 3e+02f;
-          F4 s = ld4(a.q[2], w, width);
-          for (int e = 0; e < width; ++e) s.v[e] = t0 + s.v[e];
-          st4(a.q[3], w, width, s);
-        }))
-      return;
-  }
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx - 3, j = gy - 3, k = gz;
-  if (i > g.nx + 3 || j > g.ny + 3 || k >= g.nz) return;
-  const float *th0 = fq(a.q[1]), *thP = fq(a.q[2]);
-  int64_t c = g.idx(i, j, k);
-  fq(a.q[3])[c] = (th0[k] - 3e+02f) + thP[c];
-}
+__global__ __launch_bounds__(256) void k_build_sadv(uint32_t* M, KArg a) { build_sadv_body(M, a, te_block(a)); }
 
 // apply_thterm.wgsl:111-127
 __global__ __launch_bounds__(256) void k_apply_thterm(uint32_t* M, KArg a) {
@@ -394,16 +240,7 @@ __global__ __launch_bounds__(256) void k_ppx_finish(uint32_t* M, KArg a) {
   float* ppx = fq(a.q[2]);
   ppx[c] = fq(a.q[1])[c] + ppx[c];
 }
-// ppx_finish, then the halo fill of ppx on a periodic domain (nx, ny >= 4;
-// timestep.js:1593 haloFill): each cell writes its periodic images.
-__global__ __launch_bounds__(256) void k_ppx_finish_xy(uint32_t* M, KArg a) {
-  TE_TID3
-  const Dims g = dims(a.q[0], 0);
-  if (gx >= g.nx || gy >= g.ny || gz >= g.nz) return;
-  const float* pp = fq(a.q[1]);
-  float* ppx = fq(a.q[2]);
-  update_with_halo(g, open_sides(a, 3), ppx, gx, gy, gz, 0, [&](int64_t c) { return pp[c] + ppx[c]; });
-}
+__global__ __launch_bounds__(256) void k_ppx_finish_xy(uint32_t* M, KArg a) { ppx_finish_xy_body(M, a, te_block(a)); }
 
 // diabatic_unapply.wgsl:111-140
 __global__ __launch_bounds__(256) void k_diabatic_unapply(uint32_t* M, KArg a) {
@@ -420,81 +257,11 @@ __global__ __launch_bounds__(256) void k_diabatic_unapply(uint32_t* M, KArg a) {
   }
 }
 
-// diabatic_rates.wgsl:111-137
-__global__ __launch_bounds__(256) void k_diabatic_rates(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  if (gx >= g.nx || gy >= g.ny || gz >= g.nz) return;
-  float dt = ldf(a.q[1], 0);
-  float rdt = 1.0f / dt;
-  int64_t c = g.idx(gx, gy, gz);
-  for (int q = 0; q < 4; ++q) {
-    const float* s = fq(a.q[2 + q]);
-    float* r = fq(a.q[6 + q]);
-    r[c] = (s[c] - r[c]) * rdt;
-  }
-}
+__global__ __launch_bounds__(256) void k_diabatic_rates(uint32_t* M, KArg a) { diabatic_rates_body(M, a, te_block(a)); }
 
-// pressure_tendency.wgsl:234-291
-__global__ __launch_bounds__(256) void k_pressure_tendency(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  if (gx >= g.nx || gy >= g.ny || gz >= g.nz) return;
-  const float *th = fq(a.q[1]), *qv = fq(a.q[2]), *rho = fq(a.q[3]), *ppi = fq(a.q[4]),
-              *thten = fq(a.q[5]), *qpten = fq(a.q[6]), *th0 = fq(a.q[7]), *pi0 = fq(a.q[8]),
-              *qvt = fq(a.q[13]);
-  float* ppten = fq(a.q[11]);
-  float dt = ldf(a.q[9], 0);
-  int hasDiabatic = ldi(a.q[10], 0), hasStepTend = ldi(a.q[12], 0), moist = ldi(a.q[14], 0);
-  const int k = gz;
-  int64_t c = g.idx(gx, gy, gz);
-  const float rp00 = 1.0f / P00, rddcv = RD / (CP - RD);
-  float tem = 0.0001f * 0.0001f;
-  float tht = hasStepTend != 0 ? thten[c] : 0.0f;
-  if (moist == 0) {
-    float p = 0.0f;
-    if (ab(dt * tht) > tem) {
-      float thnew = fma_(dt, tht, th[c]);
-      float pinew = fast_pow(((rho[c] * (th0[k] + thnew)) * RD) * rp00, rddcv) - pi0[k];
-      p = (pinew - ppi[c]) / dt;
-    }
-    ppten[c] = p;
-    return;
-  }
-  float qvten = qvt[c];
-  // every operand loaded with the tendencies (one wait for memory), whether
-  // or not the cell takes the update
-  const float thc = th[c], qvc = qv[c], rhoc = rho[c], ppic = ppi[c], qp = hasDiabatic != 0 ? qpten[c] : 0.0f;
-  float p = 0.0f;
-  if (ab(dt * tht) > tem || ab(dt * qvten) > 1e-14f) {
-    float thnew = fma_(dt, tht, thc);
-    float qvnew = fma_(dt, qvten, qvc);
-    float pinew = fast_pow(((rhoc * (th0[k] + thnew)) * fma_(RV, qvnew, RD)) * rp00, rddcv) - pi0[k];
-    p = (pinew - ppic) / dt;
-  }
-  if (hasDiabatic != 0) p = p + qp;
-  ppten[c] = p;
-}
+__global__ __launch_bounds__(256) void k_pressure_tendency(uint32_t* M, KArg a) { pressure_tendency_body(M, a, te_block(a)); }
 
-// update_rho_prs.wgsl:234-267
-__global__ __launch_bounds__(256) void k_update_rho_prs(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  if (gx >= g.nx || gy >= g.ny || gz >= g.nz) return;
-  int moist = ldi(a.q[1], 0);
-  const float *thP = fq(a.q[2]), *ppP = fq(a.q[3]), *th0 = fq(a.q[4]), *pi0 = fq(a.q[5]),
-              *qv = fq(a.q[6]);
-  float *prs = fq(a.q[7]), *rho = fq(a.q[8]);
-  const int k = gz;
-  int64_t c = g.idx(gx, gy, gz);
-  const float cpdrd = CP / RD;
-  float pi = pi0[k] + ppP[c];
-  float th = th0[k] + thP[c];
-  float p = P00 * fast_pow(pi, cpdrd);
-  prs[c] = p;
-  float rmix = moist != 0 ? fma_(mx(0.0f, qv[c]), RV, RD) : RD;
-  rho[c] = p / ((th * pi) * rmix);
-}
+__global__ __launch_bounds__(256) void k_update_rho_prs(uint32_t* M, KArg a) { update_rho_prs_body(M, a, te_block(a)); }
 
 // stability_max.wgsl:120-178 (adapt_dt = 1): max over the grid of the
 // squared advective Courant number c2 = x^2 + y^2 + z^2 (x = (u_i + u_i+1)

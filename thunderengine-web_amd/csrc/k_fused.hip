@@ -5,6 +5,7 @@
 #include <type_traits>
 
 #include "te_kernels.hpp"
+#include "pointwise.hpp"
 
 namespace te {
 
@@ -102,71 +103,17 @@ __global__ __launch_bounds__(256) void k_bc_open_xy(uint32_t* M, KArg a) {
     if (fill[q]) fq(a.q[1 + q])[dst] = v[q];
 }
 
-// rk_update of a scalar (stagger 1) then its halo fill (rk_update.wgsl:111-132,
-// timestep.js:1593 haloFill); arguments as rk_update's, 6 -> open x, open y.
-TE_DEV void rk_update_xy_body(uint32_t* M, const KArg& a, const Blk blk) {
-  int gx, gy, gz;
-  te_tid3(a, blk, gx, gy, gz);
-  const Dims g = dims(a.q[0], 0);
-  const int i = gx, j = gy, k = gz;
-  if (i >= g.nx || j >= g.ny || k >= g.nz) return;
-  const float *phiA = fq(a.q[2]), *tend = fq(a.q[3]);
-  const float dttmp = ldf(a.q[5], 0);
-  update_with_halo(g, open_sides(a, 6), fq(a.q[4]), i, j, k, 0, [&](int64_t c) { return fma_(dttmp, tend[c], phiA[c]); });
-}
 __global__ __launch_bounds__(256) void k_rk_update_xy(uint32_t* M, KArg a) { rk_update_xy_body(M, a, te_block(a)); }
-// the scalars of a stage in one launch
-__global__ __launch_bounds__(256) void k_rk_update_xy_batch(uint32_t* M, KBatch) {
-  const BatchPart p = te_batch_part();
-  if (p.in) rk_update_xy_body(M, p.a, te_block_at(p.a, p.w));
-}
 
-// tke_advance (levels 1 .. nz-1) then the halo fill of tke
-// (tke_advance.wgsl:111-129, timestep.js:1593 haloFill); arguments as
-// tke_advance's, 5 -> open x, open y.
-__global__ __launch_bounds__(256) void k_tke_advance_xy(uint32_t* M, KArg a) {
-  TE_TID3
-  const Dims g = dims(a.q[0], 0);
-  const int i = gx, j = gy, k = gz + 1;
-  if (i >= g.nx || j >= g.ny || k > g.nz - 1) return;
-  const float *tkea = fq(a.q[1]), *tketen = fq(a.q[2]);
-  const float dttmp = ldf(a.q[3], 0);
-  update_with_halo(g, open_sides(a, 5), fq(a.q[4]), i, j, k, 1, [&](int64_t c) {
-    const float v = fma_(dttmp, tketen[c], tkea[c]);
-    return (v < 1e-10f) ? 0.0f : v;
-  });
-}
+__global__ __launch_bounds__(256) void k_tke_advance_xy(uint32_t* M, KArg a) { tke_advance_xy_body(M, a, te_block(a)); }
 
-// turb_zero (turb_zero.wgsl, timestep.js:1070-1072) of up to 8 fields in one
-// launch over the whole grid [strideJ, strideK, nz+1].  p[1..8] fields,
-// p[9] -> field count.
-__global__ __launch_bounds__(256) void k_zero_fields(uint32_t* M, KArg a) {
-  if (te_flat(a, [&](uint32_t w, int width) {
-        const int n = ldi(a.q[9], 0);
-        F4 z;
-        z.v[0] = z.v[1] = z.v[2] = z.v[3] = 0.0f;
-        for (int q = 0; q < 8; ++q) {
-          if (q >= n) break;
-          st4(a.q[1 + q], w, width, z);
-        }
-      }))
-    return;
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  if (gx >= g.sJ || gy >= g.sK || gz > g.nz) return;
-  const int64_t c = gx + (int64_t)g.sJ * (gy + (int64_t)g.sK * gz);
-  const int n = ldi(a.q[9], 0);
-  for (int q = 0; q < 8; ++q) {
-    if (q >= n) break;
-    fq(a.q[1 + q])[c] = 0.0f;
-  }
-}
+__global__ __launch_bounds__(256) void k_zero_fields(uint32_t* M, KArg a) { zero_fields_body(M, a, te_block(a)); }
 
 // turb_add_tendency (dst = fma(scale, src, dst) over the whole grid) for up
 // to 4 independent triples: p[1..4] sources, p[5..8] destinations,
 // p[9..12] -> scales, p[13] -> count.
 __global__ __launch_bounds__(256) void k_add_fields(uint32_t* M, KArg a) {
-  if (te_flat(a, [&](uint32_t w, int width) {
+  if (te_flat(a, te_block(a), [&](uint32_t w, int width) {
         const int n = ldi(a.q[13], 0);
         for (int q = 0; q < 4; ++q) {
           if (q >= n) break;
@@ -191,48 +138,9 @@ __global__ __launch_bounds__(256) void k_add_fields(uint32_t* M, KArg a) {
   }
 }
 
-// stage_tendency_reset (stage_tendency_reset.wgsl:111-129) followed by
-// turb_add_tendency of the three SGS / damping momentum tendencies:
-// dst = fma(scale, src, 0), the bits of adding src*scale to the cleared field.
-// p: 1-3 uten vten wten, 4-6 their sources, 7 -> scale.  Grid: whole.
-__global__ __launch_bounds__(256) void k_tendency_reset_add(uint32_t* M, KArg a) {
-  if (te_flat(a, [&](uint32_t w, int width) {
-        const float sc = ldf(a.q[7], 0);
-        for (int q = 0; q < 3; ++q) {
-          F4 d = ld4(a.q[4 + q], w, width);
-          for (int e = 0; e < width; ++e) d.v[e] = fma_(sc, d.v[e], 0.0f);
-          st4(a.q[1 + q], w, width, d);
-        }
-      }))
-    return;
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx - 3, j = gy - 3, k = gz;
-  if (i > g.nx + 3 || j > g.ny + 3 || k > g.nz) return;
-  const int64_t c = g.idx(i, j, k);
-  const float scale = ldf(a.q[7], 0);
-  for (int q = 0; q < 3; ++q) fq(a.q[1 + q])[c] = fma_(scale, fq(a.q[4 + q])[c], 0.0f);
-}
+__global__ __launch_bounds__(256) void k_tendency_reset_add(uint32_t* M, KArg a) { tendency_reset_add_body(M, a, te_block(a)); }
 
-// Up to 4 buffer copies of a.n[0] words each (the state swap of
-// timestep.js:766-774): p[1..4] sources, p[5..8] destinations, p[9] -> count.
-__global__ __launch_bounds__(256) void k_copy_fields(uint32_t* M, KArg a) {
-  if (te_flat(a, [&](uint32_t w, int width) {
-        const int n = ldi(a.q[9], 0);
-        for (int f = 0; f < 4; ++f) {
-          if (f >= n) break;
-          st4(a.q[5 + f], w, width, ld4(a.q[1 + f], w, width));
-        }
-      }))
-    return;
-  const uint32_t q = (uint32_t)(te_block(a).x * TE_BX) + threadIdx.x;
-  if (q >= a.n[0]) return;
-  const int n = ldi(a.q[9], 0);
-  for (int f = 0; f < 4; ++f) {
-    if (f >= n) break;
-    a.q[5 + f][q] = a.q[1 + f][q];
-  }
-}
+__global__ __launch_bounds__(256) void k_copy_fields(uint32_t* M, KArg a) { copy_fields_body(M, a, te_block(a)); }
 
 // ---- acoustic substep
 // acoustic_pp (acoustic_pp.wgsl:131-167) at interior points, then

@@ -3,6 +3,7 @@
 // tridiagonal sweep carried in registers.
 #include "te_device.hpp"
 #include "te_kernels.hpp"
+#include "pointwise.hpp"
 
 // Column sweeps load TS_CHUNK levels ahead of their serial arithmetic.
 #ifndef TS_CHUNK
@@ -11,366 +12,24 @@
 
 namespace te {
 
-// rayleigh_damping.wgsl:111-164
-__global__ __launch_bounds__(256) void k_rayleigh_damping(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx, j = gy, k = gz;
-  if (i > g.nx || j > g.ny || k > g.nz) return;
-  const float *u = fq(a.q[1]), *v = fq(a.q[2]), *w = fq(a.q[3]), *th = fq(a.q[4]), *u0 = fq(a.q[5]),
-              *v0 = fq(a.q[6]), *tauh = fq(a.q[7]), *tauf = fq(a.q[8]), *hdx = fq(a.q[14]),
-              *hdy = fq(a.q[15]), *avg = fq(a.q[18]), *th0 = fq(a.q[19]);
-  float *uten = fq(a.q[10]), *vten = fq(a.q[11]), *wten = fq(a.q[12]), *thten = fq(a.q[13]);
-  float rdalpha = ldf(a.q[9], 0);
-  int lateral = ldi(a.q[16], 0), toAverage = ldi(a.q[17], 0);
-  const int64_t c = g.idx(i, j, k);
-  // the four fields loaded before the first store (the loads go out together)
-  const float uc = u[c], vc = v[c], thc = th[c], wc = w[c];
-  if (k < g.nz) {
-    float t = tauh[k];
-    float ur = toAverage != 0 ? avg[k] : u0[k];
-    float vr = toAverage != 0 ? avg[g.nz + k] : v0[k];
-    if (j < g.ny) uten[c] = ((-rdalpha) * t) * (uc - ur);
-    if (i < g.nx) vten[c] = ((-rdalpha) * t) * (vc - vr);
-    if (i < g.nx && j < g.ny) {
-      float d = toAverage != 0 ? (th0[k] - avg[2 * g.nz + k]) + thc : thc;
-      thten[c] = ((-rdalpha) * t) * d;
-    }
-  }
-  if (i < g.nx && j < g.ny) {
-    float tf = tauf[k];
-    if (lateral != 0 && k < g.nz) tf = mx(mx(tf, hdx[i]), hdy[j]);
-    wten[c] = ((-rdalpha) * tf) * wc;
-  }
-}
+__global__ __launch_bounds__(256) void k_rayleigh_damping(uint32_t* M, KArg a) { rayleigh_damping_body(M, a, te_block(a)); }
 
-// turb_rho_faces.wgsl:111-151
-__global__ __launch_bounds__(256) void k_turb_rho_faces(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx - 2, j = gy - 2, k = gz;
-  if (i > g.nx + 1 || j > g.ny + 1 || k > g.nz) return;
-  const float *rho = fq(a.q[1]), *c1 = fq(a.q[2]), *c2 = fq(a.q[3]);
-  float *rr = fq(a.q[4]), *rf = fq(a.q[5]);
-  const uint32_t *os = a.q[6], *ot = a.q[7];
-  const int64_t sk = g.sk(), c = g.idx(i, j, k);
-  // rf formed before either store (the loads go out together)
-  float r;
-  if (k == 0) {
-    r = fma_(ldf(os, 0), rho[c], ldf(os, 1) * rho[c + sk]);
-    if (g.nz >= 3) r = fma_(ldf(os, 2), rho[c + 2 * sk], r);
-  } else if (k == g.nz) {
-    r = fma_(ldf(ot, 0), rho[c - sk], ldf(ot, 1) * rho[c - 2 * sk]);
-    if (g.nz >= 3) r = fma_(ldf(ot, 2), rho[c - 3 * sk], r);
-  } else {
-    r = fma_(c1[k], rho[c - sk], c2[k] * rho[c]);
-  }
-  if (k < g.nz) rr[c] = 1.0f / rho[c];
-  rf[c] = r;
-}
+__global__ __launch_bounds__(256) void k_turb_rho_faces(uint32_t* M, KArg a) { turb_rho_faces_body(M, a, te_block(a)); }
 
-// turb_def_centers.wgsl:139-168
-__global__ __launch_bounds__(256) void k_turb_def_centers(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx - 1, j = gy - 1, k = gz;
-  if (i > g.nx + 1 || j > g.ny + 1 || k >= g.nz) return;
-  const float *u = fq(a.q[1]), *v = fq(a.q[2]), *w = fq(a.q[3]), *rho = fq(a.q[4]), *mh = fq(a.q[5]),
-              *hm = fq(a.q[30]);
-  const int64_t sj = g.sJ, sk = g.sk(), c = g.idx(i, j, k);
-  // every value formed before the first store (the loads go out together)
-  const float r0 = rho[c];
-  const float s11 = ((r0 * (u[c + 1] - u[c])) * g.rdx) * hm_uh(hm, g, i);
-  const float s22 = ((r0 * (v[c + sj] - v[c])) * g.rdy) * hm_vh(hm, g, j);
-  const float s33 = ((r0 * (w[c + sk] - w[c])) * g.rdz) * mh[k];
-  const float rcorner = 0.25f * ((rho[c - 1 - sj] + r0) + (rho[c - 1] + rho[c - sj]));
-  const float s12 =
-      (0.5f * fma_((u[c] - u[c - sj]) * g.rdy, hm_vf(hm, g, j), ((v[c] - v[c - 1]) * g.rdx) * hm_uf(hm, g, i))) * rcorner;
-  fq(a.q[6])[c] = s11;
-  fq(a.q[7])[c] = s22;
-  fq(a.q[8])[c] = s33;
-  fq(a.q[9])[c] = s12;
-}
+__global__ __launch_bounds__(256) void k_turb_def_centers(uint32_t* M, KArg a) { turb_def_centers_body(M, a, te_block(a)); }
 
-// turb_def_faces.wgsl:125-151
-__global__ __launch_bounds__(256) void k_turb_def_faces(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx, j = gy, k = gz + 1;
-  if (i > g.nx + 1 || j > g.ny + 1 || k > g.nz - 1) return;
-  const float *u = fq(a.q[1]), *v = fq(a.q[2]), *w = fq(a.q[3]), *rf = fq(a.q[4]), *mf = fq(a.q[5]),
-              *hm = fq(a.q[30]);
-  const int64_t sj = g.sJ, sk = g.sk(), c = g.idx(i, j, k);
-  float mfu = 0.5f * (mf[k] + mf[k]);
-  float mfv = 0.5f * (mf[k] + mf[k]);
-  // both values formed before the first store
-  const float s13 =
-      ((0.5f * fma_((w[c] - w[c - 1]) * g.rdx, hm_uf(hm, g, i), ((u[c] - u[c - sk]) * g.rdz) * mfu)) * 0.5f) * (rf[c - 1] + rf[c]);
-  const float s23 =
-      ((0.5f * fma_((w[c] - w[c - sj]) * g.rdy, hm_vf(hm, g, j), ((v[c] - v[c - sk]) * g.rdz) * mfv)) * 0.5f) * (rf[c - sj] + rf[c]);
-  fq(a.q[6])[c] = s13;
-  fq(a.q[7])[c] = s23;
-}
+__global__ __launch_bounds__(256) void k_turb_def_faces(uint32_t* M, KArg a) { turb_def_faces_body(M, a, te_block(a)); }
 
-// turb_def_assemble.wgsl:111-149
-__global__ __launch_bounds__(256) void k_turb_def_assemble(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx, j = gy, k = gz + 1;
-  if (i >= g.nx || j >= g.ny || k > g.nz - 1) return;
-  const float *s11 = fq(a.q[1]), *s22 = fq(a.q[2]), *s33 = fq(a.q[3]), *s12 = fq(a.q[4]),
-              *s13 = fq(a.q[5]), *s23 = fq(a.q[6]), *c1 = fq(a.q[7]), *c2 = fq(a.q[8]), *rf = fq(a.q[9]);
-  const int64_t sj = g.sJ, sk = g.sk(), c = g.idx(i, j, k);
-  float A = c1[k], B = c2[k];
-  float t11 = fma_(A * s11[c - sk], s11[c - sk], (B * s11[c]) * s11[c]);
-  float t22 = fma_(A * s22[c - sk], s22[c - sk], (B * s22[c]) * s22[c]);
-  float t33 = fma_(A * s33[c - sk], s33[c - sk], (B * s33[c]) * s33[c]);
-  auto sq2 = [&](int64_t p, int64_t q) { return fma_(s12[p], s12[p], s12[q] * s12[q]); };
-  float lo = sq2(c - sk, c + 1 + sj - sk) + sq2(c + sj - sk, c + 1 - sk);
-  float hi = sq2(c, c + 1 + sj) + sq2(c + sj, c + 1);
-  float t12 = 0.25f * fma_(A, lo, B * hi);
-  float t13 = 0.5f * fma_(s13[c], s13[c], s13[c + 1] * s13[c + 1]);
-  float t23 = 0.5f * fma_(s23[c], s23[c], s23[c + sj] * s23[c + sj]);
-  float rrf = 1.0f / (rf[c] * rf[c]);
-  fq(a.q[10])[c] = (4.0f * (t13 + t23)) * rrf;
-  fq(a.q[11])[c] = fma_(2.0f, (t11 + t22) + t33, 4.0f * t12) * rrf;
-}
+__global__ __launch_bounds__(256) void k_turb_def_assemble(uint32_t* M, KArg a) { turb_def_assemble_body(M, a, te_block(a)); }
 
-// saturation mixing ratios over liquid / ice (turb_nm.wgsl:204-230)
-TE_DEV float mp_rslf(float p, float t) {
-  float esl = 611.2f * fast_exp((17.67f * (t - 273.15f)) / (t - 29.65f));
-  esl = mn(esl, p * 0.5f);
-  return ((RD / RV) * esl) / (p - esl);
-}
-TE_DEV float mp_rsif(float p, float t) {
-  float esi = 611.2f * fast_exp((21.874557f * (t - 273.15f)) / (t - 7.66f));
-  esi = mn(esi, p * 0.5f);
-  return ((RD / RV) * esi) / (p - esi);
-}
+__global__ __launch_bounds__(256) void k_turb_nm(uint32_t* M, KArg a) { turb_nm_body(M, a, te_block(a)); }
 
-// turb_nm.wgsl:236-355 (moist squared buoyancy frequency)
-__global__ __launch_bounds__(256) void k_turb_nm(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx, j = gy, k = gz + 1;
-  if (i >= g.nx || j >= g.ny || k > g.nz - 1) return;
-  const float *thP = fq(a.q[1]), *ppP = fq(a.q[2]), *th0 = fq(a.q[3]), *pi0 = fq(a.q[4]),
-              *prs = fq(a.q[5]), *qv = fq(a.q[6]), *qc = fq(a.q[7]), *qr = fq(a.q[8]), *qi = fq(a.q[9]),
-              *qs = fq(a.q[10]), *qg = fq(a.q[11]), *c1 = fq(a.q[12]), *c2 = fq(a.q[13]), *mf = fq(a.q[14]);
-  float *nm = fq(a.q[15]), *sat = fq(a.q[17]);
-  int moist = ldi(a.q[16], 0), wantSat = ldi(a.q[18], 0);
-  const int64_t sk = g.sk(), c = g.idx(i, j, k);
-  const float nmsat = 1e-10f, eps = RD / RV, reps = RV / RD, gAcc = 9.81f;
-  const float LV1 = 3134708.0f, LV2 = 2.32e+03f, LS1 = 2898463.5f, LS2 = 236.0f;
-  float thA = th0[k - 1] + thP[c - sk];
-  float thB = th0[k] + thP[c];
-  if (moist == 0) {
-    if (wantSat != 0) sat[c] = 0.0f;
-    nm[c] = ((fast_log(thB / thA) * gAcc) * g.rdz) * mf[k];
-    return;
-  }
-  float piA = pi0[k - 1] + ppP[c - sk], piB = pi0[k] + ppP[c];
-  float tA = thA * piA, tB = thB * piB;
-  float qtA = ((((qv[c - sk] + qc[c - sk]) + qr[c - sk]) + qi[c - sk]) + qs[c - sk]) + qg[c - sk];
-  float qtB = ((((qv[c] + qc[c]) + qr[c]) + qi[c]) + qs[c]) + qg[c];
-  float qciA = (qv[c - sk] + qc[c - sk]) + qi[c - sk];
-  float qciB = (qv[c] + qc[c]) + qi[c];
-  float thvA = (thA * fma_(reps, qv[c - sk], 1.0f)) / (1.0f + qtA);
-  float thvB = (thB * fma_(reps, qv[c], 1.0f)) / (1.0f + qtB);
-  float rmf = g.rdz * mf[k];
-  float A = c1[k], B = c2[k];
-  float pavg = fma_(A, prs[c - sk], B * prs[c]);
-  float tavg = fma_(A, tA, B * tB);
-  float qtavg = fma_(A, qtA, B * qtB);
-  float qciavg = fma_(A, qciA, B * qciB);
-  // The three temperature ranges only choose lam's operands (liquid, ice, or
-  // both blended by ff); lam and the logarithms it needs are evaluated once,
-  // below, for the saturated points alone.
-  bool satd = false, blend = false;
-  float qvs1 = 0.0f, lh1 = 0.0f, drdt1 = 0.0f, qvs2 = 0.0f, lh2 = 0.0f, drdt2 = 0.0f, cpml = 0.0f, ff = 0.0f;
-  if (tavg >= 273.15f) {
-    float qvs = mp_rslf(pavg, tavg);
-    float ql = mx(qciavg - qvs, 0.0f);
-    if (ql > nmsat) {
-      satd = true;
-      float qvl = mx(qciavg - ql, 0.0f);
-      cpml = fma_(CPL, ql, fma_(CPV, qvl, CP));
-      qvs1 = qvs;
-      lh1 = fma_(-LV2, tavg, LV1);
-      drdt1 = ((17.67f * (273.15f - 29.65f)) * qvs) / ((tavg - 29.65f) * (tavg - 29.65f));
-    }
-  } else if (tavg <= 233.15f) {
-    float qvs = mp_rsif(pavg, tavg);
-    float qice = mx(qciavg - qvs, 0.0f);
-    if (qice > nmsat) {
-      satd = true;
-      float qvl = mx(qciavg - qice, 0.0f);
-      cpml = fma_(CPI, qice, fma_(CPV, qvl, CP));
-      qvs1 = qvs;
-      lh1 = fma_(-LS2, tavg, LS1);
-      drdt1 = ((21.874557f * (273.15f - 7.66f)) * qvs) / ((tavg - 7.66f) * (tavg - 7.66f));
-    }
-  } else {
-    ff = (tavg - 233.15f) / (273.15f - 233.15f);
-    float qvsl = mp_rslf(pavg, tavg), qvsi = mp_rsif(pavg, tavg);
-    float qvs = fma_(ff, qvsl, (1.0f - ff) * qvsi);
-    float qice = mx(0.0f, (1.0f - ff) * (qciavg - qvs));
-    float ql = mx(0.0f, ff * (qciavg - qvs));
-    if (ql + qice > nmsat) {
-      satd = blend = true;
-      float qvl = mx(0.0f, (qciavg - ql) - qice);
-      cpml = fma_(CPI, qice, fma_(CPL, ql, fma_(CPV, qvl, CP)));
-      qvs1 = qvsl;
-      lh1 = fma_(-LV2, tavg, LV1);
-      drdt1 = ((17.67f * (273.15f - 29.65f)) * qvsl) / ((tavg - 29.65f) * (tavg - 29.65f));
-      qvs2 = qvsi;
-      lh2 = fma_(-LS2, tavg, LS1);
-      drdt2 = ((21.874557f * (273.15f - 7.66f)) * qvsi) / ((tavg - 7.66f) * (tavg - 7.66f));
-    }
-  }
-  if (wantSat != 0) sat[c] = satd ? 1.0f : 0.0f;
-  float out;
-  if (satd) {
-    const float dlnT = fast_log(tB / tA) * rmf;
-    const float dlnQt = fast_log((1.0f + qtB) / (1.0f + qtA)) * rmf;
-    auto lam = [&](float qvs, float lh, float drdt) {
-      float gamma = ((gAcc * (1.0f + qtavg)) * (1.0f + (lh * qvs) / (RD * tavg))) / fma_(lh, drdt, cpml);
-      return gAcc * fma_(dlnT + gamma / tavg, 1.0f + (tavg * drdt) / (eps + qvs), -dlnQt);
-    };
-    const float n1 = lam(qvs1, lh1, drdt1);
-    out = blend ? fma_(ff, n1, (1.0f - ff) * lam(qvs2, lh2, drdt2)) : n1;
-  } else {
-    out = (gAcc * fast_log(thvB / thvA)) * rmf;
-  }
-  nm[c] = out;
-}
+__global__ __launch_bounds__(256) void k_turb_km_kh(uint32_t* M, KArg a) { turb_km_kh_at<false>(M, a, te_block(a)); }
+__global__ __launch_bounds__(256) void k_turb_km_kh_xy(uint32_t* M, KArg a) { turb_km_kh_at<true>(M, a, te_block(a)); }
 
-// turb_km_kh.wgsl:125-187; IMG: then the halo fill of kmh, kmv, khh, khv on
-// a periodic domain (nx, ny >= 4; timestep.js:1593 haloFill): each cell
-// writes its periodic images, the cells of levels 1 and nz-1 also the images
-// of levels 0 and nz (not written here; no thread of the launch reads K).
-template <bool IMG>
-__device__ __forceinline__ void turb_km_kh_body(uint32_t* M, const KArg& a) {
-  TE_TID3
-  const Dims g = dims(a.q[0], 0);
-  int i = gx, j = gy, k = gz + 1;
-  if (i >= g.nx || j >= g.ny || k > g.nz - 1) return;
-  const float *tkea = fq(a.q[1]), *nm = fq(a.q[2]), *mf = fq(a.q[3]), *hm = fq(a.q[30]);
-  float *kmh = fq(a.q[4]), *kmv = fq(a.q[5]), *khh = fq(a.q[6]), *khv = fq(a.q[7]), *lenscl = fq(a.q[8]),
-        *dissten = fq(a.q[9]);
-  float kmScale = ldf(a.q[10], 0), kmFixed = ldf(a.q[11], 0), turbfac = ldf(a.q[12], 0);
-  const int64_t c = g.idx(i, j, k);
-  const float c_m = 0.1f, c_l = 0.8165f, ri_c = 0.25f, tke_min = 1e-10f, nm_min = 1e-06f, small_len_frac = 0.001f;
-  float cmz = mx(0.001f, turbfac * c_m);
-  float ce1z = ((cmz * c_l) * c_l) * (1.0f / ri_c - 1.0f);
-  float ce2z = mx(0.0f, fma_(cmz * 3.1415927f, 3.1415927f, -ce1z));
-  float dzk = (1.0f / g.rdz) / mf[k];
-  float grdscl = fast_pow((((1.0f / g.rdx) / hm_uh(hm, g, i)) * ((1.0f / g.rdy) / hm_vh(hm, g, j))) * dzk, 0.33333334f);
-  float rgrdscl = 1.0f / grdscl;
-  // the cell's operands, loaded once before the stores below
-  const float tkc = tkea[c], nmc = nm[c], dissc = dissten[c];
-  float tk, len;
-  if (tkc <= tke_min) {
-    tk = tke_min;
-    len = small_len_frac * grdscl;
-  } else {
-    tk = tkc;
-    len = grdscl;
-    if (nmc > nm_min) {
-      len = c_l * sqrtf(tk / nmc);
-      len = mn(len, grdscl);
-      len = mx(len, small_len_frac * grdscl);
-    }
-  }
-  lenscl[c] = len;
-  dissten[c] = dissc + ((fma_(ce2z * len, rgrdscl, ce1z) * tk) * sqrtf(tk)) / len;
-  float km = kmFixed > 0.0f ? kmFixed : ((cmz * sqrtf(tk)) * len) * kmScale;
-  kmh[c] = km;
-  kmv[c] = km;
-  float prinv = 3.0f;
-  if (nmc > nm_min) prinv = mn(fma_(2.0f * len, rgrdscl, 1.0f), 3.0f);
-  khh[c] = km * prinv;
-  khv[c] = km * prinv;
-  if (IMG) {
-    float* F[4] = {kmh, kmv, khh, khv};
-    const float v[4] = {km, km, km * prinv, km * prinv};
-    const int64_t sk = g.sk(), e = k == 1 ? -sk : (k == g.nz - 1 ? sk : 0);
-    const int64_t e2 = k == 1 && k == g.nz - 1 ? sk : 0;  // nz = 2: level 1 is next to both
-    float ev[4], ev2[4];
-    for (int q = 0; q < 4; ++q) {
-      ev[q] = e != 0 ? F[q][c + e] : 0.0f;
-      ev2[q] = e2 != 0 ? F[q][c + e2] : 0.0f;
-    }
-    for (int q = 0; q < 4; ++q) {
-      halo_from<false>(g, {false, false}, F[q], i, j, c, v[q], {});
-      if (e != 0) halo_from<false>(g, {false, false}, F[q], i, j, c + e, ev[q], {});
-      if (e2 != 0) halo_from<false>(g, {false, false}, F[q], i, j, c + e2, ev2[q], {});
-    }
-  }
-}
-__global__ __launch_bounds__(256) void k_turb_km_kh(uint32_t* M, KArg a) { turb_km_kh_body<false>(M, a); }
-__global__ __launch_bounds__(256) void k_turb_km_kh_xy(uint32_t* M, KArg a) { turb_km_kh_body<true>(M, a); }
+__global__ __launch_bounds__(256) void k_turb_dissipative_heating(uint32_t* M, KArg a) { turb_dissipative_heating_body(M, a, te_block(a)); }
 
-// turb_dissipative_heating.wgsl:139-194
-__global__ __launch_bounds__(256) void k_turb_dissipative_heating(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx, j = gy, k = gz;
-  if (i >= g.nx || j >= g.ny || k >= g.nz) return;
-  const float *dissten = fq(a.q[1]), *pi0 = fq(a.q[2]), *ppi = fq(a.q[3]), *qv = fq(a.q[4]),
-              *qc = fq(a.q[5]), *qr = fq(a.q[6]), *qi = fq(a.q[7]), *qs = fq(a.q[8]), *qg = fq(a.q[9]),
-              *sfc = fq(a.q[12]);
-  float* thten = fq(a.q[10]);
-  const uint32_t* op = a.q[11];
-  int moist = ldi(op, 0), bbc3 = ldi(op, 1), zntField = ldi(op, 4);
-  float znt = ldf(op, 2), dz1 = ldf(op, 3);
-  const int64_t sk = g.sk(), c = g.idx(i, j, k);
-  const float cv = CP - RD, cvv = CPV - RV, cpdcv = CP / (CP - RD);
-  float epsd;
-  if (k == 0 && bbc3 != 0) {
-    float ust = sfc[3 * sk + g.idx(i, j, 0)];
-    float z0 = zntField != 0 ? sfc[4 * sk + g.idx(i, j, 0)] : znt;
-    epsd = (((ust * ust) * ust) * fast_log((dz1 + z0) / z0)) / (0.4f * dz1);
-  } else {
-    epsd = 0.5f * (dissten[c] + dissten[c + sk]);
-  }
-  float pi = pi0[k] + ppi[c];
-  float dheat;
-  if (moist != 0) {
-    float cvm = fma_(2106.0f, (qi[c] + qs[c]) + qg[c], fma_(4.19e+03f, qc[c] + qr[c], fma_(cvv, qv[c], cv)));
-    dheat = epsd / ((cpdcv * cvm) * pi);
-  } else {
-    dheat = epsd / (CP * pi);
-  }
-  thten[c] = thten[c] + dheat;
-}
-
-// turb_gettau.wgsl:111-143
-__global__ __launch_bounds__(256) void k_turb_gettau(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx - 1, j = gy - 1, k = gz;
-  if (i > g.nx || j > g.ny || k >= g.nz) return;
-  const float *kmh = fq(a.q[1]), *kmv = fq(a.q[2]);
-  float *t11 = fq(a.q[3]), *t22 = fq(a.q[4]), *t33 = fq(a.q[5]), *t12 = fq(a.q[6]), *t13 = fq(a.q[7]),
-        *t23 = fq(a.q[8]);
-  const int64_t sj = g.sJ, sk = g.sk(), c = g.idx(i, j, k);
-  // every operand loaded before the first store (the loads go out together;
-  // t13 / t23 and kmv at the column's first level are read but not used)
-  const float tem = kmh[c] + kmh[c + sk];
-  const float q = ((kmh[c - 1 - sj] + kmh[c]) + (kmh[c - 1] + kmh[c - sj])) +
-                  ((kmh[c - 1 - sj + sk] + kmh[c + sk]) + (kmh[c - 1 + sk] + kmh[c - sj + sk]));
-  const float a11 = t11[c], a22 = t22[c], a33 = t33[c], a12 = t12[c], a13 = t13[c], a23 = t23[c];
-  const float kv = kmv[c], kvx = kmv[c - 1], kvy = kmv[c - sj];
-  t11[c] = a11 * tem;
-  t22[c] = a22 * tem;
-  t33[c] = a33 * tem;
-  t12[c] = a12 * (0.25f * q);
-  if (k >= 1 && k <= g.nz - 1 && i >= 0 && j >= 0) {
-    t13[c] = a13 * (kvx + kv);
-    t23[c] = a23 * (kvy + kv);
-  }
-}
+__global__ __launch_bounds__(256) void k_turb_gettau(uint32_t* M, KArg a) { turb_gettau_body(M, a, te_block(a)); }
 
 // turb_sfcstress.wgsl:132-207 (free-slip and no-slip bottom; surface-flux
 // modes need the surface-layer planes and are not on this path)
@@ -458,16 +117,7 @@ __global__ __launch_bounds__(256) void k_tke_epst(uint32_t* M, KArg a) {
   }
 }
 
-// tke_sources.wgsl:111-129
-__global__ __launch_bounds__(256) void k_tke_sources(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx, j = gy, k = gz + 1;
-  if (i >= g.nx || j >= g.ny || k > g.nz - 1) return;
-  const int64_t c = g.idx(i, j, k);
-  const float *khv = fq(a.q[1]), *nm = fq(a.q[2]), *dissten = fq(a.q[3]), *epst = fq(a.q[4]);
-  fq(a.q[5])[c] = fma_(-khv[c], nm[c], -dissten[c]) + epst[c];
-}
+__global__ __launch_bounds__(256) void k_tke_sources(uint32_t* M, KArg a) { tke_sources_body(M, a, te_block(a)); }
 
 // turb_u_tendency.wgsl:146-294 / turb_v_tendency.wgsl
 template <int DIR, bool LDS>
@@ -674,8 +324,7 @@ struct WaveColumn {
   int i, j;
   bool in;  // within the op's n0 x n1
 };
-TE_DEV WaveColumn wave_column(const KArg& a, int lane) {
-  const Blk b = te_block(a);
+TE_DEV WaveColumn wave_column(const KArg& a, const Blk& b, int lane) {
   const uint32_t l = (uint32_t)b.y * a.lg[3] + (uint32_t)b.x, n0 = a.n[0];
   const uint32_t c = l * 64u + (uint32_t)lane, j = c / n0;
   return {(int)(c - j * n0), (int)j, c < n0 * a.n[1]};
@@ -732,12 +381,12 @@ TE_DEV void relay_back(WaveRelay& r, int wave, int lane, int Lq, bool top, const
 // its rows, the solution, and its levels' tendencies; all loads of a phase
 // are issued before its stores.
 template <int DIR, int LMAX>
-__device__ __forceinline__ void uv_waves(uint32_t* M, const KArg& a) {
+__device__ __forceinline__ void uv_waves(uint32_t* M, const KArg& a, const Blk& b_) {
   __shared__ WaveRelay rl;
   const int lane = (int)threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
   const Dims g = dims(a.q[0], 0);
-  const WaveColumn col = wave_column(a, lane);
+  const WaveColumn col = wave_column(a, b_, lane);
   const int i = col.i, j = col.j, nz = g.nz;
   const int Lw = (nz + AC_WAVES - 1) / AC_WAVES, k0 = wave * Lw, k1 = min(nz, k0 + Lw), Lq = max(0, k1 - k0);
   // a wave past the top (Lq = 0, when AC_WAVES does not divide nz) touches no level
@@ -928,8 +577,8 @@ __device__ __forceinline__ void uv_waves(uint32_t* M, const KArg& a) {
   }
 }
 #define UV_INST(L)                                                                                           \
-  __global__ __launch_bounds__(64 * AC_WAVES, (L) <= 10 ? 6 : 1) void k_u_waves##L(uint32_t* M, KArg a) { uv_waves<0, L>(M, a); } \
-  __global__ __launch_bounds__(64 * AC_WAVES, (L) <= 10 ? 6 : 1) void k_v_waves##L(uint32_t* M, KArg a) { uv_waves<1, L>(M, a); }
+  __global__ __launch_bounds__(64 * AC_WAVES, (L) <= 10 ? 6 : 1) void k_u_waves##L(uint32_t* M, KArg a) { uv_waves<0, L>(M, a, te_block(a)); } \
+  __global__ __launch_bounds__(64 * AC_WAVES, (L) <= 10 ? 6 : 1) void k_v_waves##L(uint32_t* M, KArg a) { uv_waves<1, L>(M, a, te_block(a)); }
 UV_INST(1) UV_INST(2) UV_INST(3) UV_INST(4) UV_INST(5) UV_INST(6) UV_INST(7) UV_INST(8) UV_INST(9) UV_INST(10)
 UV_INST(11) UV_INST(12) UV_INST(13) UV_INST(14) UV_INST(15) UV_INST(16)
 #undef UV_INST
@@ -1222,10 +871,9 @@ __device__ __forceinline__ void face_waves(WaveRelay& rl, bool live, int wave, i
 // LMAX > 0: 64 x AC_WAVES workgroups, grid (columns / 64, rows): face_waves;
 // else one lane per column
 template <bool LDS, int LMAX = 0>
-__device__ void w_tendency(uint32_t* M, const KArg& a) {
-  const Blk b_ = te_block(a);
+__device__ void w_tendency(uint32_t* M, const KArg& a, const Blk& b_) {
   const bool wv = LMAX > 0;
-  const WaveColumn col = wv ? wave_column(a, (int)threadIdx.x) : WaveColumn{0, 0, true};
+  const WaveColumn col = wv ? wave_column(a, b_, (int)threadIdx.x) : WaveColumn{0, 0, true};
   const int i = wv ? col.i : b_.x * TE_BX + (int)threadIdx.x;
   const int j = wv ? col.j : b_.y * TE_BY + (int)threadIdx.y;
   Dims g = dims(a.q[0], 0);
@@ -1272,26 +920,10 @@ __device__ void w_tendency(uint32_t* M, const KArg& a) {
   const ColStore<LDS> CA{cA, base, sk, TE_LANE, TE_NLANES, 0}, CB{cB, base, sk, TE_LANE, TE_NLANES, nz};
   face_implicit(kmh, mh, rho, mf, rf, w, CA, CB, base, sk, nz, tema, cfd1, cfdT, out);
 }
-__global__ __launch_bounds__(256) void k_turb_w_tendency(uint32_t* M, KArg a) { w_tendency<false>(M, a); }
-__global__ __launch_bounds__(256) void k_turb_w_tendency_lds(uint32_t* M, KArg a) { w_tendency<true>(M, a); }
+__global__ __launch_bounds__(256) void k_turb_w_tendency(uint32_t* M, KArg a) { w_tendency<false>(M, a, te_block(a)); }
+__global__ __launch_bounds__(256) void k_turb_w_tendency_lds(uint32_t* M, KArg a) { w_tendency<true>(M, a, te_block(a)); }
 
-// turb_scalar_flux_h.wgsl:125-148
-__global__ __launch_bounds__(256) void k_turb_scalar_flux_h(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx, j = gy, k = gz;
-  if (i > g.nx || j > g.ny || k >= g.nz) return;
-  const float *s = fq(a.q[1]), *rho = fq(a.q[2]), *khh = fq(a.q[3]), *hm = fq(a.q[30]);
-  float leNum = ldf(a.q[4], 0);
-  const int64_t sj = g.sJ, sk = g.sk(), c = g.idx(i, j, k);
-  // both fluxes formed before the first store (the loads go out together)
-  const float fx = (((((-0.125f * (rho[c] + rho[c - 1])) * leNum) * ((khh[c] + khh[c - 1]) + (khh[c + sk] + khh[c - 1 + sk]))) *
-                     (s[c] - s[c - 1])) * g.rdx) * hm_uf(hm, g, i);
-  const float fy = (((((-0.125f * (rho[c] + rho[c - sj])) * leNum) * ((khh[c] + khh[c - sj]) + (khh[c + sk] + khh[c - sj + sk]))) *
-                     (s[c] - s[c - sj])) * g.rdy) * hm_vf(hm, g, j);
-  fq(a.q[5])[c] = fx;
-  fq(a.q[6])[c] = fy;
-}
+__global__ __launch_bounds__(256) void k_turb_scalar_flux_h(uint32_t* M, KArg a) { turb_scalar_flux_h_body(M, a, te_block(a)); }
 
 // turb_scalar_vert_implicit.wgsl:210-327
 template <bool LDS>
@@ -1455,12 +1087,12 @@ __global__ __launch_bounds__(256) void k_turb_scalar_vert_implicit_lds(uint32_t*
 // row's missing super-diagonal are zeros, which give the reference's special
 // rows' bits.  cA / cB are not written (dead scratch of the fused program).
 template <int LMAX>
-__device__ __forceinline__ void svi_waves(uint32_t* M, const KArg& a) {
+__device__ __forceinline__ void svi_waves(uint32_t* M, const KArg& a, const Blk& b_) {
   __shared__ WaveRelay rl;
   const int lane = (int)threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
   const Dims g = dims(a.q[0], 0);
-  const WaveColumn col = wave_column(a, lane);
+  const WaveColumn col = wave_column(a, b_, lane);
   const int i = col.i, j = col.j, nz = g.nz;
   const int Lw = (nz + AC_WAVES - 1) / AC_WAVES, k0 = wave * Lw, k1 = min(nz, k0 + Lw), Lq = max(0, k1 - k0);
   // a wave past the top (Lq = 0, when AC_WAVES does not divide nz) touches no level
@@ -1642,7 +1274,7 @@ __device__ __forceinline__ void svi_waves(uint32_t* M, const KArg& a) {
   }
 }
 #define SVI_INST(L) \
-  __global__ __launch_bounds__(64 * AC_WAVES, (L) <= 10 ? 6 : 1) void k_svi_waves##L(uint32_t* M, KArg a) { svi_waves<L>(M, a); }
+  __global__ __launch_bounds__(64 * AC_WAVES, (L) <= 10 ? 6 : 1) void k_svi_waves##L(uint32_t* M, KArg a) { svi_waves<L>(M, a, te_block(a)); }
 SVI_INST(1) SVI_INST(2) SVI_INST(3) SVI_INST(4) SVI_INST(5) SVI_INST(6) SVI_INST(7) SVI_INST(8) SVI_INST(9)
 SVI_INST(10) SVI_INST(11) SVI_INST(12) SVI_INST(13) SVI_INST(14) SVI_INST(15) SVI_INST(16)
 #undef SVI_INST
@@ -1658,31 +1290,15 @@ const void* svi_waves_kernel(int levels_per_wave) {
   return levels_per_wave >= 1 && levels_per_wave <= 16 ? fns[levels_per_wave] : nullptr;
 }
 
-// tke_flux_h.wgsl:125-146
-__global__ __launch_bounds__(256) void k_tke_flux_h(uint32_t* M, KArg a) {
-  TE_TID3
-  Dims g = dims(a.q[0], 0);
-  int i = gx, j = gy, k = gz + 1;
-  if (i > g.nx || j > g.ny || k > g.nz - 1) return;
-  const float *t = fq(a.q[1]), *rf = fq(a.q[2]), *kmh = fq(a.q[3]), *hm = fq(a.q[30]);
-  const int64_t sj = g.sJ, c = g.idx(i, j, k);
-  // both fluxes formed before the first store
-  const float fx =
-      (((((-0.25f * (rf[c] + rf[c - 1])) * 2.0f) * (kmh[c] + kmh[c - 1])) * (t[c] - t[c - 1])) * g.rdx) * hm_uf(hm, g, i);
-  const float fy =
-      (((((-0.25f * (rf[c] + rf[c - sj])) * 2.0f) * (kmh[c] + kmh[c - sj])) * (t[c] - t[c - sj])) * g.rdy) * hm_vf(hm, g, j);
-  fq(a.q[4])[c] = fx;
-  fq(a.q[5])[c] = fy;
-}
+__global__ __launch_bounds__(256) void k_tke_flux_h(uint32_t* M, KArg a) { tke_flux_h_body(M, a, te_block(a)); }
 
 // tke_transport.wgsl:158-301
 // LMAX > 0: 64 x AC_WAVES workgroups, grid (columns / 64, rows): face_waves;
 // else one lane per column
 template <bool LDS, int LMAX = 0>
-__device__ void tke_transport(uint32_t* M, const KArg& a) {
-  const Blk b_ = te_block(a);
+__device__ void tke_transport(uint32_t* M, const KArg& a, const Blk& b_) {
   const bool wv = LMAX > 0;
-  const WaveColumn col = wv ? wave_column(a, (int)threadIdx.x) : WaveColumn{0, 0, true};
+  const WaveColumn col = wv ? wave_column(a, b_, (int)threadIdx.x) : WaveColumn{0, 0, true};
   const int i = wv ? col.i : b_.x * TE_BX + (int)threadIdx.x;
   const int j = wv ? col.j : b_.y * TE_BY + (int)threadIdx.y;
   Dims g = dims(a.q[0], 0);
@@ -1742,11 +1358,11 @@ __device__ void tke_transport(uint32_t* M, const KArg& a) {
   const ColStore<LDS> CA{cA, base, sk, TE_LANE, TE_NLANES, 0}, CB{cB, base, sk, TE_LANE, TE_NLANES, nz};
   face_implicit(kmh, mh, rho, mf, rf, t, CA, CB, base, sk, nz, tema, cfd1, cfdT, out);
 }
-__global__ __launch_bounds__(256) void k_tke_transport(uint32_t* M, KArg a) { tke_transport<false>(M, a); }
-__global__ __launch_bounds__(256) void k_tke_transport_lds(uint32_t* M, KArg a) { tke_transport<true>(M, a); }
+__global__ __launch_bounds__(256) void k_tke_transport(uint32_t* M, KArg a) { tke_transport<false>(M, a, te_block(a)); }
+__global__ __launch_bounds__(256) void k_tke_transport_lds(uint32_t* M, KArg a) { tke_transport<true>(M, a, te_block(a)); }
 #define FACE_INST(L)                                                                                      \
-  __global__ __launch_bounds__(64 * AC_WAVES, (L) <= 10 ? 6 : 1) void k_w_waves##L(uint32_t* M, KArg a) { w_tendency<true, L>(M, a); } \
-  __global__ __launch_bounds__(64 * AC_WAVES, (L) <= 10 ? 6 : 1) void k_tke_waves##L(uint32_t* M, KArg a) { tke_transport<true, L>(M, a); }
+  __global__ __launch_bounds__(64 * AC_WAVES, (L) <= 10 ? 6 : 1) void k_w_waves##L(uint32_t* M, KArg a) { w_tendency<true, L>(M, a, te_block(a)); } \
+  __global__ __launch_bounds__(64 * AC_WAVES, (L) <= 10 ? 6 : 1) void k_tke_waves##L(uint32_t* M, KArg a) { tke_transport<true, L>(M, a, te_block(a)); }
 FACE_INST(1) FACE_INST(2) FACE_INST(3) FACE_INST(4) FACE_INST(5) FACE_INST(6) FACE_INST(7) FACE_INST(8)
 FACE_INST(9) FACE_INST(10) FACE_INST(11) FACE_INST(12) FACE_INST(13) FACE_INST(14) FACE_INST(15) FACE_INST(16)
 #undef FACE_INST
@@ -1757,6 +1373,29 @@ const void* face_waves_kernel(int which, int levels_per_wave) {
 #undef E
   return levels_per_wave >= 1 && levels_per_wave <= 16 && (which == 0 || which == 1) ? fns[levels_per_wave][which]
                                                                                       : nullptr;
+}
+
+// Independent sweeps (u, v, w, scalars, TKE) in one launch: each is a few
+// hundred workgroups that mostly wait on memory and on the relay between their
+// waves, so one after the other they leave the chip idle.  Bodies: 0 u, 1 v,
+// 2 scalar, 3 w, 4 TKE; L levels per wave serve the face-level sweeps too.
+template <int L>
+__global__ __launch_bounds__(64 * AC_WAVES, L <= 10 ? 6 : 1) void k_sweep_batch(uint32_t* M, KBatch) {
+  const BatchPart p = te_batch_part();
+  if (!p.in) return;
+  const Blk b = p.blk();
+  if (p.body == 0) uv_waves<0, L>(M, p.a, b);
+  else if (p.body == 1) uv_waves<1, L>(M, p.a, b);
+  else if (p.body == 2) svi_waves<L>(M, p.a, b);
+  else if (p.body == 3) w_tendency<true, L>(M, p.a, b);
+  else tke_transport<true, L>(M, p.a, b);
+}
+const void* sweep_batch_kernel(int levels_per_wave) {
+#define E(L) (const void*)&k_sweep_batch<L>
+  static const void* const fns[] = {nullptr, E(1), E(2), E(3), E(4), E(5), E(6), E(7), E(8),
+                                    E(9), E(10), E(11), E(12), E(13), E(14), E(15), E(16)};
+#undef E
+  return levels_per_wave >= 1 && levels_per_wave <= 16 ? fns[levels_per_wave] : nullptr;
 }
 
 }  // namespace te

@@ -450,26 +450,28 @@ struct ColStore {
 #define TE_XCD_REMAP 1
 #endif
 struct Blk {
-  int x, y, z;
+  int x, y, z;     // the workgroup
+  int tx, ty, tz;  // the thread in it
 };
 TE_DEV uint32_t te_div(uint32_t l, uint32_t mlo, uint32_t mhi) {
   return (uint32_t)((((uint64_t)mhi << 32 | mlo) * (uint64_t)l) >> 40);
 }
 // the workgroup numbered w of a's grid (te_block: this launch's own)
-__device__ __forceinline__ Blk te_block_at(const KArg& a, uint32_t w) {
+__device__ __forceinline__ Blk te_block_at(const KArg& a, uint32_t w, int tx, int ty, int tz) {
   const uint32_t nbx = a.lg[3], nby = a.lg[4];
 #if TE_XCD_REMAP
   const uint32_t n = a.lg[9];
   const uint32_t q = n >> 3, r = n & 7u, x = w & 7u;
   const uint32_t l = x * q + (x < r ? x : r) + (w >> 3);
   const uint32_t yz = te_div(l, a.lg[5], a.lg[6]), z = te_div(yz, a.lg[7], a.lg[8]);
-  return Blk{(int)(l - yz * nbx), (int)(yz - z * nby), (int)z};
+  return Blk{(int)(l - yz * nbx), (int)(yz - z * nby), (int)z, tx, ty, tz};
 #else
-  return Blk{(int)(w % nbx), (int)(w / nbx % nby), (int)(w / nbx / nby)};
+  return Blk{(int)(w % nbx), (int)(w / nbx % nby), (int)(w / nbx / nby), tx, ty, tz};
 #endif
 }
 __device__ __forceinline__ Blk te_block(const KArg& a) {
-  return te_block_at(a, blockIdx.x + a.lg[3] * (blockIdx.y + a.lg[4] * blockIdx.z));
+  return te_block_at(a, blockIdx.x + a.lg[3] * (blockIdx.y + a.lg[4] * blockIdx.z), (int)threadIdx.x,
+                     (int)threadIdx.y, (int)threadIdx.z);
 }
 // Launches of independent dispatches side by side (the runtime's batches): the
 // arguments of each lie in the kernel's argument segment (a by-value array
@@ -489,6 +491,15 @@ struct BatchPart {
   int body;
   uint32_t w;
   bool in;
+  // the workgroup, its threads as the launch's
+  TE_DEV Blk blk() const { return te_block_at(a, w, (int)threadIdx.x, (int)threadIdx.y, (int)threadIdx.z); }
+  // for a launch in lines of 256 threads, re-read as a's block (powers of two);
+  // in: the thread lies in it
+  TE_DEV Blk line_blk(bool& in) const {
+    const uint32_t t = threadIdx.x, lx = 31 - __builtin_clz(a.lg[0]), ly = 31 - __builtin_clz(a.lg[1]);
+    in = t < a.lg[0] * a.lg[1] * a.lg[2];
+    return te_block_at(a, w, (int)(t & (a.lg[0] - 1)), (int)(t >> lx & (a.lg[1] - 1)), (int)(t >> (lx + ly)));
+  }
 };
 TE_DEV BatchPart te_batch_part() {
   const KBatch& B = *(const KBatch*)((const char*)__builtin_amdgcn_kernarg_segment_ptr() + 8);
@@ -513,10 +524,10 @@ TE_DEV BatchPart te_batch_part() {
 // op(word, width) for this thread's run: width 4 when whole, else 1 per word
 // of the tail, and reports whether the launch was flat.
 template <class F>
-TE_DEV bool te_flat(const KArg& a, F op) {
+TE_DEV bool te_flat(const KArg& a, const Blk& blk, F op) {
   if (a.lg[10] == 0) return false;
   const uint32_t W = a.n[0] * a.n[1] * a.n[2];
-  const uint32_t f = 4u * ((uint32_t)te_block(a).x * (uint32_t)a.lg[0] + threadIdx.x);
+  const uint32_t f = 4u * ((uint32_t)blk.x * (uint32_t)a.lg[0] + (uint32_t)blk.tx);
   if (f + 4 <= W) {
     op(f, 4);
   } else {
@@ -528,10 +539,10 @@ TE_DEV bool te_flat(const KArg& a, F op) {
 // width, k) with k the word's level (L words per level); a run of 4 that
 // straddles two levels is done word by word.
 template <class F>
-TE_DEV bool te_flat_levels(const KArg& a, uint32_t L, F op) {
+TE_DEV bool te_flat_levels(const KArg& a, const Blk& blk, uint32_t L, F op) {
   if (a.lg[10] == 0) return false;
   const uint32_t W = a.n[0] * a.n[1] * a.n[2];
-  const uint32_t f = 4u * ((uint32_t)te_block(a).x * (uint32_t)a.lg[0] + threadIdx.x);
+  const uint32_t f = 4u * ((uint32_t)blk.x * (uint32_t)a.lg[0] + (uint32_t)blk.tx);
   if (f >= W) return true;
   const uint32_t k0 = f / L, next = (k0 + 1) * L;
   if (f + 4 <= W && f + 4 <= next) {
@@ -564,22 +575,23 @@ TE_DEV void st4(uint32_t* p, uint32_t w, int width, const F4& r) {
 // not a multiple of 64: whole-field rows of nx+7, staggered rows of nx+1)
 // number the (i, j) plane's points consecutively, 256 per workgroup, with
 // the level on the grid's y axis, so no wave idles at a row's end.
-TE_DEV void te_tid3(const KArg& a, const Blk b, int& gx, int& gy, int& gz) {
+TE_DEV void te_tid3(const KArg& a, const Blk& b, int& gx, int& gy, int& gz) {
   if (a.lg[11] != 0) {
-    const uint32_t t = (uint32_t)b.x * 256u + threadIdx.x;
+    const uint32_t t = (uint32_t)b.x * 256u + (uint32_t)b.tx;
     const uint32_t row = te_div(t, a.lg[12], a.lg[13]);
     gx = (int)(t - row * a.n[0]);
     gy = (int)row;
     gz = b.y;
     return;
   }
-  gx = b.x * TE_BX + (int)threadIdx.x;
-  gy = b.y * TE_BY + (int)threadIdx.y;
-  gz = b.z * TE_BZ + (int)threadIdx.z;
+  gx = b.x * TE_BX + b.tx;
+  gy = b.y * TE_BY + b.ty;
+  gz = b.z * TE_BZ + b.tz;
 }
-#define TE_TID3                                                          \
+#define TE_TID3_OF(blk)                                                  \
   int gx, gy, gz;                                                        \
-  te_tid3(a, te_block(a), gx, gy, gz);                                   \
+  te_tid3(a, blk, gx, gy, gz);                                           \
   if (gx >= (int)a.n[0] || gy >= (int)a.n[1] || gz >= (int)a.n[2]) return;
+#define TE_TID3 TE_TID3_OF(te_block(a))
 
 }  // namespace te

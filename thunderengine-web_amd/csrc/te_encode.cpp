@@ -258,7 +258,11 @@ class Encoder {
   void setup();
   void openHalo(const std::string& n);
   void haloFill(const std::string& n);
-  void openTurbFlux();
+  void openTurbFlux(const std::string& fx, const std::string& fy);
+  void rayleighDamping();
+  // fuse = 1: the moisture scalars' SGS tendencies go to their caches, and
+  // nothing else adds to `tend` scalar by scalar
+  bool sgsCached() const { return cfg.fuse == 1 && moist && tke && cacheMT && !(hasMicro && usePT); }
   void openStress();
   void bindSurfaceFlux(std::vector<Bind>& bs, int plane);
   void turbulence();
@@ -422,10 +426,10 @@ void Encoder::haloFill(const std::string& n) {
   openHalo(n);
 }
 
-void Encoder::openTurbFlux() {
+void Encoder::openTurbFlux(const std::string& fx, const std::string& fy) {
   if (!openX && !openY) return;
   op("turb_openbc_flux", {std::max(cfg.nx, cfg.ny) + 1, cfg.nz + 1, 1},
-     {fb(1, "fx"), fb(2, "fy"), bb(3, I2(openX ? 1 : 0, openY ? 1 : 0))});
+     {fb(1, fx), fb(2, fy), bb(3, I2(openX ? 1 : 0, openY ? 1 : 0))});
 }
 
 void Encoder::openStress() {
@@ -443,6 +447,13 @@ void Encoder::bindSurfaceFlux(std::vector<Bind>& bs, int plane) {
   bs.push_back(bb(18, I1(1)));
 }
 
+void Encoder::rayleighDamping() {
+  op("rayleigh_damping", {cfg.nx + 1, cfg.ny + 1, cfg.nz + 1},
+     {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "th_a"), rb(5, "u0"), rb(6, "v0"), rb(7, "tauh"), rb(8, "tauf"),
+      bb(9, F1(cfg.rayleigh_alpha)), fb(10, "uten_t"), fb(11, "vten_t"), fb(12, "wten_t"), fb(13, "thten_t"),
+      rb(14, "tauf"), rb(15, "tauf"), bb(16, I1(0)), bb(17, I1(0)), rb(18, "tauf"), rb(19, "th0")});
+}
+
 void Encoder::turbulence() {
   const int nx = cfg.nx, ny = cfg.ny, nz = cfg.nz;
   const std::array<int, 3> full{nx, ny, nz}, whole{nx + 7, ny + 7, nz + 1}, haloWide{nx + 2, ny + 2, nz + 1},
@@ -455,90 +466,212 @@ void Encoder::turbulence() {
   if (!rayleigh)
     for (const char* n : {"uten_t", "vten_t", "wten_t", "thten_t"}) zl.push_back(n);
   for (auto& n : zl) op("turb_zero", whole, {fb(1, n)});
-  op("turb_rho_faces", {nx + 4, ny + 4, nz + 1},
-     {fb(1, "rho"), rb(2, "c1"), rb(3, "c2"), fb(4, "rr"), fb(5, "rf"), bb(6, Fx3(v.cgs)), bb(7, Fx3(v.cgt))});
-  op("turb_def_centers", haloWide,
-     {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "rho"), rb(5, "mh"), fb(6, "s11"), fb(7, "s22"), fb(8, "s33"),
-      fb(9, "s12")});
-  op("turb_def_faces", haloWide,
-     {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "rf"), rb(5, "mf"), fb(6, "s13"), fb(7, "s23")});
-  op("turb_def_assemble", full,
-     {fb(1, "s11"), fb(2, "s22"), fb(3, "s33"), fb(4, "s12"), fb(5, "s13"), fb(6, "s23"), rb(7, "c1"), rb(8, "c2"),
-      fb(9, "rf"), fb(10, "defv"), fb(11, "defh")});
-  openStress();
-  {
-    const char* ks[] = {"qv", "qc", "qr", "qi", "qs", "qg"};
-    std::vector<Bind> bs = {fb(1, "th_a"), fb(2, "pp3d"), rb(3, "th0"), rb(4, "pi0"), fb(5, "prs")};
-    for (int q = 0; q < 6; ++q) bs.push_back(fb(6 + q, moist ? species(ks[q], "_a") : "th_a"));
-    bs.push_back(rb(12, "c1")); bs.push_back(rb(13, "c2")); bs.push_back(rb(14, "mf")); bs.push_back(fb(15, "nm"));
-    bs.push_back(bb(16, I1(moist ? 1 : 0))); bs.push_back(fb(17, "nm")); bs.push_back(bb(18, I1(0)));
-    Op o;
-    op("turb_nm", full, {});
-    o = E.ops.back();
-    for (const Bind& bd : bs) o.A[4 + bd.idx] = (uint32_t)bd.off;
-    E.ops.back() = o;
-  }
-  // (open sides: four fields' copies in one launch are slower than their own)
-  const bool foldK = foldHalo && !openX && !openY;
-  op(foldK ? "turb_km_kh_xy" : "turb_km_kh", full,
-     {fb(1, "tke_a"), fb(2, "nm"), rb(3, "mf"), fb(4, "kmh"), fb(5, "kmv"), fb(6, "khh"), fb(7, "khv"), fb(8, "lenscl"),
-      fb(9, "dissten"), bb(10, F1(1.0f)), bb(11, F1(0.0f)), bb(12, F1(1.0f))});
-  if (!foldK)
-    for (const char* n : {"kmh", "kmv", "khh", "khv"}) haloFill(n);
-  if (diss) {
-    const char* ks[] = {"qv", "qc", "qr", "qi", "qs", "qg"};
-    const float dz1 = (float)(v.zf[1] - v.zf[0]);
-    Bytes dp = {(uint32_t)(moist ? 1 : 0), 0u, fbits(1.0f), fbits(dz1), 0u};
-    std::vector<Bind> bs = {fb(1, "dissten"), rb(2, "pi0"), fb(3, "ppi")};
-    for (int q = 0; q < 6; ++q) bs.push_back(fb(4 + q, moist ? species(ks[q], "_a") : "th_a"));
-    bs.push_back(fb(10, "thten_t")); bs.push_back(bb(11, dp)); bs.push_back(rb(12, "sfc"));
-    op("turb_dissipative_heating", full, {});
-    for (const Bind& bd : bs) E.ops.back().A[4 + bd.idx] = (uint32_t)bd.off;
-  }
-  op("turb_gettau", haloWide,
-     {fb(1, "kmh"), fb(2, "kmv"), fb(3, "s11"), fb(4, "s22"), fb(5, "s33"), fb(6, "s12"), fb(7, "s13"), fb(8, "s23")});
-  op("turb_sfcstress", stagCols,
-     {rb(1, "sfc"), fb(2, "rf"), fb(3, "s13"), fb(4, "s23"), bb(5, I1(0)), fb(6, "u_a"), fb(7, "v_a"),
-      bb(8, Fx2(cfg.umove, cfg.vmove)), fb(9, "kmv"), bb(10, I1(0)), rb(11, "mf")});
-  for (const char* n : {"s11", "s22", "s33", "s12", "s13", "s23"}) haloFill(n);
-  openStress();
-  op("tke_epst", full,
-     {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "s11"), fb(5, "s12"), fb(6, "s13"), fb(7, "s22"), fb(8, "s23"),
-      fb(9, "s33"), fb(10, "rf"), rb(11, "mh"), rb(12, "mf"), rb(13, "c1"), rb(14, "c2"), fb(15, "epst")});
-  op("tke_sources", full, {fb(1, "khv"), fb(2, "nm"), fb(3, "dissten"), fb(4, "epst"), fb(5, "tketen")});
+  auto rhoFaces = [&] {
+    op("turb_rho_faces", {nx + 4, ny + 4, nz + 1},
+       {fb(1, "rho"), rb(2, "c1"), rb(3, "c2"), fb(4, "rr"), fb(5, "rf"), bb(6, Fx3(v.cgs)), bb(7, Fx3(v.cgt))});
+  };
+  auto defCenters = [&] {
+    op("turb_def_centers", haloWide,
+       {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "rho"), rb(5, "mh"), fb(6, "s11"), fb(7, "s22"), fb(8, "s33"),
+        fb(9, "s12")});
+  };
+  auto defFaces = [&] {
+    op("turb_def_faces", haloWide,
+       {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "rf"), rb(5, "mf"), fb(6, "s13"), fb(7, "s23")});
+  };
+  auto defAssemble = [&] {
+    op("turb_def_assemble", full,
+       {fb(1, "s11"), fb(2, "s22"), fb(3, "s33"), fb(4, "s12"), fb(5, "s13"), fb(6, "s23"), rb(7, "c1"), rb(8, "c2"),
+        fb(9, "rf"), fb(10, "defv"), fb(11, "defh")});
+  };
+  auto nmOp = [&] {
+    {
+      const char* ks[] = {"qv", "qc", "qr", "qi", "qs", "qg"};
+      std::vector<Bind> bs = {fb(1, "th_a"), fb(2, "pp3d"), rb(3, "th0"), rb(4, "pi0"), fb(5, "prs")};
+      for (int q = 0; q < 6; ++q) bs.push_back(fb(6 + q, moist ? species(ks[q], "_a") : "th_a"));
+      bs.push_back(rb(12, "c1")); bs.push_back(rb(13, "c2")); bs.push_back(rb(14, "mf")); bs.push_back(fb(15, "nm"));
+      bs.push_back(bb(16, I1(moist ? 1 : 0))); bs.push_back(fb(17, "nm")); bs.push_back(bb(18, I1(0)));
+      Op o;
+      op("turb_nm", full, {});
+      o = E.ops.back();
+      for (const Bind& bd : bs) o.A[4 + bd.idx] = (uint32_t)bd.off;
+      E.ops.back() = o;
+    }
+  };
+  auto kmKh = [&] {
+    // (open sides: four fields' copies in one launch are slower than their own)
+    const bool foldK = foldHalo && !openX && !openY;
+    op(foldK ? "turb_km_kh_xy" : "turb_km_kh", full,
+       {fb(1, "tke_a"), fb(2, "nm"), rb(3, "mf"), fb(4, "kmh"), fb(5, "kmv"), fb(6, "khh"), fb(7, "khv"), fb(8, "lenscl"),
+        fb(9, "dissten"), bb(10, F1(1.0f)), bb(11, F1(0.0f)), bb(12, F1(1.0f))});
+    if (!foldK)
+      for (const char* n : {"kmh", "kmv", "khh", "khv"}) haloFill(n);
+  };
+  auto heating = [&] {
+    if (diss) {
+      const char* ks[] = {"qv", "qc", "qr", "qi", "qs", "qg"};
+      const float dz1 = (float)(v.zf[1] - v.zf[0]);
+      Bytes dp = {(uint32_t)(moist ? 1 : 0), 0u, fbits(1.0f), fbits(dz1), 0u};
+      std::vector<Bind> bs = {fb(1, "dissten"), rb(2, "pi0"), fb(3, "ppi")};
+      for (int q = 0; q < 6; ++q) bs.push_back(fb(4 + q, moist ? species(ks[q], "_a") : "th_a"));
+      bs.push_back(fb(10, "thten_t")); bs.push_back(bb(11, dp)); bs.push_back(rb(12, "sfc"));
+      op("turb_dissipative_heating", full, {});
+      for (const Bind& bd : bs) E.ops.back().A[4 + bd.idx] = (uint32_t)bd.off;
+    }
+  };
+  auto getTau = [&] {
+    op("turb_gettau", haloWide,
+       {fb(1, "kmh"), fb(2, "kmv"), fb(3, "s11"), fb(4, "s22"), fb(5, "s33"), fb(6, "s12"), fb(7, "s13"), fb(8, "s23")});
+  };
+  auto stressEdges = [&] {
+    op("turb_sfcstress", stagCols,
+       {rb(1, "sfc"), fb(2, "rf"), fb(3, "s13"), fb(4, "s23"), bb(5, I1(0)), fb(6, "u_a"), fb(7, "v_a"),
+        bb(8, Fx2(cfg.umove, cfg.vmove)), fb(9, "kmv"), bb(10, I1(0)), rb(11, "mf")});
+    for (const char* n : {"s11", "s22", "s33", "s12", "s13", "s23"}) haloFill(n);
+    openStress();
+  };
+  auto epst = [&] {
+    op("tke_epst", full,
+       {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "s11"), fb(5, "s12"), fb(6, "s13"), fb(7, "s22"), fb(8, "s23"),
+        fb(9, "s33"), fb(10, "rf"), rb(11, "mh"), rb(12, "mf"), rb(13, "c1"), rb(14, "c2"), fb(15, "epst")});
+    op("tke_sources", full, {fb(1, "khv"), fb(2, "nm"), fb(3, "dissten"), fb(4, "epst"), fb(5, "tketen")});
+  };
   const Bytes dtBig = F1(dtf), exZ = I1(explicitZ ? 1 : 0), open = I2(openX ? 1 : 0, openY ? 1 : 0);
-  op("turb_u_tendency", stagCols,
-     {fb(1, "u_a"), fb(2, "w_a"), fb(3, "rho"), fb(4, "rf"), fb(5, "kmv"), fb(6, "s11"), fb(7, "s12"), fb(8, "s13"),
-      rb(9, "mh"), rb(10, "mf"), bb(11, dtBig), fb(12, "cA"), fb(13, "cB"), fb(14, "dwdx"), fb(15, "uten_t"),
-      bb(16, open), bb(17, exZ)});
-  op("turb_v_tendency", stagCols,
-     {fb(1, "v_a"), fb(2, "w_a"), fb(3, "rho"), fb(4, "rf"), fb(5, "kmv"), fb(6, "s12"), fb(7, "s22"), fb(8, "s23"),
-      rb(9, "mh"), rb(10, "mf"), bb(11, dtBig), fb(12, "cA"), fb(13, "cB"), fb(14, "dwdx"), fb(15, "vten_t"),
-      bb(16, open), bb(17, exZ)});
-  op("turb_w_tendency", cols,
-     {fb(1, "w_a"), fb(2, "rho"), fb(3, "rf"), fb(4, "kmh"), fb(5, "s13"), fb(6, "s23"), fb(7, "s33"), rb(8, "mh"),
-      rb(9, "mf"), bb(10, dtBig), fb(11, "cA"), fb(12, "cB"), fb(13, "wten_t"), bb(14, open), bb(15, exZ)});
-  op("build_sadv", whole, {rb(1, "th0"), fb(2, "th_a"), fb(3, "sadv")});
-  auto scalarTurb = [&](const std::string& src, const std::string& sink, int plane) {
-    op("turb_scalar_flux_h", stag,
-       {fb(1, src), fb(2, "rho"), fb(3, "khh"), bb(4, F1(1.0f)), fb(5, "fx"), fb(6, "fy")});
-    openTurbFlux();
+  auto uTendency = [&] {
+    op("turb_u_tendency", stagCols,
+       {fb(1, "u_a"), fb(2, "w_a"), fb(3, "rho"), fb(4, "rf"), fb(5, "kmv"), fb(6, "s11"), fb(7, "s12"), fb(8, "s13"),
+        rb(9, "mh"), rb(10, "mf"), bb(11, dtBig), fb(12, "cA"), fb(13, "cB"), fb(14, "dwdx"), fb(15, "uten_t"),
+        bb(16, open), bb(17, exZ)});
+  };
+  auto vTendency = [&] {
+    op("turb_v_tendency", stagCols,
+       {fb(1, "v_a"), fb(2, "w_a"), fb(3, "rho"), fb(4, "rf"), fb(5, "kmv"), fb(6, "s12"), fb(7, "s22"), fb(8, "s23"),
+        rb(9, "mh"), rb(10, "mf"), bb(11, dtBig), fb(12, "cA"), fb(13, "cB"), fb(14, "dwdx"), fb(15, "vten_t"),
+        bb(16, open), bb(17, exZ)});
+  };
+  auto wTendency = [&] {
+    op("turb_w_tendency", cols,
+       {fb(1, "w_a"), fb(2, "rho"), fb(3, "rf"), fb(4, "kmh"), fb(5, "s13"), fb(6, "s23"), fb(7, "s33"), rb(8, "mh"),
+        rb(9, "mf"), bb(10, dtBig), fb(11, "cA"), fb(12, "cB"), fb(13, "wten_t"), bb(14, open), bb(15, exZ)});
+  };
+  auto sAdv = [&] { op("build_sadv", whole, {rb(1, "th0"), fb(2, "th_a"), fb(3, "sadv")}); };
+  // horizontal SGS fluxes of a scalar into a pair of fields, and its tendency
+  auto fluxH = [&](const std::string& src, const std::string& fx, const std::string& fy) {
+    op("turb_scalar_flux_h", stag, {fb(1, src), fb(2, "rho"), fb(3, "khh"), bb(4, F1(1.0f)), fb(5, fx), fb(6, fy)});
+  };
+  auto vert = [&](const std::string& src, const std::string& sink, int plane, const std::string& fx,
+                  const std::string& fy) {
     std::vector<Bind> bs = {fb(1, src), fb(2, "rho"), fb(3, "rr"), fb(4, "rf"), fb(5, "khv"), rb(6, "mh"), rb(7, "mf"),
-                            fb(8, "fx"), fb(9, "fy"), bb(10, dtBig), fb(11, "cA"), fb(12, "cB"), fb(13, sink)};
+                            fb(8, fx), fb(9, fy), bb(10, dtBig), fb(11, "cA"), fb(12, "cB"), fb(13, sink)};
     bindSurfaceFlux(bs, plane);
     op("turb_scalar_vert_implicit", cols, {});
     for (const Bind& bd : bs) E.ops.back().A[4 + bd.idx] = (uint32_t)bd.off;
   };
-  scalarTurb("sadv", "thten_t", 9);
+  auto tkeFlux = [&](const std::string& fx, const std::string& fy) {
+    op("tke_flux_h", stag, {fb(1, "tke_a"), fb(2, "rf"), fb(3, "kmh"), fb(4, fx), fb(5, fy)});
+  };
+  auto tkeTransport = [&](const std::string& fx, const std::string& fy) {
+    op("tke_transport", stagCols,
+       {fb(1, "tke_a"), fb(2, "rho"), fb(3, "rf"), fb(4, "kmh"), fb(5, "kmv"), rb(6, "mh"), rb(7, "mf"), bb(8, dtBig),
+        fb(9, "cA"), fb(10, "cB"), fb(11, fx), fb(12, fy), fb(13, "tketen"), bb(14, open), bb(15, exZ)});
+  };
+  if (cfg.fuse == 1) {
+    // the same dispatches with independent ones next to each other, for the
+    // runtime's batches (te_runtime): every scalar's fluxes in a pair of dead
+    // fields of its own, the moisture scalars' SGS tendencies here too (they
+    // depend on the start-of-step state only).  qv's is the one of qvten_t.
+    static const char* const pairs[][2] = {{"fx", "fy"}, {"fz", "fpk"}, {"tend", "qk"}, {"mm", "pk1"},
+                                           {"pk2", "tketen_s"}, {"rru", "rrv"}, {"rrw", "thv"}, {"ppterm", "piadv"},
+                                           {"buoy", "thterm"}};
+    constexpr size_t nPairs = sizeof(pairs) / sizeof(pairs[0]);
+    struct Sgs { std::string src, sink; int plane; };
+    std::vector<Sgs> sgs = {{"sadv", "thten_t", 9}};
+    const bool qvCopy = moist && usePT && sgsCached();
+    if (moist && usePT) sgs.push_back({"qv_a", "qvten_t", 10});
+    if (sgsCached())
+      for (size_t q = 1; q < scalars.size(); ++q)
+        if (!(qvCopy && scalars[q] == "qv"))
+          sgs.push_back({scalars[q] + "_a", "qturb_" + scalars[q], scalars[q] == "qv" ? 10 : -1});
+    for (size_t q = 1; q < sgs.size(); ++q) op("turb_zero", whole, {fb(1, sgs[q].sink)});
+    if (rayleigh) rayleighDamping();
+    rhoFaces();
+    defCenters();
+    nmOp();
+    sAdv();
+    defFaces();
+    kmKh();
+    defAssemble();
+    openStress();
+    heating();
+    for (size_t q0 = 0; q0 < sgs.size(); q0 += nPairs - 1) {  // (a pair is left for TKE)
+      const size_t q1 = std::min(sgs.size(), q0 + nPairs - 1);
+      const bool all = q0 == 0;
+      const auto& tkePair = pairs[q1 - q0];
+      for (size_t q = q0; q < q1; ++q) fluxH(sgs[q].src, pairs[q - q0][0], pairs[q - q0][1]);
+      if (all) tkeFlux(tkePair[0], tkePair[1]);
+      if (openX || openY) {
+        for (size_t q = q0; q < q1; ++q) openTurbFlux(pairs[q - q0][0], pairs[q - q0][1]);
+        if (all) openTurbFlux(tkePair[0], tkePair[1]);
+      }
+      if (all) {
+        getTau();
+        stressEdges();
+        epst();
+        wTendency();
+        tkeTransport(tkePair[0], tkePair[1]);
+      }
+      for (size_t q = q0; q < q1; ++q) {
+        vert(sgs[q].src, sgs[q].sink, sgs[q].plane, pairs[q - q0][0], pairs[q - q0][1]);
+        if (q == (sgs.size() > 3 ? 2 : 0)) {  // u and v share dwdx: one batch each, of about equal lengths
+          uTendency();
+          vTendency();
+        }
+      }
+    }
+    if (qvCopy) {
+      flushAdd();
+      flushHalo();
+      flushZero();
+      Op o;
+      std::memset(&o, 0, sizeof(o));
+      o.kid = kernel_id("copy_fields");
+      o.A[0] = (uint32_t)((size_t)E.L.sJ * E.L.sK * (nz + 1)); o.A[1] = 1; o.A[2] = 1;
+      o.A[4 + 0] = (uint32_t)dimsOff;
+      o.A[4 + 1] = (uint32_t)off("qvten_t");
+      o.A[4 + 5] = (uint32_t)off("qturb_qv");
+      o.A[4 + 9] = (uint32_t)bytes(I1(1));
+      E.ops.push_back(o);
+      E.names.push_back("copy_fields");
+    }
+    return;
+  }
+  rhoFaces();
+  defCenters();
+  defFaces();
+  defAssemble();
+  openStress();
+  nmOp();
+  kmKh();
+  heating();
+  getTau();
+  stressEdges();
+  epst();
+  uTendency();
+  vTendency();
+  wTendency();
+  sAdv();
+  fluxH("sadv", "fx", "fy");
+  openTurbFlux("fx", "fy");
+  vert("sadv", "thten_t", 9, "fx", "fy");
   if (moist && usePT) {
     op("turb_zero", whole, {fb(1, "qvten_t")});
-    scalarTurb("qv_a", "qvten_t", 10);
+    fluxH("qv_a", "fx", "fy");
+    openTurbFlux("fx", "fy");
+    vert("qv_a", "qvten_t", 10, "fx", "fy");
   }
-  op("tke_flux_h", stag, {fb(1, "tke_a"), fb(2, "rf"), fb(3, "kmh"), fb(4, "fx"), fb(5, "fy")});
-  openTurbFlux();
-  op("tke_transport", stagCols,
-     {fb(1, "tke_a"), fb(2, "rho"), fb(3, "rf"), fb(4, "kmh"), fb(5, "kmv"), rb(6, "mh"), rb(7, "mf"), bb(8, dtBig),
-      fb(9, "cA"), fb(10, "cB"), fb(11, "fx"), fb(12, "fy"), fb(13, "tketen"), bb(14, open), bb(15, exZ)});
+  tkeFlux("fx", "fy");
+  openTurbFlux("fx", "fy");
+  tkeTransport("fx", "fy");
 }
 
 // advect (timestep.js:1629-1900): fluxes, assembly, pdef, SGS and RK update of
@@ -610,7 +743,7 @@ void Encoder::advect(int nrk, const std::string& s, int stagger, const std::stri
       bs.push_back(fb(35, "tketen"));
       bs.push_back(bb(36, F1(1.0f)));
     } else if (chained) {
-      if (moistSgs && cfg.fuse != 1) moistureTurbulence(nrk, target);  // (fuse = 1: before all scalars, stages)
+      if (moistSgs && cfg.fuse != 1) moistureTurbulence(nrk, target);  // (fuse = 1: turbulence)
       int flags = 0;
       if (moist && target == scalars[0]) {
         flags |= 1;
@@ -748,7 +881,7 @@ void Encoder::moistureTurbulence(int nrk, const std::string& target) {
   if (cacheMT && nrk == 0) op("turb_zero", whole, {fb(1, sink)});
   if (!cacheMT || nrk == 0) {
     op("turb_scalar_flux_h", stag, {fb(1, qa), fb(2, "rho"), fb(3, "khh"), bb(4, F1(1.0f)), fb(5, "fx"), fb(6, "fy")});
-    openTurbFlux();
+    openTurbFlux("fx", "fy");
     std::vector<Bind> bs = {fb(1, qa), fb(2, "rho"), fb(3, "rr"), fb(4, "rf"), fb(5, "khv"), rb(6, "mh"),
                             rb(7, "mf"), fb(8, "fx"), fb(9, "fy"), bb(10, F1(dtf)), fb(11, "cA"), fb(12, "cB"),
                             fb(13, sink)};
@@ -971,8 +1104,6 @@ void Encoder::stages() {
     // (the runtime launches each group at once)
     static const char* const own[] = {"cA", "cB", "qk", "mm", "pk1", "pk2", "fpk", "fx", "fy", "fz"};
     const bool chains = cfg.fuse == 1 && moist && (!tke || cacheMT) && !(hasMicro && usePT), grouped = chains && nrk < 2;
-    if (chains && tke)
-      for (size_t q = 1; q < scalars.size(); ++q) moistureTurbulence(nrk, scalars[q]);
     for (size_t q = 0; q < scalars.size(); ++q) {
       if (q == 0) {
         if (cfg.fuse != 1) op("build_sadv", whole, {rb(1, "th0"), fb(2, scalars[0]), fb(3, "sadv")});
@@ -1078,12 +1209,7 @@ void Encoder::end() {
 
 Encoded Encoder::run() {
   setup();
-  if (rayleigh) {
-    op("rayleigh_damping", {cfg.nx + 1, cfg.ny + 1, cfg.nz + 1},
-       {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "th_a"), rb(5, "u0"), rb(6, "v0"), rb(7, "tauh"), rb(8, "tauf"),
-        bb(9, F1(cfg.rayleigh_alpha)), fb(10, "uten_t"), fb(11, "vten_t"), fb(12, "wten_t"), fb(13, "thten_t"),
-        rb(14, "tauf"), rb(15, "tauf"), bb(16, I1(0)), bb(17, I1(0)), rb(18, "tauf"), rb(19, "th0")});
-  }
+  if (rayleigh && !(tke && cfg.fuse == 1)) rayleighDamping();
   if (tke) turbulence();
   {
     const bool hasThten = tke || rayleigh;

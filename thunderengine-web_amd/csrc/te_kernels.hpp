@@ -36,6 +36,14 @@
 #define AC_UV_UNITS 4
 #define TE_WIDE_LIST(X) X(ac_column)
 
+// Dispatches that k_point_batch can run side by side (bodies: pointwise.hpp)
+#define TE_POINT_LIST(X) X(rayleigh_damping) X(turb_rho_faces) X(turb_def_centers) X(turb_def_faces) \
+  X(turb_def_assemble) X(turb_nm) X(turb_km_kh) X(turb_km_kh_xy) X(turb_dissipative_heating) X(turb_gettau) \
+  X(tke_sources) X(turb_scalar_flux_h) X(tke_flux_h) X(turb_openbc_flux) X(update_diagnostics_moist) \
+  X(update_diagnostics) X(stage_tendency_reset) X(stage_state_reset) X(massflux_div) X(build_sadv) X(ppx_finish_xy) \
+  X(diabatic_rates) X(pressure_tendency) X(update_rho_prs) X(tke_advance_xy) X(zero_fields) X(tendency_reset_add) \
+  X(copy_fields) X(rk_update_xy)
+
 namespace te {
 #define TE_DECL(n) __global__ __launch_bounds__(256) void k_##n(uint32_t* M, KArg a);
 TE_KERNEL_LIST(TE_DECL)
@@ -56,7 +64,11 @@ const void* adv_pdef_kernel(int kind, bool open);
 // and the kernel that runs a set of them (bit n: body n) side by side, or null
 int adv_body(bool pdef, int kind, int stag, bool open);
 const void* adv_batch_kernel(uint32_t bodies);
-__global__ __launch_bounds__(256) void k_rk_update_xy_batch(uint32_t* M, KBatch);
+// the body of a pointwise dispatch in k_point_batch, -1 if none
+int point_body(const char* name);
+__global__ __launch_bounds__(256) void k_point_batch(uint32_t* M, KBatch);
+// the turbulence sweeps' batch for ceil(nz / AC_WAVES) levels per wave
+const void* sweep_batch_kernel(int levels_per_wave);
 // turb_u_tendency_lds (dir 0) / turb_v_tendency_lds (dir 1) in the same form
 const void* uv_waves_kernel(int dir, int levels_per_wave);
 // turb_w_tendency_lds (which 0) / tke_transport_lds (which 1): levels 1 .. nz-1

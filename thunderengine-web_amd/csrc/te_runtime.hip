@@ -224,54 +224,113 @@ static hipError_t launch(te_ctx* c, const Op& op) {
 }
 
 // ---- batches: consecutive dispatches none of which reads or writes what
-// another one writes, run side by side by one launch (KBatch).  The fields of
-// a dispatch, by parameter:
-static void op_fields(const Op& op, std::vector<uint32_t>& reads, std::vector<uint32_t>& writes) {
-  static const int kAdvFused = kernel_id("adv_fused"), kAdvPdef = kernel_id("adv_pdef");
-  auto add = [&](std::vector<uint32_t>& to, std::initializer_list<int> ps) {
-    for (int q : ps) to.push_back(op.A[4 + q]);
-  };
-  if (op.kid == kAdvFused) {
-    add(reads, {2, 4, 6, 13, 14});
-    if (op.chain & 1) add(reads, {33, 34});
-    if (op.chain & 2) add(reads, {35});
-    if (op.chain & 4) add(reads, {37});
-    if (op.chain & 8) add(reads, {39});
-    if (op.chain & 64) add(reads, {42});
-    if (op.chain & 8) add(writes, {40});
-    else add(writes, {11});
-  } else if (op.kid == kAdvPdef) {
-    add(reads, {2, 4, 6, 13, 14, 46});
-    add(writes, {11, 22, 23, 24, 43, 44, 45});
-  } else {  // rk_update_xy
-    add(reads, {2, 3});
-    add(writes, {4});
+// another one writes, run side by side by one launch (KBatch).  The fields a
+// dispatch reads and writes, by parameter (unbound ones are skipped; fields
+// that never change in a step, as profiles, are left out).
+struct OpFields { std::vector<int> reads, writes; };
+static const OpFields* op_fields(int kid) {
+  static const std::map<int, OpFields> all = [] {
+    const std::vector<std::pair<const char*, OpFields>> l = {
+        {"rayleigh_damping", {{1, 2, 3, 4}, {10, 11, 12, 13}}},
+        {"turb_rho_faces", {{1}, {4, 5}}},
+        {"turb_def_centers", {{1, 2, 3, 4}, {6, 7, 8, 9}}},
+        {"turb_def_faces", {{1, 2, 3, 4}, {6, 7}}},
+        {"turb_def_assemble", {{1, 2, 3, 4, 5, 6, 9}, {10, 11}}},
+        {"turb_nm", {{1, 2, 5, 6, 7, 8, 9, 10, 11}, {15, 17}}},
+        {"turb_km_kh", {{1, 2, 9}, {4, 5, 6, 7, 8, 9}}},
+        {"turb_km_kh_xy", {{1, 2, 9}, {4, 5, 6, 7, 8, 9}}},
+        {"turb_dissipative_heating", {{1, 3, 4, 5, 6, 7, 8, 9, 10, 12}, {10}}},
+        {"turb_gettau", {{1, 2, 3, 4, 5, 6, 7, 8}, {3, 4, 5, 6, 7, 8}}},
+        {"tke_sources", {{1, 2, 3, 4}, {5}}},
+        {"turb_scalar_flux_h", {{1, 2, 3}, {5, 6}}},
+        {"tke_flux_h", {{1, 2, 3}, {4, 5}}},
+        {"turb_openbc_flux", {{1, 2}, {1, 2}}},
+        {"update_diagnostics_moist", {{1, 2, 9, 10, 11, 12, 13, 14}, {15, 16, 17, 18, 19}}},
+        {"update_diagnostics", {{1, 2}, {5, 6, 7, 9}}},
+        {"stage_tendency_reset", {{}, {1, 2, 3}}},
+        {"stage_state_reset", {{1, 2, 3, 4, 10}, {5, 6, 7, 8, 9}}},
+        {"massflux_div", {{1, 2, 3}, {6, 7, 8, 10}}},
+        {"build_sadv", {{2}, {3}}},
+        {"ppx_finish_xy", {{1, 2}, {2}}},
+        {"diabatic_rates", {{2, 3, 4, 5, 6, 7, 8, 9}, {6, 7, 8, 9}}},
+        {"pressure_tendency", {{1, 2, 3, 4, 5, 6, 13}, {11}}},
+        {"update_rho_prs", {{2, 3, 6}, {7, 8}}},
+        {"tke_advance_xy", {{1, 2}, {4}}},
+        {"zero_fields", {{}, {1, 2, 3, 4, 5, 6, 7, 8}}},
+        {"tendency_reset_add", {{4, 5, 6}, {1, 2, 3}}},
+        {"copy_fields", {{1, 2, 3, 4}, {5, 6, 7, 8}}},
+        {"rk_update_xy", {{2, 3}, {4}}},
+        {"turb_u_tendency_lds", {{1, 2, 3, 4, 5, 6, 7, 8, 14, 15}, {14, 15}}},
+        {"turb_v_tendency_lds", {{1, 2, 3, 4, 5, 6, 7, 8, 14, 15}, {14, 15}}},
+        {"turb_w_tendency_lds", {{1, 2, 3, 4, 5, 6, 7, 13}, {13}}},
+        {"turb_scalar_vert_implicit_lds", {{1, 2, 3, 4, 5, 8, 9, 13, 14}, {13}}},
+        {"tke_transport_lds", {{1, 2, 3, 4, 5, 11, 12, 13}, {13}}},
+        {"adv_fused", {{2, 4, 6, 13, 14}, {11, 40}}},  // and by its chain flags, below
+        {"adv_pdef", {{2, 4, 6, 13, 14, 46}, {11, 22, 23, 24, 43, 44, 45}}}};
+    std::map<int, OpFields> m;
+    for (const auto& e : l) m[kernel_id(e.first)] = e.second;
+    return m;
+  }();
+  const auto it = all.find(kid);
+  return it == all.end() ? nullptr : &it->second;
+}
+// Which batch kernel an op may join: 1 advection, 2 pointwise, 3 sweeps (body:
+// its body there), or 0.
+static int batch_family(const Op& op, int& body) {
+  static const std::map<int, int> points = [] {
+    std::map<int, int> m;
+    for (int k = 0; k < kNumKernels; ++k)
+      if (point_body(kKernels[k].name) >= 0) m[k] = point_body(kKernels[k].name);
+    return m;
+  }();
+  static const int sweeps[] = {kernel_id("turb_u_tendency_lds"), kernel_id("turb_v_tendency_lds"),
+                               kernel_id("turb_scalar_vert_implicit_lds"), kernel_id("turb_w_tendency_lds"),
+                               kernel_id("tke_transport_lds")};
+  if (row_waves(op.kid)) {
+    body = op.body;
+    return body >= 0 ? 1 : 0;
   }
+  if (wave_sweep(op.kid)) {
+    if (op.A[2] != 1 || op.nz < 4 || op.nz > AC_WAVES * 16) return 0;
+    for (int q = 0; q < 5; ++q)
+      if (sweeps[q] == op.kid) body = q;
+    return 3;
+  }
+  const auto it = points.find(op.kid);
+  if (it == points.end()) return 0;
+  body = it->second;
+  return 2;
 }
 static const void* batch_kernel(const Op* ops, int n) {
-  static const int kRk = kernel_id("rk_update_xy");
   if (n < 2 || n > TE_BATCH) return nullptr;
+  int family = 0;
   uint32_t bodies = 0;
-  for (int i = 0; i < n; ++i) {
-    if (ops[i].kid == kRk && ops[0].kid == kRk) {
-      // one block shape for all
-      if (ops[i].tuned || std::memcmp(ops[i].A, ops[0].A, 12) != 0 || ops[i].plane != ops[0].plane) return nullptr;
-    } else {
-      if (!row_waves(ops[i].kid) || ops[i].body < 0 || ops[0].kid == kRk) return nullptr;
-      bodies |= 1u << ops[i].body;
-    }
-  }
   const uint64_t words = (uint64_t)ops[0].sJ * ops[0].sK * (ops[0].nz + 1);
+  std::vector<uint32_t> r, w;
   auto meets = [&](const std::vector<uint32_t>& v, uint32_t f) {
     for (uint32_t x : v)
       if ((x > f ? x - f : f - x) < words) return true;
     return false;
   };
-  std::vector<uint32_t> r, w;
   for (int i = 0; i < n; ++i) {
-    if (ops[i].A[4] != ops[0].A[4]) return nullptr;  // one grid
+    const Op& op = ops[i];
+    int body = 0;
+    const int fam = batch_family(op, body);
+    const OpFields* fields = op_fields(op.kid);
+    if (fam == 0 || (i > 0 && fam != family) || op.A[4] != ops[0].A[4] || !fields) return nullptr;  // one grid
+    if (op.A[0] == 0 || op.A[1] == 0 || op.A[2] == 0) return nullptr;
+    family = fam;
+    if (fam == 1) bodies |= 1u << body;
     std::vector<uint32_t> ri, wi;
-    op_fields(ops[i], ri, wi);
+    auto add = [&](std::vector<uint32_t>& to, int q) {
+      if (op.A[4 + q] != 0) to.push_back(op.A[4 + q]);
+    };
+    for (int q : fields->reads) add(ri, q);
+    for (int q : fields->writes)
+      // a chained advection (chain 8) updates the field and leaves the tendency
+      if (fam != 1 || q != ((op.chain & 8) ? 11 : 40)) add(wi, q);
+    if (fam == 1)
+      for (int q : {33, 34, 35, 37, 39, 42}) add(ri, q);
     for (uint32_t f : wi)
       if (meets(r, f) || meets(w, f)) return nullptr;
     for (uint32_t f : ri)
@@ -279,7 +338,15 @@ static const void* batch_kernel(const Op* ops, int n) {
     r.insert(r.end(), ri.begin(), ri.end());
     w.insert(w.end(), wi.begin(), wi.end());
   }
-  return ops[0].kid == kRk ? (const void*)&k_rk_update_xy_batch : adv_batch_kernel(bodies);
+  if (family == 1) return adv_batch_kernel(bodies);
+  if (family == 3) return sweep_batch_kernel((ops[0].nz + AC_WAVES - 1) / AC_WAVES);
+  // Pointwise dispatches: below about 3 M words a field the drain and start
+  // between launches cost more than finding the dispatch and its arguments
+  // costs every workgroup.  us per step in batches and one by one: 64 x 64 x 40
+  // 382 and 416, 96 x 96 x 56 585 and 620, 128 x 128 x 60 775 and 805,
+  // 160 x 160 x 40 803 and 836, 192 x 192 x 80 (3.2 M words) 2855 and 2849,
+  // 300 x 300 x 90 6083 and 6016, 256 x 256 x 120 8612 and 8415.
+  return words <= (3u << 20) ? (const void*)&k_point_batch : nullptr;
 }
 static hipError_t launch_batch(te_ctx* c, const Op* ops, int n) {
   const void* fn = batch_kernel(ops, n);
@@ -294,10 +361,13 @@ static hipError_t launch_batch(te_ctx* c, const Op* ops, int n) {
     Shape s;
     const hipError_t e = shape_of(c, op, s);
     if (e != hipSuccess) return e;
-    fits = s.fn != nullptr;
+    int body = 0;
+    const int family = batch_family(op, body);
+    // pointwise blocks are re-read from lines of 256 threads
+    fits = s.fn != nullptr && (family != 2 || (s.b.x * s.b.y * s.b.z <= 256 && s.lds == 0));
     B.a[i] = s.a;
-    B.body[i] = (uint32_t)std::max(op.body, 0);
-    b = s.b;
+    B.body[i] = (uint32_t)body;
+    b = family == 2 ? dim3(256, 1, 1) : s.b;
     B.start[i] = (uint32_t)per;
     per += (s.a.lg[9] + 7) / 8;
   }
