@@ -63,35 +63,56 @@ __global__ __launch_bounds__(256) void k_openbc_uv_tendency(uint32_t* M, KArg a)
   }
 }
 
-// radbc_ew.wgsl:118-161 / radbc_ns.wgsl:118-161
+// radbc_ew.wgsl:118-161 / radbc_ns.wgsl:118-161: the mean over the levels of
+// the phase speed at either end of each row (column).  A workgroup takes
+// RADBC_ROWS of them: its threads form the levels' terms side by side, and one
+// lane per row and end adds them in the reference's order from LDS.  One
+// thread per row went through load, two divisions and sum level by level: 22 us
+// (ew) and 19 us (ns) for 120 rows of 40 levels, now 5.6 and 4.6.
+#define RADBC_ROWS 16
+#define RADBC_LEVELS 64
 template <int DIR>
-__device__ void radbc(uint32_t* M, const KArg& a, int t) {
-  Dims g = dims(a.q[0], 0);
-  if (t >= (DIR == 0 ? g.ny : g.nx)) return;
+__device__ void radbc(uint32_t* M, const KArg& a) {
+  __shared__ float term[2][RADBC_LEVELS][RADBC_ROWS];
+  const Dims g = dims(a.q[0], 0);
+  const int id = (int)threadIdx.x, r = id % RADBC_ROWS, rows = min(DIR == 0 ? g.ny : g.nx, (int)a.n[0]);
+  const int t = (int)blockIdx.x * RADBC_ROWS + r;
   const float *ua = fq(a.q[1]), *u = fq(a.q[2]), *hm = fq(a.q[30]);
-  float dt = ldf(a.q[3], 0);
-  float *lo = fq(a.q[4]), *hi = fq(a.q[5]);
+  const float dt = ldf(a.q[3], 0);
   const float umax = 3.5e+02f;
   const int nq = DIR == 0 ? g.nx : g.ny;
-  float d1 = DIR == 0 ? (1.0f / g.rdx) / hm_uf(hm, g, 1) : (1.0f / g.rdy) / hm_vf(hm, g, 1);
-  float d2 = DIR == 0 ? (1.0f / g.rdx) / hm_uf(hm, g, g.nx - 1) : (1.0f / g.rdy) / hm_vf(hm, g, g.ny - 1);
+  const float d1 = DIR == 0 ? (1.0f / g.rdx) / hm_uf(hm, g, 1) : (1.0f / g.rdy) / hm_vf(hm, g, 1);
+  const float d2 = DIR == 0 ? (1.0f / g.rdx) / hm_uf(hm, g, g.nx - 1) : (1.0f / g.rdy) / hm_vf(hm, g, g.ny - 1);
   auto at = [&](int q, int k) { return DIR == 0 ? g.idx(q, t, k) : g.idx(t, q, k); };
-  float avg1 = 0.0f, avg2 = 0.0f;
-  for (int k = 0; k < g.nz; ++k) {
-    int64_t c1 = at(1, k), c2 = at(2, k);
-    float foo = ua[c2] - ua[c1];
-    float cb1 = (d1 * (ua[c1] - u[c1])) / (dt * (copysign_mag(1e-10f, foo) + foo));
-    avg1 = avg1 + mx(mn(cb1, 0.0f), -umax);
-    int64_t ce = at(nq - 1, k), ce2 = at(nq - 2, k);
-    foo = ua[ce] - ua[ce2];
-    float cb2 = (d2 * (ua[ce] - u[ce])) / (dt * (copysign_mag(1e-10f, foo) + foo));
-    avg2 = avg2 + mn(mx(cb2, 0.0f), umax);
+  const int side = id / RADBC_ROWS;  // (of the first 2 * RADBC_ROWS lanes)
+  float avg = 0.0f;
+  for (int k0 = 0; k0 < g.nz; k0 += RADBC_LEVELS) {
+    if (t < rows) {
+#pragma unroll
+      for (int q = 0; q < RADBC_LEVELS * RADBC_ROWS / 256; ++q) {
+        const int kk = q * (256 / RADBC_ROWS) + id / RADBC_ROWS, k = k0 + kk;
+        if (k >= g.nz) continue;
+        const int64_t c1 = at(1, k), c2 = at(2, k), ce = at(nq - 1, k), ce2 = at(nq - 2, k);
+        const float a1 = ua[c1], a2 = ua[c2], u1 = u[c1], e1 = ua[ce], e2 = ua[ce2], ue = u[ce];
+        float foo = a2 - a1;
+        const float cb1 = (d1 * (a1 - u1)) / (dt * (copysign_mag(1e-10f, foo) + foo));
+        term[0][kk][r] = mx(mn(cb1, 0.0f), -umax);
+        foo = e1 - e2;
+        const float cb2 = (d2 * (e1 - ue)) / (dt * (copysign_mag(1e-10f, foo) + foo));
+        term[1][kk][r] = mn(mx(cb2, 0.0f), umax);
+      }
+    }
+    __syncthreads();
+    if (id < 2 * RADBC_ROWS && t < rows) {
+      const int n = min(RADBC_LEVELS, g.nz - k0);
+      for (int kk = 0; kk < n; ++kk) avg = avg + term[side][kk][r];
+    }
+    __syncthreads();
   }
-  lo[t] = avg1 / (float)g.nz;
-  hi[t] = avg2 / (float)g.nz;
+  if (id < 2 * RADBC_ROWS && t < rows) fq(a.q[side == 0 ? 4 : 5])[t] = avg / (float)g.nz;
 }
-__global__ __launch_bounds__(256) void k_radbc_ew(uint32_t* M, KArg a) { TE_TID3 radbc<0>(M, a, gx); }
-__global__ __launch_bounds__(256) void k_radbc_ns(uint32_t* M, KArg a) { TE_TID3 radbc<1>(M, a, gx); }
+__global__ __launch_bounds__(256) void k_radbc_ew(uint32_t* M, KArg a) { radbc<0>(M, a); }
+__global__ __launch_bounds__(256) void k_radbc_ns(uint32_t* M, KArg a) { radbc<1>(M, a); }
 
 __global__ __launch_bounds__(256) void k_turb_openbc_flux(uint32_t* M, KArg a) { turb_openbc_flux_body(M, a, te_block(a)); }
 

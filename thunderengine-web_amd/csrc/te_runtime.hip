@@ -146,6 +146,16 @@ static hipError_t shape_of(te_ctx* c, const Op& op, Shape& s) {
   static const int kTkeEpst = kernel_id("tke_epst");
   if (row_waves(op.kid)) b = dim3(64, 4, 1);  // one row of cells per wave (k_adv_fused)
   if (op.kid == kTkeEpst) a.n[2] = (a.n[2] + 1) / 2;  // two levels per thread (k_tke_epst)
+  // rows (or levels) dealt to workgroups by the kernel: radbc 16 rows, the mass
+  // sums 16 rows and one level
+  static const int kRadbcEw = kernel_id("radbc_ew"), kRadbcNs = kernel_id("radbc_ns"),
+                   kMassRows = kernel_id("mass_row_sums"), kMassLevels = kernel_id("mass_level_sums");
+  if (op.kid == kRadbcEw || op.kid == kRadbcNs || op.kid == kMassRows || op.kid == kMassLevels) {
+    const uint64_t n = (uint64_t)a.n[0] * a.n[1], per = op.kid == kMassLevels ? 1 : 16;
+    if (n >= (1u << 31)) return hipErrorInvalidConfiguration;
+    return done(kKernels[op.kid].fn, dim3((uint32_t)((n + per - 1) / per), 1, 1),
+                dim3(op.kid == kMassLevels ? 64 : 256, 1, 1), 0);
+  }
   static const int kAcColumn = kernel_id("ac_column");
   if (op.kid == kAcColumn) {  // 64 columns of a row per workgroup, AC_WAVES waves over the levels
     const uint32_t nz = op.nz, lw = (nz + AC_WAVES - 1) / AC_WAVES;
@@ -552,7 +562,7 @@ static const std::set<std::string>& own_mapping() {
       "acoustic_w_solve", "acoustic_w_solve_lds", "adv_fused", "adv_pdef", "_copy", "copy_fields", "turb_sfcstress",
       "turb_u_tendency", "turb_u_tendency_lds", "turb_v_tendency", "turb_v_tendency_lds", "turb_w_tendency",
       "turb_w_tendency_lds", "turb_scalar_vert_implicit", "turb_scalar_vert_implicit_lds", "tke_transport",
-      "tke_transport_lds", "ac_column"};
+      "tke_transport_lds", "ac_column", "radbc_ew", "radbc_ns", "mass_row_sums", "mass_level_sums"};
   return s;
 }
 
