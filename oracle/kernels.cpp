@@ -83,11 +83,11 @@ static void fill_periodic(uint32_t* w, T* v, const uint32_t* A, uint32_t f) {
   call(find_kernel("bc_periodic_y"), ky);
 }
 
-// haloFill of a cell-centred field on a domain with open sides (flags ox, oy;
+// haloFill of a field (on: 1 on x faces, 2 on y faces) on a domain with open sides (flags ox, oy;
 // word `tmp` of memory carries the open passes' stagger argument, 0, and is
 // put back): the periodic passes, then the open ones.
 template <class T>
-static void fill_halo(uint32_t* w, T* v, const uint32_t* A, uint32_t f, bool ox, bool oy, uint32_t tmp) {
+static void fill_halo(uint32_t* w, T* v, const uint32_t* A, uint32_t f, bool ox, bool oy, uint32_t tmp, int on = 0) {
   const uint32_t* dm = w + A[4];
   const uint32_t nx = dm[0], ny = dm[1], nz = dm[2];
   auto pass = [&](const char* kn, uint32_t other, bool open) {
@@ -101,8 +101,9 @@ static void fill_halo(uint32_t* w, T* v, const uint32_t* A, uint32_t f, bool ox,
   if (!ox) pass("bc_periodic_x", ny, false);
   if (!oy) pass("bc_periodic_y", nx, false);
   const uint32_t keep = w[tmp];
-  w[tmp] = 0;
+  w[tmp] = on == 1;
   if (ox) pass("bc_open_x", ny, true);
+  w[tmp] = on == 2;
   if (oy) pass("bc_open_y", nx, true);
   w[tmp] = keep;
 }
@@ -265,11 +266,39 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
       run1("acoustic_pp", full, {{2, W}, {3, PK1}, {4, PK2}, {5, QK}, {6, FPK}, {7, PP3D}, {8, PPD}, {9, PPX},
                                  {10, P(16)}});
       run1("acoustic_accumulate", whole, {{2, U}, {3, V}, {4, W}, {5, RRU}, {6, RRV}, {7, RRW}, {8, P(17)}});
+      if (P(38) != 0) {  // a side is open: w's and ppd's halos follow in ac_halo_open
+        const bool ox = w[P(38)] != 0u, oy = w[P(38) + 1] != 0u;
+        fill_halo(w, v, A, U, ox, oy, P(38), 1);
+        fill_halo(w, v, A, V, ox, oy, P(38), 2);
+        continue;
+      }
       for (uint32_t f : {PPD, U, V, W}) {
         run1("bc_periodic_x", {4, ny + 7, nz + 1}, {{1, f}});
         run1("bc_periodic_y", {4, nx + 7, nz + 1}, {{1, f}});
       }
       if (P(34) != 0 && w[P(34)] != 0u) fill_periodic(w, v, A, PP3D);  // the stage's pp3d fill, folded in
+      continue;
+    }
+    if (nm == "ac_halo_open") {  // (the oracle's ac_column has accumulated rrw's halo too)
+      const uint32_t so = A[4 + 10];
+      const bool ox = w[so] != 0u, oy = w[so + 1] != 0u;
+      for (int q : {2, 3}) fill_halo(w, v, A, A[4 + q], ox, oy, so);
+      if (w[A[4 + 9]] != 0u) fill_halo(w, v, A, A[4 + 6], ox, oy, so);
+      continue;
+    }
+    if (nm == "acoustic_uv_open") {  // openbc_uv_tendency, then acoustic_uv
+      const uint32_t* dm = w + A[4];
+      uint32_t X[64] = {0}, Y[64] = {0};
+      X[4] = Y[4] = A[4]; X[5] = Y[5] = A[5]; X[34] = Y[34] = A[34];
+      X[0] = std::max(dm[0], dm[1]); X[1] = dm[2]; X[2] = 1;
+      for (int q = 0; q < 4; ++q) X[4 + 2 + q] = A[4 + 9 + q];
+      for (int q = 0; q < 4; ++q) X[4 + 6 + q] = A[4 + 4 + q];
+      X[4 + 10] = A[4 + 8];
+      Y[0] = A[0]; Y[1] = A[1]; Y[2] = A[2];
+      for (int q = 2; q <= 8; ++q) Y[4 + q] = A[4 + q];
+      K<T> k1{w, v, X}, k2{w, v, Y};
+      call(find_kernel("openbc_uv_tendency"), k1);
+      call(find_kernel("acoustic_uv"), k2);
       continue;
     }
     if (nm == "massflux_div") {

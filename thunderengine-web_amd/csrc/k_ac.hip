@@ -77,6 +77,52 @@ __global__ __launch_bounds__(256) void k_acoustic_uv(uint32_t* M, KArg a) {
   if (!vEdge) v[c] = fma_(ac.dts, fma_(-((tem2 * (ppd[c] - ppd[c - sj])) * hm_vf(hm, g, j)), thv[c] + thv[c - sj], vten[c]), v[c]);
 }
 
+// openbc_uv_tendency (openbc_uv_tendency.wgsl:167-208), then acoustic_uv, on a
+// domain with an open side (nx, ny >= 4).  An edge face's update reads the face
+// next to it as it was before acoustic_uv, so that face's thread makes both.
+// p as acoustic_uv's, 9-12 -> the radiation speeds west, east, south, north.
+__global__ __launch_bounds__(256) void k_acoustic_uv_open(uint32_t* M, KArg a) {
+  TE_TID3
+  const Dims g = dims(a.q[0], 0);
+  const int i = gx, j = gy, k = gz;
+  if (i > g.nx || j > g.ny || k >= g.nz) return;
+  const Acoustic ac = acoustic(a.q[1], 0);
+  const float *ppd = fq(a.q[2]), *thv = fq(a.q[3]), *uten = fq(a.q[4]), *vten = fq(a.q[5]), *hm = fq(a.q[30]);
+  float *u = fq(a.q[6]), *v = fq(a.q[7]);
+  const bool openx = ldi(a.q[8], 0) != 0, openy = ldi(a.q[8], 1) != 0;
+  const int64_t sj = g.sJ, c = g.idx(i, j, k);
+  const float tem1 = (g.rdx * CP) * 0.5f, tem2 = (g.rdy * CP) * 0.5f;
+  const bool uEdge = openx && (i == 0 || i == g.nx), vEdge = openy && (j == 0 || j == g.ny);
+  const bool west = openx && i == 1 && j < g.ny, east = openx && i == g.nx - 1 && j < g.ny;
+  const bool south = openy && j == 1 && i < g.nx, north = openy && j == g.ny - 1 && i < g.nx;
+  // every load before the first store
+  const float uc = u[c], vc = v[c], pc = ppd[c], tc = thv[c];
+  const float px = ppd[c - 1], tx = thv[c - 1], py = ppd[c - sj], ty = thv[c - sj], ut = uten[c], vt = vten[c];
+  float un = 0.0f, vn = 0.0f;
+  if (west) {
+    const float e = u[c - 1];
+    un = fma_(ac.dts, fma_(((-fq(a.q[9])[j]) * (uc - e)) * g.rdx, hm_uh(hm, g, 0), uten[c - 1]), e);
+  }
+  if (east) {
+    const float e = u[c + 1];
+    un = fma_(ac.dts, fma_(((-fq(a.q[10])[j]) * (e - uc)) * g.rdx, hm_uh(hm, g, g.nx - 1), uten[c + 1]), e);
+  }
+  if (south) {
+    const float e = v[c - sj];
+    vn = fma_(ac.dts, fma_(((-fq(a.q[11])[i]) * (vc - e)) * g.rdy, hm_vh(hm, g, 0), vten[c - sj]), e);
+  }
+  if (north) {
+    const float e = v[c + sj];
+    vn = fma_(ac.dts, fma_(((-fq(a.q[12])[i]) * (e - vc)) * g.rdy, hm_vh(hm, g, g.ny - 1), vten[c + sj]), e);
+  }
+  if (!uEdge) u[c] = fma_(ac.dts, fma_(-((tem1 * (pc - px)) * hm_uf(hm, g, i)), tc + tx, ut), uc);
+  if (!vEdge) v[c] = fma_(ac.dts, fma_(-((tem2 * (pc - py)) * hm_vf(hm, g, j)), tc + ty, vt), vc);
+  if (west) u[c - 1] = un;
+  if (east) u[c + 1] = un;
+  if (south) v[c - sj] = vn;
+  if (north) v[c + sj] = vn;
+}
+
 // acoustic_fpk.wgsl:167-207
 __global__ __launch_bounds__(256) void k_acoustic_fpk(uint32_t* M, KArg a) {
   TE_TID3

@@ -60,31 +60,34 @@ __global__ __launch_bounds__(256) void k_bc_periodic_xy(uint32_t* M, KArg a) {
 // each; one launch for the 4 fields of a substep takes about what one pass did.
 // Grid as k_bc_periodic_xy.  p[1..8] fields, p[9] -> count, open x, open y and
 // per field 1 (on x faces), 2 (on y faces) or 0.
+TE_DEV bool halo_cell_at(const Dims& g, int n, int& i, int& j) {
+  const int rowCells = 7 * g.sJ;
+  if (n < rowCells) {
+    const int r = n / g.sJ;            // 0..6 -> j = -3..-1, ny..ny+3
+    i = n - r * g.sJ - 3;
+    j = r < 3 ? r - 3 : g.ny + (r - 3);
+    return true;
+  }
+  const int t = n - rowCells;          // ny rows x 7 halo columns, row by row
+  j = t / 7;
+  const int cidx = t - j * 7;
+  i = cidx < 3 ? cidx - 3 : g.nx + (cidx - 3);
+  return j < g.ny;
+}
+TE_DEV int halo_source(int q, int cells, bool open, int last) {
+  if (!open) return ((q % cells) + cells) % cells;
+  return q < 0 ? 0 : (q > last && q <= last + 3 ? last : q);
+}
 __global__ __launch_bounds__(256) void k_bc_open_xy(uint32_t* M, KArg a) {
   TE_TID3
   const Dims g = dims(a.q[0], 0);
   const int k = gy;
   if (k > g.nz) return;
-  const int rowCells = 7 * g.sJ;
   int i, j;
-  if (gx < rowCells) {
-    const int r = gx / g.sJ;           // 0..6 -> j = -3..-1, ny..ny+3
-    i = gx - r * g.sJ - 3;
-    j = r < 3 ? r - 3 : g.ny + (r - 3);
-  } else {
-    const int t = gx - rowCells;       // ny rows x 7 halo columns, row by row
-    j = t / 7;
-    const int cidx = t - j * 7;
-    if (j >= g.ny) return;
-    i = cidx < 3 ? cidx - 3 : g.nx + (cidx - 3);
-  }
+  if (!halo_cell_at(g, gx, i, j)) return;
   const uint32_t* P = a.q[9];
   const int n = ldi(P, 0);
   const bool openx = ldi(P, 1) != 0, openy = ldi(P, 2) != 0;
-  auto source = [](int q, int cells, bool open, int last) {
-    if (!open) return ((q % cells) + cells) % cells;
-    return q < 0 ? 0 : (q > last && q <= last + 3 ? last : q);
-  };
   const int64_t dst = g.idx(i, j, k);
   float v[8];
   bool fill[8];
@@ -93,7 +96,8 @@ __global__ __launch_bounds__(256) void k_bc_open_xy(uint32_t* M, KArg a) {
     fill[q] = false;
     if (q < n) {
       const int on = ldi(P, 3 + q);
-      const int64_t src = g.idx(source(i, g.nx, openx, g.nx - 1 + (on == 1)), source(j, g.ny, openy, g.ny - 1 + (on == 2)), k);
+      const int64_t src =
+          g.idx(halo_source(i, g.nx, openx, g.nx - 1 + (on == 1)), halo_source(j, g.ny, openy, g.ny - 1 + (on == 2)), k);
       fill[q] = src != dst;
       if (fill[q]) v[q] = fq(a.q[1 + q])[src];
     }
@@ -198,6 +202,10 @@ namespace te {
 // numbered level by level within a row j, so that an XCD takes the rows its
 // column workgroups read.  u at (nx, j) and v at (i, ny) of interior rows /
 // columns belong to the column workgroups, which read them.
+// OPEN: a side is open (p38); a halo cell's image is then found per field and
+// axis as by bc_open_xy, and u at (nx, j), v at (i, ny) of an open axis are
+// faces like the others.
+template <bool OPEN>
 TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t wg, int wave, int lane) {
   const uint32_t n = a.n[2], q8 = n >> 3, r8 = n & 7u, xcd = wg & 7u;  // a.n[2]: workgroups of this kind
   const uint32_t l = xcd * q8 + min(xcd, r8) + (wg >> 3);
@@ -205,12 +213,17 @@ TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t
   auto F = [&](int q) { return FieldB(reinterpret_cast<float*>(M) + a.p[q]); };
   const FieldB u = F(2), v = F(3), rru = F(13), rrv = F(14);
   const FieldB rruO = a.p[35] != 0 ? F(35) : rru, rrvO = a.p[36] != 0 ? F(36) : rrv;
+  const bool openx = OPEN && ldi(a.q[38], 0) != 0, openy = OPEN && ldi(a.q[38], 1) != 0;
+  auto source = [](int q, int cells, bool open, int last) {
+    if (!open) return q < 0 ? q + cells : q >= cells ? q - cells : q;
+    return q < 0 ? 0 : (q > last && q <= last + 3 ? last : q);
+  };
   const bool first = ldi(a.q[33], 0) != 0;
   const float tavg = ldf(a.q[17], 0), tv = tavg > 0.0f ? tavg : 1.0f;
   const uint32_t sjb = 4u * (uint32_t)g.sJ, skb = sjb * (uint32_t)g.sK;
   const int u0 = (int)(l * AC_WAVES + (uint32_t)wave) * AC_UV_UNITS;
   uint32_t h[AC_UV_UNITS];
-  int todo[AC_UV_UNITS];  // 1 rru, 2 rrv, 4 u and v from their image
+  int todo[AC_UV_UNITS];  // 1 rru, 2 rrv, 4 a halo cell, 8 u and 16 v from its image
   float uo[AC_UV_UNITS], vo[AC_UV_UNITS], ru[AC_UV_UNITS], rv[AC_UV_UNITS], us[AC_UV_UNITS], vs[AC_UV_UNITS];
 #pragma unroll
   for (int d = 0; d < AC_UV_UNITS; ++d) {
@@ -223,7 +236,7 @@ TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t
     const bool hx = i < 0 || i >= g.nx, hy = j < 0 || j >= g.ny;
     const uint32_t lv = skb * (uint32_t)k;
     h[d] = lv + 4u * (uint32_t)(i + 3) + sjb * (uint32_t)jr;
-    todo[d] = (!hy && i == g.nx ? 0 : 1) | (!hx && j == g.ny ? 0 : 2) | (hx || hy ? 4 : 0);
+    todo[d] = (!openx && !hy && i == g.nx ? 0 : 1) | (!openy && !hx && j == g.ny ? 0 : 2) | (hx || hy ? 4 : 0);
     uo[d] = u(h[d]);
     vo[d] = v(h[d]);
     ru[d] = rv[d] = 0.0f;
@@ -231,23 +244,31 @@ TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t
       ru[d] = rru(h[d]);
       rv[d] = rrv(h[d]);
     }
-    if (todo[d] & 4) {
+    if (OPEN && (todo[d] & 4)) {
+      const int su = source(i, g.nx, openx, g.nx), ju = source(j, g.ny, openy, g.ny - 1);
+      const int sv = source(i, g.nx, openx, g.nx - 1), jv = source(j, g.ny, openy, g.ny);
+      us[d] = u(lv + 4u * (uint32_t)(su + 3) + sjb * (uint32_t)(ju + 3));
+      vs[d] = v(lv + 4u * (uint32_t)(sv + 3) + sjb * (uint32_t)(jv + 3));
+      if (su != i || ju != j) todo[d] |= 8;
+      if (sv != i || jv != j) todo[d] |= 16;
+    } else if (todo[d] & 4) {
       const int si = i < 0 ? i + g.nx : i >= g.nx ? i - g.nx : i, sj = j < 0 ? j + g.ny : j >= g.ny ? j - g.ny : j;
       const uint32_t src = lv + 4u * (uint32_t)(si + 3) + sjb * (uint32_t)(sj + 3);
       us[d] = u(src);
       vs[d] = v(src);
+      todo[d] |= 24;
     }
   }
 #pragma unroll
   for (int d = 0; d < AC_UV_UNITS; ++d) {
     if (todo[d] & 1) rruO.put(h[d], (ru[d] + uo[d]) * tv);
     if (todo[d] & 2) rrvO.put(h[d], (rv[d] + vo[d]) * tv);
-    if ((todo[d] & 5) == 5) u.put(h[d], us[d]);
-    if ((todo[d] & 6) == 6) v.put(h[d], vs[d]);
+    if ((todo[d] & 9) == 9) u.put(h[d], us[d]);
+    if ((todo[d] & 18) == 18) v.put(h[d], vs[d]);
   }
 }
 
-// One acoustic substep after acoustic_uv, on a periodic domain, in one launch:
+// One acoustic substep after acoustic_uv, in one launch:
 // acoustic_fpk, acoustic_w_solve, acoustic_pp and acoustic_accumulate, then
 // the periodic halo fill of ppd, u, v and w, and on the stage's last substep
 // the one of pp3d that follows the substeps (timestep.js:2023-2054,
@@ -271,6 +292,11 @@ TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t
 // pivot before it is inverted, and takes the division only where a wave meets a
 // pivot outside the refined reciprocal's range (one uniform branch per row).
 //
+// OPEN (a side is open, p38): the halo of w, ppd and rrw is left to
+// ac_halo_open, since an open side's cells have up to 15 copies each; of a
+// periodic axis u at (nx, j) or v at (i, ny) stay here.  us per substep at
+// 120 x 120 x 40 with 7 species: 43 in six launches (edges, uv, fpk, w, pp with
+// the accumulation, halos) and 27 in three.
 // Halo cells (every halo cell of ppd, u, v, w is the image of interior cell
 // (i mod nx, j mod ny), as the halo fill leaves it), each updated by the
 // workgroup of its interior cell, at each level by the wave that owns it:
@@ -305,13 +331,14 @@ TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t
 //    too (with ppd's, group 4 below); the fields the replaced dispatches
 //    write as scratch (for expansions of this launch into them): 24 qk,
 //    25 pk1, 26 pk2, 27 mm, 28 fpk, 29 cA, 31 cB, and 32 rho0; 35-37 (if
-//    bound) the fields the accumulated rru, rrv, rrw go to instead, every word.
+//    bound) the fields the accumulated rru, rrv, rrw go to instead, every word
+//    (OPEN: but the halo of rrw); 38 -> open x, open y (OPEN only).
 // Grid: 64 x AC_WAVES threads per workgroup, ceil(nx / 64) * ny workgroups of
 // columns (padded to a multiple of 8), then a.n[2] of ac_accumulate_uv.
 // Needs nx, ny >= 4, 4 <= nz <= AC_WAVES * 16, and fields below 2^32 bytes
 // (word offsets into M are 32 bits and a program's fields share that range).
 #define AC_HALO_CELLS 40  // per workgroup: at most 7 x-images, 1 (nx, j) cell, 14 corners
-template <int L>
+template <int L, bool OPEN>
 __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   // Few levels per wave: the later phases' operands are kept or loaded ahead
   // of the sweep (registers to spare); many: the w rows wait in LDS and the
@@ -335,7 +362,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   const Dims g = dims(a.q[0], 0);
   const uint32_t solvers = (a.lg[9] + 7u) & ~7u;  // workgroups of columns, padded to the XCDs
   if (blockIdx.x >= solvers) {
-    ac_accumulate_uv(M, a, g, blockIdx.x - solvers, wave, lane);
+    ac_accumulate_uv<OPEN>(M, a, g, blockIdx.x - solvers, wave, lane);
     return;
   }
   if (blockIdx.x >= a.lg[9]) return;
@@ -361,8 +388,14 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   }
   // Halo cells of the x-images and corners of this workgroup's columns,
   // (hx, hy, 4), and (nx, j, 1): what `early` does with them
+  const bool openx = OPEN && ldi(a.q[38], 0) != 0, openy = OPEN && ldi(a.q[38], 1) != 0;
   const int ys[2] = {j >= ny - 3 ? j - ny : j, j <= 3 ? j + ny : j};
-  if (active && wave == 0) {  // (one wave: its LDS operations keep their order)
+  if (OPEN) {
+    if (active && wave == 0 && i == nx - 1 && !openx) {
+      hcell[0][0] = (short)nx; hcell[0][1] = (short)j; hcell[0][2] = 1;
+      hcnt = 1;
+    }
+  } else if (active && wave == 0) {  // (one wave: its LDS operations keep their order)
     const int xs[2] = {i >= nx - 3 ? i - nx : i, i <= 3 ? i + nx : i};
     const int nxi = (i >= nx - 3) + (i <= 3), nyi = (j >= ny - 3) + (j <= 3);
     const int n = nxi * (1 + nyi) + (i == nx - 1);
@@ -555,7 +588,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
         if (t0 + d < L && ROW(t0 + d)) f(d, at(k0 + t0 + d));
     };
 #pragma unroll 1
-    for (int r = 0; r < 2; ++r) {
+    for (int r = 0; r < (OPEN ? 0 : 2); ++r) {
       const int hy = ys[r];
       if (hy == j) continue;
       const uint32_t off = sjb * (uint32_t)(hy - j);
@@ -581,7 +614,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
     store(ia);
 #pragma unroll 1
     for (int it = lane + 64; it < items; it += 64) store(item(it));
-    if (j == ny - 1) {  // v at (i, ny)
+    if (j == ny - 1 && !openy) {  // v at (i, ny)
       const uint32_t src = sjb * (uint32_t)(-j);
 #pragma unroll
       for (int t0 = 0; t0 < L; t0 += CI) {
@@ -749,7 +782,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   // y (dy rows away), of the column in x (dx columns), and both
   const bool lo = i >= nx - 3, hi = i <= 3;
 #pragma unroll 1
-  for (int q = 1; q < 9; ++q) {
+  for (int q = 1; q < (OPEN ? 0 : 9); ++q) {
     const int xi = q % 3, yi = q / 3;
     const int dy = yi == 0 ? 0 : yi == 1 ? (j >= ny - 3 ? -ny : 0) : (j <= 3 ? ny : 0);
     if (yi > 0 && dy == 0) continue;
@@ -776,24 +809,53 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
 // instantiations by levels per wave: the runtime picks the one with
 // ceil(nz / AC_WAVES) levels (k_ac_column: 16)
 #define AC_INST(L, name, waves) \
-  __global__ __launch_bounds__(64 * AC_WAVES) __attribute__((amdgpu_waves_per_eu(waves))) void name(uint32_t* M, KArg a) { ac_column<L>(M, a); }
+  __global__ __launch_bounds__(64 * AC_WAVES) __attribute__((amdgpu_waves_per_eu(waves))) void name(uint32_t* M, KArg a) { ac_column<L, false>(M, a); } \
+  __global__ __launch_bounds__(64 * AC_WAVES) __attribute__((amdgpu_waves_per_eu(waves))) void name##_open(uint32_t* M, KArg a) { ac_column<L, true>(M, a); }
 AC_INST(1, k_ac_column1, 4) AC_INST(2, k_ac_column2, 4) AC_INST(3, k_ac_column3, 4) AC_INST(4, k_ac_column4, 4)
 AC_INST(5, k_ac_column5, 4) AC_INST(6, k_ac_column6, 4) AC_INST(7, k_ac_column7, 6) AC_INST(8, k_ac_column8, 6)
 AC_INST(9, k_ac_column9, 6) AC_INST(10, k_ac_column10, 6) AC_INST(11, k_ac_column11, 6) AC_INST(12, k_ac_column12, 6)
 AC_INST(13, k_ac_column13, 4) AC_INST(14, k_ac_column14, 4) AC_INST(15, k_ac_column15, 4) AC_INST(16, k_ac_column, 4)
 #undef AC_INST
 
-const void* ac_column_kernel(int levels_per_wave) {
-  static const void* const fns[17] = {nullptr,
-                                      (const void*)&k_ac_column1,  (const void*)&k_ac_column2,
-                                      (const void*)&k_ac_column3,  (const void*)&k_ac_column4,
-                                      (const void*)&k_ac_column5,  (const void*)&k_ac_column6,
-                                      (const void*)&k_ac_column7,  (const void*)&k_ac_column8,
-                                      (const void*)&k_ac_column9,  (const void*)&k_ac_column10,
-                                      (const void*)&k_ac_column11, (const void*)&k_ac_column12,
-                                      (const void*)&k_ac_column13, (const void*)&k_ac_column14,
-                                      (const void*)&k_ac_column15, (const void*)&k_ac_column};
-  return levels_per_wave >= 1 && levels_per_wave <= 16 ? fns[levels_per_wave] : nullptr;
+const void* ac_column_kernel(int levels_per_wave, bool open) {
+#define E(n) {(const void*)&n, (const void*)&n##_open}
+  static const void* const fns[17][2] = {{nullptr, nullptr}, E(k_ac_column1), E(k_ac_column2), E(k_ac_column3),
+                                         E(k_ac_column4), E(k_ac_column5), E(k_ac_column6), E(k_ac_column7),
+                                         E(k_ac_column8), E(k_ac_column9), E(k_ac_column10), E(k_ac_column11),
+                                         E(k_ac_column12), E(k_ac_column13), E(k_ac_column14), E(k_ac_column15),
+                                         E(k_ac_column)};
+#undef E
+  return levels_per_wave >= 1 && levels_per_wave <= 16 ? fns[levels_per_wave][open] : nullptr;
+}
+
+// The halo of w, ppd, rrw and, if asked for, pp3d after a substep of a domain
+// with an open side: rrw accumulates the old w there (the accumulation runs
+// before the fill), then w and ppd take their sources' values (k_bc_open_xy).
+// p: 1 acoustic, 2 w, 3 ppd, 4 rrw, 5 the accumulated rrw, 6 pp3d, 7 -> tavg,
+// 8 -> first substep of the stage (rrw starts as w * beta), 9 -> fill pp3d,
+// 10 -> open x, open y.  Grid as k_bc_open_xy.
+__global__ __launch_bounds__(256) void k_ac_halo_open(uint32_t* M, KArg a) {
+  TE_TID3
+  const Dims g = dims(a.q[0], 0);
+  const int k = gy;
+  if (k > g.nz) return;
+  int i, j;
+  if (!halo_cell_at(g, gx, i, j)) return;
+  const Acoustic ac = acoustic(a.q[1], 0);
+  const bool openx = ldi(a.q[10], 0) != 0, openy = ldi(a.q[10], 1) != 0, first = ldi(a.q[8], 0) != 0;
+  const bool fillP = ldi(a.q[9], 0) != 0;
+  const float tavg = ldf(a.q[7], 0);
+  const int64_t dst = g.idx(i, j, k);
+  const int64_t src = g.idx(halo_source(i, g.nx, openx, g.nx - 1), halo_source(j, g.ny, openy, g.ny - 1), k);
+  float *w = fq(a.q[2]), *ppd = fq(a.q[3]), *pp3d = fq(a.q[6]);
+  const float x = w[dst], y = first ? x * ac.beta : fq(a.q[4])[dst];
+  const float ws = w[src], ps = ppd[src], qs = fillP ? pp3d[src] : 0.0f;
+  fq(a.q[5])[dst] = tavg > 0.0f ? fma_(x, ac.alph, y) * tavg : y + x;
+  if (src != dst) {
+    w[dst] = ws;
+    ppd[dst] = ps;
+    if (fillP) pp3d[dst] = qs;
+  }
 }
 
 }  // namespace te

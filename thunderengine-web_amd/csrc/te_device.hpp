@@ -79,7 +79,7 @@ TE_DEV Sides open_sides(const KArg& a, int q) {
 // launch's stores (a load behind a store waits for it).  OPEN false: no side is
 // open; the two forms are compiled apart, as the open one in a periodic run's
 // launches cost them up to 20% (RK update at 192 x 192 x 80: 14.2, not 11.9 us).
-TE_DEV bool halo_source(Sides open, const Dims& g, int i, int j) {
+TE_DEV bool copies_halo(Sides open, const Dims& g, int i, int j) {
   const bool x = open.x ? i == 0 || i == g.nx - 1 : i <= 3 || i >= g.nx - 3;
   const bool y = open.y ? j == 0 || j == g.ny - 1 : j <= 3 || j >= g.ny - 3;
   return x || y;
@@ -89,8 +89,8 @@ template <bool OPEN>
 TE_DEV HaloOwn halo_own(const Dims& g, Sides open, const float* f, int i, int j, int64_t c) {
   HaloOwn o{0.0f, 0.0f};
   if (OPEN) {
-    if (open.x && i == g.nx - 1 && halo_source({true, open.y}, g, 1, j)) o.x = f[c + 4];
-    if (open.y && j == g.ny - 1 && halo_source({open.x, true}, g, i, 1)) o.y = f[c + 4 * (int64_t)g.sJ];
+    if (open.x && i == g.nx - 1 && copies_halo({true, open.y}, g, 1, j)) o.x = f[c + 4];
+    if (open.y && j == g.ny - 1 && copies_halo({open.x, true}, g, i, 1)) o.y = f[c + 4 * (int64_t)g.sJ];
   }
   return o;
 }
@@ -120,7 +120,7 @@ TE_DEV void halo_from(const Dims& g, Sides open, float* f, int i, int j, int64_t
     }
     return;
   }
-  if (!halo_source(open, g, i, j)) return;
+  if (!copies_halo(open, g, i, j)) return;
   const bool xe = i == 0 || i == g.nx - 1, ye = j == 0 || j == g.ny - 1;
   const int64_t dx = i == 0 ? -1 : 1, dy = j == 0 ? -sj : sj;
   auto copies = [&](float* r, float x) {  // the copies along x of the word at r

@@ -1004,10 +1004,11 @@ void Encoder::stages() {
        {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "ppi"), fb(5, "u"), fb(6, "v"), fb(7, "w"), fb(8, "pp3d"),
         fb(9, "ppd"), fb(10, "ppx")});
     acoustic = acousticBytes((double)(float)sch.dts[nrk]);
-    // fuse = 1 on a periodic domain: after acoustic_uv, one ac_column launch
+    // fuse = 1: after acoustic_uv, one ac_column launch (with an open side
+    // ac_halo_open after it, and the edges' update in acoustic_uv_open)
     // per substep (fpk, column solve, pp, accumulate, halo fill; prepare's
     // terms formed in it, begin folded into the stage's first substep)
-    const bool column = cfg.fuse == 1 && !openX && !openY && nx >= 4 && ny >= 4 && nz >= 4 && (nz + 7) / 8 <= 16;
+    const bool column = cfg.fuse == 1 && nx >= 4 && ny >= 4 && nz >= 4 && (nz + 7) / 8 <= 16;
     if (!column) {
       op("acoustic_prepare", full,
          {fb(2, "ppterm"), fb(3, "piadv"), fb(4, "thv"), rb(5, "rr0"), rb(6, "rf0"), rb(7, "mh"), rb(8, "mf"),
@@ -1023,12 +1024,18 @@ void Encoder::stages() {
       for (int d = 0; d < 3; ++d) E.ops.back().A[4 + q + d] = (uint32_t)off(out[d]);
     };
     for (int n = 0; n < nloop; ++n) {
-      if (openX || openY)
+      const bool sides = column && (openX || openY);
+      if (sides)
+        op("acoustic_uv_open", stag,
+           {fb(2, "ppd"), fb(3, "thv"), fb(4, "uten"), fb(5, "vten"), fb(6, "u"), fb(7, "v"), bb(8, open),
+            rb(9, "radbcw"), rb(10, "radbce"), rb(11, "radbcs"), rb(12, "radbcn")},
+           true);
+      else if (openX || openY)
         op("openbc_uv_tendency", {std::max(nx, ny), nz, 1},
            {rb(2, "radbcw"), rb(3, "radbce"), rb(4, "radbcs"), rb(5, "radbcn"), fb(6, "uten"), fb(7, "vten"),
             fb(8, "u"), fb(9, "v"), bb(10, open)},
            true);
-      op("acoustic_uv", stag,
+      if (!sides) op("acoustic_uv", stag,
          {fb(2, "ppd"), fb(3, "thv"), fb(4, "uten"), fb(5, "vten"), fb(6, "u"), fb(7, "v"), bb(8, open)}, true);
       if (column) {
         const float tavg = n == nloop - 1 ? (float)(1.0 / nloop) : 0.0f;
@@ -1038,9 +1045,16 @@ void Encoder::stages() {
             fb(15, "rrw"), bb(16, I1(nrk == 2 ? 1 : 0)), bb(17, F1(tavg)), rb(18, "rr0"), rb(19, "rf0"),
             rb(20, "mh"), rb(21, "mf"), rb(22, "c1"), rb(23, "c2"), fb(24, "qk"), fb(25, "pk1"), fb(26, "pk2"),
             fb(27, "mm"), fb(28, "fpk"), fb(29, "cA"), fb(31, "cB"), rb(32, "rho0"), bb(33, I1(n == 0 ? 1 : 0)),
-            bb(34, I1(foldHalo && n == nloop - 1 ? 1 : 0))},
+            bb(34, I1(foldHalo && !sides && n == nloop - 1 ? 1 : 0))},
            true);
         if (n == nloop - 1) meanOut(35);
+        if (sides) {
+          E.ops.back().A[4 + 38] = (uint32_t)bytes(open);
+          op("ac_halo_open", {7 * (nx + 7) + 7 * ny, nz + 1, 1},
+             {fb(2, "w"), fb(3, "ppd"), fb(4, "rrw"), fb(5, n == nloop - 1 ? "fz" : "rrw"), fb(6, "pp3d"),
+              bb(7, F1(tavg)), bb(8, I1(n == 0 ? 1 : 0)), bb(9, I1(n == nloop - 1 ? 1 : 0)), bb(10, open)},
+             true);
+        }
         continue;
       }
       if (cfg.fuse != 0) {  // pp + accumulate in one pass; accumulate reads no ppd, so ppd's

@@ -163,7 +163,7 @@ static hipError_t shape_of(te_ctx* c, const Op& op, Shape& s) {
     b = dim3(64, AC_WAVES, 1);
     const dim3 g((a.n[0] + 63) / 64, a.n[1], 1);
     if (!launch_shape(a, b, g)) return hipErrorInvalidConfiguration;
-    const void* fn = ac_column_kernel((int)lw);
+    const void* fn = ac_column_kernel((int)lw, op.A[4 + 38] != 0);
     // beyond 6 levels per wave the w rows wait in LDS: 2 floats per level and lane
     const size_t dyn = lw > 6 ? (size_t)2 * nz * 64 * sizeof(float) : 0;
     if (dyn > 65536) {
