@@ -430,8 +430,8 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
       prep(k, f);
       for (int q = 0; q < 6; ++q) lv[q][k] = f[q];
     }
+    __syncthreads();
   }
-  __syncthreads();
   const FieldB u = F(2), v = F(3), w = F(4), piadv = F(5), ppten = F(6), ppterm = F(7), thv = F(8), wten = F(9),
                pp3d = F(10), ppd = F(11), ppx = F(12), rru = F(13), rrv = F(14), rrw = F(15);
   const FieldB rruO = a.p[35] != 0 ? F(35) : rru, rrvO = a.p[36] != 0 ? F(36) : rrv, rrwO = a.p[37] != 0 ? F(37) : rrw;
@@ -476,6 +476,14 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
         const uint32_t o = at(min(k0 + t0 + n, nz));
         W[n] = w(o);
         PA[n] = piadv(o);
+      }
+      // AHEAD: the workgroup meets here, every load on its way, rather than
+      // before them (what the barrier guards lies in LDS: the counters and the
+      // list above)
+      if constexpr (AHEAD) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
       }
 #pragma unroll
       for (int d = 0; d < CH; ++d)
@@ -579,6 +587,8 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
       }
     };
     const Item ia = item(lane);
+    Item ib = {0u, 0, 0.0f, 0.0f, 0.0f};  // (rows with y images: more than 64 pairs)
+    if (AHEAD && items > 64) ib = item(lane + 64);
     // the row's own images, lane = column: rows t0 .. t0 + CI - 1 of the wave
     // (and level nz as row Lq), loads without a branch between them
     constexpr int CI = AHEAD ? L : 5;
@@ -612,8 +622,9 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
       }
     }
     store(ia);
+    if (AHEAD) store(ib);
 #pragma unroll 1
-    for (int it = lane + 64; it < items; it += 64) store(item(it));
+    for (int it = lane + (AHEAD ? 128 : 64); it < items; it += 64) store(item(it));
     if (j == ny - 1 && !openy) {  // v at (i, ny)
       const uint32_t src = sjb * (uint32_t)(-j);
 #pragma unroll
@@ -659,21 +670,28 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   // elimination) and for back_next == w (set by wave w+1 after its back
   // substitution; the top wave is the last of the forward chain), so each
   // wait ends once the waves below / above it have run.  The waits are
-  // bounded (2^22 polls) all the same.  What is handed over lies in LDS, whose
-  // operations a wave issues and the LDS executes in order: the flag needs the
-  // LDS counter only, not a release of the wave's global loads and stores
-  // (192 x 192 x 80: the top wave waited 43 k cycles there for rrw).
-  auto wait_for = [&](int* flag, int want) {
+  // bounded (2^22 polls) all the same.  What is handed over lies in LDS, which
+  // executes a wave's operations in the order it issues them: data written
+  // before the flag is there when the flag is, and data read after the flag,
+  // in the same poll, is valid when the flag was set.  So a hand-off waits for
+  // no counter and reads nothing after the flag; a wave whose turn is next
+  // polls without sleeping.  (450 cycles a hand-off with the flag behind a
+  // wait, the data read after it and a sleep in every poll, 16 of them a
+  // launch; a release of the wave's global accesses cost 43 k cycles at
+  // 192 x 192 x 80.)
+  auto wait_for = [&](int* flag, int want, auto&& read) {
     for (int s = 0; s < (1 << 22); ++s) {
-      const int f = __builtin_amdgcn_readfirstlane(
-          __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+      const int f0 = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      asm volatile("" ::: "memory");
+      read();
+      const int f = __builtin_amdgcn_readfirstlane(f0);
       if (f == want) break;
-      __builtin_amdgcn_s_sleep(1);
+      if (f < want - 1 || f > want + 1) __builtin_amdgcn_s_sleep(1);
     }
     asm volatile("" ::: "memory");
   };
   auto pass = [&](int* flag, int f) {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    asm volatile("" ::: "memory");
     __hip_atomic_store(flag, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
   // ---- forward elimination, wave after wave: (mm, right-hand side) of a row
@@ -701,14 +719,18 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
     for (int t = 1; t < L; ++t) R[t] = row(t, PQ[t - 1], P2Q[t - 1], PF[t - 1]);
   }
   if (upper && Lq > 0) early();
-  wait_for(&fwd_done, wave);
+  float pa = 0.0f, pb = 0.0f, x0 = 0.0f, x1 = 0.0f, x2 = 0.0f;
+  const int below = max(wave - 1, 0);
+  wait_for(&fwd_done, wave, [&]() {
+    pa = xb[0][lane];
+    pb = xb[1][lane];
+    x0 = xa[below][0][lane];
+    x1 = xa[below][1][lane];
+    x2 = xa[below][2][lane];
+  });
   if (Lq > 0) {
-    float pa = 0.0f, pb = 0.0f;
-    if (wave > 0) {
-      pa = xb[0][lane];
-      pb = xb[1][lane];
-      R[0] = row(0, xa[wave - 1][0][lane], xa[wave - 1][1][lane], xa[wave - 1][2][lane]);
-    }
+    if (wave > 0) R[0] = row(0, x0, x1, x2);
+    else pa = pb = 0.0f;
 #pragma unroll
     for (int t = 0; t < L; ++t) {
       const bool first_row = t == (L > 1 ? 1 : 0) && k0 + t == 1;
@@ -739,10 +761,10 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   if (!upper && Lq > 0) early();
   if (Lq > 0) load_rrw();
   // ---- back substitution, wave after wave downwards: CA becomes the new w
-  wait_for(&back_next, wave);
   float wnext = 0.0f;
+  wait_for(&back_next, wave, [&]() { wnext = xw[lane]; });
   if (Lq > 0) {
-    if (!top) wnext = xw[lane];
+    if (top) wnext = 0.0f;
     float wn = wnext;
 #pragma unroll
     for (int t = L - 1; t >= 0; --t)
