@@ -132,6 +132,10 @@ def alg_bytes_per_launch(run, names, A, op):
         io = [(1 + q, False, True) for q in range(3)] + [(4 + q, True, False) for q in range(3)]
     elif name == "adv_fused":
         io = adv_fused_io(run, A, op)
+    elif name == "diabatic_finish":
+        io = ([(i, True, True) for i in range(2, 10)] + [(12, False, True), (13, False, True), (14, True, True)])
+    elif name == "acoustic_uv_open":
+        io = [(i, True, False) for i in (2, 3, 4, 5)] + [(6, True, True), (7, True, True)]
     elif name == "mean_massflux":
         io = ([(i, True, False) for i in (1, 2, 3, 13)] + [(i, False, True) for i in (6, 7, 8, 10, 11, 14)])
     elif name == "adv_pdef":

@@ -279,6 +279,31 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
       if (P(34) != 0 && w[P(34)] != 0u) fill_periodic(w, v, A, PP3D);  // the stage's pp3d fill, folded in
       continue;
     }
+    if (nm == "diabatic_finish") {
+      // diabatic_unapply, update_rho_prs, diabatic_rates, ppx_finish and ppx's halo fill
+      auto P = [&](int q) { return A[4 + q]; };
+      auto run1 = [&](const char* kn, std::vector<std::pair<int, uint32_t>> ps) {
+        uint32_t X[64] = {0};
+        const uint32_t* dm = w + A[4];
+        X[0] = dm[0]; X[1] = dm[1]; X[2] = dm[2];
+        X[4] = A[4]; X[34] = A[34];
+        for (auto& pr : ps) X[4 + pr.first] = pr.second;
+        K<T> k1{w, v, X};
+        call(find_kernel(kn), k1);
+      };
+      std::vector<std::pair<int, uint32_t>> ps;
+      for (int q = 1; q <= 9; ++q) ps.push_back({q, P(q)});
+      run1("diabatic_unapply", ps);
+      const uint32_t dt = w[P(1)];
+      w[P(1)] = 1u;  // update_rho_prs' flag: a moist run
+      run1("update_rho_prs", {{1, P(1)}, {2, P(3)}, {3, P(2)}, {4, P(10)}, {5, P(11)}, {6, P(4)}, {7, P(12)}, {8, P(13)}});
+      w[P(1)] = dt;
+      run1("diabatic_rates", ps);
+      run1("ppx_finish", {{1, P(2)}, {2, P(14)}});
+      if (P(15) == 0) fill_periodic(w, v, A, P(14));
+      else fill_halo(w, v, A, P(14), w[P(15)] != 0u, w[P(15) + 1] != 0u, P(15));
+      continue;
+    }
     if (nm == "ac_halo_open") {  // (the oracle's ac_column has accumulated rrw's halo too)
       const uint32_t so = A[4 + 10];
       const bool ox = w[so] != 0u, oy = w[so + 1] != 0u;

@@ -263,6 +263,8 @@ __global__ __launch_bounds__(256) void k_pressure_tendency(uint32_t* M, KArg a) 
 
 __global__ __launch_bounds__(256) void k_update_rho_prs(uint32_t* M, KArg a) { update_rho_prs_body(M, a, te_block(a)); }
 
+__global__ __launch_bounds__(256) void k_diabatic_finish(uint32_t* M, KArg a) { diabatic_finish_body(M, a, te_block(a)); }
+
 // stability_max.wgsl:120-178 (adapt_dt = 1): max over the grid of the
 // squared advective Courant number c2 = x^2 + y^2 + z^2 (x = (u_i + u_i+1)
 // dt / (2 dx) uh, and alike) and of the squared diffusion number of kmh,

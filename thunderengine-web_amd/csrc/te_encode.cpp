@@ -260,6 +260,8 @@ class Encoder {
   void haloFill(const std::string& n);
   void openTurbFlux(const std::string& fx, const std::string& fy);
   void rayleighDamping();
+  // the step's end in one launch (diabatic_finish)
+  bool finishFused() const { return cfg.fuse == 1 && moist && usePT && !massCons && !hasMicro; }
   // fuse = 1: the moisture scalars' SGS tendencies go to their caches, and
   // nothing else adds to `tend` scalar by scalar
   bool sgsCached() const { return cfg.fuse == 1 && moist && tke && cacheMT && !(hasMicro && usePT); }
@@ -1132,7 +1134,12 @@ void Encoder::stages() {
            {bb(1, I1(1)), fb(2, scalars[q] + "_a"), fb(3, own[q - 1]), fb(4, scalars[q]), bb(5, dttmp)});
         foldSides(6);
       }
-    if (nrk == 2) {
+    if (nrk == 2 && finishFused()) {
+      op("diabatic_finish", full,
+         {bb(1, F1(dtf)), fb(2, "pp3d"), fb(3, "th"), fb(4, "qv"), fb(5, "qc"), fb(6, "qpten"), fb(7, "qtten"),
+          fb(8, "qvten"), fb(9, "qcten"), rb(10, "th0"), rb(11, "pi0"), fb(12, "prs"), fb(13, "rho"), fb(14, "ppx")});
+      foldSides(15);
+    } else if (nrk == 2) {
       if (moist && usePT)
         op("diabatic_unapply", full,
            {bb(1, F1(dtf)), fb(2, "pp3d"), fb(3, "th"), fb(4, "qv"), fb(5, "qc"), fb(6, "qpten"), fb(7, "qtten"),
@@ -1166,13 +1173,15 @@ void Encoder::end() {
     op("mp_pdefq", {nx, ny, 1}, {fb(1, "rho"), fb(2, "qv"), bb(3, F1(0.0f))});
     op("microphysics", {nx, ny, 1}, {});
   }
-  if (moist && usePT)
+  if (moist && usePT && !finishFused())
     op("diabatic_rates", full,
        {bb(1, F1(dtf)), fb(2, "pp3d"), fb(3, "th"), fb(4, "qv"), fb(5, "qc"), fb(6, "qpten"), fb(7, "qtten"),
         fb(8, "qvten"), fb(9, "qcten")});
-  op(foldHalo ? "ppx_finish_xy" : "ppx_finish", full, {fb(1, "pp3d"), fb(2, "ppx")});
-  foldSides(3);
-  if (!foldHalo) haloFill("ppx");
+  if (!finishFused()) {
+    op(foldHalo ? "ppx_finish_xy" : "ppx_finish", full, {fb(1, "pp3d"), fb(2, "ppx")});
+    foldSides(3);
+    if (!foldHalo) haloFill("ppx");
+  }
   flushAdd();
   flushHalo();
   flushZero();
