@@ -134,6 +134,8 @@ def alg_bytes_per_launch(run, names, A, op):
         io = adv_fused_io(run, A, op)
     elif name == "diabatic_finish":
         io = ([(i, True, True) for i in range(2, 10)] + [(12, False, True), (13, False, True), (14, True, True)])
+    elif name == "tke_epst_sources":
+        io = kernel_io()["tke_epst"] + [(16, True, False), (17, True, False), (18, True, False), (19, False, True)]
     elif name == "acoustic_uv_open":
         io = [(i, True, False) for i in (2, 3, 4, 5)] + [(6, True, True), (7, True, True)]
     elif name == "mean_massflux":

@@ -279,6 +279,18 @@ static int run_program(uint32_t* w, T* v, const char* const* names, const uint32
       if (P(34) != 0 && w[P(34)] != 0u) fill_periodic(w, v, A, PP3D);  // the stage's pp3d fill, folded in
       continue;
     }
+    if (nm == "tke_epst_sources") {  // tke_epst, then tke_sources
+      K<T> k1{w, v, A};
+      call(find_kernel("tke_epst"), k1);
+      const uint32_t* dm = w + A[4];
+      uint32_t X[64] = {0};
+      X[0] = dm[0]; X[1] = dm[1]; X[2] = dm[2];
+      X[4] = A[4]; X[34] = A[34];
+      X[5] = A[4 + 16]; X[6] = A[4 + 17]; X[7] = A[4 + 18]; X[8] = A[4 + 15]; X[9] = A[4 + 19];
+      K<T> k2{w, v, X};
+      call(find_kernel("tke_sources"), k2);
+      continue;
+    }
     if (nm == "diabatic_finish") {
       // diabatic_unapply, update_rho_prs, diabatic_rates, ppx_finish and ppx's halo fill
       auto P = [&](int q) { return A[4 + q]; };

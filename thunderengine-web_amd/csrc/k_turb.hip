@@ -71,7 +71,12 @@ __global__ __launch_bounds__(256) void k_turb_sfcstress(uint32_t* M, KArg a) {
 // runtime halves the launch's z extent): k0 = 2 gz + 1 and k0 + 1.  The
 // terms of the face between them (L1, the four-point L2 sum, L5 at k0) enter
 // level k0 as its upper terms and level k0 + 1 as its lower ones, formed once.
-__global__ __launch_bounds__(256) void k_tke_epst(uint32_t* M, KArg a) {
+// SOURCES: tke_sources (tke_sources.wgsl:111-129) of the levels too, from their
+// epst in registers (tketen = fma(-khv, nm, -dissten) + epst; p16 khv, 17 nm,
+// 18 dissten, 19 tketen): a pass over 5 fields and a launch less (a step of
+// 32 x 24 x 16 288.4 and 286.0 us, of 192 x 192 x 80 2983 and 2974).
+template <bool SOURCES>
+__device__ __forceinline__ void tke_epst(uint32_t* M, const KArg& a) {
   TE_TID3
   Dims g = dims(a.q[0], 0);
   const int i = gx, j = gy, k0 = 2 * gz + 1;
@@ -106,16 +111,33 @@ __global__ __launch_bounds__(256) void k_tke_epst(uint32_t* M, KArg a) {
   };
   const int64_t cd = c0 - sk, cu = c0 + sk;
   const float l1m = L1(cd), l10 = L1(c0), s2m = L2s(cd), s20 = L2s(c0), l5m = L5(cd, k0 - 1), l50 = L5(c0, k0);
+  const bool two = k0 + 1 <= g.nz - 1;
+  float h0 = 0.0f, n0 = 0.0f, d0 = 0.0f, h1 = 0.0f, n1 = 0.0f, d1 = 0.0f;
+  if (SOURCES) {
+    const float *khv = fq(a.q[16]), *nm = fq(a.q[17]), *dissten = fq(a.q[18]);
+    h0 = khv[c0];
+    n0 = nm[c0];
+    d0 = dissten[c0];
+    if (two) {
+      h1 = khv[cu];
+      n1 = nm[cu];
+      d1 = dissten[cu];
+    }
+  }
   const float e0 = level(k0, c0, l1m, l10, s2m, s20, l5m, l50);
+  float e1 = 0.0f;
+  if (two) e1 = level(k0 + 1, cu, l10, L1(cu), s20, L2s(cu), l50, L5(cu, k0 + 1));
   float* epst = fq(a.q[15]);
-  if (k0 + 1 <= g.nz - 1) {
-    const float e1 = level(k0 + 1, cu, l10, L1(cu), s20, L2s(cu), l50, L5(cu, k0 + 1));
-    epst[c0] = e0;
-    epst[cu] = e1;
-  } else {
-    epst[c0] = e0;
+  epst[c0] = e0;
+  if (two) epst[cu] = e1;
+  if (SOURCES) {
+    float* tketen = fq(a.q[19]);
+    tketen[c0] = fma_(-h0, n0, -d0) + e0;
+    if (two) tketen[cu] = fma_(-h1, n1, -d1) + e1;
   }
 }
+__global__ __launch_bounds__(256) void k_tke_epst(uint32_t* M, KArg a) { tke_epst<false>(M, a); }
+__global__ __launch_bounds__(256) void k_tke_epst_sources(uint32_t* M, KArg a) { tke_epst<true>(M, a); }
 
 __global__ __launch_bounds__(256) void k_tke_sources(uint32_t* M, KArg a) { tke_sources_body(M, a, te_block(a)); }
 

@@ -533,6 +533,13 @@ void Encoder::turbulence() {
     openStress();
   };
   auto epst = [&] {
+    if (cfg.fuse == 1) {
+      op("tke_epst_sources", full,
+         {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "s11"), fb(5, "s12"), fb(6, "s13"), fb(7, "s22"), fb(8, "s23"),
+          fb(9, "s33"), fb(10, "rf"), rb(11, "mh"), rb(12, "mf"), rb(13, "c1"), rb(14, "c2"), fb(15, "epst"),
+          fb(16, "khv"), fb(17, "nm"), fb(18, "dissten"), fb(19, "tketen")});
+      return;
+    }
     op("tke_epst", full,
        {fb(1, "u_a"), fb(2, "v_a"), fb(3, "w_a"), fb(4, "s11"), fb(5, "s12"), fb(6, "s13"), fb(7, "s22"), fb(8, "s23"),
         fb(9, "s33"), fb(10, "rf"), rb(11, "mh"), rb(12, "mf"), rb(13, "c1"), rb(14, "c2"), fb(15, "epst")});

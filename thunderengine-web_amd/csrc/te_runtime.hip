@@ -143,9 +143,9 @@ static hipError_t shape_of(te_ctx* c, const Op& op, Shape& s) {
     return hipSuccess;
   };
   dim3 b = block_for(a.n);
-  static const int kTkeEpst = kernel_id("tke_epst");
+  static const int kTkeEpst = kernel_id("tke_epst"), kTkeEpstSources = kernel_id("tke_epst_sources");
   if (row_waves(op.kid)) b = dim3(64, 4, 1);  // one row of cells per wave (k_adv_fused)
-  if (op.kid == kTkeEpst) a.n[2] = (a.n[2] + 1) / 2;  // two levels per thread (k_tke_epst)
+  if (op.kid == kTkeEpst || op.kid == kTkeEpstSources) a.n[2] = (a.n[2] + 1) / 2;  // two levels per thread (k_tke_epst)
   // rows (or levels) dealt to workgroups by the kernel: radbc 16 rows, the mass
   // sums 16 rows and one level
   static const int kRadbcEw = kernel_id("radbc_ew"), kRadbcNs = kernel_id("radbc_ns"),
