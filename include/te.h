@@ -55,6 +55,15 @@ int te_download_words(te_ctx* ctx, uint64_t word_off, uint32_t* dst, uint64_t nw
  * Full steps replay a captured HIP graph. */
 int te_run(te_ctx* ctx, int32_t nsteps, int32_t first_op, int32_t last_op);
 
+/* How te_run groups such a program's dispatches (no device, no context; mem
+ * holds the program's memory, whose parameter words name each dispatch's grid
+ * and options): consecutive dispatches none of which reads or writes a word
+ * that another one of them writes may run side by side in one launch.
+ * batch[i] = the dispatches that the launch beginning at dispatch i runs, 0
+ * for one that an earlier launch runs. */
+int te_plan_batches(uint64_t mem_words, const uint32_t* mem, int32_t nops, const char* const* names,
+                    const uint32_t* args, int32_t* batch);
+
 /* Runs nsteps full steps eagerly with a HIP event after every op on the
  * context's stream and adds each op's device duration (ms) into op_ms
  * (te_op_count floats, cleared first).  Profiling aid: no counterpart in the

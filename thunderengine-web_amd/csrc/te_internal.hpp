@@ -18,7 +18,7 @@ struct Op {
   int32_t kid;
   uint32_t A[64];
   int32_t nz = 0;  // levels of the op's grid (set before the first launch)
-  int32_t sJ = 0, sK = 0;  // its row and plane strides (set with nz)
+  int32_t nx = 0, ny = 0, sJ = 0, sK = 0;  // its cells, row and plane strides (set with nz)
   bool flat = false;  // launched flat over its words (set with nz)
   bool plane = false;  // launched over its (i, j) plane's points (set with nz)
   // launch shape chosen by te_autotune (generic 3-D kernels only)
@@ -27,11 +27,22 @@ struct Op {
   // the kernel launched in place of the op's table entry: a body specialised
   // on parameters the op fixes (set with nz; null: the table's kernel)
   const void* fn = nullptr;
-  // adv_fused, adv_pdef: the chain flags and specialised body (-1: none)
-  int32_t chain = 0, body = -1;
-  // ops, from this one on, that one launch runs side by side (set with nz)
+  // adv_fused, adv_pdef: the chain flags, accumulation and specialised body
+  // (-1: none); zero_fields, copy_fields: the fields
+  int32_t chain = 0, acc = 0, body = -1, count = 0;
+  // ops, from this one on, that one launch runs side by side, and its kernel
+  // (set with nz)
   int32_t batch = 1;
+  const void* batch_fn = nullptr;
 };
+
+// Words [at, at + n) of M, and those a dispatch reads and writes (set ops;
+// false for a kernel that no batch holds).  Two dispatches are independent if
+// neither writes a word that the other one reads or writes.
+struct Words { uint64_t at, n; };
+struct OpWords { std::vector<Words> reads, writes; };
+bool op_words(const Op& op, OpWords& w);
+bool independent(const OpWords& a, const OpWords& b);
 
 int kernel_id(const char* name);
 const char* kernel_name(int kid);

@@ -9,6 +9,7 @@
 #include <array>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <limits>
 #include <map>
 #include <mutex>
@@ -234,56 +235,8 @@ static hipError_t launch(te_ctx* c, const Op& op) {
 }
 
 // ---- batches: consecutive dispatches none of which reads or writes what
-// another one writes, run side by side by one launch (KBatch).  The fields a
-// dispatch reads and writes, by parameter (unbound ones are skipped; fields
-// that never change in a step, as profiles, are left out).
-struct OpFields { std::vector<int> reads, writes; };
-static const OpFields* op_fields(int kid) {
-  static const std::map<int, OpFields> all = [] {
-    const std::vector<std::pair<const char*, OpFields>> l = {
-        {"rayleigh_damping", {{1, 2, 3, 4}, {10, 11, 12, 13}}},
-        {"turb_rho_faces", {{1}, {4, 5}}},
-        {"turb_def_centers", {{1, 2, 3, 4}, {6, 7, 8, 9}}},
-        {"turb_def_faces", {{1, 2, 3, 4}, {6, 7}}},
-        {"turb_def_assemble", {{1, 2, 3, 4, 5, 6, 9}, {10, 11}}},
-        {"turb_nm", {{1, 2, 5, 6, 7, 8, 9, 10, 11}, {15, 17}}},
-        {"turb_km_kh", {{1, 2, 9}, {4, 5, 6, 7, 8, 9}}},
-        {"turb_km_kh_xy", {{1, 2, 9}, {4, 5, 6, 7, 8, 9}}},
-        {"turb_dissipative_heating", {{1, 3, 4, 5, 6, 7, 8, 9, 10, 12}, {10}}},
-        {"turb_gettau", {{1, 2, 3, 4, 5, 6, 7, 8}, {3, 4, 5, 6, 7, 8}}},
-        {"tke_sources", {{1, 2, 3, 4}, {5}}},
-        {"turb_scalar_flux_h", {{1, 2, 3}, {5, 6}}},
-        {"tke_flux_h", {{1, 2, 3}, {4, 5}}},
-        {"turb_openbc_flux", {{1, 2}, {1, 2}}},
-        {"update_diagnostics_moist", {{1, 2, 9, 10, 11, 12, 13, 14}, {15, 16, 17, 18, 19}}},
-        {"update_diagnostics", {{1, 2}, {5, 6, 7, 9}}},
-        {"stage_tendency_reset", {{}, {1, 2, 3}}},
-        {"stage_state_reset", {{1, 2, 3, 4, 10}, {5, 6, 7, 8, 9}}},
-        {"massflux_div", {{1, 2, 3}, {6, 7, 8, 10}}},
-        {"build_sadv", {{2}, {3}}},
-        {"ppx_finish_xy", {{1, 2}, {2}}},
-        {"diabatic_rates", {{2, 3, 4, 5, 6, 7, 8, 9}, {6, 7, 8, 9}}},
-        {"pressure_tendency", {{1, 2, 3, 4, 5, 6, 13}, {11}}},
-        {"update_rho_prs", {{2, 3, 6}, {7, 8}}},
-        {"tke_advance_xy", {{1, 2}, {4}}},
-        {"zero_fields", {{}, {1, 2, 3, 4, 5, 6, 7, 8}}},
-        {"tendency_reset_add", {{4, 5, 6}, {1, 2, 3}}},
-        {"copy_fields", {{1, 2, 3, 4}, {5, 6, 7, 8}}},
-        {"rk_update_xy", {{2, 3}, {4}}},
-        {"turb_u_tendency_lds", {{1, 2, 3, 4, 5, 6, 7, 8, 14, 15}, {14, 15}}},
-        {"turb_v_tendency_lds", {{1, 2, 3, 4, 5, 6, 7, 8, 14, 15}, {14, 15}}},
-        {"turb_w_tendency_lds", {{1, 2, 3, 4, 5, 6, 7, 13}, {13}}},
-        {"turb_scalar_vert_implicit_lds", {{1, 2, 3, 4, 5, 8, 9, 13, 14}, {13}}},
-        {"tke_transport_lds", {{1, 2, 3, 4, 5, 11, 12, 13}, {13}}},
-        {"adv_fused", {{2, 4, 6, 13, 14}, {11, 40}}},  // and by its chain flags, below
-        {"adv_pdef", {{2, 4, 6, 13, 14, 46}, {11, 22, 23, 24, 43, 44, 45}}}};
-    std::map<int, OpFields> m;
-    for (const auto& e : l) m[kernel_id(e.first)] = e.second;
-    return m;
-  }();
-  const auto it = all.find(kid);
-  return it == all.end() ? nullptr : &it->second;
-}
+// another one writes (op_words, te_plan.cpp), run side by side by one launch
+// (KBatch).
 // Which batch kernel an op may join: 1 advection, 2 pointwise, 3 sweeps (body:
 // its body there), or 0.
 static int batch_family(const Op& op, int& body) {
@@ -311,42 +264,22 @@ static int batch_family(const Op& op, int& body) {
   body = it->second;
   return 2;
 }
-static const void* batch_kernel(const Op* ops, int n) {
+// The kernel that runs ops[0 .. n-1] (w: their words) side by side, or null.
+static const void* batch_kernel(const Op* ops, const OpWords* w, int n) {
   if (n < 2 || n > TE_BATCH) return nullptr;
   int family = 0;
   uint32_t bodies = 0;
   const uint64_t words = (uint64_t)ops[0].sJ * ops[0].sK * (ops[0].nz + 1);
-  std::vector<uint32_t> r, w;
-  auto meets = [&](const std::vector<uint32_t>& v, uint32_t f) {
-    for (uint32_t x : v)
-      if ((x > f ? x - f : f - x) < words) return true;
-    return false;
-  };
   for (int i = 0; i < n; ++i) {
     const Op& op = ops[i];
     int body = 0;
     const int fam = batch_family(op, body);
-    const OpFields* fields = op_fields(op.kid);
-    if (fam == 0 || (i > 0 && fam != family) || op.A[4] != ops[0].A[4] || !fields) return nullptr;  // one grid
+    if (fam == 0 || (i > 0 && fam != family) || op.A[4] != ops[0].A[4]) return nullptr;  // one grid
     if (op.A[0] == 0 || op.A[1] == 0 || op.A[2] == 0) return nullptr;
     family = fam;
     if (fam == 1) bodies |= 1u << body;
-    std::vector<uint32_t> ri, wi;
-    auto add = [&](std::vector<uint32_t>& to, int q) {
-      if (op.A[4 + q] != 0) to.push_back(op.A[4 + q]);
-    };
-    for (int q : fields->reads) add(ri, q);
-    for (int q : fields->writes)
-      // a chained advection (chain 8) updates the field and leaves the tendency
-      if (fam != 1 || q != ((op.chain & 8) ? 11 : 40)) add(wi, q);
-    if (fam == 1)
-      for (int q : {33, 34, 35, 37, 39, 42}) add(ri, q);
-    for (uint32_t f : wi)
-      if (meets(r, f) || meets(w, f)) return nullptr;
-    for (uint32_t f : ri)
-      if (meets(w, f)) return nullptr;
-    r.insert(r.end(), ri.begin(), ri.end());
-    w.insert(w.end(), wi.begin(), wi.end());
+    for (int q = 0; q < i; ++q)
+      if (!independent(w[q], w[i])) return nullptr;
   }
   if (family == 1) return adv_batch_kernel(bodies);
   if (family == 3) return sweep_batch_kernel((ops[0].nz + AC_WAVES - 1) / AC_WAVES);
@@ -359,7 +292,7 @@ static const void* batch_kernel(const Op* ops, int n) {
   return words <= (3u << 20) ? (const void*)&k_point_batch : nullptr;
 }
 static hipError_t launch_batch(te_ctx* c, const Op* ops, int n) {
-  const void* fn = batch_kernel(ops, n);
+  const void* fn = ops[0].batch_fn;
   bool fits = fn != nullptr;
   KBatch B;
   std::memset(&B, 0, sizeof(B));
@@ -566,11 +499,56 @@ static const std::set<std::string>& own_mapping() {
   return s;
 }
 
-static int grow_guards(te_ctx* c) {
-  if (c->guard_ok) return TE_OK;
-  uint64_t need = 0;
-  std::map<uint32_t, int32_t> words;                 // parameter words already read
-  std::map<uint32_t, std::array<uint32_t, 5>> seen;  // grid parameter blocks already read
+// Reads n words from word at of the program's memory.
+using ReadWords = std::function<int(uint64_t at, uint32_t n, uint32_t* to)>;
+
+// The parameter words the plan depends on, offset -> value: each op's grid,
+// the flags that choose its kernel, the counts of the merged copies and zeros.
+static int plan_words(te_ctx* c, const ReadWords& read, std::map<uint32_t, uint32_t>* out) {
+  static const int kCopy = te::kernel_id("_copy"), kZero = te::kernel_id("zero_fields"),
+                   kCopies = te::kernel_id("copy_fields"), kStress = te::kernel_id("turb_sfcstress");
+  std::map<uint32_t, uint32_t>& w = *out;
+  auto add = [&](uint32_t at, uint32_t n) {
+    for (uint32_t q = 0; q < n; ++q)
+      if ((uint64_t)at + q < c->prog_words) w[at + q] = 0;
+  };
+  for (const Op& op : c->ops) {
+    if (op.kid == kCopy) continue;
+    add(op.A[4], 5);
+    if (te::row_waves(op.kid)) {
+      for (int q : {1, 3, 12, 32}) add(op.A[4 + q], 1);
+      if (op.A[4 + 17] != 0) add(op.A[4 + 17], 2);
+    }
+    if (op.kid == kZero || op.kid == kCopies) add(op.A[4 + 9], 1);
+    if (op.kid == kStress) add(op.A[4 + 5], 1);
+  }
+  // in a few runs: the words of a program lie close together
+  std::vector<uint32_t> buf;
+  for (auto it = w.begin(); it != w.end();) {
+    auto end = it;
+    uint32_t last = it->first;
+    while (end != w.end() && end->first - last < 4096) last = (end++)->first;
+    const uint32_t n = last - it->first + 1;
+    buf.resize(n);
+    const uint32_t at = it->first;
+    const int rc = read(at, n, buf.data());
+    if (rc != TE_OK) return rc;
+    for (; it != end; ++it) it->second = buf[it->first - at];
+  }
+  return TE_OK;
+}
+
+// Every op's grid, launch form and batch.  need: words of the largest field's
+// footprint.
+static int plan_ops(te_ctx* c, const ReadWords& read, uint64_t* need) {
+  std::map<uint32_t, uint32_t> words;
+  const int rc0 = plan_words(c, read, &words);
+  if (rc0 != TE_OK) return rc0;
+  auto word = [&](uint64_t at) {
+    const auto it = words.find((uint32_t)at);
+    return it == words.end() ? 0 : (int32_t)it->second;
+  };
+  *need = 0;
   // pointwise ops that may run flat (te_flat): kernel -> the parameters it
   // accesses in 16-byte runs (fields; profiles are read per level)
   static const std::map<std::string, std::vector<int>> flatOps = {
@@ -597,20 +575,16 @@ static int grow_guards(te_ctx* c) {
       op.flat = aligned(op, fl->second);
       continue;
     }
-    uint32_t d[5];
-    auto it = seen.find(op.A[4]);
-    if (it != seen.end()) {
-      std::memcpy(d, it->second.data(), sizeof(d));
-    } else {
-      TE_HIP(hipMemcpy(d, c->dM + op.A[4], sizeof(d), hipMemcpyDeviceToHost), "read grid");
-      seen[op.A[4]] = {d[0], d[1], d[2], d[3], d[4]};
-    }
-    const int32_t nz = (int32_t)d[2], sJ = (int32_t)d[3], sK = (int32_t)d[4];
+    const uint64_t grid = op.A[4];
+    const int32_t nx = word(grid), ny = word(grid + 1), nz = word(grid + 2), sJ = word(grid + 3), sK = word(grid + 4);
     if (nz < 1 || sJ < 1 || sK < 1 || nz > 100000 || sJ > 100000 || sK > 100000)
       return fail(c, TE_ERR_ARG, std::string("op ") + te::kernel_name(op.kid) + ": invalid grid parameters");
+    op.nx = std::max(nx, 0);
+    op.ny = std::max(ny, 0);
     op.nz = nz;
     op.sJ = sJ;
     op.sK = sK;
+    if (std::strcmp(kn, "zero_fields") == 0 || std::strcmp(kn, "copy_fields") == 0) op.count = word(op.A[4 + 9]);
     if (fl != flatOps.end()) {
       const bool wholeGrid = op.A[0] == (uint32_t)sJ && op.A[1] == (uint32_t)sK && op.A[2] == (uint32_t)(nz + 1);
       const bool words1d = std::strcmp(kn, "copy_fields") == 0 && op.A[1] == 1 && op.A[2] == 1;
@@ -628,49 +602,60 @@ static int grow_guards(te_ctx* c) {
       return fail(c, TE_ERR_UNSUPPORTED, std::string(te::kernel_name(op.kid)) + ": a level spans 2^32 bytes or more");
     if (std::strcmp(kn, "ac_column") == 0 && (uint64_t)sJ * sK * (uint64_t)(nz + 2) >= (1ull << 30))
       return fail(c, TE_ERR_UNSUPPORTED, "ac_column: a field spans 2^32 bytes or more");
-    need = std::max<uint64_t>(need, (uint64_t)sJ * sK * (uint64_t)(nz + 3));
+    *need = std::max<uint64_t>(*need, (uint64_t)sJ * sK * (uint64_t)(nz + 3));
     if (te::row_waves(op.kid)) {  // the body for its flux kind, stagger and halo fill
       const bool pdef = std::strcmp(kn, "adv_pdef") == 0;
-      int32_t stag = 0, kind = 0, chain = 0, open[2] = {0, 0};
-      auto read = [&](uint32_t at, int32_t* to, const char* what) -> int {  // each word once (they are shared)
-        const auto known = words.find(at);
-        if (known != words.end()) {
-          *to = known->second;
-          return TE_OK;
-        }
-        TE_HIP(hipMemcpy(to, c->dM + at, 4, hipMemcpyDeviceToHost), what);
-        words[at] = *to;
-        return TE_OK;
-      };
-      int rc = read(op.A[4 + 1], &stag, "read stagger");
-      if (rc == TE_OK) rc = read(op.A[4 + 3], &kind, "read flux kind");
-      if (rc == TE_OK) rc = read(op.A[4 + 32], &chain, "read chain flags");
-      for (int q = 0; q < 2 && rc == TE_OK && op.A[4 + 17] != 0; ++q) rc = read(op.A[4 + 17] + q, &open[q], "read open sides");
-      if (rc != TE_OK) return rc;
+      const int32_t stag = word(op.A[4 + 1]), kind = word(op.A[4 + 3]), chain = word(op.A[4 + 32]);
+      int32_t open[2] = {0, 0};
+      for (int q = 0; q < 2 && op.A[4 + 17] != 0; ++q) open[q] = word((uint64_t)op.A[4 + 17] + q);
       const bool side = open[0] != 0 || open[1] != 0;
       const bool openBody = side && (pdef || (chain & 32) != 0);
       op.fn = pdef ? te::adv_pdef_kernel(kind, side) : te::adv_fused_kernel(kind, stag, openBody);
       op.chain = pdef ? 0 : chain;
+      op.acc = pdef ? 0 : word(op.A[4 + 12]);
       op.body = te::adv_body(pdef, kind, stag, openBody);
     }
     if (std::strcmp(te::kernel_name(op.kid), "turb_sfcstress") == 0) {
-      int32_t mode = 0;
-      TE_HIP(hipMemcpy(&mode, c->dM + op.A[4 + 5], 4, hipMemcpyDeviceToHost), "read mode");
+      const int32_t mode = word(op.A[4 + 5]);
       if (mode != 0 && mode != 4)
         return fail(c, TE_ERR_UNSUPPORTED, "turb_sfcstress: surface-flux stress modes (bbc=3) are not on this path");
     }
   }
+  // batches: as many of the following dispatches as can join
+  std::vector<te::OpWords> w(c->ops.size());
+  std::vector<char> known(c->ops.size(), 0);
+  for (size_t i = 0; i < c->ops.size(); ++i) known[i] = te::op_words(c->ops[i], w[i]);
+  for (size_t i = 0; i < c->ops.size(); i += c->ops[i].batch) {
+    Op& op = c->ops[i];
+    op.batch = 1;
+    op.batch_fn = nullptr;
+    for (int n = 2; known[i] && i + n <= c->ops.size() && known[i + n - 1]; ++n) {
+      const void* fn = te::batch_kernel(&c->ops[i], &w[i], n);
+      if (!fn) break;
+      op.batch = n;
+      op.batch_fn = fn;
+    }
+    for (int q = 1; q < op.batch; ++q) c->ops[i + q].batch = 1;
+  }
+  return TE_OK;
+}
+
+static int grow_guards(te_ctx* c) {
+  if (c->guard_ok) return TE_OK;
+  uint64_t need = 0;
+  const int rc = plan_ops(
+      c,
+      [c](uint64_t at, uint32_t n, uint32_t* to) {
+        TE_HIP(hipMemcpyAsync(to, c->dM + at, 4 * (size_t)n, hipMemcpyDeviceToHost, c->stream), "read parameters");
+        TE_HIP(hipStreamSynchronize(c->stream), "read parameters");
+        return TE_OK;
+      },
+      &need);
+  if (rc != TE_OK) return rc;
   const uint64_t want = c->prog_words + need;
   if (want > c->words || need > c->front) {
-    int rc = alloc_memory(c, std::max(want, c->words), need);
-    if (rc != TE_OK) return rc;
-  }
-  // batches: as many of the following dispatches as can join
-  for (size_t i = 0; i < c->ops.size(); i += c->ops[i].batch) {
-    int n = 1;
-    while (i + n < c->ops.size() && te::batch_kernel(&c->ops[i], n + 1)) ++n;
-    c->ops[i].batch = n;
-    for (int q = 1; q < n; ++q) c->ops[i + q].batch = 1;
+    const int rc1 = alloc_memory(c, std::max(want, c->words), need);
+    if (rc1 != TE_OK) return rc1;
   }
   c->guard_ok = true;
   return TE_OK;
@@ -722,20 +707,12 @@ int te::run_ops_plain(te_ctx* c, int first, int last) {
   return run_ops(c, first, last);
 }
 
-extern "C" {
-
-int te_program_create(uint64_t mem_words, int32_t nops, const char* const* names, const uint32_t* args, te_ctx** out) {
-  if (!out || (nops > 0 && (!names || !args)) || mem_words == 0) return TE_ERR_ARG;
-  *out = nullptr;
-  te_ctx* c = new te_ctx();
+// The ops of a caller's program.
+static int program_ops(te_ctx* c, uint64_t mem_words, int32_t nops, const char* const* names, const uint32_t* args) {
   c->ops.resize(nops);
   for (int i = 0; i < nops; ++i) {
     int kid = te::kernel_id(names[i]);
-    if (kid < 0) {
-      int rc = fail(c, TE_ERR_UNSUPPORTED, std::string("no kernel '") + names[i] + "' on this path");
-      *out = c;
-      return rc;
-    }
+    if (kid < 0) return fail(c, TE_ERR_UNSUPPORTED, std::string("no kernel '") + names[i] + "' on this path");
     c->ops[i].kid = kid;
     c->op_names.push_back(names[i]);
     std::memcpy(c->ops[i].A, args + (size_t)i * 64, 64 * 4);
@@ -743,11 +720,44 @@ int te_program_create(uint64_t mem_words, int32_t nops, const char* const* names
       c->ops[i].A[1] = c->ops[i].A[2] = 1;
     }
   }
-  *out = c;
   c->words = c->prog_words = mem_words;
-  int rc = validate_ops(c);
+  return validate_ops(c);
+}
+
+extern "C" {
+
+int te_program_create(uint64_t mem_words, int32_t nops, const char* const* names, const uint32_t* args, te_ctx** out) {
+  if (!out || (nops > 0 && (!names || !args)) || mem_words == 0) return TE_ERR_ARG;
+  *out = nullptr;
+  te_ctx* c = new te_ctx();
+  *out = c;
+  int rc = program_ops(c, mem_words, nops, names, args);
   if (rc != TE_OK) return rc;
   return ctx_alloc(c, mem_words);
+}
+
+int te_plan_batches(uint64_t mem_words, const uint32_t* mem, int32_t nops, const char* const* names,
+                    const uint32_t* args, int32_t* batch) {
+  if (nops < 0 || (nops > 0 && (!names || !args || !batch)) || !mem || mem_words == 0) return TE_ERR_ARG;
+  te_ctx c;
+  int rc = program_ops(&c, mem_words, nops, names, args);
+  if (rc != TE_OK) return rc;
+  uint64_t need = 0;
+  rc = plan_ops(
+      &c,
+      [&](uint64_t at, uint32_t n, uint32_t* to) {
+        std::memcpy(to, mem + at, 4 * (size_t)n);
+        return TE_OK;
+      },
+      &need);
+  if (rc != TE_OK) return rc;
+  for (int32_t i = 0; i < nops;) {
+    const int32_t n = c.ops[i].batch;
+    batch[i] = n;
+    for (int32_t q = 1; q < n; ++q) batch[i + q] = 0;
+    i += n;
+  }
+  return TE_OK;
 }
 
 int te_upload_words(te_ctx* c, uint64_t off, const uint32_t* src, uint64_t n) {

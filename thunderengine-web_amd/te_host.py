@@ -90,6 +90,7 @@ def lib():
     ctx = ctypes.c_void_p
     sig = {
         "te_program_create": ([u64, ctypes.c_int32, P(ctypes.c_char_p), u32p, P(ctx)], ctypes.c_int),
+        "te_plan_batches": ([u64, u32p, ctypes.c_int32, P(ctypes.c_char_p), u32p, P(ctypes.c_int32)], ctypes.c_int),
         "te_upload_words": ([ctx, u64, u32p, u64], ctypes.c_int),
         "te_download_words": ([ctx, u64, u32p, u64], ctypes.c_int),
         "te_run": ([ctx, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32], ctypes.c_int),
@@ -164,6 +165,23 @@ def kernel_names():
     """Names of the kernels libte.so implements."""
     L = lib()
     return [L.te_kernel_name(i).decode() for i in range(L.te_kernel_count())]
+
+
+def plan_batches(memory, names, args):
+    """How a replay of the program groups its dispatches (te_plan_batches; no
+    device): per dispatch the number that the launch beginning with it runs
+    side by side, 0 for one that an earlier launch runs."""
+    n = len(names)
+    cn = (ctypes.c_char_p * n)(*[s.encode() for s in names])
+    M = np.ascontiguousarray(memory, dtype=np.uint32)
+    A = np.ascontiguousarray(args, dtype=np.uint32)
+    out = np.zeros(n, dtype=np.int32)
+    P = ctypes.POINTER
+    rc = lib().te_plan_batches(M.size, M.ctypes.data_as(P(ctypes.c_uint32)), n, cn,
+                               A.ctypes.data_as(P(ctypes.c_uint32)), out.ctypes.data_as(P(ctypes.c_int32)))
+    if rc != TE_OK:
+        raise TeError("te_plan_batches failed (%d)" % rc)
+    return out
 
 
 def selftest_math():
