@@ -350,7 +350,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   __shared__ float xw[64];               // new w at the first level of the wave above
   __shared__ int fwd_done, back_next;    // the sweep's hand-offs between waves
   __shared__ int hcnt;
-  __shared__ short hcell[AC_HALO_CELLS][3];
+  __shared__ int hcell[AC_HALO_CELLS][3];
   // acoustic_prepare's per-level factors tem, r1, r2, tem1, c1, c2: scalar
   // loads where a wave has few levels, else a table
   __shared__ float lv[AHEAD ? 1 : 6][AHEAD ? 1 : AC_WAVES * 16 + 1];
@@ -392,7 +392,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   const int ys[2] = {j >= ny - 3 ? j - ny : j, j <= 3 ? j + ny : j};
   if (OPEN) {
     if (active && wave == 0 && i == nx - 1 && !openx) {
-      hcell[0][0] = (short)nx; hcell[0][1] = (short)j; hcell[0][2] = 1;
+      hcell[0][0] = nx; hcell[0][1] = j; hcell[0][2] = 1;
       hcnt = 1;
     }
   } else if (active && wave == 0) {  // (one wave: its LDS operations keep their order)
@@ -402,7 +402,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
     if (n > 0) {
       int q = atomicAdd(&hcnt, n);
       auto put = [&](int hx, int hy, int m) {
-        hcell[q][0] = (short)hx; hcell[q][1] = (short)hy; hcell[q][2] = (short)m;
+        hcell[q][0] = hx; hcell[q][1] = hy; hcell[q][2] = m;
         ++q;
       };
       for (int by = 0; by < 3; ++by)
