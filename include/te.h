@@ -126,14 +126,22 @@ int te_last_run_ms(te_ctx* ctx, float* ms);
  * (an event after each launch, every trial from the same memory), keeps each
  * dispatch's fastest, and then keeps that set only if `reps` whole steps run
  * at least 0.5% faster with it than with the default shapes (three
- * interleaved comparisons), or always when `force` is nonzero.  The memory is restored and a captured step
- * graph captured again.  A shape only changes which thread computes which
+ * interleaved comparisons), or always when `force` is nonzero.  A dispatch is
+ * timed in a launch of its own and keeps its shape where a launch runs it side
+ * by side with others.  The memory is restored and a captured step graph
+ * captured again.  A shape only changes which thread computes which
  * point, never the arithmetic.  te_tuned_ops: dispatches left on a tuned
  * shape (0 when the comparison rejected the set); te_autotune_ms: mean eager
  * step time of the comparison, default and tuned shapes. */
 int te_autotune(te_ctx* ctx, int32_t reps, int32_t force);
 int32_t te_tuned_ops(const te_ctx* ctx);
 int te_autotune_ms(const te_ctx* ctx, float* untuned, float* tuned);
+
+/* How te_run launches op i of a context now: out[0] the dispatches that the
+ * launch beginning with it runs side by side (0: an earlier op's launch runs
+ * it), out[1..3] the block in which it numbers its threads along i, j, k (256,
+ * 1, 1 for runs of words and for the (i, j)-plane numbering). */
+int te_op_launch(te_ctx* ctx, int32_t i, int32_t out[4]);
 
 const char* te_last_error(const te_ctx* ctx);
 void te_destroy(te_ctx* ctx);

@@ -291,39 +291,50 @@ static const void* batch_kernel(const Op* ops, const OpWords* w, int n) {
   // 300 x 300 x 90 6083 and 6016, 256 x 256 x 120 8612 and 8415.
   return words <= (3u << 20) ? (const void*)&k_point_batch : nullptr;
 }
-static hipError_t launch_batch(te_ctx* c, const Op* ops, int n) {
-  const void* fn = ops[0].batch_fn;
-  bool fits = fn != nullptr;
+// The launch of a batch (ops[0].batch_fn): fits is false where a member's
+// launch has no place in it.
+struct BatchShape {
   KBatch B;
-  std::memset(&B, 0, sizeof(B));
   uint64_t per = 0;  // workgroups per XCD
   dim3 b;
-  for (int i = 0; i < n && fits; ++i) {
-    Op op = ops[i];
-    op.tuned = false;
-    Shape s;
-    const hipError_t e = shape_of(c, op, s);
+  bool fits = false;
+};
+static hipError_t batch_shape(te_ctx* c, const Op* ops, int n, BatchShape& s) {
+  std::memset(&s.B, 0, sizeof(s.B));
+  s.fits = ops[0].batch_fn != nullptr;
+  for (int i = 0; i < n && s.fits; ++i) {
+    Shape m;
+    const hipError_t e = shape_of(c, ops[i], m);
     if (e != hipSuccess) return e;
     int body = 0;
-    const int family = batch_family(op, body);
-    // pointwise blocks are re-read from lines of 256 threads
-    fits = s.fn != nullptr && (family != 2 || (s.b.x * s.b.y * s.b.z <= 256 && s.lds == 0));
-    B.a[i] = s.a;
-    B.body[i] = (uint32_t)body;
-    b = family == 2 ? dim3(256, 1, 1) : s.b;
-    B.start[i] = (uint32_t)per;
-    per += (s.a.lg[9] + 7) / 8;
+    const int family = batch_family(ops[i], body);
+    // advections are re-read from 4 rows of 64 lanes, pointwise blocks from
+    // lines of 256 threads
+    const uint32_t threads = m.b.x * m.b.y * m.b.z;
+    s.fits = m.fn != nullptr && (family == 3 || (threads <= 256 && m.lds == 0 && (family == 2 || m.b.x == 64)));
+    s.B.a[i] = m.a;
+    s.B.body[i] = (uint32_t)body;
+    s.b = family == 1 ? dim3(64, 4, 1) : family == 2 ? dim3(256, 1, 1) : m.b;
+    s.B.start[i] = (uint32_t)s.per;
+    s.per += (m.a.lg[9] + 7) / 8;
   }
-  for (int i = n; i <= TE_BATCH; ++i) B.start[i] = (uint32_t)per;
-  if (!fits || per * 8 >= (1ull << 31)) {  // one by one
+  for (int i = n; i <= TE_BATCH; ++i) s.B.start[i] = (uint32_t)s.per;
+  s.fits = s.fits && s.per * 8 < (1ull << 31);
+  return hipSuccess;
+}
+static hipError_t launch_batch(te_ctx* c, const Op* ops, int n) {
+  BatchShape s;
+  const hipError_t e = batch_shape(c, ops, n, s);
+  if (e != hipSuccess) return e;
+  if (!s.fits) {  // one by one
     for (int i = 0; i < n; ++i) {
-      const hipError_t e = launch(c, ops[i]);
-      if (e != hipSuccess) return e;
+      const hipError_t e1 = launch(c, ops[i]);
+      if (e1 != hipSuccess) return e1;
     }
     return hipSuccess;
   }
-  void* args[] = {(void*)&c->dM, (void*)&B};
-  return hipLaunchKernel(fn, dim3((uint32_t)per * 8, 1, 1), b, args, 0, c->stream);
+  void* args[] = {(void*)&c->dM, (void*)&s.B};
+  return hipLaunchKernel(ops[0].batch_fn, dim3((uint32_t)s.per * 8, 1, 1), s.b, args, 0, c->stream);
 }
 
 // region_hash (replay.js:408-418): per-lane sums of a 32-bit mix, reduced
@@ -1015,6 +1026,23 @@ int te_autotune_ms(const te_ctx* c, float* untuned, float* tuned) {
 }
 
 int32_t te_tuned_ops(const te_ctx* c) { return c ? c->tuned_ops : 0; }
+
+int te_op_launch(te_ctx* c, int32_t i, int32_t out[4]) {
+  if (!c || !c->dM || !out || i < 0 || i >= (int32_t)c->ops.size()) return fail(c, TE_ERR_ARG, "te_op_launch: bad arguments");
+  int rc = grow_guards(c);
+  if (rc != TE_OK) return rc;
+  int first = 0;  // of the launch that runs op i
+  while (first + c->ops[first].batch <= i) first += c->ops[first].batch;
+  const int n = c->ops[first].batch;
+  te::BatchShape s;
+  if (n > 1) TE_HIP(te::batch_shape(c, &c->ops[first], n, s), "launch shape");
+  te::Shape one;
+  if (!s.fits) TE_HIP(te::shape_of(c, c->ops[i], one), "launch shape");
+  const KArg& a = s.fits ? s.B.a[i - first] : one.a;
+  out[0] = !s.fits ? 1 : i == first ? n : 0;
+  for (int q = 0; q < 3; ++q) out[1 + q] = (int32_t)a.lg[q];
+  return TE_OK;
+}
 
 int te_region_hash(te_ctx* c, uint64_t off, uint64_t n, uint32_t* out) {
   if (!c || !out || n > c->words || off > c->words - n) return fail(c, TE_ERR_ARG, "hash outside memory");

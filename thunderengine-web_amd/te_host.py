@@ -107,6 +107,7 @@ def lib():
         "te_autotune": ([ctx, ctypes.c_int32, ctypes.c_int32], ctypes.c_int),
         "te_tuned_ops": ([ctx], ctypes.c_int32),
         "te_autotune_ms": ([ctx, P(ctypes.c_float), P(ctypes.c_float)], ctypes.c_int),
+        "te_op_launch": ([ctx, ctypes.c_int32, P(ctypes.c_int32)], ctypes.c_int),
         "te_kernel_count": ([], ctypes.c_int32),
         "te_kernel_name": ([ctypes.c_int32], ctypes.c_char_p),
         "te_destroy": ([ctx], None),
@@ -313,6 +314,16 @@ class _Ctx:
         a, b = ctypes.c_float(), ctypes.c_float()
         self._check(lib().te_autotune_ms(self.h, ctypes.byref(a), ctypes.byref(b)), "te_autotune_ms")
         return a.value, b.value
+
+    def launches(self):
+        """(nops, 4) of te_op_launch: the dispatches of the launch that begins
+        with each op (0: an earlier launch runs it) and its block."""
+        n = int(lib().te_op_count(self.h))
+        out = np.zeros((n, 4), dtype=np.int32)
+        for i in range(n):
+            self._check(lib().te_op_launch(self.h, i, out[i].ctypes.data_as(ctypes.POINTER(ctypes.c_int32))),
+                        "te_op_launch")
+        return out
 
     def program(self):
         """(names, (nops, 64) uint32 argument slots) of the context's program."""
