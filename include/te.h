@@ -44,7 +44,8 @@ typedef struct te_ctx te_ctx;
 int te_program_create(uint64_t mem_words, int32_t nops, const char* const* names, const uint32_t* args,
                       te_ctx** out);
 
-/* Replayer.upload / writeWords (web/replay.js:216-229,301): host -> M. */
+/* Replayer.upload / writeWords (web/replay.js:216-229,301): host -> M.  Parameter
+ * words may be uploaded between runs: a later run plans its launches by them. */
 int te_upload_words(te_ctx* ctx, uint64_t word_off, const uint32_t* src, uint64_t nwords);
 
 /* Replayer.read (web/replay.js:368-383): M -> host (synchronous). */

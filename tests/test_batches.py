@@ -223,3 +223,78 @@ def test_dependent_tape_bit_exact(gpu, at):
             prog.run(M)
         assert np.array_equal(r.read(0, WORDS), M[:WORDS])
     r.close()
+
+
+def test_a_tape_that_writes_its_own_flags_is_not_planned_by_them():
+    """A copy over the chain flags of the dispatches after it."""
+    def tape(dst):
+        t = Tape()
+        chain = t.words(0)
+        t.op("_copy", {0: slot(0), 1: dst(chain)}, (4, 1, 1))
+        for f in (1, 3):
+            t.op("turb_zero", {1: slot(f)}, (SJ, SK, NZ + 1))
+        adv = {q: t.words(0) for q in (1, 3, 5, 12, 20, 21)}
+        adv.update({2: slot(5), 4: slot(6), 6: slot(7), 13: slot(8), 14: slot(9), 17: t.words(0, 0), 30: slot(10)})
+        adv.update({q: slot(11) for q in (7, 8, 9, 10, 15, 16)})
+        t.M[adv[1]] = 1
+        for f in (12, 13):
+            t.op("adv_fused", {**adv, 11: slot(f), 32: chain})
+        return t.batches()
+    assert tape(lambda chain: slot(1)) == [1, 1, 1, 2, 0]
+    assert tape(lambda chain: chain - 2) == [1, 1, 1, 1, 1]
+
+
+def flagged_tape():
+    """An advection that stores its tendency (chain 0) or updates a field (8,
+    with its halo 40), one that advects that field, a merged copy and a reader
+    of its second destination.  Returns the tape and its flags' words."""
+    rng = np.random.default_rng(11)
+    t = Tape()
+    t.M[:FLAGS] = rng.uniform(0.5, 1.5, FLAGS).astype(np.float32).view(np.uint32)
+    chain, sides, count = t.words(0), t.words(0, 0), t.words(1)
+    one = {1: t.words(1), 3: t.words(0), 5: t.words(0), 12: t.words(0), 20: t.words(0), 21: t.words(0), 17: sides,
+           4: slot(1), 6: slot(2), 13: slot(3), 14: slot(4), 30: slot(5)}
+    one.update({q: slot(6) for q in (7, 8, 9, 10, 15, 16)})
+    one.update({22: slot(18), 23: slot(19), 24: slot(20)})  # the fluxes of the separate dispatches
+    dt = t.words(*np.array([0.01], np.float32).view(np.int32))
+    t.op("adv_fused", {**one, 2: slot(7), 11: slot(8), 32: chain, 39: slot(9), 40: slot(10), 41: dt})
+    t.op("adv_fused", {**one, 2: slot(10), 11: slot(11), 32: t.words(0)})
+    t.op("copy_fields", {1: slot(12), 5: slot(13), 2: slot(14), 6: slot(15), 9: count}, (FIELD, 1, 1))
+    t.op("build_sadv", {1: slot(16), 2: slot(15), 3: slot(17)}, (SJ, SK, NZ + 1))
+    return t, chain, sides, count
+
+
+@pytest.mark.gpu
+def test_uploaded_flags_reach_the_plan(gpu):
+    """Flags uploaded between runs: every run, alone and as a replayed graph, is
+    the oracle's, and dispatches that the new flags make dependent no longer
+    share a launch."""
+    t, chain, sides, count = flagged_tape()
+    A = np.array(t.args)
+    r = te_host.Replayer(WORDS, t.names, A)
+    r.upload(0, t.M)
+    buf = np.zeros((1 << 16) + WORDS + FIELD + 4096, np.uint32)
+    M = buf[1 << 16:]
+    M[:WORDS] = t.M
+    prog = ol.Program(t.names, A)
+    for flags, groups in ((dict(), [2, 0, 2, 0]), ({chain: 8}, [1, 1, 2, 0]), ({count: 2}, [1, 1, 1, 1]),
+                          ({chain: 40}, [1, 1, 1, 1]), ({sides: 1}, [1, 1, 1, 1]), ({sides + 1: 1}, [1, 1, 1, 1]),
+                          ({chain: 0, sides: 0, sides + 1: 0, count: 1}, [2, 0, 2, 0])):
+        print("flags", flags, flush=True)
+        for at, v in flags.items():
+            r.upload(at, np.array([v], np.uint32))
+            M[at] = v
+        assert r.launches()[:, 0].tolist() == groups
+        for n in (2, 1):
+            r.run(n)
+            r.sync()
+            for _ in range(n):
+                prog.run(M)
+            got, want = r.read(0, WORDS), M[:WORDS].copy()
+            # not stored here: the oracle's fluxes and a chained update's tendency
+            for w in (got, want):
+                w[slot(18): slot(21)] = 0
+                if M[chain] & 8:
+                    w[slot(8): slot(8) + FIELD] = 0
+            assert np.array_equal(got, want), (flags, n)
+    r.close()

@@ -84,7 +84,7 @@ namespace te {
 int run_ops_plain(te_ctx* c, int first, int last);
 // Reads every op's grid and grows the context's guard regions so that no
 // launch of its program leaves the allocation; idempotent.  Afterwards
-// c->front and c->words are final.
+// c->front and c->words are final (unless the caller uploads other grids).
 int ensure_guard(te_ctx* c);
 // Called by te_destroy for each adjoint still built on the context: the
 // adjoint forgets the context, and its calls that need it fail.
@@ -98,7 +98,8 @@ struct te_ctx {
   uint32_t* dM = nullptr;     // word 0 of the program's memory M
   uint64_t words = 0;       // allocated words (program memory + guard region)
   uint64_t prog_words = 0;  // words of the program's memory M
-  bool guard_ok = false;
+  bool guard_ok = false;    // the ops are planned, the guards large enough
+  std::map<uint32_t, uint32_t> plan_words;  // the parameter words that plan depends on, and their values
   uint32_t* dHash = nullptr;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;

@@ -552,7 +552,8 @@ static int plan_words(te_ctx* c, const ReadWords& read, std::map<uint32_t, uint3
 // Every op's grid, launch form and batch.  need: words of the largest field's
 // footprint.
 static int plan_ops(te_ctx* c, const ReadWords& read, uint64_t* need) {
-  std::map<uint32_t, uint32_t> words;
+  std::map<uint32_t, uint32_t>& words = c->plan_words;
+  words.clear();
   const int rc0 = plan_words(c, read, &words);
   if (rc0 != TE_OK) return rc0;
   auto word = [&](uint64_t at) {
@@ -632,10 +633,25 @@ static int plan_ops(te_ctx* c, const ReadWords& read, uint64_t* need) {
         return fail(c, TE_ERR_UNSUPPORTED, "turb_sfcstress: surface-flux stress modes (bbc=3) are not on this path");
     }
   }
-  // batches: as many of the following dispatches as can join
   std::vector<te::OpWords> w(c->ops.size());
   std::vector<char> known(c->ops.size(), 0);
-  for (size_t i = 0; i < c->ops.size(); ++i) known[i] = te::op_words(c->ops[i], w[i]);
+  bool fixed = true;  // no dispatch writes a word of the plan
+  for (size_t i = 0; i < c->ops.size(); ++i) {
+    const Op& op = c->ops[i];
+    known[i] = te::op_words(op, w[i]);
+    auto check = [&](uint64_t at, uint64_t n) {
+      const auto it = words.lower_bound((uint32_t)at);
+      if (it != words.end() && it->first < at + n) fixed = false;
+    };
+    for (const te::Words& x : w[i].writes) check(x.at, x.n);
+    if (std::strcmp(te::kernel_name(op.kid), "_copy") == 0) check(op.A[5], op.A[0]);
+  }
+  if (!fixed)  // every launch by itself, the advections by the kernels that read their flags
+    for (size_t i = 0; i < c->ops.size(); ++i) {
+      known[i] = 0;
+      c->ops[i].fn = nullptr;
+    }
+  // batches: as many of the following dispatches as can join
   for (size_t i = 0; i < c->ops.size(); i += c->ops[i].batch) {
     Op& op = c->ops[i];
     op.batch = 1;
@@ -683,6 +699,21 @@ static int run_ops(te_ctx* c, int first, int last) {
     i += together ? n : 1;
   }
   return TE_OK;
+}
+
+// The host writes words [off, off + n): where one that the plan depends on
+// changes, the next run plans (and captures) again.  The stream is idle.
+static void note_words(te_ctx* c, uint64_t off, const uint32_t* src, uint64_t n) {
+  if (!c->guard_ok) return;
+  for (auto it = c->plan_words.lower_bound((uint32_t)std::min<uint64_t>(off, UINT32_MAX));
+       it != c->plan_words.end() && it->first < off + n; ++it)
+    if (it->first >= off && src[it->first - off] != it->second) {
+      c->guard_ok = false;
+      if (c->graph) (void)hipGraphExecDestroy(c->graph);
+      c->graph = nullptr;
+      c->graph_failed = false;
+      return;
+    }
 }
 
 static int ensure_graph(te_ctx* c) {
@@ -775,6 +806,7 @@ int te_upload_words(te_ctx* c, uint64_t off, const uint32_t* src, uint64_t n) {
   if (!c || !src || n > c->prog_words || off > c->prog_words - n) return fail(c, TE_ERR_ARG, "upload outside memory");
   TE_HIP(hipMemcpyAsync(c->dM + off, src, n * 4, hipMemcpyHostToDevice, c->stream), "upload");
   TE_HIP(hipStreamSynchronize(c->stream), "upload sync");
+  note_words(c, off, src, n);
   return TE_OK;
 }
 
@@ -1273,7 +1305,8 @@ static int retime(te_ctx* c, float dt, int32_t nsound) {
                         c->stream),
          "upload step parameters");
   TE_HIP(hipStreamSynchronize(c->stream), "upload sync");
-  return same ? TE_OK : grow_guards(c);
+  note_words(c, pay0, c->image.data() + pay0, c->prog_words - pay0);
+  return c->guard_ok ? TE_OK : grow_guards(c);
 }
 
 int te_set_time_step(te_ctx* c, float dt, int32_t nsound) { return retime(c, dt, nsound); }
@@ -1430,6 +1463,14 @@ int te_ensemble_step(te_ensemble* e, int32_t nsteps) {
   // each on its own stream, so the device runs them concurrently
   for (int32_t s = 0; s < nsteps; ++s)
     for (te_ctx* c : e->members) {
+      if (!c->guard_ok) {  // a member's parameters were uploaded anew
+        int rc = grow_guards(c);
+        if (rc == TE_OK) rc = ensure_graph(c);
+        if (rc != TE_OK) {
+          e->err = c->err;
+          return rc;
+        }
+      }
       hipError_t r = c->graph ? hipGraphLaunch(c->graph, c->stream) : hipSuccess;
       int rc = r == hipSuccess ? (c->graph ? TE_OK : run_ops(c, 0, (int)c->ops.size() - 1)) : hip_fail(c, r, "hipGraphLaunch");
       if (rc != TE_OK) {
