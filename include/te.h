@@ -129,7 +129,8 @@ int te_last_run_ms(te_ctx* ctx, float* ms);
  * at least 0.5% faster with it than with the default shapes (three
  * interleaved comparisons), or always when `force` is nonzero.  A dispatch is
  * timed in a launch of its own and keeps its shape where a launch runs it side
- * by side with others.  The memory is restored and a captured step graph
+ * by side with others (advections that share a launch: the shape that is
+ * fastest for all of them).  The memory is restored and a captured step graph
  * captured again.  A shape only changes which thread computes which
  * point, never the arithmetic.  te_tuned_ops: dispatches left on a tuned
  * shape (0 when the comparison rejected the set); te_autotune_ms: mean eager

@@ -553,8 +553,8 @@ __device__ __forceinline__ void adv_fused_body(uint32_t* M, const KArg& a, const
   // a wave is one row of cells, so j and k are wave-uniform and branches on
   // them are scalar
   const int i = b_.x * 64 + (int)threadIdx.x,
-            j = b_.y * TE_BY + (int)__builtin_amdgcn_readfirstlane(b_.ty),
-            k = b_.z * TE_BZ + (int)__builtin_amdgcn_readfirstlane(b_.tz);
+            j = b_.y * TE_BY + (int)__builtin_amdgcn_readfirstlane(threadIdx.y),
+            k = b_.z * TE_BZ + (int)__builtin_amdgcn_readfirstlane(threadIdx.z);
   if (j >= (int)a.n[1] || k >= (int)a.n[2] || i >= (int)a.n[0]) return;
   Dims g = dims(a.q[0], 0);
   const int stag = STC != 0 ? STC : ldi(a.q[1], 0), st = stag < 0 ? -stag : stag;
@@ -707,15 +707,13 @@ __global__ __launch_bounds__(256) void k_adv_fused(uint32_t* M, KArg a) {
 // launch fills the chip once instead of draining it between them, and the
 // tiles of one place share an L2 (te_batch_part).
 // MASK: the bodies (adv_body) the launch may meet; body 0 or 8 is served by
-// 1 or 9, which take open sides too.  Blocks of 64 x 4, each dispatch's rows
-// in the shape te_autotune left it with (rows_blk).
+// 1 or 9, which take open sides too.  Blocks of 64 x Y x Z, the same for every
+// dispatch of the launch (te_autotune chooses one for all of them).
 template <uint32_t MASK>
 __global__ __launch_bounds__(256) void k_adv_batch(uint32_t* M, KBatch) {
   const BatchPart p = te_batch_part();
   if (!p.in) return;
-  bool in;
-  const Blk b = p.rows_blk(in);
-  if (!in) return;
+  const Blk b = p.blk();
   auto is = [&](int v, int alt = -1) {
     return (MASK >> v & 1u) != 0 && (p.body == v || (alt >= 0 && !(MASK >> alt & 1u) && p.body == alt));
   };

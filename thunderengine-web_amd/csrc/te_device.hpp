@@ -493,13 +493,6 @@ struct BatchPart {
   bool in;
   // the workgroup, its threads as the launch's
   TE_DEV Blk blk() const { return te_block_at(a, w, (int)threadIdx.x, (int)threadIdx.y, (int)threadIdx.z); }
-  // for a launch of 64 x 4 threads whose waves are rows, re-read as a's block of
-  // 64 x Y x Z (powers of two, Y * Z <= 4); in: the wave is one of its rows
-  TE_DEV Blk rows_blk(bool& in) const {
-    const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.y), ly = 31 - __builtin_clz(a.lg[1]);
-    in = t < a.lg[1] * a.lg[2];
-    return te_block_at(a, w, (int)threadIdx.x, (int)(t & (a.lg[1] - 1)), (int)(t >> ly));
-  }
   // for a launch in lines of 256 threads, re-read as a's block (powers of two);
   // in: the thread lies in it
   TE_DEV Blk line_blk(bool& in) const {

@@ -308,13 +308,14 @@ static hipError_t batch_shape(te_ctx* c, const Op* ops, int n, BatchShape& s) {
     if (e != hipSuccess) return e;
     int body = 0;
     const int family = batch_family(ops[i], body);
-    // advections are re-read from 4 rows of 64 lanes, pointwise blocks from
-    // lines of 256 threads
-    const uint32_t threads = m.b.x * m.b.y * m.b.z;
-    s.fits = m.fn != nullptr && (family == 3 || (threads <= 256 && m.lds == 0 && (family == 2 || m.b.x == 64)));
+    // pointwise blocks are re-read from lines of 256 threads; the others are
+    // the launch's
+    const dim3 b = family == 2 ? dim3(256, 1, 1) : m.b;
+    s.fits = m.fn != nullptr && (family != 2 || (m.b.x * m.b.y * m.b.z <= 256 && m.lds == 0)) &&
+             (i == 0 || (b.x == s.b.x && b.y == s.b.y && b.z == s.b.z));
     s.B.a[i] = m.a;
     s.B.body[i] = (uint32_t)body;
-    s.b = family == 1 ? dim3(64, 4, 1) : family == 2 ? dim3(256, 1, 1) : m.b;
+    s.b = b;
     s.B.start[i] = (uint32_t)s.per;
     s.per += (m.a.lg[9] + 7) / 8;
   }
@@ -967,6 +968,11 @@ int te_autotune(te_ctx* c, int32_t reps, int32_t force) {
   } onExit{undo};
   std::vector<te::Op> best = base;
   std::vector<float> bestMs(n, 1e30f), ms(n);
+  // advections that share a launch share its block: together[i] ops from i on
+  // take the shape that is fastest for all of them
+  std::vector<int> together(n, 1);
+  for (int i = 0; i < n; i += c->ops[i].batch)
+    if (te::row_waves(c->ops[i].kid)) together[i] = c->ops[i].batch;
 
   // each candidate in context: `reps` eager steps from the same memory with
   // an event after every launch, so each dispatch is timed with the caches
@@ -998,11 +1004,17 @@ int te_autotune(te_ctx* c, int32_t reps, int32_t force) {
         ms[i] += t;
       }
     }
-    for (int i = 0; i < n; ++i)
-      if (eligible[i] && (cand < 0 || c->ops[i].tuned) && ms[i] < bestMs[i]) {
-        bestMs[i] = ms[i];
-        best[i] = c->ops[i];
+    for (int i = 0; i < n; i += together[i]) {
+      bool all = true;
+      float t = 0.0f;
+      for (int q = i; q < i + together[i]; ++q) {
+        all = all && eligible[q] && (cand < 0 || c->ops[q].tuned);
+        t += ms[q];
       }
+      if (!all || t >= bestMs[i]) continue;
+      bestMs[i] = t;
+      std::copy(c->ops.begin() + i, c->ops.begin() + i + together[i], best.begin() + i);
+    }
   }
 
   // keep the per-dispatch choices only if whole steps are faster with them
