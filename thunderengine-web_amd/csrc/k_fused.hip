@@ -350,7 +350,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
   __shared__ float xw[64];               // new w at the first level of the wave above
   __shared__ int fwd_done, back_next;    // the sweep's hand-offs between waves
   __shared__ int hcnt;
-  __shared__ int hcell[AC_HALO_CELLS][3];
+  __shared__ uint32_t hcell[AC_HALO_CELLS];
   // acoustic_prepare's per-level factors tem, r1, r2, tem1, c1, c2: scalar
   // loads where a wave has few levels, else a table
   __shared__ float lv[AHEAD ? 1 : 6][AHEAD ? 1 : AC_WAVES * 16 + 1];
@@ -386,13 +386,15 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
     back_next = AC_WAVES - 1;
     hcnt = 0;
   }
-  // Halo cells of the x-images and corners of this workgroup's columns,
-  // (hx, hy, 4), and (nx, j, 1): what `early` does with them
+  // Halo cells of the x-images and corners of this workgroup's columns, and
+  // (nx, j) (low bit set): byte offsets within a level
   const bool openx = OPEN && ldi(a.q[38], 0) != 0, openy = OPEN && ldi(a.q[38], 1) != 0;
   const int ys[2] = {j >= ny - 3 ? j - ny : j, j <= 3 ? j + ny : j};
+  const uint32_t sjb = 4u * (uint32_t)g.sJ, skb = sjb * (uint32_t)g.sK;
+  auto cell = [&](int x, int y) { return 4u * (uint32_t)(x + 3) + sjb * (uint32_t)(y + 3); };
   if (OPEN) {
     if (active && wave == 0 && i == nx - 1 && !openx) {
-      hcell[0][0] = nx; hcell[0][1] = j; hcell[0][2] = 1;
+      hcell[0] = cell(nx, j) | 1u;
       hcnt = 1;
     }
   } else if (active && wave == 0) {  // (one wave: its LDS operations keep their order)
@@ -401,17 +403,13 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
     const int n = nxi * (1 + nyi) + (i == nx - 1);
     if (n > 0) {
       int q = atomicAdd(&hcnt, n);
-      auto put = [&](int hx, int hy, int m) {
-        hcell[q][0] = hx; hcell[q][1] = hy; hcell[q][2] = m;
-        ++q;
-      };
       for (int by = 0; by < 3; ++by)
         for (int bx = 0; bx < 2; ++bx) {
           const int hx = xs[bx], hy = by == 0 ? j : ys[by - 1];
           if (hx == i || (by > 0 && hy == j)) continue;
-          put(hx, hy, 4);
+          hcell[q++] = cell(hx, hy);
         }
-      if (i == nx - 1) put(nx, j, 1);
+      if (i == nx - 1) hcell[q] = cell(nx, j) | 1u;
     }
   }
   auto prep = [&](int k, float f[6]) {
@@ -436,8 +434,7 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
                pp3d = F(10), ppd = F(11), ppx = F(12), rru = F(13), rrv = F(14), rrw = F(15);
   const FieldB rruO = a.p[35] != 0 ? F(35) : rru, rrvO = a.p[36] != 0 ? F(36) : rrv, rrwO = a.p[37] != 0 ? F(37) : rrw;
   // byte offset of this lane's column at level k (the same in every field)
-  const uint32_t sjb = 4u * (uint32_t)g.sJ, skb = sjb * (uint32_t)g.sK;
-  const uint32_t o00 = 4u * (uint32_t)(ic + 3) + sjb * (uint32_t)(j + 3);
+  const uint32_t o00 = cell(ic, j);
   auto at = [&](int k) { return o00 + skb * (uint32_t)k; };
   const float asq = ac.alph * ac.alph;
   const float temx = (ac.dts * 0.5f) * g.rdx, temy = (ac.dts * 0.5f) * g.rdy;
@@ -563,17 +560,17 @@ __device__ __forceinline__ void ac_column(uint32_t* M, const KArg& a) {
     auto item = [&](int it) {
       Item c = {0u, 0, 0.0f, 0.0f, 0.0f};
       if (it < items) {
-        const int kk = it / nc, q = it - kk * nc, hx = hcell[q][0], hy = hcell[q][1];
-        const uint32_t l0 = skb * (uint32_t)(k0 + kk) + 12u + sjb * 3u;
-        c.m = hcell[q][2];
-        c.h = l0 + 4u * (uint32_t)hx + sjb * (uint32_t)hy;
+        const int kk = it / nc;
+        const uint32_t e = hcell[it - kk * nc], lv = skb * (uint32_t)(k0 + kk);
+        c.m = e & 1u ? 1 : 4;
+        c.h = lv + (e & ~3u);
         if (c.m == 4) {
           c.x = w(c.h);
           c.y = first ? c.x * ac.beta : rrw(c.h);
         } else {
           c.x = u(c.h);
           c.y = first ? 0.0f : rru(c.h);
-          c.z = u(l0 + sjb * (uint32_t)j);  // u at (0, j)
+          c.z = u(lv + cell(0, j));
         }
       }
       return c;
