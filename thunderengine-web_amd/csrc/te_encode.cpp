@@ -282,6 +282,11 @@ class Encoder {
   void end();
 };
 
+// A dispatch names its operands by 32-bit word offsets.
+static void checkWords(uint64_t words) {
+  if (words > (1ull << 32)) throw std::runtime_error("the step's memory exceeds 2^32 words");
+}
+
 void Encoder::setup() {
   const int nx = cfg.nx, ny = cfg.ny, nz = cfg.nz;
   if (nx < 4 || ny < 4 || nz < 4) throw std::runtime_error("grid must be at least 4 x 4 x 4");
@@ -401,6 +406,8 @@ void Encoder::setup() {
   }
   L.fields = fl;
   L.arena = (E.image.size() + 63) / 64 * 64;
+  // (before the image takes the arena's memory; run() checks the whole)
+  checkWords(L.arena + L.field_words * fl.size());
   if (withArena) {
     E.image.resize(L.arena + L.field_words * fl.size(), 0u);
   } else {  // the image holds the words below the arena and the payloads above it
@@ -1254,6 +1261,7 @@ Encoded Encoder::run() {
   stages();
   end();
   E.L.words = (E.image.size() + E.skipped + 63) / 64 * 64;
+  checkWords(E.L.words);
   E.image.resize(E.L.words - E.skipped, 0u);
   return std::move(E);
 }
