@@ -1021,12 +1021,12 @@ void Encoder::stages() {
         fb(9, "ppd"), fb(10, "ppx")});
     acoustic = acousticBytes((double)(float)sch.dts[nrk]);
     // fuse = 1: after acoustic_uv, one ac_column launch (with an open side
-    // ac_halo_open after it, and the edges' update in acoustic_uv_open; fields
-    // of 2^32 bytes, which it cannot address, keep the separate launches there)
+    // ac_halo_open after it, and the edges' update in acoustic_uv_open)
     // per substep (fpk, column solve, pp, accumulate, halo fill; prepare's
-    // terms formed in it, begin folded into the stage's first substep)
-    const bool column = cfg.fuse == 1 && nx >= 4 && ny >= 4 && nz >= 4 && (nz + 7) / 8 <= 16 &&
-                        ((!openX && !openY) || (uint64_t)(nx + 7) * (ny + 7) * (nz + 2) < (1ull << 30));
+    // terms formed in it, begin folded into the stage's first substep).  Its
+    // fields must span less than 2^32 bytes: a step has dozens of them within
+    // 2^32 words (checkWords).
+    const bool column = cfg.fuse == 1 && nx >= 4 && ny >= 4 && nz >= 4 && (nz + 7) / 8 <= 16;
     if (!column) {
       op("acoustic_prepare", full,
          {fb(2, "ppterm"), fb(3, "piadv"), fb(4, "thv"), rb(5, "rr0"), rb(6, "rf0"), rb(7, "mh"), rb(8, "mf"),
