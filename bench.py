@@ -8,8 +8,10 @@ hodograph + 2 K bubble, synthetic).  The state is resident in HBM before the
 timed region; a step is one full large step (a replay of its captured HIP
 graph).
 
-Prints one JSON line.  `roofline` is for the kernel with the largest device
-time per step, timed live with HIP events on the stream it runs on;
+Prints one JSON line.  `roofline` and `top_kernels_*` time the step's dispatches
+one by one with HIP events on the stream they run on (the timed steps run
+independent ones side by side in one launch, where a kernel's own time cannot
+be told); `roofline` is for the kernel with the largest sum per step;
 `cpu_baseline` times the oracle on this host's cores on a bounded sample.
 """
 import argparse

@@ -67,7 +67,8 @@ int te_plan_batches(uint64_t mem_words, const uint32_t* mem, int32_t nops, const
 
 /* Runs nsteps full steps eagerly with a HIP event after every op on the
  * context's stream and adds each op's device duration (ms) into op_ms
- * (te_op_count floats, cleared first).  Profiling aid: no counterpart in the
+ * (te_op_count floats, cleared first).  Every op is a launch of its own here,
+ * also where te_run runs several side by side (te_op_launch).  Profiling aid: no counterpart in the
  * reference, whose replayer only times whole steps. */
 int te_profile_ops(te_ctx* ctx, int32_t nsteps, float* op_ms);
 
@@ -180,8 +181,9 @@ typedef struct te_config {
   int32_t initial_tke;     /* init3d testcase of the t=0 TKE profile: 0 none, 3, 4, 5, 9, 11
                               (scenario.js:347-369) */
   int32_t fuse;            /* 1 (default): merged / fused launches where the step allows them
-                              (same state bits; scratch fields may differ), on periodic domains one
-                              launch per acoustic substep after acoustic_uv; 2: the same with the
+                              (same state bits; scratch fields may differ), up to 128 levels one
+                              launch per acoustic substep after acoustic_uv (and one for the halo of
+                              w, ppd and rrw where a side is open); 2: the same with the
                               acoustic substep as separate launches (the program the adjoint
                               recomputes); 0: the reference's dispatch list one for one */
   uint64_t sounding_seed;  /* perturbed soundings (ensemble members): seed of the draws below */

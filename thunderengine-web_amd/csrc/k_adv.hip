@@ -704,8 +704,9 @@ __global__ __launch_bounds__(256) void k_adv_fused(uint32_t* M, KArg a) {
 
 // Independent advections (adv_fused, adv_pdef) in one launch.  A stage's u, v,
 // w and TKE, and its scalars, read common fields and write their own: one
-// launch fills the chip once instead of draining it between them, and the
-// tiles of one place share an L2 (te_batch_part).
+// launch fills the chip once instead of draining it between them.  Each XCD
+// takes one dispatch after the other (KBatch: side by side tile by tile was
+// slower).
 // MASK: the bodies (adv_body) the launch may meet; body 0 or 8 is served by
 // 1 or 9, which take open sides too.  Blocks of 64 x Y x Z, the same for every
 // dispatch of the launch (te_autotune chooses one for all of them).

@@ -14,8 +14,8 @@ enum {
 #undef TE_ID
 };
 
-// All bodies in one kernel: none needs more than 50 registers, so the widest
-// does not cost the others waves, and a launch brings in the code of its own
+// All bodies in one kernel: 55 VGPRs in all, 8 waves per SIMD, so the widest
+// body does not cost the others waves, and a launch brings in the code of its own
 // dispatches only.  What it saves is the drain and start between them, 2 to 4
 // us each: a stage's diagnostics, tendency reset, mass fluxes and pressure
 // tendency, and the end of a step, are 3 to 5 launches of 3.5-6 us each at

@@ -320,10 +320,12 @@ TE_DEV void ac_accumulate_uv(uint32_t* M, const KArg& a, const Dims& g, uint32_t
 // in turn after the sweep, halos last): 300 cycles to eliminate a row and 150 to
 // substitute it back, 45 k cycles in a row without y images and 60 k in one
 // with them at 64 x 64 x 40, 125 k and 180 k at 192 x 192 x 80; now 120 and 60
-// per row, 26 k and 32 k, 105 k and 145 k.  us per launch, before and now:
-// 64 x 64 x 40 24.3 and 15.0, 192 x 192 x 80 69 and 51, 256 x 256 x 120 203 and
-// 164 (1 level of loads in flight for 9 to 12 levels per wave: 2 spill, and a
-// reload behind stores waits for them, 58 us at 192 x 192 x 80).
+// per row, 26 k and 32 k, 105 k and 145 k.  us per launch within a step, before
+// and now: 64 x 64 x 40 24.3 and 13.9, 192 x 192 x 80 69 and 56, 256 x 256 x 120
+// 203 and 165.  A reload of a spilled register behind stores waits for them, so 9
+// to 12 levels per wave have 1 level of loads in flight: these instances still
+// spill 3 to 12 VGPRs (open sides: 0 to 2), with 2 levels more (7 us longer a
+// launch at 192 x 192 x 80).
 // p: 0 dims, 1 acoustic, 2 u, 3 v, 4 w, 5 piadv, 6 ppten, 7 ppterm, 8 thv,
 //    9 wten, 10 pp3d, 11 ppd, 12 ppx, 13 rru, 14 rrv, 15 rrw, 16 -> save ppx,
 //    17 -> tavg, 18 rr0, 19 rf0, 20 mh, 21 mf, 22 c1, 23 c2, 30 metric,

@@ -74,7 +74,8 @@ __global__ __launch_bounds__(256) void k_turb_sfcstress(uint32_t* M, KArg a) {
 // SOURCES: tke_sources (tke_sources.wgsl:111-129) of the levels too, from their
 // epst in registers (tketen = fma(-khv, nm, -dissten) + epst; p16 khv, 17 nm,
 // 18 dissten, 19 tketen): a pass over 5 fields and a launch less (a step of
-// 32 x 24 x 16 288.4 and 286.0 us, of 192 x 192 x 80 2983 and 2974).
+// 32 x 24 x 16 288.4 and 286.0 us, of 192 x 192 x 80 2983 and 2974, for 92
+// instead of 67 VGPRs).
 template <bool SOURCES>
 __device__ __forceinline__ void tke_epst(uint32_t* M, const KArg& a) {
   TE_TID3

@@ -283,12 +283,15 @@ static const void* batch_kernel(const Op* ops, const OpWords* w, int n) {
   }
   if (family == 1) return adv_batch_kernel(bodies);
   if (family == 3) return sweep_batch_kernel((ops[0].nz + AC_WAVES - 1) / AC_WAVES);
-  // Pointwise dispatches: below about 3 M words a field the drain and start
-  // between launches cost more than finding the dispatch and its arguments
-  // costs every workgroup.  us per step in batches and one by one: 64 x 64 x 40
-  // 382 and 416, 96 x 96 x 56 585 and 620, 128 x 128 x 60 775 and 805,
-  // 160 x 160 x 40 803 and 836, 192 x 192 x 80 (3.2 M words) 2855 and 2849,
-  // 300 x 300 x 90 6083 and 6016, 256 x 256 x 120 8612 and 8415.
+  // Pointwise dispatches: on small fields the drain and start between launches
+  // cost more than finding the dispatch and its arguments costs every
+  // workgroup, on large ones less.  us per step in batches and one by one, by
+  // the field's words (M = 2^20), steps with TKE / moist without / open sides, 7
+  // species and TKE: 1.06 M 1059, 1109 / 757, 783 / 1539, 1626; 1.73 M 1631,
+  // 1663 / 1186, 1202 / 2375, 2437; 2.45 M 2267, 2278 / 1620, 1631 / 3148, 3178;
+  // 2.76 M 2514, 2507 / 1798, 1807 / 3482, 3510; 3.06 M 2779, 2763 / 1997, 1994 /
+  // 3821, 3828; 3.57 M 3540, 3510 / 2649, 2648 / 4782, 4771; 5.34 M 4988, 4877 /
+  // 3663, 3630 / 6701, 6580.  They cross at 2.6, 3.0 and 3.2 M words.
   return words <= (3u << 20) ? (const void*)&k_point_batch : nullptr;
 }
 // The launch of a batch (ops[0].batch_fn): fits is false where a member's

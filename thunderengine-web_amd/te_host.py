@@ -289,7 +289,8 @@ class _Ctx:
         self._check(lib().te_sync(self.h), "te_sync")
 
     def profile_ops(self, nsteps=1):
-        """Per-op device milliseconds summed over nsteps eager steps (HIP events)."""
+        """Per-op device milliseconds summed over nsteps eager steps (HIP events),
+        every op in a launch of its own."""
         n = int(lib().te_op_count(self.h))
         out = np.zeros(n, dtype=np.float32)
         self._check(lib().te_profile_ops(self.h, nsteps, out.ctypes.data_as(ctypes.POINTER(ctypes.c_float))),
