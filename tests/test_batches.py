@@ -298,3 +298,35 @@ def test_uploaded_flags_reach_the_plan(gpu):
                     w[slot(8): slot(8) + FIELD] = 0
             assert np.array_equal(got, want), (flags, n)
     r.close()
+
+
+@pytest.mark.gpu
+def test_uploaded_flags_reach_an_ensemble_member(gpu):
+    """w's buoyancy switched off (chain flag 64) between steps of an ensemble:
+    its next step is the oracle's of the changed program."""
+    import ctypes
+
+    import runs
+    cfg = te_host.config(nx=18, ny=12, nz=14, tke=1, initial_tke=3)
+    ens = te_host.Ensemble([cfg, te_host.config(nx=12, ny=10, nz=8)])
+    member = te_host.lib().te_ensemble_member(ens.h, 0)
+    ref = runs.OracleRun(cfg, fused=True)
+    end = runs.arena_end(ref.enc)
+    keep = runs.state_mask(ref.enc)
+    chains = {int(A[4 + 32]) for n, A in zip(ref.names, ref.args) if n == "adv_fused" and ref.M[A[4 + 32]] & 64}
+    assert chains
+    for off in (False, True):
+        if off:
+            for at in chains:
+                v = np.array([int(ref.M[at]) & ~64], np.uint32)
+                ref.M[at] = v[0]
+                assert te_host.lib().te_upload_words(member, at, v.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)),
+                                                     1) == te_host.TE_OK
+        ens.step(2)
+        ens.sync()
+        ref.step(2)
+        got, want = ens.member_words(0, 0, end), ref.M[:end].copy()
+        got[~keep] = 0
+        want[~keep] = 0
+        assert np.array_equal(got, want), (off, runs.first_difference(ref, got, want))
+    ens.close()
